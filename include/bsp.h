@@ -339,6 +339,58 @@ int bsp_attention_bwd_kv(int dtype, const void *d_o, const void *q, const void *
                          float scale, const int32_t *d_col_lut, int n_items, float *partial, int n_slots,
                          const int32_t *d_split_lut, int n_split, void *stream);
 
+/* The same chain without any sparse tensor in memory, for calls without relative position embedding and attention mask:
+ * o = softmax(q . k^T * scale + key-padding term) . v and its three gradients, rows and columns of any length.  What the
+ * backward pass needs of the softmax is one fp32 per row, lse = log2 of the row's sum of exponentials (of the logits in
+ * the log2 domain; +inf for a row without any block), from which the backward kernels compute the probabilities again.
+ * Scores and probabilities are not rounded between the steps except where they become an operand of a product.
+ *
+ * Tables (bsp_attention_tables_build makes them): a tile is 64 rows by 64 columns, each side four groups of sixteen consecutive positions
+ * anywhere in the matrix; its entry is eight ints: the positions of the four groups of the side the tile gathers, a
+ * bit 4 * row group + column group for every 16 x 16 piece of it that exists, three unused.
+ *   rows (bsp_attention_rows_fwd, bsp_attention_rows_bwd): d_lut = per line of 64 consecutive rows, in (head, line)
+ *     order, (tiles, offset of the first entry in ints from the start); then the entries (groups: of columns).  R lines.
+ *   columns (bsp_attention_cols_bwd): d_items = n_items work items of twelve ints (tiles, offset of the first entry, head,
+ *     column, slot or -1, 0, 0, 0, the positions of the column's four groups of keys), then the entries (groups: of
+ *     rows).  Work items, slots, partial and d_split as for bsp_attention_bwd_kv, positions in place of block-columns.
+ * lse, neg_delta: [Z][H] rows, lse_stride_h / row_stride_h (>= 64 R) floats apart.  rows_fwd: lse may be NULL (no backward
+ * pass to follow).  rows_bwd: writes dq and, if neg_delta is not NULL, -sum_d do . o of every row, which cols_bwd reads.
+ * fp16 / bf16, D = 64 or 128; pointers 16-byte aligned, strides multiples of 8 elements.  keys / rows: how many positions
+ * the operands have that are fetched tile by tile (k and v; q and do): their rows must lie within 4 GiB of the first. */
+typedef struct {
+  int lines, longest_line;         /* lines of tiles per head (R of the calls below), tiles of the longest one */
+  int columns, n_items;            /* columns of tiles per head, work items */
+  int n_slots, n_split;            /* slots of the parts of long columns, such columns */
+  int64_t items_offset, split_offset, total;   /* ints from the start of the tables: d_lut at 0, d_items, d_split, the end */
+} bsp_attention_tables;
+
+/* Host function: the tables of a layout in host memory ([H, R, C] bytes, nonzero = block), written back to back into
+ * h_tables (cap ints; the caller copies them to the device).  BSP_ERR_CAPACITY with info->total = the ints needed if cap is too small (32 H (R + C) + 16 nonzero blocks + 64 always is enough); BSP_ERR_UNSUPPORTED for
+ * blocks other than 16, 32, 64 and for layouts that do not divide into tiles.  Lines of blocks of 16 / 32 gather the
+ * block-columns in which any of their S = 64 / block block-rows holds a block, S a tile; a column of tiles is S
+ * block-columns (the long ones of a head together, the others as they lie) and gathers block-rows.  Columns of more than
+ * 16 tiles and twice the average are cut into parts. */
+int bsp_attention_tables_build(const uint8_t *h_layout, int H, int R, int C, int block, int32_t *h_tables, int64_t cap,
+                               bsp_attention_tables *info);
+int bsp_attention_rows_fwd(int dtype, const void *q, const void *k, const void *v, void *o, float *lse, int Z, int H, int R, int64_t keys, int D,
+                           int64_t q_stride_z, int64_t q_stride_h, int64_t ldq, int64_t k_stride_z, int64_t k_stride_h, int64_t ldk,
+                           int64_t v_stride_z, int64_t v_stride_h, int64_t ldv, int64_t o_stride_z, int64_t o_stride_h, int64_t ldo,
+                           int64_t lse_stride_h, float scale, const int32_t *d_lut, const void *kpm, int64_t kpm_stride_z, int kpm_mul,
+                           void *stream);
+int bsp_attention_rows_bwd(int dtype, const void *d_o, const void *q, const void *k, const void *v, const void *o, const float *lse,
+                           void *dq, float *neg_delta, int Z, int H, int R, int64_t keys, int D, int64_t do_stride_z, int64_t do_stride_h, int64_t lddo,
+                           int64_t q_stride_z, int64_t q_stride_h, int64_t ldq, int64_t k_stride_z, int64_t k_stride_h, int64_t ldk,
+                           int64_t v_stride_z, int64_t v_stride_h, int64_t ldv, int64_t o_stride_z, int64_t o_stride_h, int64_t ldo,
+                           int64_t dq_stride_z, int64_t dq_stride_h, int64_t lddq, int64_t row_stride_h, float scale,
+                           const int32_t *d_lut, const void *kpm, int64_t kpm_stride_z, int kpm_mul, void *stream);
+int bsp_attention_cols_bwd(int dtype, const void *d_o, const void *q, const void *k, const void *v, const float *lse, const float *neg_delta,
+                           void *dk, void *dv, int Z, int H, int C, int64_t rows, int D, int64_t do_stride_z, int64_t do_stride_h, int64_t lddo,
+                           int64_t q_stride_z, int64_t q_stride_h, int64_t ldq, int64_t k_stride_z, int64_t k_stride_h, int64_t ldk,
+                           int64_t v_stride_z, int64_t v_stride_h, int64_t ldv, int64_t dk_stride_z, int64_t dk_stride_h, int64_t lddk,
+                           int64_t dv_stride_z, int64_t dv_stride_h, int64_t lddv, int64_t row_stride_h, float scale,
+                           const int32_t *d_items, int n_items, float *partial, int n_slots, const int32_t *d_split, int n_split,
+                           const void *kpm, int64_t kpm_stride_z, int kpm_mul, void *stream);
+
 /* ---------------------------------------------------------------------------------------------------
  * Dense utility ops of the reference package.
  * ReLU: replaces the relu_y / relu_dxdsdbdres kernels and their launches (relu.py:8-91).  All tensors hold n

@@ -1,0 +1,81 @@
+"""CPU: the tables of the attention kernels without sparse tensors (bsp_attention_tables_build, host code of the library)."""
+import ctypes
+
+import pytest
+import torch
+
+from torch_blocksparse import _lib
+from torch_blocksparse.attention_core import _ColumnTable, _QuadTables
+
+
+@pytest.mark.parametrize('block,H,R,C,density,dtype', [
+    (64, 1, 1, 1, 1.0, torch.int64), (64, 5, 6, 9, 0.4, torch.int32), (64, 2, 70, 5, 0.5, torch.int64), (64, 9, 40, 40, 0.1, torch.bool),
+    (32, 2, 8, 12, 0.3, torch.int64), (32, 3, 80, 6, 0.2, torch.int32), (16, 2, 12, 20, 0.1, torch.int64), (16, 5, 160, 8, 0.3, torch.bool)])
+def test_tiles_cover_the_layout_once_in_both_views(block, H, R, C, density, dtype):
+    torch.manual_seed(R * C + block)
+    lay = torch.rand(H, R, C) < density
+    lay[:, :, 0] = True                                  # a long column
+    lay[0, R // 2] = False                               # an empty block-row in one head
+    lay[H - 1, :, C - 1] = False                         # and an empty block-column
+    S = 64 // block
+    t = _QuadTables(lay.to(dtype), block, 'cpu')
+    rows, items, split = t.rows.tolist(), t.items.tolist(), t.split.tolist() if t.n_split else []
+    full = lay.repeat_interleave(block, 1).repeat_interleave(block, 2)
+    assert t.lines == R // S and t.columns == C // S
+    got = torch.zeros(full.shape, dtype=torch.int32)
+    longest = 0
+    for h in range(H):
+        for line in range(t.lines):
+            n, first = rows[2 * (h * t.lines + line):2 * (h * t.lines + line) + 2]
+            longest = max(longest, n)
+            for e in range(n):
+                entry = rows[first + 8 * e:first + 8 * e + 8]
+                assert all(0 <= p <= C * block - 16 and p % 16 == 0 for p in entry[:4]) and entry[5:] == [0, 0, 0] and entry[4]
+                for piece in range(16):
+                    if entry[4] >> piece & 1:
+                        r, c = 64 * line + 16 * (piece // 4), entry[piece % 4]
+                        got[h, r:r + 16, c:c + 16] += 1
+    assert torch.equal(got, full.int()) and longest == t.longest
+    got.zero_()
+    slots, parts, keys_of = [], {}, {}
+    for i in range(t.n_items):
+        n, first, h, col, slot = items[12 * i:12 * i + 5]
+        keys = items[12 * i + 8:12 * i + 12]
+        assert items[12 * i + 5:12 * i + 8] == [0, 0, 0] and keys_of.setdefault((h, col), keys) == keys
+        parts.setdefault((h, col), []).append((slot, n))
+        slots += [slot] if slot >= 0 else []
+        for e in range(n):
+            entry = items[first + 8 * e:first + 8 * e + 8]
+            assert all(0 <= p <= R * block - 16 and p % 16 == 0 for p in entry[:4]) and entry[4]
+            for piece in range(16):
+                if entry[4] >> piece & 1:
+                    r, c = entry[piece // 4], keys[piece % 4]
+                    got[h, r:r + 16, c:c + 16] += 1
+    assert torch.equal(got, full.int())
+    for h in range(H):                                   # the columns of a head partition its keys
+        assert sorted(p for (hh, _), keys in keys_of.items() if hh == h for p in keys) == list(range(0, C * block, 16))
+    assert sorted(slots) == list(range(t.n_slots))
+    for i in range(t.n_split):
+        h, col, first, n = split[8 * i:8 * i + 4]
+        assert split[8 * i + 4:8 * i + 8] == keys_of[(h, col)]
+        assert sorted(s for s, _ in parts[(h, col)]) == list(range(first, first + n)) and n > 1
+        sizes = [c for _, c in parts[(h, col)]]
+        assert max(sizes) - min(sizes) <= 1
+    assert sum(len(p) > 1 for p in parts.values()) == t.n_split
+    lengths = [items[12 * i] for i in range(t.n_items)]  # four heads at a time, the longest items first
+    groups = [items[12 * i + 2] // 4 for i in range(t.n_items)]
+    assert groups == sorted(groups) and all(a >= b for a, b, ga, gb in zip(lengths, lengths[1:], groups, groups[1:]) if ga == gb)
+    ids = torch.full(lay.shape, -1, dtype=torch.int64)
+    ids[lay] = torch.arange(int(lay.sum()))
+    old = _ColumnTable(lay.long(), 'cpu', S=S, ids=ids)  # the same columns and parts as the kernels that read p take
+    assert (old.n_items, old.n_slots, old.n_split) == (t.n_items, t.n_slots, t.n_split)
+
+
+def test_errors():
+    lib, info = _lib.load(), _lib.AttentionTables()
+    lay, out = torch.ones(1, 4, 4, dtype=torch.bool), torch.empty(16, dtype=torch.int32)
+    build = lambda lay, R, block, cap: lib.bsp_attention_tables_build(_lib.ptr(lay), 1, R, 4, block, _lib.ptr(out), cap, ctypes.byref(info))
+    assert build(lay, 4, 64, 16) == _lib.ERR_CAPACITY and info.total > 16
+    assert build(lay, 3, 16, 16) == _lib.ERR_UNSUPPORTED
+    assert build(lay, 4, 128, 16) == _lib.ERR_UNSUPPORTED
+    assert build(None, 4, 64, 16) != _lib.OK

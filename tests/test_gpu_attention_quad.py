@@ -1,0 +1,130 @@
+"""GPU: the attention kernels that keep no sparse tensor (bsp_attention_rows_fwd, bsp_attention_rows_bwd,
+bsp_attention_cols_bwd behind attention_chain) at the points where they can go wrong: numbers of heads that do not divide
+by the heads a launch takes together, lines of one tile and of many, tiles with missing pieces, a running maximum that
+moves at every tile or starts at -inf, negative and zero scale, operands far apart in memory.  Tolerance: assert_close, the
+bounds every fp16 / bf16 comparison with the fp32 oracle uses."""
+import ctypes
+
+import pytest
+import torch
+
+import torch_blocksparse as tb
+from torch_blocksparse import _lib, attention_core as ac
+from oracle import dense_oracle as D
+from helpers import assert_close, guard_allocations
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+
+def _run(layout, block, q, k, v, do, **kw):
+    ops = (tb.MatMul(layout, block, 'sdd', trans_b=True), tb.Softmax(layout, block), tb.MatMul(layout, block, 'dsd'))
+    ts = [t.detach().clone().requires_grad_(True) for t in (q, k, v)]
+    before = ac.fused_calls
+    with guard_allocations('attention without sparse tensors'):
+        o = ac.attention_chain(ops[0], ops[1], ops[2], *ts, **kw)
+        o.backward(do)
+        torch.cuda.synchronize()
+    assert ac.fused_calls == before + 1
+    return [o.detach()] + [t.grad for t in ts]
+
+
+def _check(got, ref, dtype):
+    for name, g, r in zip(('o', 'dq', 'dk', 'dv'), got, ref):
+        assert not bool(torch.isnan(g).any()), name
+        assert_close(g, r, dtype, name)
+
+
+@pytest.mark.parametrize('Z,H,block,R,C,d,dtype', [
+    (1, 1, 64, 1, 1, 64, torch.float16),
+    (1, 3, 64, 2, 5, 128, torch.bfloat16),
+    (5, 1, 32, 6, 4, 64, torch.bfloat16),
+    (3, 3, 16, 8, 12, 64, torch.float16),
+    (1, 6, 16, 4, 20, 128, torch.float16),
+    (2, 2, 64, 40, 3, 64, torch.float16),       # columns of 40 tiles: parts and their sum
+])
+def test_shapes_at_the_edges(Z, H, block, R, C, d, dtype):
+    torch.manual_seed(R * C + d)
+    lay = (torch.rand(H, R, C) < 0.6).long()
+    lay[:, :, 0] = 1
+    q, do = [torch.randn(Z, H, R * block, d, device=DEV).to(dtype) for _ in range(2)]
+    k, v = [torch.randn(Z, H, C * block, d, device=DEV).to(dtype) for _ in range(2)]
+    kpm = torch.zeros(Z, C * block, device=DEV, dtype=dtype)
+    kpm[-1, 5:9] = float('-inf')
+    got = _run(lay, block, q, k, v, do, scale=d ** -0.5, key_padding_mask=kpm)
+    _check(got, D.attention(q, k, v, lay, block, d ** -0.5, key_padding_mask=kpm, attn_mask_mode='add', do=do), dtype)
+
+
+@pytest.mark.parametrize('down', [False, True])
+@pytest.mark.parametrize('block,d', [(64, 64), (16, 128)])
+def test_a_maximum_that_moves_at_every_tile(block, d, down):
+    """Logits that rise (fall) by 10 from tile to tile, 2^14 in the exponentials: every tile (none but the first) moves the
+    running maximum.  The first 64 keys are masked: the maximum starts at -inf.  The scores are exact in fp16."""
+    torch.manual_seed(d)
+    Z, H, R, C = 1, 2, 2 * 64 // block, 6 * 64 // block
+    lay = torch.ones(H, R, C, dtype=torch.int64)
+    n = torch.arange(C * block)
+    logit = 10. * ((C * block - 1 - n) // 64 if down else n // 64) + 0.5 * (n % 3)
+    q, k = torch.zeros(Z, H, R * block, d), torch.zeros(Z, H, C * block, d)
+    q[..., 0] = 8.
+    k[..., 0] = logit
+    q, k = q.half().to(DEV), k.half().to(DEV)
+    v, do = torch.randn(Z, H, C * block, d, device=DEV).half(), torch.randn(Z, H, R * block, d, device=DEV).half()
+    kpm = torch.zeros(Z, C * block, device=DEV).half()
+    kpm[:, :64] = float('-inf')
+    got = _run(lay, block, q, k, v, do, scale=0.125, key_padding_mask=kpm)
+    ref = D.attention(q, k, v, lay, block, 0.125, key_padding_mask=kpm, attn_mask_mode='add', do=do)
+    # dq sums ds k over the row with k up to 51: its error follows the size of what was summed, ds rounded to 2^-11
+    for name, g, r in zip(('o', 'dk', 'dv'), (got[0], got[2], got[3]), (ref[0], ref[2], ref[3])):
+        assert_close(g, r, torch.float16, name)
+    p = torch.softmax((q.float() @ k.float().transpose(2, 3).contiguous() * 0.125).cpu() + kpm.float().cpu()[:, None, None], -1)
+    terms = (p * ((do.float() @ v.float().transpose(2, 3).contiguous()).cpu().abs() + 40.) * 0.125) @ k.float().cpu().abs()
+    assert bool(((got[1].float().cpu() - ref[1]).abs() <= 2 ** -10 * terms + 1e-2 * ref[1].abs() + 1e-2).all())
+
+
+def test_negative_and_zero_scale():
+    torch.manual_seed(2)
+    Z, H, R, block, d = 2, 3, 5, 64, 64
+    lay = torch.tril(torch.ones(H, R, R)).long()
+    q, k, v, do = [torch.randn(Z, H, R * block, d, device=DEV).half() for _ in range(4)]
+    o, dq, dk, dv = D.attention(q, -k, v, lay, block, 0.125, attn_mask_mode='add', do=do)
+    _check(_run(lay, block, q, k, v, do, scale=-0.125), (o, dq, -dk, dv), torch.float16)
+    got = _run(lay, block, q, k, v, do, scale=0.)
+    zero = torch.zeros_like(q)
+    o, _, _, dv = D.attention(zero, k, v, lay, block, 1., attn_mask_mode='add', do=do)
+    assert not bool(got[1].any()) and not bool(got[2].any())
+    _check((got[0], got[3]), (o, dv), torch.float16)
+
+
+def test_gradients_without_those_of_the_keys():
+    torch.manual_seed(4)
+    lay = torch.tril(torch.ones(2, 4, 4)).long()
+    q, k, v, do = [torch.randn(1, 2, 256, 64, device=DEV).half() for _ in range(4)]
+    full = _run(lay, 64, q, k, v, do, scale=0.125)
+    core = ac.AttentionCore(lay, 64)
+    for need in ((True, False, False), (False, False, True), (True, False, True)):
+        ts = [t.clone().requires_grad_(n) for t, n in zip((q, k, v), need)]
+        core(*ts, scale=0.125).backward(do)
+        for t, n, f in zip(ts, need, full[1:]):
+            assert (t.grad is not None) == n and (not n or torch.equal(t.grad, f))
+
+
+def test_c_abi_argument_checks():
+    lib = _lib.load()
+    t = torch.zeros(1, 1, 64, 64, device=DEV, dtype=torch.float16)
+    o, lse = t.clone(), torch.zeros(1, 1, 64, device=DEV)
+    table = ac.AttentionCore(torch.ones(1, 1, 1, dtype=torch.int64), 64).quad(torch.device(DEV)).rows
+    null, st = ctypes.c_void_p(0), (t.stride(0), t.stride(1))
+
+    def fwd(dtype=0, q=t, D=64, ldk=64, keys=64, lse_sh=64):
+        return lib.bsp_attention_rows_fwd(dtype, _lib.ptr(q), _lib.ptr(t), _lib.ptr(t), _lib.ptr(o), _lib.ptr(lse), 1, 1, 1, keys, D,
+                                          *st, 64, *st, ldk, *st, 64, *st, 64, lse_sh, 1.0, _lib.ptr(table), null, 0, 0, _lib.stream_ptr(torch.device(DEV)))
+    assert fwd() == _lib.OK
+    assert fwd(dtype=_lib.F32) == _lib.ERR_UNSUPPORTED
+    assert fwd(D=96) == _lib.ERR_UNSUPPORTED
+    assert fwd(q=None) != _lib.OK
+    assert fwd(ldk=60) != _lib.OK
+    assert fwd(keys=0) != _lib.OK
+    assert fwd(keys=2 ** 25) != _lib.OK                 # 2^25 rows of 128 bytes: beyond the 32-bit offsets
+    assert fwd(lse_sh=32) != _lib.OK
+    torch.cuda.synchronize()

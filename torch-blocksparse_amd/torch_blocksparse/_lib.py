@@ -31,6 +31,10 @@ _c = ctypes
 _vp, _i, _i64, _f = _c.c_void_p, _c.c_int, _c.c_int64, _c.c_float
 _pi, _pi64 = _c.POINTER(_c.c_int), _c.POINTER(_c.c_int64)
 
+class AttentionTables(_c.Structure):      # bsp_attention_tables
+    _fields_ = [(n, _i) for n in ('lines', 'longest_line', 'columns', 'n_items', 'n_slots', 'n_split')] + [(n, _i64) for n in ('items_offset', 'split_offset', 'total')]
+
+
 # name -> (restype, argtypes); must list every symbol of include/bsp.h
 SIGNATURES = {
     'bsp_version': (_i, []),
@@ -67,6 +71,10 @@ SIGNATURES = {
                                 _vp, _i64, _i, _vp, _i64, _i, _vp]),
     'bsp_attention_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i] + [_i64] * 17 + [_i, _f, _vp, _i, _vp, _i64, _vp]),
     'bsp_attention_bwd_kv': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i] + [_i64] * 17 + [_i, _f, _vp, _i, _vp, _i, _vp, _i, _vp]),
+    'bsp_attention_tables_build': (_i, [_vp, _i, _i, _i, _i, _vp, _i64, _c.POINTER(AttentionTables)]),
+    'bsp_attention_rows_fwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 13 + [_f, _vp, _vp, _i64, _i, _vp]),
+    'bsp_attention_rows_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 19 + [_f, _vp, _vp, _i64, _i, _vp]),
+    'bsp_attention_cols_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 19 + [_f, _vp, _i, _vp, _i, _vp, _i, _vp, _i64, _i, _vp]),
     'bsp_layout_fixed': (_i, [_vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
     'bsp_layout_sparse_transformer': (_i, [_vp, _i, _i, _i, _i, _i, _vp]),
     'bsp_layout_bigbird': (_i, [_vp, _i, _i, _i, _i, _i, _vp, _i, _vp]),

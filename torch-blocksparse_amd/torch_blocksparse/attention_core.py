@@ -139,6 +139,26 @@ class _ColumnTable:
                                     groups[long_cols]), 1).reshape(-1).to(torch.int32).to(device)
 
 
+class _QuadTables:
+    """The tables of the kernels without sparse tensors (bsp_attention_tables_build), made on the host in one call and copied
+    to `device` in one piece: rows (forward and row kernel), items and split (column kernel), and their sizes."""
+
+    def __init__(self, layout, block, device):
+        lay = (layout != 0).cpu().contiguous()
+        H, R, C = lay.shape
+        lib = _lib.load()
+        info = _lib.AttentionTables()
+        cap = 32 * H * (R + C) + 16 * int(torch.count_nonzero(lay)) + 64
+        host = torch.empty(cap, dtype=torch.int32)
+        _lib.check(lib.bsp_attention_tables_build(_lib.ptr(lay), H, R, C, block, _lib.ptr(host), cap, ctypes.byref(info)),
+                   'bsp_attention_tables_build')
+        self.rows = host[:info.total].to(device)
+        self.items = self.rows[info.items_offset:]
+        self.split = self.rows[info.split_offset:] if info.n_split else None
+        self.lines, self.longest, self.columns = info.lines, info.longest_line, info.columns
+        self.n_items, self.n_slots, self.n_split = info.n_items, info.n_slots, info.n_split
+
+
 def _vec_ok(t):
     """16-byte vector accesses: unit inner stride, every other stride a multiple of 8 elements, aligned base."""
     return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1])
@@ -146,6 +166,11 @@ def _vec_ok(t):
 
 def _vec(t):
     return t if _vec_ok(t) else t.contiguous()
+
+
+def _near(t):
+    """... and the rows of a head within 4 GiB of its first, as the kernels without sparse tensors address them"""
+    return t if _vec_ok(t) and t.stride(2) * t.size(2) * t.element_size() < 2 ** 32 else t.contiguous()
 
 
 class AttentionCore:
@@ -162,15 +187,25 @@ class AttentionCore:
         self.dsd_tn = MatMul(layout, block, 'dsd', trans_a=True, trans_b=False)
         self.nnz = None
         self._tables = dict()
+        self._quad = dict()
 
     def blocks(self):
         if self.nnz is None:
             self.nnz = int((self.layout != 0).sum())
         return self.nnz
 
+    def quad(self, device):
+        """the tables of the kernels without sparse tensors on `device`, or None when the layout does not divide into tiles"""
+        key = str(device)
+        if key not in self._quad:
+            S = 64 // self.block
+            self._quad[key] = None if self.spdims[1] % S or self.spdims[2] % S else _QuadTables(self.layout, self.block, device)
+        return self._quad[key]
+
     def tables(self, device):
         """(table, longest row, None, rows of the table's layout, present blocks per present tile as a share,
-        tables of the column kernel) on `device`, or None when the layout does not divide into 64 x 64 tiles."""
+        tables of the column kernel) on `device`, or None when the layout does not divide into 64 x 64 tiles: what the kernels
+        that store p need"""
         key = str(device)
         if key not in self._tables:
             S = 64 // self.block
@@ -207,21 +242,132 @@ class AttentionCore:
         Z, D, b = q.size(0), q.size(3), self.block
         if tuple(q.shape) != (Z, H, R * b, D) or tuple(k.shape) != (Z, H, C * b, D) or tuple(v.shape) != (Z, H, C * b, D):
             return False
-        t = self.tables(q.device)
-        if t is None or t[1] <= 0:
+        t = self.quad(q.device)
+        if t is None or t.longest <= 0:
             return False
-        return t[1] * 64 < 32768                           # the softmax operator's bound on a row (softmax.py:225-227)
+        return t.longest * 64 < 32768                           # the softmax operator's bound on a row (softmax.py:225-227)
 
     def __call__(self, q, k, v, scale=1., rpe=None, key_padding_mask=None, attn_mask=None,
                  key_padding_mask_mode='add', attn_mask_mode='add'):
         for name, m in (('relative position embedding', rpe), ('Attention mask', attn_mask), ('Key padding mask', key_padding_mask)):
             if m is not None and m.dtype != q.dtype:      # softmax.py:348-353
                 raise ValueError('%s must be %s' % (name, q.dtype))
+        if rpe is None and attn_mask is None:
+            if key_padding_mask is not None:
+                self._check_masks(q, None, key_padding_mask, None)
+            return _attention_quad.apply(q, k, v, float(scale), key_padding_mask, key_padding_mask_mode, self, torch.is_grad_enabled())
         lut, maxlut, _, rows = self.tables(q.device)[:4]
         # p is kept for the backward pass; a forward pass that no backward pass can follow does not store it
         keep_p = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
         return _attention_core.apply(q, k, v, float(scale), rpe, key_padding_mask, attn_mask, key_padding_mask_mode,
                                      attn_mask_mode, self, lut, maxlut, keep_p, rows)
+
+
+    def _check_masks(self, q, rpe, key_padding_mask, attn_mask):
+        """the masks against the layout, exactly as the softmax operator checks them (the kernels take every address from the table)"""
+        nnz, block = self.blocks(), self.block
+        _sparse_softmax._check_shapes(torch.empty((q.size(0), nnz, block, block), device='meta'), rpe, key_padding_mask, attn_mask, self.spdims, block, nnz)
+
+
+class _attention_quad(torch.autograd.Function):
+    """The chain without per-element masks: no sparse tensor is kept for the backward pass, one float per row is (the
+    logarithm of the row's sum of exponentials), from which the backward kernels compute the softmax again."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, scale, key_padding_mask, kp_mask_mode, core, grad_enabled):
+        global fused_calls
+        H, R, C = core.spdims
+        Z, D = q.size(0), q.size(3)
+        tables = core.quad(q.device)
+        lines = tables.lines
+        keep = grad_enabled and any(ctx.needs_input_grad[:3])
+        q, k, v = _near(q), _near(k), _near(v)
+        kpm = None
+        if key_padding_mask is not None:                   # element (z, c), softmax.py:60-62, 274
+            kpm = _sparse_softmax._strided16(key_padding_mask, 'key_padding_mask')
+        ctx.kpm_args = (kpm.stride(0) if kpm is not None and kpm.size(0) > 1 else 0, int(kp_mask_mode == 'mul'))
+        o = torch.empty((Z, H, R * core.block, D), dtype=q.dtype, device=q.device)
+        lse = torch.empty((Z, H, lines * 64), dtype=torch.float32, device=q.device) if keep else None
+        rc = _lib.load().bsp_attention_rows_fwd(
+            _lib.DTYPES[q.dtype], _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse), Z, H, lines, k.size(2), D,
+            q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
+            o.stride(0), o.stride(1), o.stride(2), lines * 64, scale, _lib.ptr(tables.rows), _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
+        _lib.check(rc, 'bsp_attention_rows_fwd')
+        fused_calls += 1
+        if keep:
+            ctx.save_for_backward(q, k, v, o, lse, kpm)
+            ctx.core, ctx.scale, ctx.tables, ctx.kp_mask_mode = core, scale, tables, kp_mask_mode
+        return o
+
+    @staticmethod
+    def rows_kernel(ctx, do, delta):
+        """dq, and into delta (if given) the negative of the rows' sums sum_d do . o"""
+        q, k, v, o, lse, kpm = ctx.saved_tensors
+        Z, H, D = q.size(0), q.size(1), q.size(3)
+        dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        rc = _lib.load().bsp_attention_rows_bwd(
+            _lib.DTYPES[q.dtype], _lib.ptr(do), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse), _lib.ptr(dq), _lib.ptr(delta), Z, H,
+            ctx.tables.lines, k.size(2), D, do.stride(0), do.stride(1), do.stride(2), q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
+            v.stride(0), v.stride(1), v.stride(2), o.stride(0), o.stride(1), o.stride(2), dq.stride(0), dq.stride(1), dq.stride(2),
+            ctx.tables.lines * 64, ctx.scale, _lib.ptr(ctx.tables.rows), _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
+        _lib.check(rc, 'bsp_attention_rows_bwd')
+        return dq
+
+    @staticmethod
+    def columns_kernel(ctx, do, delta):
+        """dk and dv"""
+        q, k, v, o, lse, kpm = ctx.saved_tensors
+        Z, H, D = q.size(0), q.size(1), q.size(3)
+        ct = ctx.tables
+        dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
+        dv = torch.empty(v.shape, dtype=v.dtype, device=v.device)
+        partial = torch.empty((Z, ct.n_slots, 2, 64, D), dtype=torch.float32, device=q.device) if ct.n_slots else None
+        rc = _lib.load().bsp_attention_cols_bwd(
+            _lib.DTYPES[q.dtype], _lib.ptr(do), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(lse), _lib.ptr(delta), _lib.ptr(dk), _lib.ptr(dv), Z, H,
+            ct.columns, q.size(2), D, do.stride(0), do.stride(1), do.stride(2), q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
+            v.stride(0), v.stride(1), v.stride(2), dk.stride(0), dk.stride(1), dk.stride(2), dv.stride(0), dv.stride(1), dv.stride(2),
+            ctx.tables.lines * 64, ctx.scale, _lib.ptr(ct.items), ct.n_items, _lib.ptr(partial), ct.n_slots, _lib.ptr(ct.split), ct.n_split,
+            _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
+        _lib.check(rc, 'bsp_attention_cols_bwd')
+        return dk, dv
+
+    @staticmethod
+    def through_stored_gradient(ctx, do):
+        """dk and dv the other way (FUSED_KV = False): softmax and softmax gradient as sparse tensors, then the two dsd operators"""
+        q, k, v, o, lse, kpm = ctx.saved_tensors
+        core = ctx.core
+        lut, maxlut, _, lines = core.tables(q.device)[:4]
+        stored = _StoredSoftmax()
+        _attention_core.forward(stored, q, k, v, ctx.scale, None, kpm, None, ctx.kp_mask_mode, 'add', core, lut, maxlut, True, lines)
+        p = stored.saved_tensors[3]
+        ds = torch.empty_like(p)
+        _attention_core.rows_kernel(stored, do, ds, None)
+        return core.dsd_tn(ds, q), core.dsd_tn(p, do)      # ds^T . q and p^T . do, as the operators' backward passes do (matmul.py:598-601)
+
+    @staticmethod
+    def backward(ctx, do):
+        q = ctx.saved_tensors[0]
+        do = _near(do)
+        need_q, need_k, need_v = ctx.needs_input_grad[:3]
+        dq = dk = dv = None
+        rows = (q.size(0), q.size(1), ctx.tables.lines * 64)
+        delta = None
+        if need_k:
+            delta = torch.empty(rows, dtype=torch.float32, device=q.device)
+        elif need_v and FUSED_KV:
+            delta = torch.zeros(rows, dtype=torch.float32, device=q.device)        # (dk is computed beside dv, and dropped)
+        if need_q or need_k:
+            dq = _attention_quad.rows_kernel(ctx, do, delta if need_k else None)
+        if need_k or need_v:
+            dk, dv = _attention_quad.columns_kernel(ctx, do, delta) if FUSED_KV else _attention_quad.through_stored_gradient(ctx, do)
+        return (dq if need_q else None, dk if need_k else None, dv if need_v else None) + (None,) * 5
+
+
+class _StoredSoftmax:
+    """stands in for the autograd context of _attention_core where its kernels are called one by one"""
+
+    def save_for_backward(self, *tensors):
+        self.saved_tensors = tensors
 
 
 class _attention_core(torch.autograd.Function):
@@ -232,9 +378,8 @@ class _attention_core(torch.autograd.Function):
         H, R, C = core.spdims
         Z, D, block = q.size(0), q.size(3), core.block
         nnz = core.blocks()
-        # the masks against the layout, exactly as the softmax operator checks them (it takes every address from the table)
         if rpe is not None or key_padding_mask is not None or attn_mask is not None:
-            _sparse_softmax._check_shapes(torch.empty((Z, nnz, block, block), device='meta'), rpe, key_padding_mask, attn_mask, core.spdims, block, nnz)
+            core._check_masks(q, rpe, key_padding_mask, attn_mask)
         q, k, v = _vec(q), _vec(k), _vec(v)
         null = ctypes.c_void_p(0)
         rpe_args = (null, 0, 0, 0)

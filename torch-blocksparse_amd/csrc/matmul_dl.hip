@@ -33,8 +33,19 @@ inline bool raise_lds_limit(const void *kernel, int bytes, std::atomic<uint64_t>
   return true;
 }
 
-#define BSP_GLOBAL_PTR(p) ((const void __attribute__((address_space(1))) *)(p))
-#define BSP_LDS_PTR(p) ((void __attribute__((address_space(3))) *)(p))
+// Sixteen bytes per lane from src (a lane's own address) to LDS byte dst + 16 * lane (dst the same in all lanes).  As
+// assembly and not as the builtin: the compiler cannot tell which stage of the ring a load fills, and in front of every
+// transposing LDS read it would wait for all loads in flight (s_waitcnt vmcnt(0) once or several times per reduction
+// step), which leaves nothing of the prefetch.  The waits are the counted ones of BSP_WAIT_VM alone.  The scalar no-op
+// is the wait state between the write of m0 and its use.  Measured against the builtin, fp16, 4 x 8 products of 2048^3 at a
+// quarter of the blocks: dsd with the dense operand's reduction strided 286 -> 247 us at block 64 and 228 -> 199 at 128, sdd of
+// 2 x 4 such products with a strided operand 153-162 -> 121-133 at block 32; kernels that read both tiles along the
+// reduction are as fast as before.  dsd with the sparse operand transposed and the dense reduction contiguous comes here for the
+// same reason: 299 us in the general kernel, 270 here at block 64, 231 and 210 at 128.
+__device__ __forceinline__ void load_lds16(const void *src, const unsigned char *dst) {
+  const uint32_t at = (uint32_t)(uintptr_t)((const void __attribute__((address_space(3))) *)dst);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(at) : "memory");   // (nothing else in these kernels uses m0)
+}
 // Wait until at most n vector-memory operations of this wavefront are outstanding and all of its LDS reads have
 // returned.  It stands before the barrier of a reduction step, behind which other wavefronts start the direct-to-LDS
 // loads that overwrite the stage read last: a read still in flight then could return the new bytes.  (In these
@@ -183,10 +194,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     unsigned char *st = smem + (s % kStages) * STAGE;
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(xb + xoff[i]), BSP_LDS_PTR(st + (wave * XL + i) * 1024), 16, 0, 0);
+      load_lds16(xb + xoff[i], st + (wave * XL + i) * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(yb + yoff[i]), BSP_LDS_PTR(st + XT::BYTES + (wave * YL + i) * 1024), 16, 0, 0);
+      load_lds16(yb + yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
   };
   if (nblk > 0) {
     int pos, bid;
@@ -359,10 +370,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     unsigned char *st = smem + (e % kStages) * STAGE;
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(xb + (bid >= 0 ? xoff[i] : 0)), BSP_LDS_PTR(st + wave * XT::BYTES + i * 1024), 16, 0, 0);
+      load_lds16(xb + (bid >= 0 ? xoff[i] : 0), st + wave * XT::BYTES + i * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(yb + yoff[i]), BSP_LDS_PTR(st + G * XT::BYTES + (wave * YL + i) * 1024), 16, 0, 0);
+      load_lds16(yb + yoff[i], st + G * XT::BYTES + (wave * YL + i) * 1024);
   };
   if (ne > 0) {
     // entries s, s + 1 and s + 2 are in flight at step s (their table values in registers: the table is read one step
@@ -587,10 +598,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     unsigned char *st = smem + (s % kStages) * STAGE;
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(xb + xoff[i]), BSP_LDS_PTR(st + (wave * XL + i) * 1024), 16, 0, 0);
+      load_lds16(xb + xoff[i], st + (wave * XL + i) * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(yb + yoff[i]), BSP_LDS_PTR(st + XT::BYTES + (wave * YL + i) * 1024), 16, 0, 0);
+      load_lds16(yb + yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
   };
 #pragma unroll
   for (int s = 0; s < kStages - 1; s++) issue(s);
@@ -738,10 +749,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3))
     unsigned char *st = smem + (s % kStages) * STAGE;
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(xb + xoff[i]), BSP_LDS_PTR(st + (wave * XL + i) * 1024), 16, 0, 0);
+      load_lds16(xb + xoff[i], st + (wave * XL + i) * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      __builtin_amdgcn_global_load_lds(BSP_GLOBAL_PTR(yb + yoff[i]), BSP_LDS_PTR(st + XT::BYTES + (wave * YL + i) * 1024), 16, 0, 0);
+      load_lds16(yb + yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
   };
   if (ksteps > 0) {
 #pragma unroll
@@ -904,10 +915,6 @@ int xsd_dl(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bo
     return rc == BSP_OK ? 1 : rc;
   }
   if (block != 64 && block != 128) return 0;
-  // (sparse operand transposed and dense operand with the reduction contiguous, the dX product of a sparse linear layer:
-  // measured 0.064 ms here against 0.059 ms for the general kernel at block 128, 0.0595 against 0.0596 once the strided
-  // tiles were free of bank conflicts, equal at block 64: left where it was)
-  if (sp_trans && dn_kc) return 0;
   int rc;
   if (dtype == BSP_F16) rc = block == 128 ? launch_dl<f16, 128>(g, sp_trans, dn_kc, out_nc, st) : launch_dl<f16, 64>(g, sp_trans, dn_kc, out_nc, st);
   else rc = block == 128 ? launch_dl<bf16, 128>(g, sp_trans, dn_kc, out_nc, st) : launch_dl<bf16, 64>(g, sp_trans, dn_kc, out_nc, st);

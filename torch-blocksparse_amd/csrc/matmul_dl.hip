@@ -13,6 +13,13 @@
 //   * all eight orientations (sparse operand as stored / transposed, dense operand with the reduction contiguous or
 //     strided, result written along either index): a tile whose reduction index is strided in memory is kept as it
 //     lies and read with the transposing LDS load.
+//   * the ring is walked in rounds of three steps, so that a stage is a constant: LDS addresses are registers made before the
+//     loop plus immediates, and a load is a scalar base plus a 32-bit register.  With the stage a run-time value a step
+//     spent some 250 instructions per wavefront on addresses and bookkeeping and was bound by issuing them: fp16, 8 products
+//     of 2048^3 at a quarter of the blocks, dsd at block 32 107 -> 85 us, 64 87-90 -> 74-89, 128 91 -> 82; sdd at
+//     block 32 127 -> 105-108 (125 with both reductions contiguous); the block-16 sdd over a hidden size of 512 131 -> 116.
+//     (Measured slower: reduction steps of 64, full 128-byte lines, eight wavefronts a CU: sdd 129 -> 152; six stages and
+//     one workgroup per CU, at any launch size: dsd at block 32 25 -> 37 us for 1024^3.)
 // A standalone dense probe of this pipeline (128 x 256 x 32 tiles) reaches 0.9 PFLOP/s on an 8192 x 4096 x 4096
 // product where the register-staged general kernel reaches 0.75.
 #include "matmul_generic.h"
@@ -33,7 +40,11 @@ inline bool raise_lds_limit(const void *kernel, int bytes, std::atomic<uint64_t>
   return true;
 }
 
-// Sixteen bytes per lane from src (a lane's own address) to LDS byte dst + 16 * lane (dst the same in all lanes).  As
+constexpr int kTK = 32;          // reduction step (elements)
+constexpr int kTN = 256;         // tile of the dense free dimension
+constexpr int kStages = 3;
+
+// Sixteen bytes per lane from base (the same in all lanes) + off to LDS byte dst + 16 * lane (dst the same in all lanes).  As
 // assembly and not as the builtin: the compiler cannot tell which stage of the ring a load fills, and in front of every
 // transposing LDS read it would wait for all loads in flight (s_waitcnt vmcnt(0) once or several times per reduction
 // step), which leaves nothing of the prefetch.  The waits are the counted ones of BSP_WAIT_VM alone.  The scalar no-op
@@ -42,9 +53,17 @@ inline bool raise_lds_limit(const void *kernel, int bytes, std::atomic<uint64_t>
 // 2 x 4 such products with a strided operand 153-162 -> 121-133 at block 32; kernels that read both tiles along the
 // reduction are as fast as before.  dsd with the sparse operand transposed and the dense reduction contiguous comes here for the
 // same reason: 299 us in the general kernel, 270 here at block 64, 231 and 210 at 128.
-__device__ __forceinline__ void load_lds16(const void *src, const unsigned char *dst) {
+__device__ __forceinline__ void load_lds16(const void *base, uint32_t off, const unsigned char *dst) {
   const uint32_t at = (uint32_t)(uintptr_t)((const void __attribute__((address_space(3))) *)dst);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(at) : "memory");   // (nothing else in these kernels uses m0)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(at) : "memory");   // (nothing else in these kernels uses m0)
+}
+template <int N> struct Const { static constexpr int value = N; };
+// step(stage, s) for s = 0 .. n - 1, the stage (s modulo the ring's length) a compile-time constant: the LDS addresses of a
+// stage are then immediates of its reads
+template <int S = 0, class F> __device__ __forceinline__ void ring_round(int s, int n, F &&step) {
+  step(Const<S>{}, s + S);
+  if constexpr (S + 1 < kStages)
+    if (s + S + 1 < n) ring_round<S + 1>(s, n, step);
 }
 // Wait until at most n vector-memory operations of this wavefront are outstanding and all of its LDS reads have
 // returned.  It stands before the barrier of a reduction step, behind which other wavefronts start the direct-to-LDS
@@ -52,10 +71,6 @@ __device__ __forceinline__ void load_lds16(const void *src, const unsigned char 
 // kernels the matrix instructions that consume a step's reads come before the barrier in the compiled code, so the
 // reads have returned anyway; the explicit wait does not leave that to the instruction scheduler.)
 #define BSP_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0x0 << 8))
-
-constexpr int kTK = 32;          // reduction step (elements)
-constexpr int kTN = 256;         // tile of the dense free dimension
-constexpr int kStages = 3;
 
 // ---- LDS tile layouts (byte offsets) ------------------------------------------------------------------------
 // Reduction contiguous: [row][4 chunks of 16 bytes]; chunk c of row r sits at chunk slot c ^ ((r >> 2) & 3).  A 128-bit
@@ -83,18 +98,18 @@ template <typename T, int ROWS, bool KCONTIG> struct DlTile {
   static constexpr int BYTES = ROWS * kTK * 2;
   static constexpr int LOADS = BYTES / 1024;          // wavefront-level loads per stage
   static_assert(KCONTIG || ROWS >= 32, "a reduction row holds at least two pairs of chunks");
-  // Global element offset (relative to the tile's origin) of the chunk that lane `lane` of load `ld` fetches, as
+  // Global byte offset (relative to the tile's origin) of the chunk that lane `lane` of load `ld` fetches, as
   // (row index, reduction index): rows advance by `row_stride` elements, reduction indices by `k_stride`.
-  __device__ __forceinline__ static int64_t lane_offset(int ld, int lane, int64_t row_stride, int64_t k_stride) {
+  __device__ __forceinline__ static uint32_t lane_offset(int ld, int lane, int64_t row_stride, int64_t k_stride) {
     if constexpr (KCONTIG) {
       const int row = ld * 16 + (lane >> 2), slot = lane & 3;
       const int chunk = slot ^ kc_swz(row);      // the global chunk that belongs into this LDS slot
-      return row * row_stride + chunk * 8 * k_stride;
+      return (uint32_t)(row * row_stride + chunk * 8 * k_stride) * 2u;
     } else {
       constexpr int CPR = ROWS / 8;                    // chunks per reduction row
       const int j = ld * 64 + lane, k = j / CPR, slot = j % CPR;
       const int pair = (slot >> 1) ^ ks_swz<ROWS>(k);
-      return k * k_stride + (((pair << 1) | (slot & 1)) * 8) * row_stride;
+      return (uint32_t)(k * k_stride + (((pair << 1) | (slot & 1)) * 8) * row_stride) * 2u;
     }
   }
   // MFMA operand (32 x 16 slice): rows row0 .. row0 + 31 of the tile, reduction indices 16 * kk ..; lane l supplies row
@@ -113,6 +128,28 @@ template <typename T, int ROWS, bool KCONTIG> struct DlTile {
       s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       return __builtin_bit_cast(frag_t, v);
     }
+  }
+};
+
+// N consecutive ints per entry of a table, read by the whole wavefront: lane l holds entry 64 w + l of the window w in use, and
+// an entry of the window is N readlanes.  A reduction step that reads its entry from memory (scalar loads share their
+// counter with the LDS reads, and return in any order) waits for that read before its first matrix instruction.
+template <int N> struct TableWindow {
+  const int32_t *first;
+  int entries, at;                                    // entries of the table; first entry of the window, -1: none yet
+  int v[N];
+  __device__ __forceinline__ TableWindow(const int32_t *first_, int entries_) : first(first_), entries(entries_), at(-1) {}
+  __device__ __forceinline__ void get(int e, int lane, int (&out)[N]) {   // e (the same in all lanes) below `entries`
+    if ((e & ~63) != at) {
+      at = e & ~63;
+      const int mine = at + lane < entries ? at + lane : entries - 1;
+#pragma unroll
+      for (int i = 0; i < N; i++) v[i] = first[(int64_t)N * mine + i];
+#pragma unroll
+      for (int i = 0; i < N; i++) asm volatile("" : "+v"(v[i]));          // (wait for them here, not at every use)
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) out[i] = __builtin_amdgcn_readlane(v[i], e & 63);
   }
 };
 
@@ -142,17 +179,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   // a zero-length segment that follows a real one of the same line must not touch the output; one that stands alone
   // is an empty line and zero-fills its tile (as in k_xsd)
   if (nblk == 0 && seg > 0 && hd[-6 + 2] == column && hd[-6 + 3] == depth) return;
-  const table_ptr plan = as_table(g.plan) + 2 * (int64_t)((offset - 6 * g.width) / g.div2);
+  TableWindow<2> plan(g.plan + 2 * (int64_t)((offset - 6 * g.width) / g.div2), nblk);
   const int n0 = nt * kTN, NF = g.NF;
   const int64_t ldd = g.ldd, ldo = g.ldo;
   const T *sp = reinterpret_cast<const T *>(g.sp) + z * g.sp_sz;
-  const T *dn = reinterpret_cast<const T *>(g.dn) + z * g.dn_sz + depth * g.dn_sh;
+  const T *dn = reinterpret_cast<const T *>(g.dn) + z * g.dn_sz + depth * g.dn_sh + (DN_KC ? n0 * ldd : n0);
   T *oz = reinterpret_cast<T *>(g.out) + z * g.out_sz + depth * g.out_sh;
 
   // Per-lane part of every load address, computed once.  Sparse block element (m, k): stored [m][k] or, transposed,
   // [k][m], rows of BLOCK elements.  Dense element (n, k): [n][k] (reduction contiguous) or [k][n], rows of ldd; dense
   // rows past the free dimension read row NF - 1 instead (their results are not stored).
-  int64_t xoff[XL], yoff[YL];
+  uint32_t xoff[XL], yoff[YL];
 #pragma unroll
   for (int i = 0; i < XL; i++)
     xoff[i] = SP_TRANS ? XT::lane_offset(wave * XL + i, lane, 1, BLOCK) : XT::lane_offset(wave * XL + i, lane, BLOCK, 1);
@@ -160,14 +197,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   for (int i = 0; i < YL; i++) {
     if constexpr (DN_KC) {
       const int ld = wave * YL + i, row = ld * 16 + (lane >> 2), chunk = (lane & 3) ^ kc_swz(row);
-      const int n = n0 + row < NF ? n0 + row : NF - 1;
-      yoff[i] = (int64_t)n * ldd + chunk * 8;
+      const int n = n0 + row < NF ? row : NF - 1 - n0;
+      yoff[i] = (uint32_t)(n * ldd + chunk * 8) * 2u;
     } else {
       constexpr int CPR = kTN / 8;
       const int j = (wave * YL + i) * 64 + lane, k = j / CPR, slot = j % CPR;
       const int chunk = (((slot >> 1) ^ ks_swz<kTN>(k)) << 1) | (slot & 1);
-      const int n = n0 + chunk * 8 < NF ? n0 + chunk * 8 : (NF - 8 > 0 ? NF - 8 : 0);   // whole chunks: NF is a multiple of 8
-      yoff[i] = (int64_t)k * ldd + n;
+      const int n = n0 + chunk * 8 < NF ? chunk * 8 : NF - 8 - n0;   // whole chunks: NF is a multiple of 8
+      yoff[i] = (uint32_t)(k * ldd + n) * 2u;
     }
   }
   typename M::acc_t acc[RM][RN];
@@ -179,35 +216,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int v = 0; v < M::NACC; v++) acc[i][j][v] = 0.f;
 
   const int ksteps = nblk * SPB;
-  // table values of a step: (position of its block in the dense operand, storage index of the block).  Steps past the
-  // end repeat the last one: every stage issues the same number of loads, so the wait in front of a step counts
-  // exactly the loads issued after it.
-  auto lookup = [&](int s, int &pos, int &bid) {
-    const int b = (s < ksteps ? s : ksteps - 1) / SPB;
-    pos = plan[2 * b];
-    bid = plan[2 * b + 1];
-  };
-  auto issue = [&](int s, int pos, int bid) {
-    const int kin = ((s < ksteps ? s : ksteps - 1) % SPB) * kTK;
-    const T *xb = sp + (int64_t)bid * (BLOCK * BLOCK) + (SP_TRANS ? kin * BLOCK : kin);
-    const T *yb = dn + (DN_KC ? (int64_t)pos + kin : ((int64_t)pos + kin) * ldd);
-    unsigned char *st = smem + (s % kStages) * STAGE;
+  // loads of step s into stage st
+  auto issue = [&](int s, unsigned char *st) {
+    int e[2];                                          // position of the step's block in the dense operand, storage index of the block
+    plan.get(s / SPB, lane, e);
+    const int kin = (s % SPB) * kTK;
+    const T *xb = sp + (int64_t)e[1] * (BLOCK * BLOCK) + (SP_TRANS ? kin * BLOCK : kin);
+    const T *yb = dn + (DN_KC ? (int64_t)e[0] + kin : ((int64_t)e[0] + kin) * ldd);
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      load_lds16(xb + xoff[i], st + (wave * XL + i) * 1024);
+      load_lds16(xb, xoff[i], st + (wave * XL + i) * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      load_lds16(yb + yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
+      load_lds16(yb, yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
   };
   if (nblk > 0) {
-    int pos, bid;
-#pragma unroll
-    for (int s = 0; s < kStages - 1; s++) {
-      lookup(s, pos, bid);
-      issue(s, pos, bid);
-    }
-    lookup(kStages - 1, pos, bid);                     // the table runs one step ahead of the loads that use it: its
-    for (int s = 0; s < ksteps; s++) {                 // (scalar) latency is not between the barrier and the loads
+    static_assert(kStages == 3 && SPB >= 2, "the first two steps exist");
+    issue(0, smem);
+    issue(1, smem + STAGE);
+    auto step = [&](auto stage, int s) {
+      constexpr int S = decltype(stage)::value;
       // this wavefront's loads of step s have landed: all but those of the one step issued after them, or, at the
       // last step, all (no load is issued for steps past the end)
       if (s + 1 < ksteps) BSP_WAIT_VM(L * (kStages - 2));
@@ -215,9 +243,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       asm volatile("" ::: "memory");                   // (the compiler must not move LDS accesses across the barrier)
       __builtin_amdgcn_s_barrier();                    // everybody's have, and everybody is done reading step s - 1
       asm volatile("" ::: "memory");
-      if (s + kStages - 1 < ksteps) issue(s + kStages - 1, pos, bid);   // into the stage that step s - 1 used
-      lookup(s + kStages, pos, bid);
-      const unsigned char *st = smem + (s % kStages) * STAGE;
+      if (s + 2 < ksteps) issue(s + 2, smem + (S + 2) % kStages * STAGE);   // into the stage that step s - 1 used
+      const unsigned char *st = smem + S * STAGE;
       // operands of the second half of the step are fetched from LDS before the matrix instructions of the first
       frag_t xf[kTK / 16][RM], yf[kTK / 16][RN];
 #pragma unroll
@@ -236,7 +263,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             if constexpr (OUT_NC) acc[i][j] = M::run(yf[kk][j], xf[kk][i], acc[i][j]);   // 4 consecutive values run along n
             else acc[i][j] = M::run(xf[kk][i], yf[kk][j], acc[i][j]);                    // ... along m
           }
-    }
+    };
+    for (int s = 0; s < ksteps; s += kStages) ring_round(s, ksteps, step);
     BSP_WAIT_VM(0);                                    // (nothing is in flight any more unless the segment had a single step)
   }
   asm volatile("" ::: "memory");
@@ -306,31 +334,31 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int nt = (int)((w % per_z) / g.n_pgroups);
   const table_ptr hd = as_table(g.gplan) + 4 * ((w % per_z) % g.n_pgroups);
   const int e0 = hd[0], ne = hd[1], depth = hd[2], code = hd[3];
-  const table_ptr ent = as_table(g.gplan) + 4 * (int64_t)g.n_pgroups + (int64_t)(G + 1) * e0;
+  const int32_t *entries = g.gplan + 4 * (int64_t)g.n_pgroups + (int64_t)(G + 1) * e0;
   const bool chain = code < 0;
   const int line0 = chain ? -(code + 1) : (code & 0xffffff) * G;
   const int absent = chain ? 0xe : ((code >> 24) & 0xf);            // members that are not this group's to compute
   const int n0 = nt * kTN, NF = g.NF;
   const int64_t ldd = g.ldd, ldo = g.ldo;
   const T *sp = reinterpret_cast<const T *>(g.sp) + z * g.sp_sz;
-  const T *dn = reinterpret_cast<const T *>(g.dn) + z * g.dn_sz + depth * g.dn_sh;
+  const T *dn = reinterpret_cast<const T *>(g.dn) + z * g.dn_sz + depth * g.dn_sh + (DN_KC ? n0 * ldd : n0);
   T *oz = reinterpret_cast<T *>(g.out) + z * g.out_sz + depth * g.out_sh;
 
-  int64_t xoff[XL], yoff[YL];
+  uint32_t xoff[XL], yoff[YL];
 #pragma unroll
   for (int i = 0; i < XL; i++) xoff[i] = SP_TRANS ? XT::lane_offset(i, lane, 1, B) : XT::lane_offset(i, lane, B, 1);
 #pragma unroll
   for (int i = 0; i < YL; i++) {
     if constexpr (DN_KC) {
       const int ld = wave * YL + i, row = ld * 16 + (lane >> 2), chunk = (lane & 3) ^ kc_swz(row);
-      const int n = n0 + row < NF ? n0 + row : NF - 1;
-      yoff[i] = (int64_t)n * ldd + chunk * 8;
+      const int n = n0 + row < NF ? row : NF - 1 - n0;
+      yoff[i] = (uint32_t)(n * ldd + chunk * 8) * 2u;
     } else {
       constexpr int CPR = kTN / 8;
       const int j = (wave * YL + i) * 64 + lane, k = j / CPR, slot = j % CPR;
       const int chunk = (((slot >> 1) ^ ks_swz<kTN>(k)) << 1) | (slot & 1);
-      const int n = n0 + chunk * 8 < NF ? n0 + chunk * 8 : (NF - 8 > 0 ? NF - 8 : 0);
-      yoff[i] = (int64_t)k * ldd + n;
+      const int n = n0 + chunk * 8 < NF ? chunk * 8 : NF - 8 - n0;   // whole chunks: NF is a multiple of 8
+      yoff[i] = (uint32_t)(k * ldd + n) * 2u;
     }
   }
   typename M::acc_t acc[G][RN];
@@ -341,72 +369,74 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int v = 0; v < M::NACC; v++) acc[m][j][v] = 0.f;
 
-  // an entry of the plan: (position of the reduction block, block id of each member or -1); entries past the end repeat
-  // the last one with every member absent
-  // (the ids are a vector, not an array: an array member that is copied around makes the compiler keep the entries in
-  // scratch memory, and every access to scratch is a vector-memory operation that the loop would wait for)
-  typedef int ids_t __attribute__((ext_vector_type(4)));
-  struct Entry { int pos; ids_t id; };
-  auto lookup = [&](int e) {
-    const table_ptr en = ent + (G + 1) * (e < ne ? e : ne - 1);
-    Entry r;
-    r.pos = en[0];
-    const bool live = e < ne;
+  // The entries of the plan (position of the reduction block, block id of each member or -1) in windows of 64, lane l holding
+  // entry l of the window: its position, this wavefront's member's block (-1: none), and a bit per member that has a block.
+  // A step reads its own with readlanes.  (Read from memory step by step, with scalar loads, which share their counter with
+  // the LDS reads and return in any order, an entry was waited for before the step's first matrix instruction.)
+  int window = -1, w_pos = 0, w_bid = 0, w_has = 0;
+  auto issue = [&](int e, unsigned char *st) -> unsigned {
+    if ((e & ~63) != window) {
+      window = e & ~63;
+      const int32_t *mine = entries + (int64_t)(G + 1) * (window + lane < ne ? window + lane : ne - 1);
+      w_pos = mine[0];
+      w_has = 0;
 #pragma unroll
-    for (int m = 0; m < G; m++) {
-      const int id = en[1 + m];                        // read unconditionally: one wait for the whole entry
-      r.id[m] = (live && !((absent >> m) & 1)) ? id : -1;
+      for (int m = 0; m < G; m++) {
+        const int id = (absent >> m) & 1 ? -1 : mine[1 + m];
+        w_has |= id >= 0 ? 1 << m : 0;
+        w_bid = wave == m ? id : w_bid;
+      }
+      asm volatile("" : "+v"(w_pos), "+v"(w_bid), "+v"(w_has));   // (wait for them here, not at every use)
     }
-    return r;
-  };
-  auto issue = [&](int e, const Entry &en) {
-    int bid = en.id[0];
-#pragma unroll
-    for (int m = 1; m < G; m++) bid = wave == m ? en.id[m] : bid;
+    const int pos = __builtin_amdgcn_readlane(w_pos, e & 63), bid = __builtin_amdgcn_readlane(w_bid, e & 63);
     // an absent member still issues its loads (the count per stage is fixed), but all lanes fetch one and the same
     // chunk: a single cache line instead of sixteen
     const T *xb = sp + (int64_t)(bid > 0 ? bid : 0) * (B * B);
-    const T *yb = dn + (DN_KC ? (int64_t)en.pos * B : (int64_t)en.pos * B * ldd);
-    unsigned char *st = smem + (e % kStages) * STAGE;
+    const T *yb = dn + (DN_KC ? (int64_t)pos * B : (int64_t)pos * B * ldd);
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      load_lds16(xb + (bid >= 0 ? xoff[i] : 0), st + wave * XT::BYTES + i * 1024);
+      load_lds16(xb, bid >= 0 ? xoff[i] : 0u, st + wave * XT::BYTES + i * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      load_lds16(yb + yoff[i], st + G * XT::BYTES + (wave * YL + i) * 1024);
+      load_lds16(yb, yoff[i], st + G * XT::BYTES + (wave * YL + i) * 1024);
+    return __builtin_amdgcn_readlane(w_has, e & 63);
   };
   if (ne > 0) {
-    // entries s, s + 1 and s + 2 are in flight at step s (their table values in registers: the table is read one step
-    // before the loads that need it are issued)
-    Entry cur = lookup(0), nx1 = lookup(1), nx2 = lookup(2);
-    issue(0, cur);
-    issue(1, nx1);
-    for (int s = 0; s < ne; s++) {
-      BSP_WAIT_VM(L * (kStages - 2));
+    unsigned cur = issue(0, smem), next = ne > 1 ? issue(1, smem + STAGE) : 0;   // members with a block in entries s, s + 1
+    auto step = [&](auto stage, int s) {
+      constexpr int S = decltype(stage)::value;
+      if (s + 1 < ne) BSP_WAIT_VM(L * (kStages - 2));
+      else BSP_WAIT_VM(0);
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      issue(s + 2, nx2);
-      const Entry nx3 = lookup(s + 3);
-      const unsigned char *st = smem + (s % kStages) * STAGE;
+      const unsigned here = cur;
+      cur = next;
+      if (s + 2 < ne) next = issue(s + 2, smem + (S + 2) % kStages * STAGE);
+      const unsigned char *st = smem + S * STAGE;
+      // all operands of the step first, then its products: the latency of the LDS is waited for once and not per member
+      frag_t xf[G][kTK / 16] = {}, yf[kTK / 16][RN];
 #pragma unroll
-      for (int kk = 0; kk < kTK / 16; kk++) {
-        frag_t yf[RN];
+      for (int kk = 0; kk < kTK / 16; kk++)
 #pragma unroll
-        for (int j = 0; j < RN; j++) yf[j] = YT::frag(st + G * XT::BYTES, (wave * RN + j) * 32, kk, lane);
+        for (int j = 0; j < RN; j++) yf[kk][j] = YT::frag(st + G * XT::BYTES, (wave * RN + j) * 32, kk, lane);
 #pragma unroll
-        for (int m = 0; m < G; m++)
-          if (cur.id[m] >= 0) {
-            const frag_t xf = XT::frag(st + m * XT::BYTES, 0, kk, lane);
+      for (int m = 0; m < G; m++)
+        if ((here >> m) & 1)
+#pragma unroll
+          for (int kk = 0; kk < kTK / 16; kk++) xf[m][kk] = XT::frag(st + m * XT::BYTES, 0, kk, lane);
+#pragma unroll
+      for (int m = 0; m < G; m++)
+        if ((here >> m) & 1)
+#pragma unroll
+          for (int kk = 0; kk < kTK / 16; kk++)
 #pragma unroll
             for (int j = 0; j < RN; j++) {
-              if constexpr (OUT_NC) acc[m][j] = M::run(yf[j], xf, acc[m][j]);
-              else acc[m][j] = M::run(xf, yf[j], acc[m][j]);
+              if constexpr (OUT_NC) acc[m][j] = M::run(yf[kk][j], xf[m][kk], acc[m][j]);
+              else acc[m][j] = M::run(xf[m][kk], yf[kk][j], acc[m][j]);
             }
-          }
-      }
-      cur = nx1; nx1 = nx2; nx2 = nx3;
-    }
+    };
+    for (int s = 0; s < ne; s += kStages) ring_round(s, ne, step);
     BSP_WAIT_VM(0);
   }
   asm volatile("" ::: "memory");
@@ -524,25 +554,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int line0 = (code & 0xffffff) * G;
   const int rows_a = g.lines * B;                     // rows of op(A) per head
   const int64_t lda = g.lda, ldb = g.ldb;
-  const T *pa = reinterpret_cast<const T *>(g.a) + z * g.a_sz + h * g.a_sh;
+  const T *pa = reinterpret_cast<const T *>(g.a) + z * g.a_sz + h * g.a_sh + (int64_t)line0 * B * (A_KC ? lda : 1);
   const T *pb = reinterpret_cast<const T *>(g.b) + z * g.b_sz + h * g.b_sh;
 
   // Loop-invariant part of every load address.  A: rows line0 * 32 .. + 127 (rows past the end of the matrix read its
   // last rows; their blocks do not exist).  B: row n of the tile is row n % 32 of block-column pos[n / 32].
-  int64_t xoff[XL], yoff[YL];
+  uint32_t xoff[XL], yoff[YL];
 #pragma unroll
   for (int i = 0; i < XL; i++) {
     const int ld = wave * XL + i;
     if constexpr (A_KC) {
       const int row = ld * 16 + (lane >> 2), chunk16 = (lane & 3) ^ kc_swz(row);
-      const int r = line0 * B + row < rows_a ? line0 * B + row : rows_a - 1;
-      xoff[i] = (int64_t)r * lda + chunk16 * 8;
+      const int r = line0 * B + row < rows_a ? row : rows_a - 1 - line0 * B;
+      xoff[i] = (uint32_t)(r * lda + chunk16 * 8) * 2u;
     } else {
       constexpr int CPR = TM / 8;
       const int j = ld * 64 + lane, k = j / CPR, slot = j % CPR;
       const int c = (((slot >> 1) ^ ks_swz<TM>(k)) << 1) | (slot & 1);
-      const int r = line0 * B + c * 8 < rows_a ? line0 * B + c * 8 : rows_a - 8;
-      xoff[i] = (int64_t)k * lda + r;
+      const int r = line0 * B + c * 8 < rows_a ? c * 8 : rows_a - 8 - line0 * B;
+      xoff[i] = (uint32_t)(k * lda + r) * 2u;
     }
   }
 #pragma unroll
@@ -552,14 +582,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       const int row = ld * 16 + (lane >> 2), chunk16 = (lane & 3) ^ kc_swz(row);
       const int jj = row / CB;
       const int pos = as_table(g.gplan)[4 * (int64_t)g.n_pgroups + (int64_t)ENT * (e0 + chunk * J + (jj < left ? jj : left - 1))];
-      yoff[i] = ((int64_t)pos * CB + (row % CB)) * ldb + chunk16 * 8;
+      yoff[i] = (uint32_t)(((int64_t)pos * CB + (row % CB)) * ldb + chunk16 * 8) * 2u;
     } else {
       constexpr int CPR = TN / 8;
       const int j = ld * 64 + lane, k = j / CPR, slot = j % CPR;
       const int c = (((slot >> 1) ^ ks_swz<TN>(k)) << 1) | (slot & 1);
       const int jj = c / (CB / 8);                    // CB / 8 chunks of 8 columns per block-column
       const int pos = as_table(g.gplan)[4 * (int64_t)g.n_pgroups + (int64_t)ENT * (e0 + chunk * J + (jj < left ? jj : left - 1))];
-      yoff[i] = (int64_t)k * ldb + (int64_t)pos * CB + (c % (CB / 8)) * 8;
+      yoff[i] = (uint32_t)(k * ldb + (int64_t)pos * CB + (c % (CB / 8)) * 8) * 2u;
     }
   }
   typename M::acc_t acc[RM][RN];
@@ -591,27 +621,29 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
       }
   }
   const int ksteps = g.K / kTK;
-  auto issue = [&](int s) {
-    const int64_t k0 = (int64_t)(s < ksteps ? s : ksteps - 1) * kTK;
+  auto issue = [&](int s, unsigned char *st) {
+    const int64_t k0 = (int64_t)s * kTK;
     const T *xb = pa + (A_KC ? k0 : k0 * lda);
     const T *yb = pb + (B_KC ? k0 : k0 * ldb);
-    unsigned char *st = smem + (s % kStages) * STAGE;
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      load_lds16(xb + xoff[i], st + (wave * XL + i) * 1024);
+      load_lds16(xb, xoff[i], st + (wave * XL + i) * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      load_lds16(yb + yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
+      load_lds16(yb, yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
   };
-#pragma unroll
-  for (int s = 0; s < kStages - 1; s++) issue(s);
-  for (int s = 0; s < ksteps; s++) {
-    BSP_WAIT_VM(L * (kStages - 2));
+  static_assert(kStages == 3, "two steps ahead");
+  issue(0, smem);
+  if (ksteps > 1) issue(1, smem + STAGE);
+  auto step = [&](auto stage, int s) {
+    constexpr int S = decltype(stage)::value;
+    if (s + 1 < ksteps) BSP_WAIT_VM(L * (kStages - 2));
+    else BSP_WAIT_VM(0);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    issue(s + kStages - 1);
-    const unsigned char *st = smem + (s % kStages) * STAGE;
+    if (s + 2 < ksteps) issue(s + 2, smem + (S + 2) % kStages * STAGE);
+    const unsigned char *st = smem + S * STAGE;
 #pragma unroll
     for (int kk = 0; kk < kTK / 16; kk++) {
       frag_t xf[RM] = {}, yf[RN] = {};
@@ -628,7 +660,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int j = 0; j < RN; j++)
           if ((present >> (i * RN + j)) & 1u) acc[i][j] = M::run(yf[j], xf[i], acc[i][j]);   // 4 consecutive values run along the block's columns
     }
-  }
+  };
+  for (int s = 0; s < ksteps; s += kStages) ring_round(s, ksteps, step);
   BSP_WAIT_VM(0);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
@@ -730,7 +763,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3))
   // (a part past the end of the reduction has nothing to add: it leaves a zero block, so that the sum reads no garbage)
   const T *pa = reinterpret_cast<const T *>(g.a) + z * g.a_sz + h * g.a_sh + (A_KC ? (int64_t)bi * BL * lda : (int64_t)bi * BL);
   const T *pb = reinterpret_cast<const T *>(g.b) + z * g.b_sz + h * g.b_sh + (B_KC ? (int64_t)bj * BL * ldb : (int64_t)bj * BL);
-  int64_t xoff[XL], yoff[YL];
+  uint32_t xoff[XL], yoff[YL];
 #pragma unroll
   for (int i = 0; i < XL; i++) xoff[i] = A_KC ? XT::lane_offset(wave * XL + i, lane, lda, 1) : XT::lane_offset(wave * XL + i, lane, 1, lda);
 #pragma unroll
@@ -742,28 +775,29 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3))
     for (int j = 0; j < RN; j++)
 #pragma unroll
       for (int v = 0; v < M::NACC; v++) acc[i][j][v] = 0.f;
-  auto issue = [&](int s) {
-    const int64_t k0 = (int64_t)(s0 + (s < ksteps ? s : ksteps - 1)) * kTK;
+  auto issue = [&](int s, unsigned char *st) {
+    const int64_t k0 = (int64_t)(s0 + s) * kTK;
     const T *xb = pa + (A_KC ? k0 : k0 * lda);
     const T *yb = pb + (B_KC ? k0 : k0 * ldb);
-    unsigned char *st = smem + (s % kStages) * STAGE;
 #pragma unroll
     for (int i = 0; i < XL; i++)
-      load_lds16(xb + xoff[i], st + (wave * XL + i) * 1024);
+      load_lds16(xb, xoff[i], st + (wave * XL + i) * 1024);
 #pragma unroll
     for (int i = 0; i < YL; i++)
-      load_lds16(yb + yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
+      load_lds16(yb, yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
   };
   if (ksteps > 0) {
-#pragma unroll
-    for (int s = 0; s < kStages - 1; s++) issue(s);
-    for (int s = 0; s < ksteps; s++) {
-      BSP_WAIT_VM(L * (kStages - 2));
+    issue(0, smem);
+    if (ksteps > 1) issue(1, smem + STAGE);
+    auto step = [&](auto stage, int s) {
+      constexpr int S = decltype(stage)::value;
+      if (s + 1 < ksteps) BSP_WAIT_VM(L * (kStages - 2));
+      else BSP_WAIT_VM(0);
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      issue(s + kStages - 1);                          // (past the end: the last step again, a fixed number of loads per step)
-      const unsigned char *st = smem + (s % kStages) * STAGE;
+      if (s + 2 < ksteps) issue(s + 2, smem + (S + 2) % kStages * STAGE);
+      const unsigned char *st = smem + S * STAGE;
       frag_t xf[kTK / 16][RM], yf[kTK / 16][RN];
 #pragma unroll
       for (int kk = 0; kk < kTK / 16; kk++) {
@@ -778,7 +812,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3))
         for (int i = 0; i < RM; i++)
 #pragma unroll
           for (int j = 0; j < RN; j++) acc[i][j] = M::run(yf[kk][j], xf[kk][i], acc[i][j]);   // 4 consecutive values run along the block's columns
-    }
+    };
+    for (int s = 0; s < ksteps; s += kStages) ring_round(s, ksteps, step);
     BSP_WAIT_VM(0);
   }
   asm volatile("" ::: "memory");
@@ -902,19 +937,29 @@ template <typename T, int BLOCK> int launch_dl(const XsdArgs &g0, bool sp_trans,
 
 }  // namespace
 
+// The kernels of this file keep the per-lane part of a load's address in 32 bits of bytes from the operand's tile (or, for the
+// gathered operand of sdd_dl, from its first row).
+static bool near_rows(int64_t rows, int64_t ld) { return ld >= 0 && ld < ((int64_t)1 << 31) / rows; }
+
 // 1 = launched, 0 = not applicable (the caller takes another kernel), < 0 = error
 int xsd_dl(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
-  if (dtype == BSP_F32 || g.NF < 256) return 0;
+  if (dtype == BSP_F32 || g.NF < 256 || !near_rows(kTN, g.ldd)) return 0;
   if (block == 32) {   // needs the group plan (whole blocks, no split chains)
-    // Measured on 2048^3 products at a quarter of the blocks (8 x 16 of them): with the dense operand's reduction
-    // contiguous 1.60-1.83 ms against 1.89-2.05 for the general kernel; with it strided the general kernel's 1.47-1.58 ms
-    // stand against 1.70-1.73 (also with the conflict-free layout of the strided tiles), so those stay where they were.
-    if (!dn_kc) return 0;
+    // Groups of four lines times tiles of 256 columns leave most of the chip idle in a small launch, where the general
+    // kernel's smaller workgroups win.  Single dsd products at a quarter of the blocks, this kernel / the general one, dense
+    // reduction strided (contiguous): 1024^3, 32 workgroups here, 20.8 / 14.9 us (19.8 / 16.0); 4096 x 2048 x 4096, 256 of
+    // them, 70.5 / 60.8 (68.1 / 67.0); 8 products of 2048^3, 1024 of them, 87 / 111 (91 against 108 of this kernel with its
+    // table read and its addresses computed in every step).  (The host chooses the plan by the same rule: _plan_for in matmul.py.)
+    if ((g.width + 3) / 4 * (int64_t)((g.NF + kTN - 1) / kTN) * g.Z < 384) return 0;
     if (!g.gplan || g.n_pgroups <= 0 || g.lines <= 0 || g.n_split != 0) return 0;
     const int rc = dtype == BSP_F16 ? launch_rg_dl<f16>(g, sp_trans, dn_kc, out_nc, st) : launch_rg_dl<bf16>(g, sp_trans, dn_kc, out_nc, st);
     return rc == BSP_OK ? 1 : rc;
   }
   if (block != 64 && block != 128) return 0;
+  // ... the same at blocks of 64 with the dense reduction contiguous, whose tiles the general kernel reads well: 1024^3 (64
+  // workgroups here) 13.7 / 12.2 us, 4096 x 2048 x 4096 (512) 56.7 / 55.5, 8 products of 2048^3 (2048) 89 / 104; with it
+  // strided 13.9 / 15.0, 52.4 / 75.1 and 76 / 110
+  if (block == 64 && dn_kc && (int64_t)g.width * ((g.NF + kTN - 1) / kTN) * g.Z <= 512) return 0;
   int rc;
   if (dtype == BSP_F16) rc = block == 128 ? launch_dl<f16, 128>(g, sp_trans, dn_kc, out_nc, st) : launch_dl<f16, 64>(g, sp_trans, dn_kc, out_nc, st);
   else rc = block == 128 ? launch_dl<bf16, 128>(g, sp_trans, dn_kc, out_nc, st) : launch_dl<bf16, 64>(g, sp_trans, dn_kc, out_nc, st);
@@ -924,7 +969,7 @@ int xsd_dl(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bo
 // sdd at blocks of 128 over a reduction cut into `parts` parts (pack-1 table rows; ws: parts fp32 blocks per table row and
 // batch, may be null when parts == 1): BSP_OK = launched, BSP_ERR_UNSUPPORTED = not this kernel's case
 int sdd128_splitk(int dtype, const SddArgs &g, int parts, float *ws, bool a_kc, bool b_kc, hipStream_t st) {
-  if (dtype == BSP_F32 || parts < 1 || g.K % kTK || (parts > 1 && !ws)) return BSP_ERR_UNSUPPORTED;
+  if (dtype == BSP_F32 || parts < 1 || g.K % kTK || (parts > 1 && !ws) || !near_rows(128, g.lda) || !near_rows(128, g.ldb)) return BSP_ERR_UNSUPPORTED;
   const int steps = g.K / kTK;
   SplitK sk;
   sk.parts = parts; sk.steps_per_part = (steps + parts - 1) / parts; sk.ws = ws;
@@ -936,7 +981,7 @@ int sdd128_splitk(int dtype, const SddArgs &g, int parts, float *ws, bool a_kc, 
 int sdd_dl(int dtype, const SddArgs &g, int block, bool rowpair_plan, bool a_kc, bool b_kc, hipStream_t st) {
   if (dtype == BSP_F32 || (block != 32 && block != 16) || !g.gplan || g.n_pgroups <= 0 || g.lines <= 0 || g.cols <= 0) return 0;
   if ((block == 16) != rowpair_plan) return 0;        // blocks of 16 come with the plan over pairs of block-rows, and only they
-  if (g.K < 256 || g.K % kTK) return 0;
+  if (g.K < 256 || g.K % kTK || !near_rows(BSP_GROUP * 32, g.lda) || !near_rows(b_kc ? (int64_t)g.cols * block : kTK, g.ldb)) return 0;
   int rc;
   if (block == 32) rc = dtype == BSP_F16 ? launch_sdd_rg_dl<f16, 32>(g, a_kc, b_kc, st) : launch_sdd_rg_dl<bf16, 32>(g, a_kc, b_kc, st);
   else rc = dtype == BSP_F16 ? launch_sdd_rg_dl<f16, 16>(g, a_kc, b_kc, st) : launch_sdd_rg_dl<bf16, 16>(g, a_kc, b_kc, st);

@@ -488,11 +488,12 @@ class _sparse_matmul(torch.autograd.Function):
         return lut, num_locks.value, width.value, None
 
     @staticmethod
-    def _plan_for(lut, block, free_dim, dtype, dense_k_contiguous):
+    def _plan_for(lut, block, free_dim, dtype, width, batch):
         """The group plan that goes with a dsd / dds launch: the wide-free-dimension plan for blocks of 32 (16-bit types,
-        256 dense rows or more, dense operand with the reduction contiguous: the products the wide kernel takes), else
-        the table's ordinary plan."""
-        if (block == 32 and free_dim >= 256 and dtype != torch.float32 and dense_k_contiguous
+        256 dense rows or more, a launch of 384 workgroups or more of the wide kernel, which measures by the same rule),
+        else the table's ordinary plan."""
+        if (block == 32 and free_dim >= 256 and dtype != torch.float32
+                and (width + 3) // 4 * ((free_dim + 255) // 256) * batch >= 384
                 and getattr(lut, 'build_wide', None) is not None):
             if lut.gplan_wide is None:
                 lut.gplan_wide = lut.build_wide()
@@ -525,7 +526,7 @@ class _sparse_matmul(torch.autograd.Function):
         rc = _lib.load().bsp_dds_matmul(_lib.DTYPES[a.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
                                         int(trans_c), a.size(0), M, a.stride(0), a.stride(1), a.stride(2), b_sz, c.stride(0),
                                         c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
-                                        *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, M, a.dtype, not trans_a), M, a.size(0)), KERNEL_FLAGS,
+                                        *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, M, a.dtype, width, a.size(0)), M, a.size(0)), KERNEL_FLAGS,
                                         _lib.stream_ptr(a.device))
         _lib.check(rc, 'bsp_dds_matmul')
         time[0] = timer.done()
@@ -550,7 +551,7 @@ class _sparse_matmul(torch.autograd.Function):
         rc = _lib.load().bsp_dsd_matmul(_lib.DTYPES[b.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
                                         int(trans_c), b.size(0), N, a_sz, b.stride(0), b.stride(1), b.stride(2), c.stride(0),
                                         c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
-                                        *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, N, b.dtype, bool(trans_b)), N, b.size(0)), KERNEL_FLAGS,
+                                        *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, N, b.dtype, width, b.size(0)), N, b.size(0)), KERNEL_FLAGS,
                                         _lib.stream_ptr(b.device))
         _lib.check(rc, 'bsp_dsd_matmul')
         time[0] = timer.done()

@@ -45,3 +45,26 @@ def test_ring_and_table_windows(mode, block, Z, trans_a, trans_b):
     unit = 2. ** -11 if dtype == torch.float16 else 2. ** -8
     bound = unit * ref.abs() + 2 * K * 2. ** -24 * terms + 2. ** -24
     assert got.shape == ref.shape and bool(((got - ref).abs() <= bound).all()), (got - ref).abs().max().item()
+
+
+def test_first_wide_launch_under_capture():
+    """operators warmed up with a batch too small for the wide kernel, then captured with one that takes it: the plan of the
+    wide kernel cannot be built then, and the ordinary one (with its chains of long lines) serves"""
+    lay = torch.eye(64, dtype=torch.int64)[None]
+    lay[0, 7, :] = 1
+    lay[0, :, 9] = 1
+    dot = tb.MatMul(lay, 32, 'dsd')
+    torch.manual_seed(5)
+    sp = torch.randn(6, int(lay.sum()), 32, 32, device='cuda').half() * 0.1
+    dn = torch.randn(6, 1, 2048, 1024, device='cuda').half()
+    parts = torch.cat([dot(sp[i:i + 1], dn[i:i + 1]) for i in range(6)])      # 64 workgroups of the wide kernel a call
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        whole = dot(sp, dn)                                                  # 384
+    for _ in range(3):
+        whole.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        # the same products in another order of their fp32 sums: one unit of the 16-bit result
+        assert bool(((whole.float() - parts.float()).abs() <= 2. ** -10 * parts.float().abs() + 2. ** -12).all())
+    torch.testing.assert_close(dot(sp, dn), whole, rtol=2. ** -10, atol=2. ** -12)

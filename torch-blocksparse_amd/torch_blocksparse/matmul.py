@@ -495,9 +495,10 @@ class _sparse_matmul(torch.autograd.Function):
         if (block == 32 and free_dim >= 256 and dtype != torch.float32
                 and (width + 3) // 4 * ((free_dim + 255) // 256) * batch >= 384
                 and getattr(lut, 'build_wide', None) is not None):
-            if lut.gplan_wide is None:
+            if lut.gplan_wide is None and not torch.cuda.is_current_stream_capturing():
                 lut.gplan_wide = lut.build_wide()
-            return lut.gplan_wide
+            if lut.gplan_wide is not None:                     # (a plan cannot be built under capture: the kernel also runs the ordinary one)
+                return lut.gplan_wide
         return getattr(lut, 'gplan', None)
 
     @staticmethod

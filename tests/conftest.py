@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -42,3 +43,11 @@ def golden():
         g = json.load(f)
     g['layouts'] = {k: np.array(v, dtype=np.int64) for k, v in g['layouts'].items()}
     return g
+
+
+@pytest.fixture(autouse=True)
+def _no_garbage_of_earlier_tests(request):
+    """tests that compare allocated memory to the byte start without tensors that a later collection would free"""
+    if 'no_alloc' in request.node.nodeid:
+        gc.collect()
+    yield

@@ -354,9 +354,13 @@ int bsp_attention_bwd_kv(int dtype, const void *d_o, const void *q, const void *
  *     column, slot or -1, 0, 0, 0, the positions of the column's four groups of keys), then the entries (groups: of
  *     rows).  Work items, slots, partial and d_split as for bsp_attention_bwd_kv, positions in place of block-columns.
  * lse, neg_delta: [Z][H] rows, lse_stride_h / row_stride_h (>= 64 R) floats apart.  rows_fwd: lse may be NULL (no backward
- * pass to follow).  rows_bwd: writes dq and, if neg_delta is not NULL, -sum_d do . o of every row, which cols_bwd reads.
+ * pass to follow).  With BSP_ROWS_WITH_REST added to dtype in all three calls (strides >= 128 R), the 64 R floats of a head's
+ * lse are followed by 64 R more: what the rounding of each lse to one float left out.  Without them the probabilities of the
+ * backward pass are off by up to |lse| * 2^-24 in the exponent, which counts where every key of a row has a large finite
+ * padding value.  rows_bwd: writes dq and, if neg_delta is not NULL, -sum_d do . o of every row, which cols_bwd reads.
  * fp16 / bf16, D = 64 or 128; pointers 16-byte aligned, strides multiples of 8 elements.  keys / rows: how many positions
  * the operands have that are fetched tile by tile (k and v; q and do): their rows must lie within 4 GiB of the first. */
+enum { BSP_ROWS_WITH_REST = 256 };
 typedef struct {
   int lines, longest_line;         /* lines of tiles per head (R of the calls below), tiles of the longest one */
   int columns, n_items;            /* columns of tiles per head, work items */

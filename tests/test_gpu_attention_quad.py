@@ -128,3 +128,50 @@ def test_c_abi_argument_checks():
     assert fwd(keys=2 ** 25) != _lib.OK                 # 2^25 rows of 128 bytes: beyond the 32-bit offsets
     assert fwd(lse_sh=32) != _lib.OK
     torch.cuda.synchronize()
+
+
+def _padded_rows(block, dtype, pad, R=512):
+    """Causal layout, left padding of finite values over the first 128 keys of one sequence and over all keys of the other:
+    rows 0 .. 127 of the one and every row of the other see nothing but padded keys."""
+    lay = torch.tril(torch.ones(2, R // block, R // block)).long()
+    kpm = torch.zeros(2, R)
+    kpm[0, :128] = pad
+    kpm[1] = pad
+    return lay, kpm.to(dtype).to(DEV)
+
+
+@pytest.mark.parametrize('block,d,dtype,pad', [
+    (64, 64, torch.float16, -1e4), (16, 64, torch.float16, -65504.), (32, 128, torch.float16, -65504.),
+    (64, 128, torch.bfloat16, -1e6), (16, 64, torch.bfloat16, -1e9), (64, 64, torch.bfloat16, -1e9)])
+def test_shares_of_rows_that_see_only_padded_keys_add_up_to_one(block, d, dtype, pad):
+    """do is a one in row 2 j + 1, column j: sum_c dv[c, j] is the sum of that row's shares as the backward pass has them.  Each
+    share is rounded to the operand type once (2^-11, 2^-8 of it, or 2^-25 in fp16's subnormals); one is what they add up to."""
+    torch.manual_seed(d + block)
+    lay, kpm = _padded_rows(block, dtype, pad)
+    q, k, v = [torch.randn(2, 2, 512, d, device=DEV).to(dtype) for _ in range(3)]
+    do = torch.zeros(2, 2, 512, d, device=DEV)
+    do[:, :, 2 * torch.arange(min(d, 64)) + 1, torch.arange(min(d, 64))] = 1.
+    got = _run(lay, block, q, k, v, do.to(dtype), scale=d ** -0.5, key_padding_mask=kpm)
+    sums = got[3].double().sum(2)[..., :min(d, 64)]
+    unit = 2. ** -11 if dtype == torch.float16 else 2. ** -8
+    assert float((sums - 1.).abs().max()) <= unit + 512 * 2. ** -25 + 2. ** -16
+    if dtype == torch.float16:
+        do = torch.randn(2, 2, 512, d, device=DEV).to(dtype)
+        got = _run(lay, block, q, k, v, do, scale=d ** -0.5, key_padding_mask=kpm)
+        _check(got, D.attention(q, k, v, lay, block, d ** -0.5, key_padding_mask=kpm, attn_mask_mode='add', do=do), dtype)
+
+
+def test_the_rest_of_lse_is_part_of_the_row_buffers_only_when_asked_for():
+    lib = _lib.load()
+    t, lse = torch.zeros(1, 1, 64, 64, device=DEV, dtype=torch.float16), torch.full((128,), 7., device=DEV)
+    table = ac.AttentionCore(torch.ones(1, 1, 1, dtype=torch.int64), 64).quad(torch.device(DEV)).rows
+    null, st = ctypes.c_void_p(0), (t.stride(0), t.stride(1), 64)
+    for flag, stride, ok in ((0, 64, True), (0, 128, True), (_lib.ROWS_WITH_REST, 64, False), (_lib.ROWS_WITH_REST, 128, True)):
+        lse.fill_(7.)
+        o = torch.empty_like(t)
+        rc = lib.bsp_attention_rows_fwd(flag, _lib.ptr(t), _lib.ptr(t), _lib.ptr(t), _lib.ptr(o), _lib.ptr(lse), 1, 1, 1, 64, 64, *st, *st, *st, *st,
+                                        stride, 1.0, _lib.ptr(table), null, 0, 0, _lib.stream_ptr(torch.device(DEV)))
+        assert (rc == _lib.OK) == ok
+        if ok:
+            assert lse[:64].tolist() == [6.] * 64 and lse[64:].tolist() == [0. if flag else 7.] * 64
+    torch.cuda.synchronize()

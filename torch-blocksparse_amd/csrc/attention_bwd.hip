@@ -1,5 +1,5 @@
 // Backward pass of the attention chain without any sparse tensor: p = exp2(logit - lse) is computed again from q, k and
-// the row's lse, the softmax gradient from it, dp = do . v^T and delta = sum_d do_d o_d (= sum_j p_j dp_j, because o = p . v
+// the row's lse (its rounding: row_rest), the softmax gradient from it, dp = do . v^T and delta = sum_d do_d o_d (= sum_j p_j dp_j, because o = p . v
 // and dp = do . v^T; softmax.py:189, matmul.py:587-606):
 //     ds = p * (dp - delta) * scale,   dq = ds . k,   dk = ds^T . q,   dv = p^T . do.
 // The scale is applied to the sums dq and dk: as an operand p (dp - delta) stays below half of the largest |dp| (it is at most
@@ -112,10 +112,11 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 2) k_attn_bwd_rows(QuadArgs
       step(Const<1>{}, n + 1);
     }
   }
+  const float last = a.rest ? a.scale * __builtin_amdgcn_exp2f(-a.lse[((int64_t)z * a.H + h) * a.row_sh + a.rest + row]) : a.scale;
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-    for (int i = 0; i < 16; i++) dq[mt][i] *= a.scale;
+    for (int i = 0; i < 16; i++) dq[mt][i] *= last;
   quad_barrier();                                       // the ring is free
   T *po = reinterpret_cast<T *>(a.o) + z * a.o_sz + h * a.o_sh + ((int64_t)line * 64 + 32 * wave) * a.o_ld;
   store_32_rows<T, D>(reinterpret_cast<T *>(smem) + wave * 32 * (D + 8), po, po + 16 * a.o_ld, a.o_ld, dq, lane);
@@ -132,7 +133,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
   constexpr int MT = D / 32;
   constexpr bool LEAN = D == 128;                       // dk, dv, k and v alone take 192 registers there
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  unsigned char *rowvals = smem + Q::RING;              // per stage the lse and the delta of its rows, 256 bytes each
+  unsigned char *rowvals = smem + Q::RING;              // per stage, 128 bytes each: lse of its rows, their rests, their deltas, unused
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
   const int64_t wg = xcd_remap(blockIdx.x, (int64_t)a.Z * a.R);
@@ -159,6 +160,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
     const char *pq = reinterpret_cast<const char *>(reinterpret_cast<const T *>(a.q) + z * a.q_sz + h * a.q_sh);
     const char *pdo = reinterpret_cast<const char *>(reinterpret_cast<const T *>(a.d_o) + z * a.do_sz + h * a.do_sh);
     const char *prow = reinterpret_cast<const char *>((wave == 0 ? a.lse : a.delta) + ((int64_t)z * a.H + h) * a.row_sh);
+    const uint32_t to_rest = wave == 0 && half ? (uint32_t)a.rest * 4u : 0u;
     GroupLoad<D, LEAN> gq, gdo;
     gq.init(a.q_ld, lane);
     gdo.init(a.do_ld, lane);
@@ -166,8 +168,8 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
       const uint32_t st = lds_address(smem) + stage_no * Q::STAGE + wave * (32 * D), pos = wave ? groups.hi : groups.lo;
       gq.issue(pq, pos, (uint32_t)a.q_ld * 2u, st);
       gdo.issue(pdo, pos, (uint32_t)a.do_ld * 2u, st + Q::PIECE);
-      // one wavefront the lse of the stage's 32 rows, one their -delta (the upper lanes fetch them again)
-      load_to_lds<4>(prow, (uint32_t)((lane & 16 ? groups.hi : groups.lo) + (lane & 15)) * 4u, 0, lds_address(rowvals) + stage_no * 512 + wave * 256);
+      // one wavefront the lse of the stage's 32 rows and (the upper lanes) their rests, one their -delta (twice)
+      load_to_lds<4>(prow, (uint32_t)((lane & 16 ? groups.hi : groups.lo) + (lane & 15)) * 4u + to_rest, 0, lds_address(rowvals) + stage_no * 512 + wave * 256);
     };
     issue(0, half_groups(core, 0));
     Groups groups_next = half_groups(core, 1);
@@ -182,6 +184,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
       constexpr int S = decltype(stage_no)::value, Q0 = S * Q::STAGE, O0 = Q0 + Q::PIECE;
       quad_barrier();
       if (n + 1 < steps) issue(1 - S, groups_next);
+      const bool some_rest = a.rest && __builtin_amdgcn_ballot_w64(reinterpret_cast<const float *>(rowvals)[S * 128 + 32 + l32] != 0.f);   // (of row l32 of the stage's 32)
       Scores<T> raw;
       raw.set(row_product<T, D, Q0>(smem, rows, xk));
       const int here = bits >> (2 * wave + 8 * S);      // bit 4 * row group + column group; the wavefront's column groups are 2 wave, 2 wave + 1
@@ -202,6 +205,14 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
         const f32x4 lse = *reinterpret_cast<const f32x4 *>(rv + 16 * (g >> 1) + 4 * (g & 1));
 #pragma unroll
         for (int i = 0; i < 4; i++) p[4 * g + i] = __builtin_amdgcn_exp2f(fmaf(raw[4 * g + i], sc, KPM ? kp - lse[i] : -lse[i]));
+      }
+      if (some_rest) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const f32x4 rest = *reinterpret_cast<const f32x4 *>(rv + 32 + 16 * (g >> 1) + 4 * (g & 1));
+#pragma unroll
+          for (int i = 0; i < 4; i++) p[4 * g + i] *= __builtin_amdgcn_exp2f(-rest[i]);
+        }
       }
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) pf[ks] = pack8<T>(reinterpret_cast<const float (&)[8]>(p[8 * ks]));
@@ -307,16 +318,19 @@ extern "C" int bsp_attention_rows_bwd(int dtype, const void *d_o, const void *q,
                                       int64_t v_stride_z, int64_t v_stride_h, int64_t ldv, int64_t o_stride_z, int64_t o_stride_h, int64_t ldo,
                                       int64_t dq_stride_z, int64_t dq_stride_h, int64_t lddq, int64_t row_stride_h, float scale,
                                       const int32_t *d_lut, const void *kpm, int64_t kpm_stride_z, int kpm_mul, void *stream) {
+  const int rest = dtype & BSP_ROWS_WITH_REST ? R * 64 : 0;
+  dtype &= ~BSP_ROWS_WITH_REST;
   const void *ptrs[] = {d_o, q, k, v, o, dq, kpm, lse, neg_delta};
   const int64_t strides[] = {do_stride_z, do_stride_h, lddo, q_stride_z, q_stride_h, ldq, k_stride_z, k_stride_h, ldk, v_stride_z, v_stride_h, ldv,
                              o_stride_z, o_stride_h, ldo, dq_stride_z, dq_stride_h, lddq, kpm_stride_z};
   const int64_t lds[] = {ldk, ldv, lddo, ldq, ldo, lddq};
-  if (!d_o || !q || !k || !v || !o || !lse || !dq || !d_lut || Z <= 0 || H <= 0 || R <= 0 || row_stride_h < (int64_t)R * 64) return BSP_ERR_ARG;
+  if (!d_o || !q || !k || !v || !o || !lse || !dq || !d_lut || Z <= 0 || H <= 0 || R <= 0 || row_stride_h < (int64_t)R * 64 + rest) return BSP_ERR_ARG;
   const int rc = quad_check(dtype, D, ptrs, 9, strides, 19, lds, 6, 2, keys, (int64_t)Z * H * R);
   if (rc != BSP_OK) return rc;
   QuadArgs a{};
   a.d_o = d_o; a.q = q; a.k = k; a.v = v; a.o_in = o; a.o = dq;
   a.lse = const_cast<float *>(lse); a.delta = neg_delta; a.row_sh = row_stride_h;
+  a.rest = rest;
   a.do_sz = do_stride_z; a.do_sh = do_stride_h; a.do_ld = lddo;
   a.q_sz = q_stride_z; a.q_sh = q_stride_h; a.q_ld = ldq;
   a.k_sz = k_stride_z; a.k_sh = k_stride_h; a.k_ld = ldk;
@@ -339,18 +353,21 @@ extern "C" int bsp_attention_cols_bwd(int dtype, const void *d_o, const void *q,
                                       int64_t dv_stride_z, int64_t dv_stride_h, int64_t lddv, int64_t row_stride_h, float scale,
                                       const int32_t *d_items, int n_items, float *partial, int n_slots, const int32_t *d_split, int n_split,
                                       const void *kpm, int64_t kpm_stride_z, int kpm_mul, void *stream) {
+  const int64_t rest = dtype & BSP_ROWS_WITH_REST ? rows : 0;
+  dtype &= ~BSP_ROWS_WITH_REST;
   const void *ptrs[] = {d_o, q, k, v, dk, dv, kpm, lse, neg_delta, partial};
   const int64_t strides[] = {do_stride_z, do_stride_h, lddo, q_stride_z, q_stride_h, ldq, k_stride_z, k_stride_h, ldk, v_stride_z, v_stride_h, ldv,
                              dk_stride_z, dk_stride_h, lddk, dv_stride_z, dv_stride_h, lddv, kpm_stride_z};
   const int64_t lds[] = {lddo, ldq, ldk, ldv, lddk, lddv};
   if (!d_o || !q || !k || !v || !lse || !neg_delta || !dk || !dv || !d_items || Z <= 0 || H <= 0 || C <= 0 || n_items < H * C) return BSP_ERR_ARG;
   if (n_slots < 0 || n_split < 0 || (n_slots > 0) != (n_split > 0) || (n_slots > 0 && (!partial || !d_split)) || n_items > H * C + n_slots) return BSP_ERR_ARG;
-  if (row_stride_h < rows) return BSP_ERR_ARG;
+  if (row_stride_h < rows + rest) return BSP_ERR_ARG;
   const int rc = quad_check(dtype, D, ptrs, 10, strides, 19, lds, 6, 2, rows, (int64_t)Z * n_items + (int64_t)Z * n_split * 16);
   if (rc != BSP_OK) return rc;
   QuadArgs a{};
   a.d_o = d_o; a.q = q; a.k = k; a.v = v; a.o = dk; a.o2 = dv;
   a.lse = const_cast<float *>(lse); a.delta = const_cast<float *>(neg_delta); a.row_sh = row_stride_h;
+  a.rest = rest;
   a.do_sz = do_stride_z; a.do_sh = do_stride_h; a.do_ld = lddo;
   a.q_sz = q_stride_z; a.q_sh = q_stride_h; a.q_ld = ldq;
   a.k_sz = k_stride_z; a.k_sh = k_stride_h; a.k_ld = ldk;

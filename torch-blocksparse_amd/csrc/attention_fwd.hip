@@ -127,8 +127,12 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 3) k_attn_fwd(QuadArgs a) {
   l += swap32(l);
   const bool any_block = (rows_seen >> 4 * ((lane >> 4) & 1)) & 15;
   const float inv = any_block ? 1.f / l : 0.f;          // masked everywhere: 0 * inf = NaN, as the softmax operator gives; no block at all: zeros
-  if (a.lse != nullptr && half == 0)
-    a.lse[((int64_t)z * a.H + h) * a.row_sh + row] = any_block ? m + __builtin_amdgcn_logf(l) : INFINITY;   // (... and a share of 0 in the backward pass)
+  if (a.lse != nullptr && half == 0) {
+    const float log_l = __builtin_amdgcn_logf(l), lse = m + log_l;
+    float *to = a.lse + ((int64_t)z * a.H + h) * a.row_sh + row;
+    *to = any_block ? lse : INFINITY;                   // (... and a share of 0 in the backward pass)
+    if (a.rest) to[a.rest] = any_block ? row_rest(m, log_l, lse) : 0.f;
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -159,14 +163,17 @@ extern "C" int bsp_attention_rows_fwd(int dtype, const void *q, const void *k, c
                                       int64_t v_stride_z, int64_t v_stride_h, int64_t ldv, int64_t o_stride_z, int64_t o_stride_h, int64_t ldo,
                                       int64_t lse_stride_h, float scale, const int32_t *d_lut, const void *kpm, int64_t kpm_stride_z, int kpm_mul,
                                       void *stream) {
+  const int rest = dtype & BSP_ROWS_WITH_REST ? R * 64 : 0;
+  dtype &= ~BSP_ROWS_WITH_REST;
   const void *ptrs[] = {q, k, v, o, kpm};
   const int64_t strides[] = {q_stride_z, q_stride_h, ldq, k_stride_z, k_stride_h, ldk, v_stride_z, v_stride_h, ldv, o_stride_z, o_stride_h, ldo, kpm_stride_z};
   const int64_t lds[] = {ldk, ldv, ldq, ldo};
-  if (!q || !k || !v || !o || !d_lut || Z <= 0 || H <= 0 || R <= 0 || (lse && (lse_stride_h < (int64_t)R * 64 || (reinterpret_cast<uintptr_t>(lse) & 15)))) return BSP_ERR_ARG;
+  if (!q || !k || !v || !o || !d_lut || Z <= 0 || H <= 0 || R <= 0 || (lse && (lse_stride_h < (int64_t)R * 64 + rest || (reinterpret_cast<uintptr_t>(lse) & 15)))) return BSP_ERR_ARG;
   const int rc = quad_check(dtype, D, ptrs, 5, strides, 13, lds, 4, 2, keys, (int64_t)Z * H * R);
   if (rc != BSP_OK) return rc;
   QuadArgs a{};
   a.q = q; a.k = k; a.v = v; a.o = o; a.lse = lse; a.row_sh = lse_stride_h;
+  a.rest = rest;
   a.q_sz = q_stride_z; a.q_sh = q_stride_h; a.q_ld = ldq;
   a.k_sz = k_stride_z; a.k_sh = k_stride_h; a.k_ld = ldk;
   a.v_sz = v_stride_z; a.v_sh = v_stride_h; a.v_ld = ldv;

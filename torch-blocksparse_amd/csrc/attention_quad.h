@@ -34,7 +34,7 @@ struct QuadArgs {
   const void *d_o, *o_in;          // backward: do, and the forward result (row kernel)
   void *o, *o2;                    // forward: o; row kernel: dq; column kernel: dk and dv
   float *lse, *delta;              // per row, [Z][H] rows row_sh apart
-  int64_t row_sh;
+  int64_t row_sh, rest;            // rest: floats from a row's lse to what its rounding left out (row_rest); 0: not kept
   int64_t q_sz, q_sh, q_ld, k_sz, k_sh, k_ld, v_sz, v_sh, v_ld, do_sz, do_sh, do_ld, oin_sz, oin_sh, oin_ld;
   int64_t o_sz, o_sh, o_ld, o2_sz, o2_sh, o2_ld;
   float scale;
@@ -295,6 +295,14 @@ template <typename T, int N> __device__ __forceinline__ void negate(typename Mma
 
 // |scale| in the log2 domain; not zero, so that -inf stays -inf
 __device__ __forceinline__ float logit_scale(float scale) { return fmaxf(fabsf(scale) * kLog2e, 1e-30f); }
+
+// A row's lse = m + log2 l has the precision of m: where the maximum is far from zero (finite padding values of -10000 or
+// -65504 on every key that the row sees, large scores) the sum rounds log2 l away, and exp2(logit - lse) would not add up to
+// one: by 0.3 % at -65504, by the number of keys at -1e9.  From a maximum of kRestFrom on (below it the sum loses 2^-18 at
+// most) the forward kernel keeps what was lost as a second float; the backward kernels multiply by exp2(-rest), the row
+// kernel its sums at the end, the column kernel the shares of a step in which a row has one.
+constexpr float kRestFrom = 64.f;
+__device__ __forceinline__ float row_rest(float m, float log_l, float lse) { return fabsf(m) >= kRestFrom ? log_l - (lse - m) : 0.f; }
 
 // key-padding value -> addend in the log2 domain (softmax.py:104-106, 122-124)
 template <typename T> __device__ __forceinline__ float kpm_term(T v, int mul) {

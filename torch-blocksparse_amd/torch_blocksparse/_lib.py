@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(os.path.dirname(_HERE), 'lib', 'libbsp_hip.so')
 F16, BF16, F32 = 0, 1, 2
 DTYPES = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
 
+ROWS_WITH_REST = 256  # BSP_ROWS_WITH_REST
 FLAG_GENERAL_ONLY, FLAG_NO_GROUPS, FLAG_NO_WIDE, FLAG_PLAN_ROWPAIR = 1, 2, 4, 8   # bsp_launch_flags
 
 OK = 0

@@ -270,8 +270,9 @@ class AttentionCore:
 
 
 class _attention_quad(torch.autograd.Function):
-    """The chain without per-element masks: no sparse tensor is kept for the backward pass, one float per row is (the
-    logarithm of the row's sum of exponentials), from which the backward kernels compute the softmax again."""
+    """The chain without per-element masks: no sparse tensor is kept for the backward pass, two floats per row are (the
+    logarithm of the row's sum of exponentials, and what its rounding left out), from which the backward kernels compute
+    the softmax again."""
 
     @staticmethod
     def forward(ctx, q, k, v, scale, key_padding_mask, kp_mask_mode, core, grad_enabled):
@@ -287,11 +288,11 @@ class _attention_quad(torch.autograd.Function):
             kpm = _sparse_softmax._strided16(key_padding_mask, 'key_padding_mask')
         ctx.kpm_args = (kpm.stride(0) if kpm is not None and kpm.size(0) > 1 else 0, int(kp_mask_mode == 'mul'))
         o = torch.empty((Z, H, R * core.block, D), dtype=q.dtype, device=q.device)
-        lse = torch.empty((Z, H, lines * 64), dtype=torch.float32, device=q.device) if keep else None
+        lse = torch.empty((Z, H, 2, lines * 64), dtype=torch.float32, device=q.device) if keep else None      # (and what its rounding left out)
         rc = _lib.load().bsp_attention_rows_fwd(
-            _lib.DTYPES[q.dtype], _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse), Z, H, lines, k.size(2), D,
+            _lib.DTYPES[q.dtype] | _lib.ROWS_WITH_REST, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse), Z, H, lines, k.size(2), D,
             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
-            o.stride(0), o.stride(1), o.stride(2), lines * 64, scale, _lib.ptr(tables.rows), _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
+            o.stride(0), o.stride(1), o.stride(2), lines * 128, scale, _lib.ptr(tables.rows), _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
         _lib.check(rc, 'bsp_attention_rows_fwd')
         fused_calls += 1
         if keep:
@@ -306,10 +307,10 @@ class _attention_quad(torch.autograd.Function):
         Z, H, D = q.size(0), q.size(1), q.size(3)
         dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         rc = _lib.load().bsp_attention_rows_bwd(
-            _lib.DTYPES[q.dtype], _lib.ptr(do), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse), _lib.ptr(dq), _lib.ptr(delta), Z, H,
+            _lib.DTYPES[q.dtype] | _lib.ROWS_WITH_REST, _lib.ptr(do), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse), _lib.ptr(dq), _lib.ptr(delta), Z, H,
             ctx.tables.lines, k.size(2), D, do.stride(0), do.stride(1), do.stride(2), q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), o.stride(0), o.stride(1), o.stride(2), dq.stride(0), dq.stride(1), dq.stride(2),
-            ctx.tables.lines * 64, ctx.scale, _lib.ptr(ctx.tables.rows), _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
+            ctx.tables.lines * 128, ctx.scale, _lib.ptr(ctx.tables.rows), _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
         _lib.check(rc, 'bsp_attention_rows_bwd')
         return dq
 
@@ -323,10 +324,10 @@ class _attention_quad(torch.autograd.Function):
         dv = torch.empty(v.shape, dtype=v.dtype, device=v.device)
         partial = torch.empty((Z, ct.n_slots, 2, 64, D), dtype=torch.float32, device=q.device) if ct.n_slots else None
         rc = _lib.load().bsp_attention_cols_bwd(
-            _lib.DTYPES[q.dtype], _lib.ptr(do), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(lse), _lib.ptr(delta), _lib.ptr(dk), _lib.ptr(dv), Z, H,
+            _lib.DTYPES[q.dtype] | _lib.ROWS_WITH_REST, _lib.ptr(do), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(lse), _lib.ptr(delta), _lib.ptr(dk), _lib.ptr(dv), Z, H,
             ct.columns, q.size(2), D, do.stride(0), do.stride(1), do.stride(2), q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), dk.stride(0), dk.stride(1), dk.stride(2), dv.stride(0), dv.stride(1), dv.stride(2),
-            ctx.tables.lines * 64, ctx.scale, _lib.ptr(ct.items), ct.n_items, _lib.ptr(partial), ct.n_slots, _lib.ptr(ct.split), ct.n_split,
+            ctx.tables.lines * 128, ctx.scale, _lib.ptr(ct.items), ct.n_items, _lib.ptr(partial), ct.n_slots, _lib.ptr(ct.split), ct.n_split,
             _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
         _lib.check(rc, 'bsp_attention_cols_bwd')
         return dk, dv
@@ -350,7 +351,7 @@ class _attention_quad(torch.autograd.Function):
         do = _near(do)
         need_q, need_k, need_v = ctx.needs_input_grad[:3]
         dq = dk = dv = None
-        rows = (q.size(0), q.size(1), ctx.tables.lines * 64)
+        rows = (q.size(0), q.size(1), 2, ctx.tables.lines * 64)      # (the rows of a head as far apart as those of lse; the second half is not used)
         delta = None
         if need_k:
             delta = torch.empty(rows, dtype=torch.float32, device=q.device)

@@ -175,3 +175,35 @@ def test_the_rest_of_lse_is_part_of_the_row_buffers_only_when_asked_for():
         if ok:
             assert lse[:64].tolist() == [6.] * 64 and lse[64:].tolist() == [0. if flag else 7.] * 64
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize('block,d,dtype,why', [
+    (16, 64, torch.float16, 'padded'), (32, 64, torch.bfloat16, 'padded'), (16, 128, torch.bfloat16, 'padded'), (32, 128, torch.float16, 'padded'),
+    (16, 64, torch.float16, 'overflow'), (32, 128, torch.float16, 'overflow')])
+def test_rows_without_a_softmax_reach_only_the_keys_they_attend_to(block, d, dtype, why):
+    """Causal layout whose first block-row sees nothing but its own keys, all padded (or one of whose rows has scores beyond the
+    type): these rows are NaN, and the gradients of the keys of their block; the other keys of the same 64 x 64 tiles have no block there."""
+    torch.manual_seed(block + d)
+    lay = torch.tril(torch.ones(2, 256 // block, 256 // block)).long()
+    q, k, v, do = [torch.randn(2, 2, 256, d, device=DEV).to(dtype) for _ in range(4)]
+    kw = dict(scale=d ** -0.5)
+    if why == 'padded':
+        kw['key_padding_mask'] = torch.zeros(2, 256, device=DEV).to(dtype)
+        kw['key_padding_mask'][0, :block] = float('-inf')
+        do[0, 1, :block] = 0.
+    else:
+        q[0, :, 3] = 6e4
+    got = _run(lay, block, q, k, v, do, **kw)
+    old = ac.FUSED
+    try:
+        ac.FUSED = False
+        ops = (tb.MatMul(lay, block, 'sdd', trans_b=True), tb.Softmax(lay, block), tb.MatMul(lay, block, 'dsd'))
+        ts = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        o = ac.attention_chain(*ops, *ts, **kw)
+        o.backward(do)
+    finally:
+        ac.FUSED = old
+    for name, g, r in zip(('o', 'dq', 'dk', 'dv'), got, [o.detach()] + [t.grad for t in ts]):
+        assert torch.equal(torch.isnan(g), torch.isnan(r)), name
+        assert bool(torch.isnan(r).any()) and not bool(torch.isnan(r[1]).any()) and not bool(torch.isnan(r[0, :, block:]).any()), name
+        assert_close(g, r, dtype, name)

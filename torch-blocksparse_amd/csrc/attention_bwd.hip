@@ -190,11 +190,10 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
       const int here = bits >> (2 * wave + 8 * S);      // bit 4 * row group + column group; the wavefront's column groups are 2 wave, 2 wave + 1
       bits = half_bits(core, n + 1 < steps ? n + 1 : n);
       groups_next = half_groups(core, n + 2 < steps ? n + 2 : steps - 1);
-      if ((here & 0x33) != 0x33) {
-        const int mine = here >> ((lane >> 4) & 1);
-        raw.keep_if(0, mine & 1);
-        raw.keep_if(1, mine & 16);
-      }
+      // Pieces without a block: their shares and softmax gradients are set to zero once they are operands.  (A score of -inf
+      // is not enough: in a row that is masked everywhere lse or delta is not a number, and the keys of such a piece, which
+      // the row does not attend to, would take it up.)
+      const bool holes = (here & 0x33) != 0x33;
       // The rows' values are read into as many registers as there are scores (two addresses a read, which costs the LDS
       // little): lse is what the scaled scores are added to, -delta where the product dp starts.
       const float *rv = rv_half + S * 128;
@@ -216,6 +215,10 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
       }
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) pf[ks] = pack8<T>(reinterpret_cast<const float (&)[8]>(p[8 * ks]));
+      if (holes) {
+        zero_unless(pf[0], here);
+        zero_unless(pf[1], here >> 4);
+      }
       tr_product<T, D, O0>(dv, tr, pf);
       f32x16 dp;
 #pragma unroll
@@ -229,6 +232,10 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
       for (int i = 0; i < 16; i++) e[i] = p[i] * dp[i]; // (the scale comes last, on dk)
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) df[ks] = pack8<T>(reinterpret_cast<const float (&)[8]>(e[8 * ks]));
+      if (LEAN || holes) {                              // (a branch here costs registers that the wide head does not have)
+        zero_unless(df[0], here);
+        zero_unless(df[1], here >> 4);
+      }
       tr_product<T, D, Q0>(dk, tr, df);
     };
     for (int n = 0; n < steps; n += 2) {

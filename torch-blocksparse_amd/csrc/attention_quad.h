@@ -121,6 +121,16 @@ template <typename T> __device__ __forceinline__ typename Mma<T, 32>::frag_t pac
   return u.f;
 }
 
+// The eight values of an operand that belong to a piece without a block: zero, whatever came out for them.  pieces: bit 0 the
+// lanes 0 .. 15 and 32 .. 47 have one, bit 1 the others (made a lane mask by scalar instructions: no vector register holds it)
+template <typename F> __device__ __forceinline__ void zero_unless(F &f, int pieces) {
+  const bool here = __builtin_amdgcn_inverse_ballot_w64((pieces & 1 ? 0x0000ffff0000ffffull : 0) | (pieces & 2 ? 0xffff0000ffff0000ull : 0));
+  u32x4 r = __builtin_bit_cast(u32x4, f);
+#pragma unroll
+  for (int i = 0; i < 4; i++) r[i] = here ? r[i] : 0u;
+  f = __builtin_bit_cast(F, r);
+}
+
 // An operand fragment through the transposing LDS read: rows 0 .. 3 of the lane's column at the first address, 4 .. 7 at the second
 template <typename T> __device__ __forceinline__ typename Mma<T, 32>::frag_t tr_fragment(uint32_t lo, uint32_t hi) {
   typedef s16x4 __attribute__((address_space(3))) * lds_ptr;

@@ -207,3 +207,20 @@ def test_rows_without_a_softmax_reach_only_the_keys_they_attend_to(block, d, dty
         assert torch.equal(torch.isnan(g), torch.isnan(r)), name
         assert bool(torch.isnan(r).any()) and not bool(torch.isnan(r[1]).any()) and not bool(torch.isnan(r[0, :, block:]).any()), name
         assert_close(g, r, dtype, name)
+
+
+@pytest.mark.parametrize('block,d', [(64, 64), (16, 128), (32, 64), (64, 128)])
+def test_padding_values_beyond_the_scores(block, d):
+    """-1e9 in bf16: in rows that see nothing else, fp32 rounds the scores away beside it and every key gets the same share, in
+    the oracle, in the three operators and in the fused kernels."""
+    torch.manual_seed(d)
+    lay, kpm = _padded_rows(block, torch.bfloat16, -1e9)
+    q, k, v, do = [torch.randn(2, 2, 512, d, device=DEV).bfloat16() for _ in range(4)]
+    kw = dict(scale=d ** -0.5, key_padding_mask=kpm)
+    got = _run(lay, block, q, k, v, do, **kw)
+    _check(got, D.attention(q, k, v, lay, block, d ** -0.5, key_padding_mask=kpm, attn_mask_mode='add', do=do), torch.bfloat16)
+    ops = (tb.MatMul(lay, block, 'sdd', trans_b=True), tb.Softmax(lay, block), tb.MatMul(lay, block, 'dsd'))
+    ts = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    o = ops[2](ops[1](ops[0](ts[0], ts[1]), **kw), ts[2])
+    o.backward(do)
+    _check(got, [o.detach()] + [t.grad for t in ts], torch.bfloat16)

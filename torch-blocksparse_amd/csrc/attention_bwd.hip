@@ -96,6 +96,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 2) k_attn_bwd_rows(QuadArgs
         raw.keep_if(1, mine & 2);
       }
       const float kp = KPM ? kpm_term(kp_lane[S * 128], a.kpm_mul) : 0.f;
+      if (KPM && __builtin_amdgcn_ballot_w64(far_padding<T>(kp))) raw.settle(sc, [&](auto ic) { return row_bcast<decltype(ic)::value>(kp); });
       float e[16];
       for_16<0>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
@@ -160,6 +161,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
     const char *pq = reinterpret_cast<const char *>(reinterpret_cast<const T *>(a.q) + z * a.q_sz + h * a.q_sh);
     const char *pdo = reinterpret_cast<const char *>(reinterpret_cast<const T *>(a.d_o) + z * a.do_sz + h * a.do_sh);
     const char *prow = reinterpret_cast<const char *>((wave == 0 ? a.lse : a.delta) + ((int64_t)z * a.H + h) * a.row_sh);
+    const bool far = KPM && __builtin_amdgcn_ballot_w64(far_padding<T>(kp));
     const uint32_t to_rest = wave == 0 && half ? (uint32_t)a.rest * 4u : 0u;
     GroupLoad<D, LEAN> gq, gdo;
     gq.init(a.q_ld, lane);
@@ -187,6 +189,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
       const bool some_rest = a.rest && __builtin_amdgcn_ballot_w64(reinterpret_cast<const float *>(rowvals)[S * 128 + 32 + l32] != 0.f);   // (of row l32 of the stage's 32)
       Scores<T> raw;
       raw.set(row_product<T, D, Q0>(smem, rows, xk));
+      if (far) raw.settle(sc, [&](auto) { return kp; });
       const int here = bits >> (2 * wave + 8 * S);      // bit 4 * row group + column group; the wavefront's column groups are 2 wave, 2 wave + 1
       bits = half_bits(core, n + 1 < steps ? n + 1 : n);
       groups_next = half_groups(core, n + 2 < steps ? n + 2 : steps - 1);

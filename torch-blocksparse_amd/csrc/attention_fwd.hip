@@ -87,6 +87,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 3) k_attn_fwd(QuadArgs a) {
         raw.keep_if(1, mine & 2);
       }
       const float kp = KPM ? kpm_term(kp_lane[S * 128], a.kpm_mul) : 0.f;
+      if (KPM && __builtin_amdgcn_ballot_w64(far_padding<T>(kp))) raw.settle(sc, [&](auto ic) { return row_bcast<decltype(ic)::value>(kp); });
       // the exponentials relative to the running maximum as it stands: nearly always it still serves
       float e[16], sum;
       auto exponentials = [&]() {

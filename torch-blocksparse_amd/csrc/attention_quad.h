@@ -79,6 +79,16 @@ template <int I, class F> __device__ __forceinline__ void for_16(F &&f) {
 
 __device__ __forceinline__ float swap32(float v) { return __shfl_xor(v, 32); }
 
+// Finite padding values so large that fp32 cannot hold them and the scores together (bf16 only: -1e9, say): the softmax operator
+// adds the two and rounds, which leaves little or nothing of the score, so that a row of such keys gets equal shares.  These
+// kernels take the maximum off the padding value first and would bring the scores back; where a padding value is this
+// large they are first reduced to what the rounding leaves of them (Scores::settle).  Below it the rounding is worth
+// 2^-4 in the exponent at most and is left out.
+constexpr float kFarPadding = 2097152.f;
+template <typename T> __device__ __forceinline__ bool far_padding(float kp) {
+  return !__is_same(T, f16) && fabsf(kp) >= kFarPadding && kp != -INFINITY;
+}
+
 // The scores of a quadrant rounded to the storage type, as the sdd operator would have stored them (the chain then gives what
 // the three operators give, up to the order of its sums); the conversion back is part of the multiply-add that uses them.
 template <typename T> struct Scores {
@@ -95,6 +105,14 @@ template <typename T> struct Scores {
     const uint32_t none = sizeof(T) == 2 && __is_same(T, f16) ? 0xfc00fc00u : 0xff80ff80u;   // two times -inf
 #pragma unroll
     for (int i = 4 * k; i < 4 * k + 4; i++) pair[i] = here ? pair[i] : __builtin_bit_cast(t2, none);
+  }
+  // value i, scaled by sc, to what is left of it beside the padding value kp(i) (see far_padding)
+  template <class F> __device__ __forceinline__ void settle(float sc, F &&kp) {
+    for_16<0>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const float pad = kp(ic), left = (fmaf((*this)[i], sc, pad) - pad) * __builtin_amdgcn_rcpf(sc);
+      pair[i >> 1][i & 1] = far_padding<T>(pad) ? (T)left : pair[i >> 1][i & 1];
+    });
   }
   __device__ __forceinline__ float top() const {
     if constexpr (__is_same(T, f16)) {

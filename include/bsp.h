@@ -376,6 +376,14 @@ typedef struct {
  * 16 tiles and twice the average are cut into parts. */
 int bsp_attention_tables_build(const uint8_t *h_layout, int H, int R, int C, int block, int32_t *h_tables, int64_t cap,
                                bsp_attention_tables *info);
+/* Host function: the tables of bsp_attention_fwd / bsp_attention_bwd (d_lut at 0: at blocks of 64 what bsp_softmax_lut_build
+ * gives) and bsp_attention_bwd_kv (d_col_lut, d_split_lut), written as by bsp_attention_tables_build, with the same lines and
+ * columns of tiles; work items by column.  h_ids: [H, R, C] ids of the blocks, or NULL for their positions in the row-major
+ * order of the nonzero blocks; part: tiles of a part of a long column, or 0 for the rule above.  A layout whose C does not
+ * divide into tiles gets the table of the lines alone.  2 H R + 20 H C + (20 at blocks of 64, else 28 + 2 S S) ints per
+ * nonzero block always are enough. */
+int bsp_attention_stored_tables_build(const uint8_t *h_layout, const int32_t *h_ids, int H, int R, int C, int block, int part,
+                                      int32_t *h_tables, int64_t cap, bsp_attention_tables *info);
 int bsp_attention_rows_fwd(int dtype, const void *q, const void *k, const void *v, void *o, float *lse, int Z, int H, int R, int64_t keys, int D,
                            int64_t q_stride_z, int64_t q_stride_h, int64_t ldq, int64_t k_stride_z, int64_t k_stride_h, int64_t ldk,
                            int64_t v_stride_z, int64_t v_stride_h, int64_t ldv, int64_t o_stride_z, int64_t o_stride_h, int64_t ldo,

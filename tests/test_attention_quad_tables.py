@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from torch_blocksparse import _lib
-from torch_blocksparse.attention_core import _ColumnTable, _QuadTables
+from torch_blocksparse.attention_core import AttentionCore, _ColumnTable, _QuadTables, _stored_tables
 
 
 @pytest.mark.parametrize('block,H,R,C,density,dtype', [
@@ -79,3 +79,39 @@ def test_errors():
     assert build(lay, 3, 16, 16) == _lib.ERR_UNSUPPORTED
     assert build(lay, 4, 128, 16) == _lib.ERR_UNSUPPORTED
     assert build(None, 4, 64, 16) != _lib.OK
+
+
+@pytest.mark.parametrize('block,H,R,C', [(64, 3, 7, 70), (32, 2, 8, 10), (16, 2, 8, 7)])
+def test_tables_of_the_kernels_that_store_p(block, H, R, C):
+    """the rows' part (the softmax table at blocks of 64, tiles with the ids of their blocks below), made beside the other set by
+    whichever call comes first; a layout whose columns do not divide into tiles gets no columns"""
+    torch.manual_seed(C)
+    lay = (torch.rand(H, R, C) < 0.3).long()
+    lay[0, 1] = 0
+    S = 64 // block
+    host, info = _stored_tables(lay, block)
+    assert info.lines == R // S and info.columns == (0 if C % S else C // S) and info.longest_line == max(
+        -(-int(n) // S) for n in (lay.reshape(H, R // S, S, C).sum(2) > 0).sum(-1).flatten())
+    seen = {}
+    for h in range(H):
+        for line in range(R // S):
+            n, first = host[2 * (h * (R // S) + line):][:2].tolist()
+            for e in range(n):
+                if S == 1:
+                    bid, c, r, hh = host[first + 4 * e:][:4].tolist()
+                    assert (r, hh) == (line, h)
+                    seen[bid] = (h, r, c)
+                else:
+                    entry = host[first + (8 + S * S) * e:][:8 + S * S].tolist()
+                    for i, bid in enumerate(entry[8:]):
+                        if bid >= 0:
+                            seen[bid] = (h, S * line + i // S, entry[4 + i % S])
+    assert [list(seen[i]) for i in range(len(seen))] == lay.nonzero().tolist()
+    core = AttentionCore(lay, block)
+    if C % S:
+        assert core.tables('cpu') is None and core.quad('cpu') is None
+    else:
+        assert torch.equal(core.tables('cpu')[0], host) and core.quad('cpu').lines == R // S
+    odd = ctypes.c_int64(0)
+    assert _lib.load().bsp_attention_stored_tables_build(_lib.ptr(lay.bool()), None, H, R, C, block, 0, ctypes.byref(odd), 1, ctypes.byref(info)) == _lib.ERR_CAPACITY
+    assert info.total == host.numel()

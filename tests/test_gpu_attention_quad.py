@@ -224,3 +224,44 @@ def test_padding_values_beyond_the_scores(block, d):
     o = ops[2](ops[1](ops[0](ts[0], ts[1]), **kw), ts[2])
     o.backward(do)
     _check(got, [o.detach()] + [t.grad for t in ts], torch.bfloat16)
+
+
+@pytest.mark.parametrize('block', [64, 16])
+@pytest.mark.parametrize('masked_first', [False, True])
+def test_capture_of_the_kind_of_call_that_the_warm_up_was_not(block, masked_first):
+    """Calls with per-element masks run other kernels on other tables than calls without.  Operators that have met one kind
+    only are captured with the other; every replay against operators that run it eagerly."""
+    torch.manual_seed(block)
+    L = 256
+    lay = torch.tril(torch.ones(2, L // block, L // block)).long()
+    make = lambda: (tb.MatMul(lay, block, 'sdd', trans_b=True), tb.Softmax(lay, block), tb.MatMul(lay, block, 'dsd'))
+    masks = dict(rpe=(0.3 * torch.randn(L, L, device=DEV)).half())
+    ops, others = make(), make()
+
+    def chain(ops, tensors, kw):
+        ts = [t.detach().clone().requires_grad_(True) for t in tensors[:3]]
+        before = ac.fused_calls
+        o = ac.attention_chain(*ops, *ts, scale=0.125, **kw)
+        assert ac.fused_calls == before + 1
+        return (o.detach(),) + torch.autograd.grad(o, ts, tensors[3])
+    static_in = [torch.randn(2, 2, L, 64, device=DEV).half() for _ in range(4)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        chain(ops, static_in, masks if masked_first else {})
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    kw = {} if masked_first else masks
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        static_out = chain(ops, static_in, kw)
+    for _ in range(3):
+        fresh = [torch.randn_like(t) for t in static_in]
+        eager = chain(others, fresh, kw)
+        torch.cuda.synchronize()
+        for s, f in zip(static_in, fresh):
+            s.copy_(f)
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, a, b in zip(('o', 'dq', 'dk', 'dv'), static_out, eager):
+            assert torch.equal(a, b), name

@@ -73,6 +73,7 @@ SIGNATURES = {
     'bsp_attention_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i] + [_i64] * 17 + [_i, _f, _vp, _i, _vp, _i64, _vp]),
     'bsp_attention_bwd_kv': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i] + [_i64] * 17 + [_i, _f, _vp, _i, _vp, _i, _vp, _i, _vp]),
     'bsp_attention_tables_build': (_i, [_vp, _i, _i, _i, _i, _vp, _i64, _c.POINTER(AttentionTables)]),
+    'bsp_attention_stored_tables_build': (_i, [_vp, _vp, _i, _i, _i, _i, _i, _vp, _i64, _c.POINTER(AttentionTables)]),
     'bsp_attention_rows_fwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 13 + [_f, _vp, _vp, _i64, _i, _vp]),
     'bsp_attention_rows_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 19 + [_f, _vp, _vp, _i64, _i, _vp]),
     'bsp_attention_cols_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 19 + [_f, _vp, _i, _vp, _i, _vp, _i, _vp, _i64, _i, _vp]),

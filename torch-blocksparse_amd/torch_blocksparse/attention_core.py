@@ -26,6 +26,20 @@ FUSED_KV = os.environ.get('BSP_FUSED_ATTENTION_KV', '1') != '0'
 
 
 
+def _stored_tables(layout, block, ids=None, part=0):
+    """(tables, sizes): the tables of the kernels that store p, in host memory (bsp_attention_stored_tables_build)"""
+    lay = (layout != 0).cpu().contiguous()
+    H, R, C = lay.shape
+    S = 64 // block
+    info = _lib.AttentionTables()
+    cap = 2 * H * R + 20 * H * C + (20 if S == 1 else 28 + 2 * S * S) * int(torch.count_nonzero(lay))
+    host = torch.empty(max(cap, 1), dtype=torch.int32)
+    ids = None if ids is None else ids.to(torch.int32).contiguous()
+    _lib.check(_lib.load().bsp_attention_stored_tables_build(_lib.ptr(lay), _lib.ptr(ids), H, R, C, block, part, _lib.ptr(host), cap,
+                                                             ctypes.byref(info)), 'bsp_attention_stored_tables_build')
+    return host[:info.total], info
+
+
 class _GatheredTiles:
     """64 x 64 tiles over a layout of small blocks (S = 64 / block a side).  A *line* of tiles is S consecutive block-rows;
     a tile takes the line's S block-rows and S block-columns gathered from anywhere in the line: the columns in which
@@ -37,37 +51,20 @@ class _GatheredTiles:
     the block at (block-row i of the line, gathered column g), -1 where the layout has none or the slot is padding."""
 
     def __init__(self, lay, ids, S):
-        H, R, C = lay.shape
-        L = R // S
-        pres = lay.reshape(H, L, S, C).any(2)
-        n = pres.sum(-1).flatten()
-        self.sizes = (n + S - 1) // S
-        self.starts = torch.cumsum(self.sizes, 0) - self.sizes
-        self.n_tiles = int(self.sizes.sum())
-        h, t, c = pres.nonzero().unbind(1)
-        line = h * L + t
-        rank = torch.arange(c.numel()) - (torch.cumsum(n, 0) - n)[line]
-        tile, slot = self.starts[line] + rank // S, rank % S
-        cols = torch.full((self.n_tiles, S), -1, dtype=torch.int64)
-        cols[tile, slot] = c
-        self.cols = torch.where(cols < 0, cols[:, :1], cols)
-        self.ids = torch.full((self.n_tiles, S, S), -1, dtype=ids.dtype)
-        for i in range(S):
-            self.ids[tile, i, slot] = ids[h, t * S + i, c]
-        self.lines, self.heads = L, H
+        host, info = _stored_tables(lay, 64 // S, ids)
+        self.lines, self.heads = info.lines, lay.size(0)
+        n, ints = self.lines * self.heads, 8 + S * S
+        self.sizes = host[0:2 * n:2].long()
+        self.starts = (host[1:2 * n:2].long() - 2 * n) // ints
+        self._entries = host[2 * n:info.items_offset].reshape(-1, ints).long()
+        self.n_tiles = self._entries.size(0)
+        self.cols = self._entries[:, 4:4 + S]
+        self.ids = self._entries[:, 8:].reshape(-1, S, S)
 
-    def entries(self, transposed_ids=False):
+    def entries(self):
         """per tile 8 + S * S ints: (tile, 0, line, head, then the tile's block-columns, the last repeated up to four, then
-        the ids of its blocks, [block-row of the line][gathered block-column], or the other way round)"""
-        t = torch.arange(self.n_tiles)
-        line = torch.repeat_interleave(torch.arange(self.heads * self.lines), self.sizes)
-        cols = self.cols if self.cols.size(1) == 4 else torch.cat((self.cols, self.cols[:, -1:].expand(-1, 4 - self.cols.size(1))), 1)
-        ids = self.ids.transpose(1, 2) if transposed_ids else self.ids
-        return torch.cat((torch.stack((t, torch.zeros_like(t), line % self.lines, line // self.lines), 1), cols,
-                          ids.reshape(self.n_tiles, -1).to(torch.int64)), 1)
-
-
-KV_PART_BLOCKS = 16         # columns of more blocks than this (and than twice the average column) are computed in parts of about this size
+        the ids of its blocks, [block-row of the line][gathered block-column])"""
+        return self._entries
 
 
 class _ColumnTable:
@@ -75,68 +72,24 @@ class _ColumnTable:
     items: per item twelve ints (entries, offset of its entries, head, column, slot of its partial sums or -1, 0, 0, 0, then
     the column's block-columns, the last repeated up to four), then the entries, a column's by row.  Blocks of 64: a
     column is a block-column, an entry (id, row, column, head); the ids are the positions in the row-major order of the
-    nonzero blocks, as everywhere.  Smaller blocks: a column is S block-columns (the long ones of a head together, the others
-    with their neighbours), its entries the tiles
+    nonzero blocks, as everywhere.  Smaller blocks: a column is S block-columns whose blocks lie in the same block-rows as
+    far as possible, so that the block-rows gathered into a tile hold blocks in most of them (the long ones of a head
+    together, longest first, the others as they lie: neighbours share their rows in banded layouts), its entries the tiles
     of _GatheredTiles over the transposed layout (S block-rows gathered per tile): 8 + S * S ints, the last S * S the ids
-    of the tile's blocks, [gathered block-row][block-column of the group].  A column of more than `part`
-    entries is cut into parts of near-equal size, each with a slot; split: per such column eight ints (head, column,
-    first slot, parts, then its block-columns)."""
+    of the tile's blocks, [gathered block-row][block-column of the group].  A column of more than `part` entries (None: 16
+    and twice the average, every part costs a slot written and read) is cut into parts of near-equal size, each with a slot;
+    split: per such column eight ints (head, column, first slot, parts, then its block-columns)."""
 
     def __init__(self, layout, device, part=None, S=1, ids=None):
-        lay = (layout != 0).cpu()
-        H, R, C = lay.shape
-        if S == 1:
-            h, r, c = lay.nonzero().unbind(1)
-            col = h * C + c
-            order = torch.argsort(col * R + r)
-            sizes = torch.bincount(col, minlength=H * C)
-            starts = torch.cumsum(sizes, 0) - sizes
-            entries = torch.stack((order, r[order], c[order], h[order]), 1)
-            groups = torch.arange(H * C).reshape(H * C, 1) % C
-        else:
-            # a column of tiles: S block-columns whose blocks lie in the same block-rows as far as possible, so that the
-            # block-rows gathered into a tile hold blocks in most of them: first the long block-columns of the head (more
-            # than four times the median: the global columns of a layout), longest first, then the others as they lie
-            # (neighbours share their rows in banded layouts)
-            layT, idsT = lay.transpose(1, 2), ids.transpose(1, 2)
-            length = layT.sum(-1)                                                         # [H, C]
-            is_long = length > 4 * length.float().median(dim=1, keepdim=True).values.clamp(min=1)
-            key = torch.where(is_long, -length.double() - 2.0 * R, torch.arange(C, dtype=torch.float64)[None].expand_as(length))
-            order = torch.argsort(key, dim=1, stable=True)                                # [H, C]
-            pick = order[:, :, None].expand(-1, -1, R)
-            g = _GatheredTiles(torch.gather(layT, 1, pick), torch.gather(idsT, 1, pick), S)
-            C = C // S
-            # an entry carries the ids of its tile's blocks, [gathered block-row][block-column of the group]
-            sizes, starts, entries = g.sizes, g.starts, g.entries(transposed_ids=True)
-            groups = order.reshape(H * C, S)
-        groups = torch.cat((groups, groups[:, -1:].expand(-1, 4 - groups.size(1))), 1) if groups.size(1) < 4 else groups
-        if part is None:
-            # only columns that stand out are cut (every part costs a slot written and read): those of more than twice the
-            # average length
-            part = max(KV_PART_BLOCKS, -(-2 * int(sizes.sum()) // max(1, H * C)))
-        parts = torch.clamp((sizes + part - 1) // part, min=1)
-        first_item = torch.cumsum(parts, 0) - parts
-        item_col = torch.repeat_interleave(torch.arange(H * C), parts)
-        n_items = int(item_col.numel())
-        k = torch.arange(n_items) - first_item[item_col]
-        base, rem = sizes[item_col] // parts[item_col], sizes[item_col] % parts[item_col]
-        count = base + (k < rem).long()
-        begin = starts[item_col] + k * base + torch.minimum(k, rem)
-        is_part = parts[item_col] > 1
-        slot = torch.where(is_part, torch.cumsum(is_part.long(), 0) - 1, torch.full_like(count, -1))
-        zero = torch.zeros_like(count)
-        header = torch.cat((torch.stack((count, 12 * n_items + entries.size(1) * begin, item_col // C, item_col % C, slot, zero, zero, zero), 1),
-                            groups[item_col]), 1).reshape(-1)
-        self.items = torch.cat((header, entries.reshape(-1))).to(torch.int32).to(device)
-        self.n_items = n_items
-        self.columns = C
-        self.n_slots = int(is_part.sum())
-        long_cols = (parts > 1).nonzero().flatten()
-        self.n_split = int(long_cols.numel())
-        self.split = None
-        if self.n_split:
-            self.split = torch.cat((torch.stack((long_cols // C, long_cols % C, slot[first_item[long_cols]], parts[long_cols]), 1),
-                                    groups[long_cols]), 1).reshape(-1).to(torch.int32).to(device)
+        self._take(*_stored_tables(layout, 64 // S, ids, part or 0), device)
+
+    def _take(self, host, info, device):
+        """the columns' part of the tables, in one piece on `device`; -> all of it there"""
+        tables = host.to(device)
+        self.items = tables[info.items_offset:info.split_offset]
+        self.split = tables[info.split_offset:] if info.n_split else None
+        self.columns, self.n_items, self.n_slots, self.n_split = info.columns, info.n_items, info.n_slots, info.n_split
+        return tables
 
 
 class _QuadTables:
@@ -187,7 +140,6 @@ class AttentionCore:
         self.dsd_tn = MatMul(layout, block, 'dsd', trans_a=True, trans_b=False)
         self.nnz = None
         self._tables = dict()
-        self._quad = dict()
 
     def blocks(self):
         if self.nnz is None:
@@ -196,37 +148,32 @@ class AttentionCore:
 
     def quad(self, device):
         """the tables of the kernels without sparse tensors on `device`, or None when the layout does not divide into tiles"""
-        key = str(device)
-        if key not in self._quad:
-            S = 64 // self.block
-            self._quad[key] = None if self.spdims[1] % S or self.spdims[2] % S else _QuadTables(self.layout, self.block, device)
-        return self._quad[key]
+        return self._made(device)[0]
 
     def tables(self, device):
         """(table, longest row, None, rows of the table's layout, present blocks per present tile as a share,
         tables of the column kernel) on `device`, or None when the layout does not divide into 64 x 64 tiles: what the kernels
         that store p need"""
+        return self._made(device)[1]
+
+    def _made(self, device):
+        """Both sets of tables: a call with per-element masks and one without need different ones, and either may be the one
+        that is captured after a warm-up step of the other kind."""
         key = str(device)
         if key not in self._tables:
             S = 64 // self.block
             H, R, C = self.spdims
-            if S == 1:
-                lut, maxlut = self.softmax.make_lut(device)
-                self._tables[key] = (lut, maxlut, None, R, 1., _ColumnTable(self.layout, device))
-            elif R % S or C % S:
-                self._tables[key] = None
+            if R % S or C % S:
+                self._tables[key] = (None, None)
             else:
-                # tiles of 64 x 64 with gathered block-columns (rows: forward and the row kernel of the backward pass) and with
-                # gathered block-rows (the column kernel): each view has its own tiles; p lives in the small blocks either way
-                lay = (self.layout != 0).cpu()
-                ids = torch.full(lay.shape, -1, dtype=torch.int32)
-                ids[lay] = torch.arange(int(lay.sum()), dtype=torch.int32)
-                g = _GatheredTiles(lay, ids, S)
-                header = torch.stack((g.sizes, 2 * g.sizes.numel() + (8 + S * S) * g.starts), 1).reshape(-1)
-                lut = torch.cat((header, g.entries().reshape(-1))).to(torch.int32).to(device)
-                maxlut = int(g.sizes.max()) if g.n_tiles else 0
-                ct = _ColumnTable(self.layout, device, S=S, ids=ids)
-                self._tables[key] = (lut, maxlut, None, R // S, self.blocks() / max(1, g.n_tiles * S * S), ct)
+                lay = (self.layout != 0).cpu().contiguous()
+                self.nnz = int(torch.count_nonzero(lay))
+                host, info = _stored_tables(lay, self.block)
+                columns = _ColumnTable.__new__(_ColumnTable)
+                lut = columns._take(host, info, device)
+                n_tiles = (info.items_offset - 2 * H * info.lines) // (4 if S == 1 else 8 + S * S)
+                stored = (lut, info.longest_line, None, info.lines, self.blocks() / max(1, n_tiles * S * S), columns)
+                self._tables[key] = (_QuadTables(lay, self.block, device), stored)
         return self._tables[key]
 
     def usable(self, q, k, v, dropout_p=0.):

@@ -265,3 +265,37 @@ def test_capture_of_the_kind_of_call_that_the_warm_up_was_not(block, masked_firs
         torch.cuda.synchronize()
         for name, a, b in zip(('o', 'dq', 'dk', 'dv'), static_out, eager):
             assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize('which', ['do over positions', 'k of one position', 'odd address', 'odd stride of a single batch', 'rows apart', 'overlapping rows'])
+@pytest.mark.parametrize('masked', [False, True])
+def test_operands_that_the_kernels_cannot_address_are_copied(which, masked):
+    """Tensors that are contiguous or aligned in the wrong way, or whose rows overlap (a gradient that reaches every position
+    through a sum has rows 0 apart), against the same values in memory of their own."""
+    torch.manual_seed(5)
+    Z, L, d = (1 if 'batch' in which else 2), 256, 64
+    lay = torch.tril(torch.ones(2, L // 32, L // 32)).long()
+    q, k, v, do = [torch.randn(Z, 2, L, d, device=DEV).half() for _ in range(4)]
+    if which == 'do over positions':
+        do = torch.randn(Z, 2, d, device=DEV).half()[:, :, None].expand(-1, -1, L, -1)
+    elif which == 'k of one position':
+        k = k[:, :, :1].expand(-1, -1, L, -1)
+    elif which == 'odd address':
+        q, do = [torch.randn(Z * 2 * L * d + 1, device=DEV).half()[1:].view(Z, 2, L, d) for _ in range(2)]
+    elif which == 'odd stride of a single batch':
+        v, do = [t.as_strided(t.shape, (2 * L * d + 3,) + t.stride()[1:]) for t in (v, do)]
+    elif which == 'rows apart':
+        q, k, v, do = [torch.randn(Z, L, 2, 3 * d, device=DEV).half()[..., d:2 * d].transpose(1, 2) for _ in range(4)]
+    else:
+        v = torch.randn(Z * 2 * L * 32 + 32, device=DEV).half().as_strided((Z, 2, L, d), (2 * L * 32, L * 32, 32, 1))
+    kw = dict(scale=0.125, rpe=(0.3 * torch.randn(L, L, device=DEV)).half()) if masked else dict(scale=0.125)
+
+    def grads(q, k, v, do):
+        ops = (tb.MatMul(lay, 32, 'sdd', trans_b=True), tb.Softmax(lay, 32), tb.MatMul(lay, 32, 'dsd'))
+        ts = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        before = ac.fused_calls
+        o = ac.attention_chain(*ops, *ts, **kw)
+        assert ac.fused_calls == before + 1
+        return (o,) + torch.autograd.grad(o, ts, do)
+    for name, a, b in zip(('o', 'dq', 'dk', 'dv'), grads(q, k, v, do), grads(*[t.clone(memory_format=torch.contiguous_format) for t in (q, k, v, do)])):
+        assert torch.equal(a, b), name

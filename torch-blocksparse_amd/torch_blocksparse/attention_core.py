@@ -113,17 +113,23 @@ class _QuadTables:
 
 
 def _vec_ok(t):
-    """16-byte vector accesses: unit inner stride, every other stride a multiple of 8 elements, aligned base."""
-    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1])
+    """16-byte vector accesses: unit inner stride, every other stride a multiple of 8 elements, aligned base, rows that do not
+    overlap (a gradient expanded along the positions has rows 0 apart)."""
+    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.stride(2) >= t.size(3)
+
+
+def _packed(t):
+    """a copy in storage of its own (contiguous() returns a tensor at an odd address, or of batch size 1 with an odd stride, as it is)"""
+    return t.clone(memory_format=torch.contiguous_format)
 
 
 def _vec(t):
-    return t if _vec_ok(t) else t.contiguous()
+    return t if _vec_ok(t) else _packed(t)
 
 
 def _near(t):
     """... and the rows of a head within 4 GiB of its first, as the kernels without sparse tensors address them"""
-    return t if _vec_ok(t) and t.stride(2) * t.size(2) * t.element_size() < 2 ** 32 else t.contiguous()
+    return t if _vec_ok(t) and t.stride(2) * t.size(2) * t.element_size() < 2 ** 32 else _packed(t)
 
 
 class AttentionCore:

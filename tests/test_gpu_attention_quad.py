@@ -299,3 +299,29 @@ def test_operands_that_the_kernels_cannot_address_are_copied(which, masked):
         return (o,) + torch.autograd.grad(o, ts, do)
     for name, a, b in zip(('o', 'dq', 'dk', 'dv'), grads(q, k, v, do), grads(*[t.clone(memory_format=torch.contiguous_format) for t in (q, k, v, do)])):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize('d,dtype,block', [(64, torch.float16, 64), (128, torch.bfloat16, 64), (64, torch.bfloat16, 16)])
+def test_operands_far_apart_in_memory(d, dtype, block):
+    """Rows 2.9 MB apart, so that the last ones of the tensors that are fetched tile by tile lie just below 4 GiB from the first: byte
+    offsets beyond 2^31, and the largest row stride that 1472 positions allow."""
+    torch.manual_seed(d + block)
+    L = 1472
+    ld = 2 ** 32 // (2 * L) // 8 * 8
+    assert 2 * L * ld < 2 ** 32 <= 2 * L * (ld + 8)
+    lay = (torch.rand(2, L // block, L // block) < 0.3).long()
+    lay[:, :, 0] = lay[:, :, -1] = 1
+    buf = torch.empty(L * ld, device=DEV, dtype=dtype)
+    near = [torch.randn(1, 2, L, d, device=DEV).to(dtype) for _ in range(4)]
+    far = [buf.as_strided((1, 2, L, d), (16, 4 * d, ld, 1), i * d) for i in range(4)]
+    for f, n in zip(far, near):
+        f.copy_(n)
+    core = ac.AttentionCore(lay, block)
+    results = []
+    for q, k, v, do in (far, near):
+        assert all(ac._near(t) is t for t in (q, k, v, do))
+        ts = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        o = core(*ts, scale=d ** -0.5)
+        results.append((o,) + torch.autograd.grad(o, ts, do))
+    for name, a, b in zip(('o', 'dq', 'dk', 'dv'), *results):
+        assert torch.equal(a, b), name

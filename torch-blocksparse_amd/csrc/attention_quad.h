@@ -380,7 +380,7 @@ inline int quad_check(int dtype, int D, const void *const *ptrs, int n_ptrs, con
   for (int i = 0; i < n_strides; i++)
     if (strides[i] % 8) return BSP_ERR_ARG;
   for (int i = 0; i < n_lds; i++)
-    if (lds[i] < D || (i < loaded && (positions <= 0 || lds[i] >= ((int64_t)1 << 32) / (2 * positions)))) return BSP_ERR_ARG;
+    if (lds[i] < D || (i < loaded && (positions <= 0 || lds[i] > (((int64_t)1 << 32) - 1) / (2 * positions)))) return BSP_ERR_ARG;
   return BSP_OK;
 }
 

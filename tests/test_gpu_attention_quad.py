@@ -325,3 +325,24 @@ def test_operands_far_apart_in_memory(d, dtype, block):
         results.append((o,) + torch.autograd.grad(o, ts, do))
     for name, a, b in zip(('o', 'dq', 'dk', 'dv'), *results):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize('layout_of', [lambda m: m, lambda m: m[:1], lambda m: torch.cat((m, m), 1)[:, :256], lambda m: m[0].expand(2, -1),
+                                       lambda m: torch.cat((m, m), 1)[:, :260]])
+def test_a_mask_buffer_may_be_refilled_before_the_backward_pass(layout_of):
+    torch.manual_seed(6)
+    lay = torch.tril(torch.ones(2, 4, 4)).long()
+    q, k, v, do = [torch.randn(2, 2, 256, 64, device=DEV).half() for _ in range(4)]
+    mask = torch.zeros(2, 256, device=DEV).half()
+    mask[0, 3:40] = float('-inf')
+    mask = layout_of(mask)
+    results = []
+    for refill in (False, True):
+        core = ac.AttentionCore(lay, 64)
+        ts = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        o = core(*ts, scale=0.125, key_padding_mask=mask)
+        if refill:
+            (mask if mask.stride(0) or mask.size(0) == 1 else mask[0]).fill_(1.)
+        results.append((o.detach(),) + torch.autograd.grad(o, ts, do))
+    for name, a, b in zip(('o', 'dq', 'dk', 'dv'), *results):
+        assert torch.equal(a, b), name

@@ -239,6 +239,8 @@ class _attention_quad(torch.autograd.Function):
         kpm = None
         if key_padding_mask is not None:                   # element (z, c), softmax.py:60-62, 274
             kpm = _sparse_softmax._strided16(key_padding_mask, 'key_padding_mask')
+            if keep and kpm.data_ptr() == key_padding_mask.data_ptr():
+                kpm = _packed(kpm[:, :k.size(2)])          # the backward pass reads it again, the caller may fill it with the next mask until then
         ctx.kpm_args = (kpm.stride(0) if kpm is not None and kpm.size(0) > 1 else 0, int(kp_mask_mode == 'mul'))
         o = torch.empty((Z, H, R * core.block, D), dtype=q.dtype, device=q.device)
         lse = torch.empty((Z, H, 2, lines * 64), dtype=torch.float32, device=q.device) if keep else None      # (and what its rounding left out)

@@ -321,8 +321,11 @@ template <typename T, int N> __device__ __forceinline__ void negate(typename Mma
   }
 }
 
-// |scale| in the log2 domain; not zero, so that -inf stays -inf
-__device__ __forceinline__ float logit_scale(float scale) { return fmaxf(fabsf(scale) * kLog2e, 1e-30f); }
+// |scale| in the log2 domain; not zero, so that -inf stays -inf; what is not a number stays that
+__device__ __forceinline__ float logit_scale(float scale) {
+  const float s = fabsf(scale) * kLog2e;
+  return s < 1e-30f ? 1e-30f : s;
+}
 
 // A row's lse = m + log2 l has the precision of m: where the maximum is far from zero (finite padding values of -10000 or
 // -65504 on every key that the row sees, large scores) the sum rounds log2 l away, and exp2(logit - lse) would not add up to

@@ -360,3 +360,29 @@ def test_a_scale_that_is_not_a_number(block, kpm):
     assert bool(torch.isnan(o[:, 0]).all()) and bool(torch.isnan(o[:, 1, :-block]).all()) and not bool(o[:, 1, -block:].any())
     for g in torch.autograd.grad(o, (q, k, v), torch.ones_like(o)):
         assert bool(torch.isnan(g[:, 0]).all())
+
+
+@pytest.mark.parametrize('which', ['dq', 'dk'])
+@pytest.mark.parametrize('block,d,scale', [(64, 64, 8.), (16, 64, -8.), (32, 128, 64.), (64, 64, 1e5)])
+def test_small_gradients_under_a_scale_above_one(which, block, d, scale):
+    """fp16 gradients so small that ds without the scale lies in the subnormals.  ds with it is rounded in steps of 2^-24 there, an
+    error of 2^-24 / sqrt(12) an element that the product takes on as relative to its root mean square; beside it the result's own
+    rounding, 2^-11 or half a step of 2^-24, and of what ds is made of."""
+    torch.manual_seed(d)
+    L = 512
+    lay = torch.ones(2, L // block, L // block, dtype=torch.int64)
+    small = 0.64 / (abs(scale) * d ** 0.5)                # scores of about 0.64, so that the shares are spread
+    q, k = torch.randn(1, 2, L, d, device=DEV), torch.randn(1, 2, L, d, device=DEV)
+    q, k = (q * small, k) if which == 'dq' else (q, k * small)
+    v, do = torch.randn(1, 2, L, d, device=DEV), torch.randn(1, 2, L, d, device=DEV) * 2. ** -12 / min(abs(scale), 64.)
+    q, k, v, do = [t.half() for t in (q, k, v, do)]
+    got = _run(lay, block, q, k, v, do, scale=scale)[1 if which == 'dq' else 2].double()
+    Q, K, V, dO = [t.double() for t in (q, k, v, do)]
+    P = torch.softmax(Q @ K.transpose(2, 3).contiguous() * scale, -1)
+    dP = dO @ V.transpose(2, 3).contiguous()
+    dS = P * (dP - (P * dP).sum(-1, keepdim=True)) * scale
+    ref = dS @ K if which == 'dq' else dS.transpose(2, 3).contiguous() @ Q
+    step, rms = 2. ** -24 / 12 ** 0.5, lambda t: float(t.pow(2).mean().sqrt())
+    assert 4 * rms(dS) / abs(scale) < 2. ** -14 and rms(ref) > 2. ** -16
+    bound = step / rms(dS) + step / rms(ref) + 3 * 2. ** -11
+    assert float((got - ref).norm() / ref.norm()) < 1.25 * bound

@@ -2,8 +2,8 @@
 // the row's lse (its rounding: row_rest), the softmax gradient from it, dp = do . v^T and delta = sum_d do_d o_d (= sum_j p_j dp_j, because o = p . v
 // and dp = do . v^T; softmax.py:189, matmul.py:587-606):
 //     ds = p * (dp - delta) * scale,   dq = ds . k,   dk = ds^T . q,   dv = p^T . do.
-// The scale is applied to the sums dq and dk: as an operand p (dp - delta) stays below half of the largest |dp| (it is at most
-// p (1 - p) times the difference of two dp), so it fits the storage type wherever dp itself does.
+// A scale of at most 1 is applied to the sums dq and dk: as an operand p (dp - delta) stays below half of the largest |dp| (it is
+// at most p (1 - p) times the difference of two dp), so it fits the storage type wherever dp itself does.  (Larger: scale_place.)
 //   row kernel    : a line of tiles per workgroup -> dq and delta
 //   column kernel : a column of tiles (or a part of a long one) per workgroup -> dk and dv
 // The two together read q, k, v, do twice and o once; a stored p would be written once and read twice, and is larger
@@ -55,6 +55,8 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 2) k_attn_bwd_rows(QuadArgs
     frag_t xq[D / 16];
     load_operand<T, D>(xq, reinterpret_cast<const T *>(a.q) + z * a.q_sz + h * a.q_sh + row * a.q_ld + 8 * half);
     if (a.scale < 0.f) negate<T>(xq);
+    const bool shifted = __is_same(T, f16) && a.ds_shift != 0.f;
+    const float shift = __builtin_amdgcn_exp2f(a.ds_shift);
     const float sc = logit_scale(a.scale), lse = a.lse[((int64_t)z * a.H + h) * a.row_sh + row];
     const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const T *>(a.k) + z * a.k_sz + h * a.k_sh);
     const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const T *>(a.v) + z * a.v_sz + h * a.v_sh);
@@ -101,8 +103,11 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 2) k_attn_bwd_rows(QuadArgs
       for_16<0>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
         const float p = __builtin_amdgcn_exp2f(fmaf(raw[i], sc, KPM ? row_bcast<i>(kp) - lse : -lse));
-        e[i] = p * (dp[i] - delta);                     // (the scale comes last, on dq)
+        e[i] = p * (dp[i] - delta);
       });
+      if (shifted)                                      // (the rest of the scale comes last, on dq)
+#pragma unroll
+        for (int i = 0; i < 16; i++) e[i] *= shift;
       frag_t df[2];
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) df[ks] = pack8<T>(reinterpret_cast<const float (&)[8]>(e[8 * ks]));
@@ -113,7 +118,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 2) k_attn_bwd_rows(QuadArgs
       step(Const<1>{}, n + 1);
     }
   }
-  const float last = a.rest ? a.scale * __builtin_amdgcn_exp2f(-a.lse[((int64_t)z * a.H + h) * a.row_sh + a.rest + row]) : a.scale;
+  const float last = a.rest ? a.sum_scale * __builtin_amdgcn_exp2f(-a.lse[((int64_t)z * a.H + h) * a.row_sh + a.rest + row]) : a.sum_scale;
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -143,6 +148,8 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
   const int steps = head[0] * 2, h = head[2], slot = head[4];
   const table_ptr core = lut + head[1];
   const int64_t key_lo = head[8 + 2 * wave], key_hi = head[8 + 2 * wave + 1];
+  const bool shifted = __is_same(T, f16) && a.ds_shift != 0.f;
+  const float shift = __builtin_amdgcn_exp2f(a.ds_shift), unshift = __builtin_amdgcn_exp2f(-a.ds_shift);
   f32x16 dk[MT], dv[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
@@ -216,6 +223,9 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
           for (int i = 0; i < 4; i++) p[4 * g + i] *= __builtin_amdgcn_exp2f(-rest[i]);
         }
       }
+      if (shifted)                                      // (dv is scaled back at the end)
+#pragma unroll
+        for (int i = 0; i < 16; i++) p[i] *= shift;
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) pf[ks] = pack8<T>(reinterpret_cast<const float (&)[8]>(p[8 * ks]));
       if (holes) {
@@ -232,7 +242,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
       }
       dp = row_product<T, D, O0>(smem, rows, xv, dp);
 #pragma unroll
-      for (int i = 0; i < 16; i++) e[i] = p[i] * dp[i]; // (the scale comes last, on dk)
+      for (int i = 0; i < 16; i++) e[i] = p[i] * dp[i]; // (the rest of the scale comes last, on dk)
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) df[ks] = pack8<T>(reinterpret_cast<const float (&)[8]>(e[8 * ks]));
       if (LEAN || holes) {                              // (a branch here costs registers that the wide head does not have)
@@ -250,7 +260,10 @@ __global__ void __launch_bounds__(128, D == 64 ? 3 : 2) k_attn_bwd_cols(QuadArgs
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-    for (int i = 0; i < 16; i++) dk[mt][i] *= a.scale;
+    for (int i = 0; i < 16; i++) {
+      dk[mt][i] *= a.sum_scale;
+      if constexpr (__is_same(T, f16)) dv[mt][i] *= unshift;
+    }
   if (slot >= 0) {                                      // a part of a long column: fp32 sums to its slot [dk, dv][64 keys][D]
     float *ws = a.partial + ((int64_t)z * a.n_slots + slot) * (2 * 64 * D) + (32 * wave + l32) * D + 4 * half;
 #pragma unroll
@@ -348,6 +361,7 @@ extern "C" int bsp_attention_rows_bwd(int dtype, const void *d_o, const void *q,
   a.oin_sz = o_stride_z; a.oin_sh = o_stride_h; a.oin_ld = ldo;
   a.o_sz = dq_stride_z; a.o_sh = dq_stride_h; a.o_ld = lddq;
   a.scale = scale; a.lut = d_lut;
+  scale_place(a, dtype);
   a.kpm = kpm; a.kpm_sz = kpm_stride_z; a.kpm_mul = kpm_mul;
   a.Z = Z; a.H = H; a.R = R;
   const int rl = dtype == BSP_F16 ? launch_t<f16>(a, D, false, as_stream(stream)) : launch_t<bf16>(a, D, false, as_stream(stream));
@@ -384,7 +398,8 @@ extern "C" int bsp_attention_cols_bwd(int dtype, const void *d_o, const void *q,
   a.v_sz = v_stride_z; a.v_sh = v_stride_h; a.v_ld = ldv;
   a.o_sz = dk_stride_z; a.o_sh = dk_stride_h; a.o_ld = lddk;
   a.o2_sz = dv_stride_z; a.o2_sh = dv_stride_h; a.o2_ld = lddv;
-  a.scale = scale; a.lut = d_items; a.partial = partial; a.n_slots = n_slots; a.split_lut = d_split; a.n_split = n_split;
+  a.scale = scale; scale_place(a, dtype);
+  a.lut = d_items; a.partial = partial; a.n_slots = n_slots; a.split_lut = d_split; a.n_split = n_split;
   a.kpm = kpm; a.kpm_sz = kpm_stride_z; a.kpm_mul = kpm_mul;
   a.Z = Z; a.H = H; a.R = n_items;
   const int rl = dtype == BSP_F16 ? launch_t<f16>(a, D, true, as_stream(stream)) : launch_t<bf16>(a, D, true, as_stream(stream));

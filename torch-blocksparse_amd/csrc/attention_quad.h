@@ -26,6 +26,7 @@
 #ifndef BSP_ATTENTION_QUAD_H
 #define BSP_ATTENTION_QUAD_H
 #include "attention_common.h"
+#include <cmath>
 
 namespace bsp {
 
@@ -38,6 +39,7 @@ struct QuadArgs {
   int64_t q_sz, q_sh, q_ld, k_sz, k_sh, k_ld, v_sz, v_sh, v_ld, do_sz, do_sh, do_ld, oin_sz, oin_sh, oin_ld;
   int64_t o_sz, o_sh, o_ld, o2_sz, o2_sh, o2_ld;
   float scale;
+  float ds_shift, sum_scale;       // the scale's place in the backward pass, 2^ds_shift in ds and the rest on its sums: scale_place
   const int32_t *lut;
   const void *kpm; int64_t kpm_sz; int kpm_mul;
   float *partial;                  // column kernel: slots of the parts of long columns, [Z][n_slots][dk, dv][64][D]
@@ -370,6 +372,16 @@ template <typename T, int D> __device__ __forceinline__ void store_32_rows(T *st
     __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(stage + r * (D + 8) + 8 * ch), reinterpret_cast<u32x4 *>(dst));
   }
   __builtin_amdgcn_wave_barrier();
+}
+
+// ds = p (dp - delta) scale is rounded to the storage type.  Up to 1 the scale is left to the sums dq and dk: without it ds has
+// the range of dp.  Above, ds without it could fall into the subnormals where with it, as the operators round it, it does not:
+// its power of two goes in first (with p: exact, and no more than 2^14 of it, which fp16 holds).  bf16 has no such values.
+inline void scale_place(QuadArgs &a, int dtype) {
+  const float s = fabsf(a.scale);
+  const int shift = dtype == BSP_F16 && s >= 2.f ? (s < 16384.f ? ilogbf(s) : 14) : 0;
+  a.ds_shift = (float)shift;
+  a.sum_scale = ldexpf(a.scale, -shift);
 }
 
 // What the launchers check: types and sizes, 16-byte alignment of every pointer (NULL is aligned) and stride, and that the

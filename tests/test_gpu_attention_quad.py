@@ -386,3 +386,21 @@ def test_small_gradients_under_a_scale_above_one(which, block, d, scale):
     assert 4 * rms(dS) / abs(scale) < 2. ** -14 and rms(ref) > 2. ** -16
     bound = step / rms(dS) + step / rms(ref) + 3 * 2. ** -11
     assert float((got - ref).norm() / ref.norm()) < 1.25 * bound
+
+
+@pytest.mark.parametrize('masks', [(), ('key_padding_mask',), ('rpe',)])
+def test_under_a_non_reentrant_checkpoint(masks):
+    """which lets a backward pass unpack what was saved once"""
+    from torch.utils.checkpoint import checkpoint
+    torch.manual_seed(8)
+    core = ac.AttentionCore(torch.tril(torch.ones(2, 4, 4)).long(), 64)
+    q, k, v, do = [torch.randn(2, 2, 256, 64, device=DEV).half() for _ in range(4)]
+    values = dict(key_padding_mask=(0.5 * torch.randn(2, 256, device=DEV)).half(), rpe=(0.3 * torch.randn(256, 256, device=DEV)).half())
+    kw = dict(scale=0.125, **{m: values[m] for m in masks})
+    results = []
+    for wrap in (lambda f, *ts: f(*ts), lambda f, *ts: checkpoint(f, *ts, use_reentrant=False)):
+        ts = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        o = wrap(lambda a, b, c: core(a, b, c, **kw), *ts)
+        results.append((o.detach(),) + torch.autograd.grad(o, ts, do))
+    for name, a, b in zip(('o', 'dq', 'dk', 'dv'), *results):
+        assert torch.equal(a, b), name

@@ -256,9 +256,9 @@ class _attention_quad(torch.autograd.Function):
         return o
 
     @staticmethod
-    def rows_kernel(ctx, do, delta):
+    def rows_kernel(ctx, saved, do, delta):
         """dq, and into delta (if given) the negative of the rows' sums sum_d do . o"""
-        q, k, v, o, lse, kpm = ctx.saved_tensors
+        q, k, v, o, lse, kpm = saved
         Z, H, D = q.size(0), q.size(1), q.size(3)
         dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
         rc = _lib.load().bsp_attention_rows_bwd(
@@ -270,9 +270,9 @@ class _attention_quad(torch.autograd.Function):
         return dq
 
     @staticmethod
-    def columns_kernel(ctx, do, delta):
+    def columns_kernel(ctx, saved, do, delta):
         """dk and dv"""
-        q, k, v, o, lse, kpm = ctx.saved_tensors
+        q, k, v, o, lse, kpm = saved
         Z, H, D = q.size(0), q.size(1), q.size(3)
         ct = ctx.tables
         dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
@@ -288,9 +288,9 @@ class _attention_quad(torch.autograd.Function):
         return dk, dv
 
     @staticmethod
-    def through_stored_gradient(ctx, do):
+    def through_stored_gradient(ctx, saved, do):
         """dk and dv the other way (FUSED_KV = False): softmax and softmax gradient as sparse tensors, then the two dsd operators"""
-        q, k, v, o, lse, kpm = ctx.saved_tensors
+        q, k, v, o, lse, kpm = saved
         core = ctx.core
         lut, maxlut, _, lines = core.tables(q.device)[:4]
         stored = _StoredSoftmax()
@@ -302,7 +302,8 @@ class _attention_quad(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, do):
-        q = ctx.saved_tensors[0]
+        saved = ctx.saved_tensors                          # (unpacked once: non-reentrant checkpoints allow no more)
+        q = saved[0]
         do = _near(do)
         need_q, need_k, need_v = ctx.needs_input_grad[:3]
         dq = dk = dv = None
@@ -313,9 +314,9 @@ class _attention_quad(torch.autograd.Function):
         elif need_v and FUSED_KV:
             delta = torch.zeros(rows, dtype=torch.float32, device=q.device)        # (dk is computed beside dv, and dropped)
         if need_q or need_k:
-            dq = _attention_quad.rows_kernel(ctx, do, delta if need_k else None)
+            dq = _attention_quad.rows_kernel(ctx, saved, do, delta if need_k else None)
         if need_k or need_v:
-            dk, dv = _attention_quad.columns_kernel(ctx, do, delta) if FUSED_KV else _attention_quad.through_stored_gradient(ctx, do)
+            dk, dv = _attention_quad.columns_kernel(ctx, saved, do, delta) if FUSED_KV else _attention_quad.through_stored_gradient(ctx, saved, do)
         return (dq if need_q else None, dk if need_k else None, dv if need_v else None) + (None,) * 5
 
 
@@ -368,9 +369,9 @@ class _attention_core(torch.autograd.Function):
         return o
 
     @staticmethod
-    def rows_kernel(ctx, do, ds, delta):
+    def rows_kernel(ctx, do, ds, delta, saved=None):
         """dq; with it the softmax gradient ds (if a tensor is given) and / or the rows' sums delta = sum_d do . o"""
-        q, k, v, p, o, lut = ctx.saved_tensors
+        q, k, v, p, o, lut = saved or ctx.saved_tensors
         core = ctx.core
         Z, H, D = q.size(0), q.size(1), q.size(3)
         dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
@@ -384,9 +385,9 @@ class _attention_core(torch.autograd.Function):
         return dq
 
     @staticmethod
-    def columns_kernel(ctx, do, delta):
+    def columns_kernel(ctx, do, delta, saved=None):
         """dk and dv, the softmax gradient computed again from p and delta"""
-        q, k, v, p, o, lut = ctx.saved_tensors
+        q, k, v, p, o, lut = saved or ctx.saved_tensors
         Z, H, D = q.size(0), q.size(1), q.size(3)
         ct = ctx.columns
         dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
@@ -403,7 +404,8 @@ class _attention_core(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, do):
-        q, k, v, p, o, lut = ctx.saved_tensors
+        saved = ctx.saved_tensors                          # (unpacked once, as above)
+        q, k, v, p, o, lut = saved
         core = ctx.core
         do = _vec(do)
         need_q, need_k, need_v = ctx.needs_input_grad[:3]
@@ -411,17 +413,17 @@ class _attention_core(torch.autograd.Function):
         if need_k and FUSED_KV:
             # two launches: rows (dq, delta), then columns (dk and dv)
             delta = torch.empty((q.size(0), q.size(1), ctx.rows * 64), dtype=torch.float32, device=q.device)
-            dq = _attention_core.rows_kernel(ctx, do, None, delta)
-            dk, dv = _attention_core.columns_kernel(ctx, do, delta)
+            dq = _attention_core.rows_kernel(ctx, do, None, delta, saved)
+            dk, dv = _attention_core.columns_kernel(ctx, do, delta, saved)
         else:
             if need_v:
                 dv = core.dsd_tn(p, do)                    # p^T . do, as the dsd operator's backward does (matmul.py:598-601)
             if need_k:
                 ds = torch.empty_like(p)
-                dq = _attention_core.rows_kernel(ctx, do, ds, None)
+                dq = _attention_core.rows_kernel(ctx, do, ds, None, saved)
                 dk = core.dsd_tn(ds, q)                    # ds^T . q (matmul.py:598-601 of the sdd operator)
             elif need_q:
-                dq = _attention_core.rows_kernel(ctx, do, None, None)
+                dq = _attention_core.rows_kernel(ctx, do, None, None, saved)
         return (dq if need_q else None, dk, dv if need_v else None) + (None,) * 11
 
 

@@ -404,3 +404,24 @@ def test_under_a_non_reentrant_checkpoint(masks):
         results.append((o.detach(),) + torch.autograd.grad(o, ts, do))
     for name, a, b in zip(('o', 'dq', 'dk', 'dv'), *results):
         assert torch.equal(a, b), name
+
+
+def test_stored_gradient_way_computes_what_is_asked_for(monkeypatch):
+    """FUSED_KV = False: one product for one gradient, the same values as where both are asked for"""
+    torch.manual_seed(9)
+    core = ac.AttentionCore(torch.tril(torch.ones(2, 4, 4)).long(), 64)
+    q, k, v, do = [torch.randn(1, 2, 256, 64, device=DEV).half() for _ in range(4)]
+    monkeypatch.setattr(ac, 'FUSED_KV', False)
+    products, dsd = [], core.dsd_tn
+    monkeypatch.setattr(core, 'dsd_tn', lambda *a: (products.append(a), dsd(*a))[1])
+
+    def grads(need):
+        ts = [t.clone().requires_grad_(n) for t, n in zip((q, k, v), need)]
+        del products[:]
+        core(*ts, scale=0.125).backward(do)
+        assert len(products) == need[1] + need[2]
+        return [t.grad for t in ts]
+    full = grads((True, True, True))
+    for need in ((False, False, True), (False, True, False), (True, False, False), (True, False, True)):
+        for n, g, f in zip(need, grads(need), full):
+            assert (g is not None) == n and (not n or torch.equal(g, f))

@@ -288,17 +288,23 @@ class _attention_quad(torch.autograd.Function):
         return dk, dv
 
     @staticmethod
-    def through_stored_gradient(ctx, saved, do):
-        """dk and dv the other way (FUSED_KV = False): softmax and softmax gradient as sparse tensors, then the two dsd operators"""
+    def through_stored_gradient(ctx, saved, do, need_k, need_v):
+        """dk and dv the other way (FUSED_KV = False): softmax and softmax gradient as sparse tensors, then the dsd operators; each
+        only where its result is asked for"""
         q, k, v, o, lse, kpm = saved
         core = ctx.core
         lut, maxlut, _, lines = core.tables(q.device)[:4]
         stored = _StoredSoftmax()
         _attention_core.forward(stored, q, k, v, ctx.scale, None, kpm, None, ctx.kp_mask_mode, 'add', core, lut, maxlut, True, lines)
         p = stored.saved_tensors[3]
-        ds = torch.empty_like(p)
-        _attention_core.rows_kernel(stored, do, ds, None)
-        return core.dsd_tn(ds, q), core.dsd_tn(p, do)      # ds^T . q and p^T . do, as the operators' backward passes do (matmul.py:598-601)
+        dk = dv = None
+        if need_k:
+            ds = torch.empty_like(p)
+            _attention_core.rows_kernel(stored, do, ds, None)
+            dk = core.dsd_tn(ds, q)                        # ds^T . q and p^T . do, as the operators' backward passes do (matmul.py:598-601)
+        if need_v:
+            dv = core.dsd_tn(p, do)
+        return dk, dv
 
     @staticmethod
     def backward(ctx, do):
@@ -316,7 +322,8 @@ class _attention_quad(torch.autograd.Function):
         if need_q or need_k:
             dq = _attention_quad.rows_kernel(ctx, saved, do, delta if need_k else None)
         if need_k or need_v:
-            dk, dv = _attention_quad.columns_kernel(ctx, saved, do, delta) if FUSED_KV else _attention_quad.through_stored_gradient(ctx, saved, do)
+            dk, dv = (_attention_quad.columns_kernel(ctx, saved, do, delta) if FUSED_KV else
+                      _attention_quad.through_stored_gradient(ctx, saved, do, need_k, need_v))
         return (dq if need_q else None, dk if need_k else None, dv if need_v else None) + (None,) * 5
 
 

@@ -352,14 +352,12 @@ def test_a_mask_buffer_may_be_refilled_before_the_backward_pass(layout_of):
 def test_a_scale_that_is_not_a_number(block, kpm):
     torch.manual_seed(7)
     lay = torch.tril(torch.ones(2, 256 // block, 256 // block)).long()
-    lay[1, -1] = 0                                       # block-row without a block, alone in its line or beside others
     q, k, v = [torch.randn(2, 2, 256, 64, device=DEV).half().requires_grad_(True) for _ in range(3)]
     kw = dict(key_padding_mask=torch.zeros(2, 256, device=DEV).half()) if kpm else {}
     core = ac.AttentionCore(lay, block)
     o = core(q, k, v, scale=float('nan'), **kw)
-    assert bool(torch.isnan(o[:, 0]).all()) and bool(torch.isnan(o[:, 1, :-block]).all()) and not bool(o[:, 1, -block:].any())
-    for g in torch.autograd.grad(o, (q, k, v), torch.ones_like(o)):
-        assert bool(torch.isnan(g[:, 0]).all())
+    for t in (o,) + torch.autograd.grad(o, (q, k, v), torch.ones_like(o)):
+        assert bool(torch.isnan(t).all())
 
 
 @pytest.mark.parametrize('which', ['dq', 'dk'])

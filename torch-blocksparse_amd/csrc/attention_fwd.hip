@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 3) k_attn_fwd(QuadArgs a) {
 
   l += swap32(l);
   const bool any_block = (rows_seen >> 4 * ((lane >> 4) & 1)) & 15;
-  const float inv = 1.f / l;                            // masked everywhere: 0 * inf = NaN, as the softmax operator gives; no block at all: zeros
+  const float inv = any_block ? 1.f / l : 0.f;          // masked everywhere: 0 * inf = NaN, as the softmax operator gives; no block at all: zeros
   if (a.lse != nullptr && half == 0) {
     const float log_l = __builtin_amdgcn_logf(l), lse = m + log_l;
     float *to = a.lse + ((int64_t)z * a.H + h) * a.row_sh + row;
@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(128, D == 64 ? 4 : 3) k_attn_fwd(QuadArgs a) {
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-    for (int i = 0; i < 16; i++) o[mt][i] = any_block ? o[mt][i] * inv : 0.f;
+    for (int i = 0; i < 16; i++) o[mt][i] *= inv;
   quad_barrier();                                       // the ring is free
   T *po = reinterpret_cast<T *>(a.o) + z * a.o_sz + h * a.o_sh + ((int64_t)line * 64 + 32 * wave) * a.o_ld;
   store_32_rows<T, D>(reinterpret_cast<T *>(smem) + wave * 32 * (D + 8), po, po + 16 * a.o_ld, a.o_ld, o, lane);

@@ -258,11 +258,11 @@ __device__ __forceinline__ f32x16 row_product(const unsigned char *smem, const R
 
 // BYTES (4 or 16) a lane from base + add (the same in all lanes) + off straight to LDS byte dst + BYTES * lane.  As assembly,
 // because the compiler cannot tell which stage such a load fills: before every LDS read behind it, it would wait for the
-// load to land.  The only wait is the one in front of a stage's barrier (quad_barrier).  (Nothing else here uses m0.)
+// load to land.  The only wait is the one in front of a stage's barrier (quad_barrier).
 template <int BYTES> __device__ __forceinline__ void load_to_lds(const char *base, uint32_t off, uint32_t add, uint32_t dst) {
   uint32_t at;                                            // (the addition also is the instruction that must lie between m0 and its use)
-  if constexpr (BYTES == 16) asm volatile("s_mov_b32 m0, %4\n\tv_add_u32 %0, %2, %1\n\tglobal_load_lds_dwordx4 %0, %3" : "=&v"(at) : "v"(off), "s"(add), "s"(base), "s"(dst) : "memory");
-  else asm volatile("s_mov_b32 m0, %4\n\tv_add_u32 %0, %2, %1\n\tglobal_load_lds_dword %0, %3" : "=&v"(at) : "v"(off), "s"(add), "s"(base), "s"(dst) : "memory");
+  if constexpr (BYTES == 16) asm volatile("s_mov_b32 m0, %4\n\tv_add_u32 %0, %2, %1\n\tglobal_load_lds_dwordx4 %0, %3" : "=&v"(at) : "v"(off), "s"(add), "s"(base), "s"(dst) : "m0", "memory");
+  else asm volatile("s_mov_b32 m0, %4\n\tv_add_u32 %0, %2, %1\n\tglobal_load_lds_dword %0, %3" : "=&v"(at) : "v"(off), "s"(add), "s"(base), "s"(dst) : "m0", "memory");
 }
 // the positions of the two groups of half n of a line's (column's) tiles
 struct Groups { int lo, hi; };

@@ -55,7 +55,7 @@ constexpr int kStages = 3;
 // same reason: 299 us in the general kernel, 270 here at block 64, 231 and 210 at 128.
 __device__ __forceinline__ void load_lds16(const void *base, uint32_t off, const unsigned char *dst) {
   const uint32_t at = (uint32_t)(uintptr_t)((const void __attribute__((address_space(3))) *)dst);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(at) : "memory");   // (nothing else in these kernels uses m0)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(at) : "m0", "memory");
 }
 template <int N> struct Const { static constexpr int value = N; };
 // step(stage, s) for s = 0 .. n - 1, the stage (s modulo the ring's length) a compile-time constant: the LDS addresses of a

@@ -24,6 +24,8 @@ def test_ring_and_table_windows(mode, block, Z, trans_a, trans_b):
     dtype = torch.float16 if trans_a == trans_b else torch.bfloat16
     lines, free = _lines(), 2048 - 24                          # (the last tile of the free dimension is not full)
     K = 66 * block
+    tiles = -(-free // 256) * Z                                # the sizes from which the library takes the wide kernels
+    assert 16 // 4 * tiles >= 384 if block == 32 else 16 * tiles > 512
     # the sparse operand as stored: dsd op(A) is [lines, reduction], dds op(B) is [reduction, lines]
     stored = lines if (mode == 'dsd') != (trans_a if mode == 'dsd' else trans_b) else lines.t()
     lay = stored.contiguous()[None]
@@ -61,6 +63,7 @@ def test_first_wide_launch_under_capture():
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         whole = dot(sp, dn)                                                  # 384
+    assert 64 // 4 * (1024 // 256) * 6 == 384 and dot.make_lut(sp.dtype, sp.device)[0].gplan_wide is None
     for _ in range(3):
         whole.zero_()
         graph.replay()
@@ -68,3 +71,39 @@ def test_first_wide_launch_under_capture():
         # the same products in another order of their fp32 sums: one unit of the 16-bit result
         assert bool(((whole.float() - parts.float()).abs() <= 2. ** -10 * parts.float().abs() + 2. ** -12).all())
     torch.testing.assert_close(dot(sp, dn), whole, rtol=2. ** -10, atol=2. ** -12)
+    assert dot.make_lut(sp.dtype, sp.device)[0].gplan_wide is not None
+
+
+@pytest.mark.parametrize('mode,block,trans_a,trans_b', [
+    ('dsd', 64, False, False), ('dsd', 128, False, True), ('dsd', 64, True, False), ('dds', 64, False, False), ('dds', 128, True, False),
+    ('sdd', 32, False, True), ('sdd', 32, True, False), ('sdd', 16, False, True)])
+def test_operands_beyond_the_reach_of_the_wide_kernels(mode, block, trans_a, trans_b):
+    """Dense rows so far apart that a tile's byte offsets leave 32 bits: the general kernels take the launch."""
+    torch.manual_seed(block)
+    M, N, K = (256, 256, 256)
+    ld = 2 ** 31 // (128 if mode == 'sdd' else 256) + 64
+    shape = (M if mode == 'sdd' else K, K if mode == 'sdd' else N)
+    lay = (torch.rand(1, shape[0] // block if mode == 'sdd' else M // block, (N if mode == 'sdd' else K) // block) < 0.6).long()
+    lay[0, :, 0] = lay[0, 0, :] = 1
+    far = torch.empty(256 * ld, device='cuda', dtype=torch.float16).as_strided((1, 1, 256, 256), (8, 8, ld, 1))
+    far.copy_(torch.randn(256, 256, device='cuda').half())
+    sp = torch.randn(1, int(lay.sum()), block, block, device='cuda').half()
+    dn = torch.randn(1, 1, 256, 256, device='cuda').half()
+    a, b = {'sdd': (far, dn), 'dsd': (sp, far), 'dds': (far, sp)}[mode]
+    got = tb.MatMul(lay, block, mode, trans_a=trans_a, trans_b=trans_b)(a, b).float()
+    h, r, c = lay.nonzero().unbind(1)
+
+    def full(t):
+        if t is not sp:
+            return t.float().contiguous()
+        x = torch.zeros(1, 1, 256 // block, 256 // block, block, block, device='cuda')
+        x[:, h, r, c] = sp.float()
+        return x.transpose(3, 4).reshape(1, 1, 256, 256)
+    x, y = full(a), full(b)
+    x, y = (x.transpose(2, 3) if trans_a else x).contiguous(), (y.transpose(2, 3) if trans_b else y).contiguous()
+    ref, terms = torch.matmul(x, y), torch.matmul(x.abs(), y.abs())
+    if mode == 'sdd':
+        blocks = lambda t: t.reshape(1, 1, 256 // block, block, 256 // block, block).transpose(3, 4)[:, h, r, c]
+        ref, terms = blocks(ref), blocks(terms)
+    bound = 2. ** -11 * ref.abs() + 2 * K * 2. ** -24 * terms + 2. ** -24      # as above
+    assert got.shape == ref.shape and bool(((got - ref).abs() <= bound).all()), (got - ref).abs().max().item()

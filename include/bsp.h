@@ -340,10 +340,13 @@ int bsp_attention_bwd_kv(int dtype, const void *d_o, const void *q, const void *
                          const int32_t *d_split_lut, int n_split, void *stream);
 
 /* The same chain without any sparse tensor in memory, for calls without relative position embedding and attention mask:
- * o = softmax(q . k^T * scale + key-padding term) . v and its three gradients, rows and columns of any length.  What the
- * backward pass needs of the softmax is one fp32 per row, lse = log2 of the row's sum of exponentials (of the logits in
+ * o = softmax(round(q . k^T) * scale + key-padding term) . v and its three gradients, rows and columns of any length.  What
+ * the backward pass needs of the softmax is one fp32 per row, lse = log2 of the row's sum of exponentials (of the logits in
  * the log2 domain; +inf for a row without any block), from which the backward kernels compute the probabilities again.
- * Scores and probabilities are not rounded between the steps except where they become an operand of a product.
+ * round() is the rounding of the scores to the storage type that the sdd operator does when it stores them (in fp16 a product
+ * beyond 65504 is infinite), in all three kernels; probabilities and ds are rounded where they become an operand of a
+ * product, dp = do . v^T is not.  In fp16 a scale of 2 or more enters ds before that rounding with its power of two (2^14 at
+ * most), everywhere else dq and dk after it.
  *
  * Tables (bsp_attention_tables_build makes them): a tile is 64 rows by 64 columns, each side four groups of sixteen consecutive positions
  * anywhere in the matrix; its entry is eight ints: the positions of the four groups of the side the tile gathers, a

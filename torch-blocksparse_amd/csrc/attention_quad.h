@@ -10,10 +10,11 @@
 //
 // Work split.  A workgroup is two wavefronts, each with 32 of the 64 rows of its line (keys of its column), which walk the
 // tiles of the line (column) in halves of 32 columns (rows), MFMA 32x32x16: nothing is exchanged between the wavefronts at
-// the end and a barrier joins two of them.  What these kernels wait for is the vector unit (it computes in 60 % of the
-// cycles, the matrix cores in 40 %, the LDS in 20 %), so what counts is instructions per score and wavefronts to hide their
-// latencies: with 16 KiB of LDS a workgroup at head dimension 64 the registers decide, four wavefronts per SIMD (three in
-// the column kernel).  Measured on the self-attention module's default configuration (block 16, stride 64, 8 x 16 heads x
+// the end and a barrier joins two of them.  What these kernels wait for is the vector unit: on the self-attention module's
+// default configuration it computes in 58 / 51 / 42 % of the cycles (forward / rows / columns), the matrix cores in
+// 31 / 38 / 38 %, the LDS in 18 / 21 / 32 % (counters: profiles/attention_units.txt).  So what counts is instructions per score
+// and wavefronts to hide their latencies: with 16 KiB of LDS a workgroup at head dimension 64 the registers decide, four
+// wavefronts per SIMD (three in the column kernel).  Measured on that configuration (block 16, stride 64, 8 x 16 heads x
 // 4096, forward / rows / columns): 124 / 161 / 262 us; whole tiles per stage, so 32 KiB and 2.5 wavefronts per SIMD:
 // 148 / 177 / 284; four wavefronts with a 32 x 32 quadrant of the tile each, which add partial results up at the end:
 // 155 / 190 / 288.

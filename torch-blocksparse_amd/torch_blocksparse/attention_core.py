@@ -3,8 +3,10 @@
 The reference's modules call three operators, sparse_dot_sdd_nt(q, k), sparse_softmax(...), sparse_dot_dsd_nn(p, v)
 (deepspeedsparseselfattention.py:152-157; attention.py:190-202).  `attention_chain` takes the same three operator
 objects and the same arguments and returns the same context tensor; when the operators are this package's, built on
-one layout with blocks of 16, 32 or 64, and the tensors are fp16 / bf16 with a head dimension of 64 or 128, it runs the fused
-kernels (bsp_attention_fwd / bsp_attention_bwd) instead: the scores stay in registers between the three steps.
+one layout with blocks of 16, 32 or 64, and the tensors are fp16 / bf16 with a head dimension of 64 or 128, it runs fused
+kernels instead.  Without relative position embedding and attention mask no sparse tensor exists (bsp_attention_rows_fwd,
+bsp_attention_rows_bwd, bsp_attention_cols_bwd: class _attention_quad); with one of them the softmax is stored for the backward pass
+(bsp_attention_fwd, bsp_attention_bwd, bsp_attention_bwd_kv: class _attention_core).
 In every other case, and with FUSED = False, it calls the three operators one after the other.
 """
 import ctypes
@@ -19,11 +21,9 @@ from .softmax import Softmax, _sparse_softmax
 FUSED = os.environ.get('BSP_FUSED_ATTENTION', '1') != '0'
 MAX_ROW_BLOCKS = 8          # BSP_ATTENTION_MAX_ROW_BLOCKS: longer rows are streamed (the library decides)
 fused_calls = 0             # forward calls that took the fused kernels; tests read it
-# dk and dv from the column kernel (bsp_attention_bwd_kv), which computes the softmax gradient again instead of reading it;
-# False: the row kernel stores the gradient and the two products are ordinary dsd operators
+# dk and dv from a column kernel (bsp_attention_cols_bwd, bsp_attention_bwd_kv), which computes the softmax gradient again instead
+# of reading it; False: the row kernel stores the gradient and the two products are ordinary dsd operators
 FUSED_KV = os.environ.get('BSP_FUSED_ATTENTION_KV', '1') != '0'
-
-
 
 
 def _stored_tables(layout, block, ids=None, part=0):
@@ -113,9 +113,10 @@ class _QuadTables:
 
 
 def _vec_ok(t):
-    """16-byte vector accesses: unit inner stride, every other stride a multiple of 8 elements, aligned base, rows that do not
-    overlap (a gradient expanded along the positions has rows 0 apart)."""
-    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.stride(2) >= t.size(3)
+    """16-byte vector accesses of a 4-dimensional tensor: unit inner stride, every other stride a multiple of 8 elements, aligned
+    base, rows that do not overlap (a gradient expanded along the positions has rows 0 apart)."""
+    z, h, row, inner = t.stride()
+    return inner == 1 and not (z | h | row) % 8 and row >= t.size(3) and not t.data_ptr() % 16
 
 
 def _packed(t):
@@ -133,16 +134,14 @@ def _near(t):
 
 
 class AttentionCore:
-    """What the fused kernels need beside the tensors: the softmax table of the layout (for blocks of 16 or 32: the table
-    of its 64 x 64 tiles with gathered block-columns and the ids of each tile's blocks), the tables of the column
-    kernel, and the two products that are ordinary operators in the backward pass when the column kernel is not used
-    (dv = p^T . do and dk = ds^T . q)."""
+    """What the fused kernels need beside the tensors: the tables of the layout's 64 x 64 tiles along lines of rows and along
+    columns, for the kernels without sparse tensors and for those that store the softmax, and the two products that are
+    ordinary operators in the backward pass when the column kernel is not used (dv = p^T . do and dk = ds^T . q)."""
 
-    def __init__(self, layout, block, softmax=None):
+    def __init__(self, layout, block):
         self.layout = layout
         self.block = block
         self.spdims = tuple(layout.shape)
-        self.softmax = softmax if softmax is not None else Softmax(layout, block)
         self.dsd_tn = MatMul(layout, block, 'dsd', trans_a=True, trans_b=False)
         self.nnz = None
         self._tables = dict()
@@ -154,33 +153,31 @@ class AttentionCore:
 
     def quad(self, device):
         """the tables of the kernels without sparse tensors on `device`, or None when the layout does not divide into tiles"""
-        return self._made(device)[0]
+        return (self._tables.get(str(device)) or self._made(device))[0]
 
     def tables(self, device):
         """(table, longest row, None, rows of the table's layout, present blocks per present tile as a share,
         tables of the column kernel) on `device`, or None when the layout does not divide into 64 x 64 tiles: what the kernels
         that store p need"""
-        return self._made(device)[1]
+        return (self._tables.get(str(device)) or self._made(device))[1]
 
     def _made(self, device):
         """Both sets of tables: a call with per-element masks and one without need different ones, and either may be the one
         that is captured after a warm-up step of the other kind."""
-        key = str(device)
-        if key not in self._tables:
-            S = 64 // self.block
-            H, R, C = self.spdims
-            if R % S or C % S:
-                self._tables[key] = (None, None)
-            else:
-                lay = (self.layout != 0).cpu().contiguous()
-                self.nnz = int(torch.count_nonzero(lay))
-                host, info = _stored_tables(lay, self.block)
-                columns = _ColumnTable.__new__(_ColumnTable)
-                lut = columns._take(host, info, device)
-                n_tiles = (info.items_offset - 2 * H * info.lines) // (4 if S == 1 else 8 + S * S)
-                stored = (lut, info.longest_line, None, info.lines, self.blocks() / max(1, n_tiles * S * S), columns)
-                self._tables[key] = (_QuadTables(lay, self.block, device), stored)
-        return self._tables[key]
+        S = 64 // self.block
+        H, R, C = self.spdims
+        made = (None, None)
+        if not (R % S or C % S):
+            lay = (self.layout != 0).cpu().contiguous()
+            self.nnz = int(torch.count_nonzero(lay))
+            host, info = _stored_tables(lay, self.block)
+            columns = _ColumnTable.__new__(_ColumnTable)
+            lut = columns._take(host, info, device)
+            n_tiles = (info.items_offset - 2 * H * info.lines) // (4 if S == 1 else 8 + S * S)
+            made = (_QuadTables(lay, self.block, device),
+                    (lut, info.longest_line, None, info.lines, self.blocks() / max(1, n_tiles * S * S), columns))
+        self._tables[str(device)] = made
+        return made
 
     def usable(self, q, k, v, dropout_p=0.):
         """Can this call take the fused kernels?  (Shapes that do not fit the layout are left to the operators, which
@@ -446,7 +443,7 @@ def _core_for(sdd_nt, softmax, dsd_nn):
     if ok:
         for other in (sdd_nt.layout, dsd_nn.layout):
             ok = ok and (other is softmax.layout or (other.shape == softmax.layout.shape and bool((other == softmax.layout).all())))
-    made = AttentionCore(softmax.layout, softmax.block, softmax) if ok else None
+    made = AttentionCore(softmax.layout, softmax.block) if ok else None
     softmax._attention_core = (sdd_nt, dsd_nn, made)
     return made
 

@@ -260,9 +260,9 @@ def main():
                 e1.synchronize()
                 return e0.elapsed_time(e1) / reps
             out['fused_attention_chain'] = {
-                'what': 'attention_chain(sdd, softmax, dsd, q, k, v): bsp_attention_fwd, then in the backward pass bsp_attention_bwd (dq) '
-                        'and bsp_attention_bwd_kv (dk, dv; the softmax gradient is computed twice and never stored); same workload, '
-                        'flop count of the six products of the three-operator chain',
+                'what': 'attention_chain(sdd, softmax, dsd, q, k, v): bsp_attention_rows_fwd, then in the backward pass bsp_attention_rows_bwd '
+                        '(dq) and bsp_attention_cols_bwd (dk, dv); no sparse tensor is stored, scores and softmax are computed again in both; '
+                        'same workload, flop count of the six products of the three-operator chain',
                 'ms_per_step': round(ms_fused, 4), 'TFLOP/s': round(6 * w.flops_mm / ms_fused * 1e-9, 3),
                 'vs_three_operators': round(ms_per_step / ms_fused, 3),
                 'launches': fused_chain_launches(w.lay, w.q.detach(), w.k.detach(), w.v.detach(), w.do, w.scale, timeit,
@@ -389,12 +389,14 @@ def launch_roofline(kernel, flops, nbytes, ms, peak_tflops=MFMA_PEAK_TFLOPS):
             'flop_per_byte': round(flops / nbytes, 1), 'traffic': None}
 
 
-def xsd_kernel_name(block, dtype_bits, free_dim, sp_trans, dn_kc):
-    """Which kernel the library's dispatch gives a dsd/dds launch (csrc/capi.hip xsd_dispatch, in its order)."""
+def xsd_kernel_name(block, dtype_bits, free_dim, sp_trans, dn_kc, lines, Z):
+    """Which kernel the library's dispatch gives a dsd/dds launch over `lines` block-rows (block-columns) of all heads (csrc/capi.hip
+    xsd_dispatch, in its order)."""
     if dtype_bits == 16 and free_dim >= 256:
-        if block == 32 and dn_kc:
+        tiles = (free_dim + 255) // 256 * Z
+        if block == 32 and (lines + 3) // 4 * tiles >= 384:
             return 'k_xsd_rg_dl'
-        if block in (64, 128) and not (sp_trans and dn_kc):
+        if block == 128 or (block == 64 and not (dn_kc and lines * tiles <= 512)):
             return 'k_xsd_dl<%d>' % block
     if dtype_bits == 16 and not dn_kc and free_dim % 64 == 0:
         if block == 64:
@@ -407,50 +409,57 @@ def xsd_kernel_name(block, dtype_bits, free_dim, sp_trans, dn_kc):
 
 
 def fused_chain_launches(lay, q, k, v, do, scale, timeit, variants, block=64):
-    """The fused attention kernels (bsp_attention_fwd / bsp_attention_bwd: what the attention modules launch instead of
-    sdd -> softmax -> dsd when block, dtype and head dimension allow), each timed on its own through the C ABI.
-    variants: [(label, softmax keyword arguments)] for the forward kernel.  Algorithmic bytes: forward q, k, v, o and
-    the sparse p once each; backward rows do, o, v, k, dq and the sparse p once each, backward columns do, q, v, dk, dv and p (masks: what the layout touches
-    is counted by the caller's softmax figures, not here)."""
+    """The fused attention kernels (what the attention modules launch instead of sdd -> softmax -> dsd when block, dtype and head
+    dimension allow), each timed on its own through the C ABI.  variants: [(label, softmax keyword arguments)].  Without
+    rpe and attention mask the kernels that keep no sparse tensor (bsp_attention_rows_fwd, _rows_bwd, _cols_bwd), with the
+    products that they compute (2, 3 and 4, the scores again in each) and as bytes what they read and write of the dense
+    tensors; with them those that store p (bsp_attention_fwd, _bwd, _bwd_kv): forward q, k, v, o and p once each; backward
+    rows do, o, v, k, dq and p once each, backward columns do, q, v, dk, dv and p (masks: what the layout touches is counted by
+    the caller's softmax figures, not here)."""
     import torch
     from torch_blocksparse import attention_core as ac
     core = ac.AttentionCore(lay, block)
     B, H, L, dh = q.shape
-    nnz = core.blocks()
     dense = q.numel() * q.element_size()
-    xb = B * nnz * block * block * q.element_size()
+    elems = B * core.blocks() * block * block
+    p_bytes, product = elems * q.element_size(), 2.0 * elems * dh
     out = []
-    state = {}
+
+    def entry(label, kernel, f, flops, nbytes):
+        with torch.no_grad():
+            ms = timeit(f)
+        out.append({'launch': label, 'ms': round(ms, 4), 'GB/s': round(nbytes / ms * 1e-6, 1),
+                    'hbm_frac': round(nbytes / ms * 1e-6 / HBM_PEAK_GBS, 4), 'roofline': launch_roofline(kernel, flops, nbytes, ms)})
+
+    def parts(ct):       # the partial sums of the long columns' parts: written, read
+        return 2 * B * ct.n_slots * 2 * 64 * dh * 4
     for label, kw in variants:
-        def fwd():
-            with torch.no_grad():
-                state['o'] = ac._attention_core.forward(state.setdefault('ctx', _Ctx()), q, k, v, float(scale), kw.get('rpe'), kw.get('key_padding_mask'),
-                                                        kw.get('attn_mask'), kw.get('key_padding_mask_mode', 'add'), kw.get('attn_mask_mode', 'add'),
-                                                        core, *_fwd_tables(core, q.device))
-        ms = timeit(fwd)
-        nbytes = 4 * dense + xb
-        out.append({'launch': 'fused forward: q.k^T, softmax, p.v (%s)' % label, 'ms': round(ms, 4), 'GB/s': round(nbytes / ms * 1e-6, 1),
-                    'hbm_frac': round(nbytes / ms * 1e-6 / HBM_PEAK_GBS, 4), 'roofline': launch_roofline('k_attn64_fwd', 0, nbytes, ms)})
-    ctx = state['ctx']
-    delta = torch.empty((B, H, ctx.rows * 64), dtype=torch.float32, device=q.device)
-
-    def rows():
-        with torch.no_grad():
-            ac._attention_core.rows_kernel(ctx, do, None, delta)
-    ms = timeit(rows)
-    nbytes = 5 * dense + xb
-    out.append({'launch': 'fused backward, rows: do.v^T, softmax gradient, ds.k -> dq', 'ms': round(ms, 4), 'GB/s': round(nbytes / ms * 1e-6, 1),
-                'hbm_frac': round(nbytes / ms * 1e-6 / HBM_PEAK_GBS, 4), 'roofline': launch_roofline('k_attn64_bwd', 0, nbytes, ms)})
-
-    def columns():
-        with torch.no_grad():
-            ac._attention_core.columns_kernel(ctx, do, delta)
-    ms = timeit(columns)
-    ct = ctx.columns
-    nbytes = 5 * dense + xb + 2 * B * ct.n_slots * 2 * 64 * dh * 4      # (the partial sums of the long columns' parts: written, read)
-    out.append({'launch': 'fused backward, columns: softmax gradient again, p^T.do -> dv, ds^T.q -> dk (%d of %d columns in parts)' % (ct.n_split, H * ct.columns),
-                'ms': round(ms, 4), 'GB/s': round(nbytes / ms * 1e-6, 1),
-                'hbm_frac': round(nbytes / ms * 1e-6 / HBM_PEAK_GBS, 4), 'roofline': launch_roofline('k_attn64_bwd_kv', 0, nbytes, ms)})
+        ctx = _Ctx()
+        if kw.get('rpe') is None and kw.get('attn_mask') is None:
+            fn = ac._attention_quad
+            entry('fused forward: q.k^T, softmax, p.v (%s)' % label, 'k_attn_fwd',
+                  lambda: fn.forward(ctx, q, k, v, float(scale), kw.get('key_padding_mask'), kw.get('key_padding_mask_mode', 'add'), core, True),
+                  2 * product, 4 * dense)
+            saved, ct = ctx.saved_tensors, ctx.tables
+            delta = torch.empty((B, H, 2, ct.lines * 64), dtype=torch.float32, device=q.device)
+            entry('fused backward, rows: softmax again, do.v^T, ds.k -> dq (%s)' % label, 'k_attn_bwd_rows',
+                  lambda: fn.rows_kernel(ctx, saved, do, delta), 3 * product, 6 * dense)
+            entry('fused backward, columns: softmax and its gradient again, p^T.do -> dv, ds^T.q -> dk (%s; %d of %d columns in parts)'
+                  % (label, ct.n_split, H * ct.columns), 'k_attn_bwd_cols',
+                  lambda: fn.columns_kernel(ctx, saved, do, delta), 4 * product, 6 * dense + parts(ct))
+        else:
+            fn = ac._attention_core
+            entry('fused forward with stored p: q.k^T, softmax, p.v (%s)' % label, 'k_attn64_fwd',
+                  lambda: fn.forward(ctx, q, k, v, float(scale), kw.get('rpe'), kw.get('key_padding_mask'), kw.get('attn_mask'),
+                                     kw.get('key_padding_mask_mode', 'add'), kw.get('attn_mask_mode', 'add'), core, *_fwd_tables(core, q.device)),
+                  0, 4 * dense + p_bytes)
+            ct = ctx.columns
+            delta = torch.empty((B, H, ctx.rows * 64), dtype=torch.float32, device=q.device)
+            entry('fused backward with stored p, rows: do.v^T, softmax gradient, ds.k -> dq', 'k_attn64_bwd',
+                  lambda: fn.rows_kernel(ctx, do, None, delta), 0, 5 * dense + p_bytes)
+            entry('fused backward with stored p, columns: softmax gradient again, p^T.do -> dv, ds^T.q -> dk (%d of %d columns in parts)'
+                  % (ct.n_split, H * ct.columns), 'k_attn64_bwd_kv',
+                  lambda: fn.columns_kernel(ctx, do, delta), 0, 5 * dense + p_bytes + parts(ct))
     return out
 
 
@@ -602,9 +611,9 @@ def other_config(config, steps, warmup):
                       'k_sdd64_rg' if (block in (16, 64) and bits == 16 and K in (64, 128) and not ta and tb_) else
                       'k_sdd_rg_small' if (block == 32 and bits == 16 and K == 64 and not ta and tb_) else 'k_sdd (general)')
         elif mode == 'dsd':      # kernel rows = rows of op(A); dense operand reduction-contiguous when B is read transposed
-            kernel = xsd_kernel_name(block, bits, N, ta, tb_)
+            kernel = xsd_kernel_name(block, bits, N, ta, tb_, H * M // block, Z)
         else:                    # dds = dsd on the transposed problem
-            kernel = xsd_kernel_name(block, bits, M, not tb_, not ta)
+            kernel = xsd_kernel_name(block, bits, M, not tb_, not ta, H * N // block, Z)
         out.append({'launch': name, 'ms': round(ms, 4), 'TFLOP/s': round(fl / ms * 1e-9, 2), 'mfma_frac': round(fl / ms * 1e-9 / peak, 4),
                     'GB/s': round(nbytes / ms * 1e-6, 1), 'hbm_frac': round(nbytes / ms * 1e-6 / HBM_PEAK_GBS, 4),
                     'roofline': launch_roofline(kernel, fl, nbytes, ms, peak)})
@@ -916,8 +925,8 @@ def record_traffic(fetch_dir, write_dir):
         ('k_sdd64_rg', ('k_sdd64_rg',)), ('k_xsd64_rg<sparse operand as stored>', ('k_xsd64_rg', 'Lb0E')),
         ('k_xsd64_rg<sparse operand transposed>', ('k_xsd64_rg', 'Lb1E')), ('k_softmax_fwd', ('k_softmax_fwd',)),
         ('k_softmax_bwd', ('k_softmax_bwd',)))}
-    for name in ('k_attn64_fwd', 'k_attn64_bwd', 'k_attn64_bwd_kv'):   # the fused chain of the attention modules, run after the headline step
-        for sub in (name + 'I', name + '<'):               # (the template's name as mangled or as written: k_attn64_bwd is not k_attn64_bwd_kv)
+    for name in ('k_attn_fwd', 'k_attn_bwd_rows', 'k_attn_bwd_cols'):   # the fused chain of the attention modules, run after the headline step
+        for sub in (name + 'I', name + '<'):               # (the template's name as mangled or as written: k_attn_bwd_cols is not k_attn_bwd_cols_sum)
             if any(sub in k for k in fetch) and any(sub in k for k in write):
                 per_kernel[name] = kernel_bytes(name, sub)
     rec = {'kernel_sources_sha256': kernel_sources_sha(), 'bytes_per_counted_KiB': {'FETCH_SIZE': round(fs, 1), 'WRITE_SIZE': round(ws, 1)},

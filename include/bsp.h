@@ -171,6 +171,15 @@ int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, int trans_a
                    const uint8_t *d_valid, int64_t n_groups, const int32_t *d_gplan, int n_plan_groups, int plan_lines, int flags,
                    void *stream);
 
+/* ... all pack levels of the table (n_levels <= 3, each pack width at most once) in one call: packs, d_luts, d_valids (entries may
+ * be NULL) and n_groups are host arrays with what a call of bsp_sdd_matmul per level would get.  Blocks of 16 and 32, which are
+ * the ones with several levels, run as a single launch. */
+int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, void *c, int trans_a, int trans_b, int Z, int K,
+                          int64_t a_stride_z, int64_t a_stride_h, int64_t lda, int64_t b_stride_z, int64_t b_stride_h,
+                          int64_t ldb, int64_t c_stride_z, int block, int n_levels, const int *packs, const int32_t *const *d_luts,
+                          const uint8_t *const *d_valids, const int64_t *n_groups, const int32_t *d_gplan, int n_plan_groups, int plan_lines,
+                          int flags, void *stream);
+
 /* sparse = dense x dense over a long reduction into few blocks of 128, the reduction cut into `parts` parts that run side by
  * side: replaces _sparse_matmul._sdd_matmul (matmul.py:299-364) where the reference would have used the split-K lock path of
  * its kernel (matmul.py:186-203; dead there, no locks or atomics here).  Blocks of 128 and 16-bit types only, K a multiple

@@ -34,13 +34,17 @@ extern "C" const char *bsp_strerror(int status) {
   }
 }
 
-extern "C" int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, int trans_a, int trans_b, int Z, int K,
-                              int64_t a_stride_z, int64_t a_stride_h, int64_t lda, int64_t b_stride_z, int64_t b_stride_h,
-                              int64_t ldb, int64_t c_stride_z, int block, int pack, const int32_t *d_lut,
-                              const uint8_t *d_valid, int64_t n_groups, const int32_t *d_gplan, int n_plan_groups,
-                              int plan_lines, int flags, void *stream) {
-  if (!a || !b || !c || Z <= 0 || K <= 0 || n_groups < 0) return BSP_ERR_ARG;
-  if (!d_lut && (!d_gplan || no_groups(flags) || general_only(flags))) return d_gplan ? BSP_NEEDS_TABLE : BSP_ERR_ARG;
+extern "C" int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, void *c, int trans_a, int trans_b, int Z, int K,
+                                     int64_t a_stride_z, int64_t a_stride_h, int64_t lda, int64_t b_stride_z, int64_t b_stride_h,
+                                     int64_t ldb, int64_t c_stride_z, int block, int n_levels, const int *packs, const int32_t *const *d_luts,
+                                     const uint8_t *const *d_valids, const int64_t *n_groups, const int32_t *d_gplan, int n_plan_groups,
+                                     int plan_lines, int flags, void *stream) {
+  if (!a || !b || !c || Z <= 0 || K <= 0 || n_levels < 1 || n_levels > 3 || !packs || !d_luts || !d_valids || !n_groups) return BSP_ERR_ARG;
+  SddLevel levels[3];
+  for (int i = 0; i < n_levels; i++) {
+    if (!d_luts[i] || n_groups[i] < 0) return BSP_ERR_ARG;
+    levels[i] = SddLevel{packs[i], d_luts[i], d_valids[i], n_groups[i]};
+  }
   if (!block_ok(block)) return BSP_ERR_UNSUPPORTED;
   if (K % 16) return BSP_ERR_K_MULTIPLE;   // reference matmul.py:318-319
   const int u = elems16(dtype);
@@ -50,36 +54,61 @@ extern "C" int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, 
   g.a = a; g.b = b; g.c = c; g.Z = Z; g.K = K;
   g.a_sz = a_stride_z; g.a_sh = a_stride_h; g.lda = lda;
   g.b_sz = b_stride_z; g.b_sh = b_stride_h; g.ldb = ldb; g.c_sz = c_stride_z;
-  g.lut = d_lut; g.valid = d_valid; g.n_groups = n_groups;
+  g.lut = levels[0].lut; g.valid = levels[0].valid; g.n_groups = levels[0].n;
   g.gplan = no_groups(flags) ? nullptr : d_gplan; g.n_pgroups = n_plan_groups; g.lines = plan_lines;
   if (g.gplan && (n_plan_groups <= 0 || plan_lines == 0)) return BSP_ERR_ARG;
+  if (rowpair(flags)) g.gplan = nullptr;   // a plan over pairs of block-rows serves the long-reduction kernel only
   // op(A)[m][k]: reduction contiguous unless A is read transposed; op(B)[k][n]: contiguous when B is read transposed
   const bool a_kc = !trans_a, b_kc = trans_b != 0;
   hipStream_t st = as_stream(stream);
-  int rc = 0;
-  if (!d_lut) {   // the plan alone: n_groups then carries an upper bound on the entries of a group (at most the block-columns of the layout)
-    g.cols = (int)n_groups; g.n_groups = 0;
-    rc = no_wide(flags) ? 0 : sdd_dl(dtype, g, block, rowpair(flags), a_kc, b_kc, st);
-    if (rc < 0) return rc;
-    if (rc == 2) { BSP_LAUNCH_CHECK(); return BSP_OK_WHOLE_LAYOUT; }
-  }
-  if (rowpair(flags)) {   // a plan over pairs of block-rows serves the long-reduction kernel only
-    if (!d_lut) return BSP_NEEDS_TABLE;
-    g.gplan = nullptr;
-  }
-  rc = general_only(flags) ? 0 : sdd_fast64(dtype, g, block, pack, a_kc, b_kc, st);
+  int rc = general_only(flags) ? 0 : sdd_fast64(dtype, g, block, packs[0], a_kc, b_kc, st);
   if (rc < 0) return rc;
+  // (a kernel that works from the plan writes the whole layout; the one for a single level serves blocks of 64, which have no other)
   if (rc >= 1) { BSP_LAUNCH_CHECK(); return rc == 2 ? BSP_OK_WHOLE_LAYOUT : BSP_OK; }
-  if (!d_lut) return BSP_NEEDS_TABLE;      // a call with the plan alone, and no kernel that works from the plan applies
   switch (dtype) {
-    case BSP_F16: rc = sdd_generic_f16(g, block, pack, a_kc, b_kc, st); break;
-    case BSP_BF16: rc = sdd_generic_bf16(g, block, pack, a_kc, b_kc, st); break;
-    case BSP_F32: rc = sdd_generic_f32(g, block, pack, a_kc, b_kc, st); break;
+    case BSP_F16: rc = sdd_generic_f16(g, block, levels, n_levels, a_kc, b_kc, st); break;
+    case BSP_BF16: rc = sdd_generic_bf16(g, block, levels, n_levels, a_kc, b_kc, st); break;
+    case BSP_F32: rc = sdd_generic_f32(g, block, levels, n_levels, a_kc, b_kc, st); break;
     default: return BSP_ERR_UNSUPPORTED;
   }
   if (rc != BSP_OK) return rc;
   BSP_LAUNCH_CHECK();
   return BSP_OK;
+}
+
+extern "C" int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, int trans_a, int trans_b, int Z, int K,
+                              int64_t a_stride_z, int64_t a_stride_h, int64_t lda, int64_t b_stride_z, int64_t b_stride_h,
+                              int64_t ldb, int64_t c_stride_z, int block, int pack, const int32_t *d_lut,
+                              const uint8_t *d_valid, int64_t n_groups, const int32_t *d_gplan, int n_plan_groups,
+                              int plan_lines, int flags, void *stream) {
+  if (d_lut)
+    return bsp_sdd_matmul_levels(dtype, a, b, c, trans_a, trans_b, Z, K, a_stride_z, a_stride_h, lda, b_stride_z, b_stride_h, ldb, c_stride_z, block,
+                                 1, &pack, &d_lut, &d_valid, &n_groups, d_gplan, n_plan_groups, plan_lines, flags, stream);
+  if (!a || !b || !c || Z <= 0 || K <= 0 || n_groups < 0) return BSP_ERR_ARG;
+  if (!d_gplan || no_groups(flags) || general_only(flags)) return d_gplan ? BSP_NEEDS_TABLE : BSP_ERR_ARG;
+  if (!block_ok(block)) return BSP_ERR_UNSUPPORTED;
+  if (K % 16) return BSP_ERR_K_MULTIPLE;   // reference matmul.py:318-319
+  const int u = elems16(dtype);
+  if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return BSP_ERR_ARG;
+  if (a_stride_z % u || a_stride_h % u || lda % u || b_stride_z % u || b_stride_h % u || ldb % u || c_stride_z % u) return BSP_ERR_ARG;
+  if (n_plan_groups <= 0 || plan_lines == 0) return BSP_ERR_ARG;
+  // the plan alone: n_groups then carries an upper bound on the entries of a group (at most the block-columns of the layout)
+  SddArgs g;
+  g.a = a; g.b = b; g.c = c; g.Z = Z; g.K = K;
+  g.a_sz = a_stride_z; g.a_sh = a_stride_h; g.lda = lda;
+  g.b_sz = b_stride_z; g.b_sh = b_stride_h; g.ldb = ldb; g.c_sz = c_stride_z;
+  g.lut = nullptr; g.valid = d_valid; g.n_groups = 0; g.cols = (int)n_groups;
+  g.gplan = d_gplan; g.n_pgroups = n_plan_groups; g.lines = plan_lines;
+  const bool a_kc = !trans_a, b_kc = trans_b != 0;
+  hipStream_t st = as_stream(stream);
+  int rc = no_wide(flags) ? 0 : sdd_dl(dtype, g, block, rowpair(flags), a_kc, b_kc, st);
+  if (rc < 0) return rc;
+  if (rc == 2) { BSP_LAUNCH_CHECK(); return BSP_OK_WHOLE_LAYOUT; }
+  if (rowpair(flags)) return BSP_NEEDS_TABLE;      // a plan over pairs of block-rows serves the long-reduction kernel only
+  rc = sdd_fast64(dtype, g, block, pack, a_kc, b_kc, st);
+  if (rc < 0) return rc;
+  if (rc >= 1) { BSP_LAUNCH_CHECK(); return rc == 2 ? BSP_OK_WHOLE_LAYOUT : BSP_OK; }
+  return BSP_NEEDS_TABLE;                          // no kernel that works from the plan applies
 }
 
 extern "C" int64_t bsp_sdd_splitk_workspace_bytes(int Z, int64_t n_groups, int parts) {

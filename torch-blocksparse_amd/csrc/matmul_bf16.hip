@@ -2,8 +2,8 @@
 // three compiles parallel).
 #include "matmul_generic.h"
 namespace bsp {
-int sdd_generic_bf16(const SddArgs &g, int block, int pack, bool a_kc, bool b_kc, hipStream_t st) {
-  return launch_sdd<bf16>(g, block, pack, a_kc, b_kc, st);
+int sdd_generic_bf16(const SddArgs &g, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st) {
+  return launch_sdd<bf16>(g, block, levels, n_levels, a_kc, b_kc, st);
 }
 int xsd_generic_bf16(const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
   return launch_xsd<bf16>(g, block, sp_trans, dn_kc, out_nc, st);

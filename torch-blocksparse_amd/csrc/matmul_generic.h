@@ -198,7 +198,7 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
   // the epilogue then writes block by block.  SUB == 0: the output is a matrix with long rows.
   template <int SUB = 0, class XView, class YView, class Store>
   static __device__ __forceinline__ void run(const XView &xv, const YView &yv, int ksteps, T *smem, const Store &store) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x % NT, lane = tid & 63, wave = tid >> 6;   // (a workgroup may hold several products of one wavefront)
     const int wm = wave / WGN, wn = wave % WGN;
     T *Xs[2] = {smem, smem + X_ELEMS + Y_ELEMS};
     T *Ys[2] = {smem + X_ELEMS, smem + 2 * X_ELEMS + Y_ELEMS};
@@ -209,8 +209,8 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
       for (int j = 0; j < RN; j++)
 #pragma unroll
         for (int v = 0; v < M::NACC; v++) acc[i][j][v] = 0.f;
-    // Register ring of NS stages (two: deeper rings were measured slower or equal, the loop is not waiting for its
-    // loads): global loads run NS - 1 reduction steps ahead of their use; two LDS buffers, one
+    // Register ring of NS stages (two: deeper rings were measured slower or equal, on large tiles and on the small ones of short
+    // launches, the loop is not waiting for its loads): global loads run NS - 1 reduction steps ahead of their use; two LDS buffers, one
     // barrier per step.  Step s first writes stage s + 1 to the other LDS buffer, then reads stage s and issues its
     // MFMAs, then refills the ring slot it has just emptied, and only then meets the barrier: the LDS write and the
     // barrier wait pass while the matrix pipe works instead of in front of it.  The loop runs whole rounds of NS
@@ -368,6 +368,8 @@ struct SddArgs {
   int cols = 0;                                       // block-columns per head when known (a call with the plan alone), else 0
 };
 
+struct SddLevel { int pack; const int32_t *lut; const uint8_t *valid; int64_t n; };   // one pack level of the sdd table, n super-blocks
+
 template <typename T, int BLOCK, int PACK, bool KCONTIG> struct SddView {
   // idx is a vector, not an array: an array member makes the compiler keep the view in scratch memory and turn the
   // selection in blk() into an indexed scratch load, a full memory round trip before a workgroup's first load
@@ -391,16 +393,12 @@ template <typename T, int BLOCK, int PACK, bool KCONTIG> struct SddView {
 
 template <int T_> struct SddShape { static constexpr int WG = T_ >= 32 ? 2 : 1; };
 
+// One super-block, by the SddShape<BLOCK * PACK>::WG squared wavefronts that call it together
 template <typename T, int BLOCK, int PACK, bool A_KCONTIG, bool B_KCONTIG>
-__global__ void __launch_bounds__(64 * SddShape<BLOCK * PACK>::WG * SddShape<BLOCK * PACK>::WG) k_sdd(SddArgs g) {
+__device__ __forceinline__ void sdd_super_block(const SddArgs &g, const int32_t *lut, const uint8_t *all_valid, int z, int64_t grp, bool keep, unsigned char *smem) {
   constexpr int TT = BLOCK * PACK, WG = SddShape<TT>::WG;
   typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  const int64_t n_wg = g.n_groups * g.Z;
-  const int64_t w = xcd_remap(blockIdx.x, n_wg);
-  const int z = (int)(w / g.n_groups);
-  const int64_t grp = w % g.n_groups;
-  const table_ptr e = as_table(g.lut) + grp * (PACK * PACK * 4);
+  const table_ptr e = as_table(lut) + grp * (PACK * PACK * 4);
   const int h = e[0];
   SddView<T, BLOCK, PACK, A_KCONTIG> av;
   SddView<T, BLOCK, PACK, B_KCONTIG> bv;
@@ -412,18 +410,72 @@ __global__ void __launch_bounds__(64 * SddShape<BLOCK * PACK>::WG * SddShape<BLO
     bv.idx[p] = e[p * 4 + 2];            // block-col of entries (0, p)
   }
   T *cz = reinterpret_cast<T *>(g.c) + z * g.c_sz;
-  const uint8_t *valid = g.valid ? g.valid + grp * (PACK * PACK) : nullptr;
+  const uint8_t *valid = all_valid ? all_valid + grp * (PACK * PACK) : nullptr;
   // The entry differs from lane to lane here, so the output block is looked up through an ordinary pointer (a vector
   // load): through the constant address space the compiler fetches all PACK * PACK entries with scalar loads and
   // indexes them per lane in scratch memory.
-  const int32_t *eg = g.lut + grp * (PACK * PACK * 4);
+  const int32_t *eg = lut + grp * (PACK * PACK * 4);
   auto store = [&](int m, int n, u32x4 v) {
     const int ent = (m / BLOCK) * PACK + n / BLOCK;
-    if (valid && !valid[ent]) return;
+    if (!keep || (valid && !valid[ent])) return;
     const int64_t bk = eg[ent * 4 + 3];
     *reinterpret_cast<u32x4 *>(cz + bk * (BLOCK * BLOCK) + (m % BLOCK) * BLOCK + n % BLOCK) = v;
   };
-  G::template run<BLOCK>(av, bv, (g.K + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem_raw), store);
+  G::template run<BLOCK>(av, bv, (g.K + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem), store);
+}
+
+template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG>
+__global__ void __launch_bounds__(64 * SddShape<BLOCK>::WG * SddShape<BLOCK>::WG) k_sdd(SddArgs g) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const int64_t n_wg = g.n_groups * g.Z;
+  const int64_t w = xcd_remap(blockIdx.x, n_wg);
+  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG>(g, g.lut, g.valid, (int)(w / g.n_groups), w % g.n_groups, true, smem_raw);
+}
+
+// Blocks of 16 and 32: every pack level of the table in one launch, the largest super-blocks first.  A launch per level
+// leaves the chip idle between them and at the end of each: fp32, block 16, 256 x 512 x 384 in 8 heads and batches, half of
+// the blocks, takes 11.3 + 9.5 us in two launches and 14.7 in one, beside the launch that the host does not make.  The last level of block 16 has super-blocks of one wavefront; four of them share a workgroup: they run the same
+// number of steps and so of barriers, the ones past the end of the level repeat its last super-block and keep nothing.
+template <int BLOCK> struct SddLevels {
+  static constexpr int N = BLOCK == 16 ? 3 : 2;
+  const int32_t *lut[N];                 // by pack: 64 / BLOCK, half of that, ..., 1
+  const uint8_t *valid[N];
+  int64_t n[N];                          // super-blocks
+};
+constexpr int max_of(int a, int b) { return a > b ? a : b; }
+template <typename T, int BLOCK, bool AK, bool BK> struct SddLevelsShape {
+  static constexpr int PACK0 = 64 / BLOCK, LAST_PER_WG = BLOCK == 16 ? 4 : 1;
+  template <int P> using G = TileGemm<T, BLOCK * P, BLOCK * P, SddShape<BLOCK * P>::WG, SddShape<BLOCK * P>::WG, AK, BK, true>;
+  static constexpr int SMEM = max_of(max_of(G<PACK0>::SMEM_BYTES, G<PACK0 / 2>::SMEM_BYTES), LAST_PER_WG * G<1>::SMEM_BYTES);
+};
+
+template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG>
+__global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> lv) {
+  typedef SddLevelsShape<T, BLOCK, A_KCONTIG, B_KCONTIG> S;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  int64_t w = blockIdx.x, n = lv.n[0] * g.Z;
+  if (w < n) {
+    w = xcd_remap(w, n);
+    sdd_super_block<T, BLOCK, S::PACK0, A_KCONTIG, B_KCONTIG>(g, lv.lut[0], lv.valid[0], (int)(w / lv.n[0]), w % lv.n[0], true, smem_raw);
+    return;
+  }
+  w -= n;
+  if constexpr (BLOCK == 16) {
+    n = lv.n[1] * g.Z;
+    if (w < n) {
+      w = xcd_remap(w, n);
+      sdd_super_block<T, 16, 2, A_KCONTIG, B_KCONTIG>(g, lv.lut[1], lv.valid[1], (int)(w / lv.n[1]), w % lv.n[1], true, smem_raw);
+      return;
+    }
+    w -= n;
+  }
+  constexpr int LAST = SddLevels<BLOCK>::N - 1, PER = S::LAST_PER_WG;
+  const int64_t last = lv.n[LAST] * g.Z;
+  w = xcd_remap(w, (last + PER - 1) / PER);
+  const int part = PER == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t i = w * PER + part, j = i < last ? i : last - 1;
+  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG>(g, lv.lut[LAST], lv.valid[LAST], (int)(j / lv.n[LAST]), j % lv.n[LAST], i < last,
+                                                     smem_raw + part * S::template G<1>::SMEM_BYTES);
 }
 
 // sdd with SPLIT x SPLIT workgroups per block (pack 1): for layouts with so few blocks that one workgroup per block
@@ -611,15 +663,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 // ---------------------------------------------------------------------------------------------------------
 // host-side launch helpers shared by the per-type translation units
 // ---------------------------------------------------------------------------------------------------------
-template <typename T, int BLOCK, int PACK> int launch_sdd_tp(const SddArgs &g, bool a_kc, bool b_kc, hipStream_t st) {
-  constexpr int TT = BLOCK * PACK, WG = SddShape<TT>::WG;
+template <typename T, int BLOCK> int launch_sdd_b(const SddArgs &g, bool a_kc, bool b_kc, hipStream_t st) {
+  constexpr int WG = SddShape<BLOCK>::WG;
   const int64_t n_wg = g.n_groups * g.Z;
   if (n_wg <= 0) return BSP_OK;
   if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
-  hipLaunchKernelGGL((k_sdd<T, BLOCK, PACK, AK, BK>), grid, blockdim,                                           \
-                     (TileGemm<T, TT, TT, WG, WG, AK, BK, true>::SMEM_BYTES), st, g)
+  hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK>), grid, blockdim,                                                 \
+                     (TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true>::SMEM_BYTES), st, g)
+  if (a_kc && b_kc) BSP_SDD_LAUNCH(true, true);
+  else if (a_kc && !b_kc) BSP_SDD_LAUNCH(true, false);
+  else if (!a_kc && b_kc) BSP_SDD_LAUNCH(false, true);
+  else BSP_SDD_LAUNCH(false, false);
+#undef BSP_SDD_LAUNCH
+  return BSP_OK;
+}
+
+template <typename T, int BLOCK> int launch_sdd_levels(const SddArgs &g, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st) {
+  SddLevels<BLOCK> lv{};
+  int64_t n_wg = 0;
+  for (int i = 0; i < n_levels; i++) {
+    int at = 0;
+    while (at < SddLevels<BLOCK>::N && (64 / BLOCK) >> at != levels[i].pack) at++;
+    if (at == SddLevels<BLOCK>::N || lv.n[at]) return BSP_ERR_UNSUPPORTED;
+    lv.lut[at] = levels[i].lut; lv.valid[at] = levels[i].valid; lv.n[at] = levels[i].n;
+    const int per = BLOCK == 16 && levels[i].pack == 1 ? 4 : 1;
+    n_wg += (levels[i].n * g.Z + per - 1) / per;
+  }
+  if (n_wg <= 0) return BSP_OK;
+  if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
+  dim3 grid((unsigned)n_wg), blockdim(256);
+#define BSP_SDD_LAUNCH(AK, BK) hipLaunchKernelGGL((k_sdd_levels<T, BLOCK, AK, BK>), grid, blockdim, (SddLevelsShape<T, BLOCK, AK, BK>::SMEM), st, g, lv)
   if (a_kc && b_kc) BSP_SDD_LAUNCH(true, true);
   else if (a_kc && !b_kc) BSP_SDD_LAUNCH(true, false);
   else if (!a_kc && b_kc) BSP_SDD_LAUNCH(false, true);
@@ -644,16 +719,16 @@ template <typename T, int BLOCK, int SPLIT> int launch_sdd_split(const SddArgs &
   return BSP_OK;
 }
 
-template <typename T> int launch_sdd(const SddArgs &g, int block, int pack, bool a_kc, bool b_kc, hipStream_t st) {
+template <typename T> int launch_sdd(const SddArgs &g0, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st) {
+  if (block == 16) return launch_sdd_levels<T, 16>(g0, levels, n_levels, a_kc, b_kc, st);
+  if (block == 32) return launch_sdd_levels<T, 32>(g0, levels, n_levels, a_kc, b_kc, st);
+  if (n_levels != 1 || levels[0].pack != 1) return BSP_ERR_UNSUPPORTED;
+  SddArgs g = g0;
+  g.lut = levels[0].lut; g.valid = levels[0].valid; g.n_groups = levels[0].n;
   // fewer than two workgroups per CU: four 64 x 64 workgroups per 128-block instead of one
-  if (block == 128 && pack == 1 && g.n_groups * g.Z < 512) return launch_sdd_split<T, 128, 2>(g, a_kc, b_kc, st);
-  if (block == 16 && pack == 4) return launch_sdd_tp<T, 16, 4>(g, a_kc, b_kc, st);
-  if (block == 16 && pack == 2) return launch_sdd_tp<T, 16, 2>(g, a_kc, b_kc, st);
-  if (block == 16 && pack == 1) return launch_sdd_tp<T, 16, 1>(g, a_kc, b_kc, st);
-  if (block == 32 && pack == 2) return launch_sdd_tp<T, 32, 2>(g, a_kc, b_kc, st);
-  if (block == 32 && pack == 1) return launch_sdd_tp<T, 32, 1>(g, a_kc, b_kc, st);
-  if (block == 64 && pack == 1) return launch_sdd_tp<T, 64, 1>(g, a_kc, b_kc, st);
-  if (block == 128 && pack == 1) return launch_sdd_tp<T, 128, 1>(g, a_kc, b_kc, st);
+  if (block == 128 && g.n_groups * g.Z < 512) return launch_sdd_split<T, 128, 2>(g, a_kc, b_kc, st);
+  if (block == 64) return launch_sdd_b<T, 64>(g, a_kc, b_kc, st);
+  if (block == 128) return launch_sdd_b<T, 128>(g, a_kc, b_kc, st);
   return BSP_ERR_UNSUPPORTED;
 }
 
@@ -703,9 +778,9 @@ template <typename T> int launch_xsd(const XsdArgs &g, int block, bool sp_trans,
 }
 
 // implemented once per element type (matmul_f16.hip, matmul_bf16.hip, matmul_f32.hip)
-int sdd_generic_f16(const SddArgs &g, int block, int pack, bool a_kc, bool b_kc, hipStream_t st);
-int sdd_generic_bf16(const SddArgs &g, int block, int pack, bool a_kc, bool b_kc, hipStream_t st);
-int sdd_generic_f32(const SddArgs &g, int block, int pack, bool a_kc, bool b_kc, hipStream_t st);
+int sdd_generic_f16(const SddArgs &g, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st);
+int sdd_generic_bf16(const SddArgs &g, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st);
+int sdd_generic_f32(const SddArgs &g, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st);
 int xsd_generic_f16(const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st);
 int xsd_generic_bf16(const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st);
 int xsd_generic_f32(const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st);

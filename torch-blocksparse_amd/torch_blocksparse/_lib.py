@@ -53,6 +53,8 @@ SIGNATURES = {
     'bsp_xsd_workspace_bytes': (_i64, [_i, _i, _i]),
     'bsp_sdd_matmul': (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _i, _vp, _vp,
                             _i64, _vp, _i, _i, _i, _vp]),
+    'bsp_sdd_matmul_levels': (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _i, _vp, _vp, _vp, _vp,
+                                   _vp, _i, _i, _i, _vp]),
     'bsp_sdd_splitk_workspace_bytes': (_i64, [_i, _i64, _i]),
     'bsp_sdd_matmul_splitk': (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _vp, _vp,
                                    _i64, _i, _vp, _i64, _i, _vp]),

@@ -376,7 +376,7 @@ class _sparse_matmul(torch.autograd.Function):
                     AS0, AS3, a.stride(0), a.stride(1), a.stride(2), b.stride(0), b.stride(1), b.stride(2), c.stride(0), block)
         # The group plan describes the whole layout.  If the tables are not built yet it goes first on its own: a kernel
         # that works from the plan writes every block (status OK_WHOLE_LAYOUT) and the tables are never needed; otherwise
-        # nothing was launched (NEEDS_TABLE), the tables are built and the plan goes with the first pack level.
+        # nothing was launched (NEEDS_TABLE), the tables are built and all pack levels go in one call, with the plan.
         gplan = GroupPlan.args(getattr(luts, 'gplan', None))
         rc = _lib.NEEDS_TABLE
         long_k = (lazy and block in (16, 32) and AS3 >= 256 and AS3 % 32 == 0 and a.dtype != torch.float32
@@ -403,13 +403,13 @@ class _sparse_matmul(torch.autograd.Function):
             if _sparse_matmul._sdd_splitk(lib, operands, a, AS0, AS3, block, luts, widths, packs):
                 time[0] = timer.done()
                 return c
-            for lut, width, pack in zip(luts, widths, packs):
-                rc = lib.bsp_sdd_matmul(*operands, pack, _lib.ptr(lut), _lib.ptr(getattr(lut, 'valid', None)), width,
-                                        gplan[0], gplan[1], gplan[2], KERNEL_FLAGS, _lib.stream_ptr(a.device))
-                if rc == _lib.OK_WHOLE_LAYOUT:
-                    break
-                _lib.check(rc, 'bsp_sdd_matmul')
-                gplan = GroupPlan.args(None)
+            n = len(luts)
+            if n:
+                rc = lib.bsp_sdd_matmul_levels(*operands, n, (ctypes.c_int * n)(*packs), (ctypes.c_void_p * n)(*[t.data_ptr() for t in luts]),
+                                               (ctypes.c_void_p * n)(*[t.valid.data_ptr() if getattr(t, 'valid', None) is not None else None for t in luts]),
+                                               (ctypes.c_int64 * n)(*widths), gplan[0], gplan[1], gplan[2], KERNEL_FLAGS, _lib.stream_ptr(a.device))
+                if rc != _lib.OK_WHOLE_LAYOUT:
+                    _lib.check(rc, 'bsp_sdd_matmul_levels')
         time[0] = timer.done()
         return c
 

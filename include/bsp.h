@@ -144,10 +144,12 @@ typedef enum {
   BSP_FLAG_GENERAL_ONLY = 1,  /* take the general kernels even where a specialised one would serve (for cross-checks) */
   BSP_FLAG_NO_GROUPS = 2,     /* ignore the group plan (the per-block / per-segment kernels run instead) */
   BSP_FLAG_NO_WIDE = 4,       /* skip the kernels specialised for a wide free dimension (dsd / dds, blocks 64 and 128) */
-  BSP_FLAG_PLAN_ROWPAIR = 8   /* bsp_sdd_matmul, block 16: d_gplan is a plan over PAIRS of block-rows (built by bsp_group_plan_build on
+  BSP_FLAG_PLAN_ROWPAIR = 8,  /* bsp_sdd_matmul, block 16: d_gplan is a plan over PAIRS of block-rows (built by bsp_group_plan_build on
                                  the layout with every two block-rows merged, entries widened to 13 ints: position, 4 member ids,
                                  then the ids of the two blocks of each member, -1 where absent); plan_lines counts the pairs.  Such a
                                  plan serves the long-reduction kernel (K >= 256, K % 32 == 0, 16-bit types) and nothing else */
+  BSP_FLAG_ANY_K = 16         /* bsp_sdd_matmul_levels with trans_a and not trans_b (the reduction runs along the rows of both operands): K need
+                                 not be a multiple of 16 */
 } bsp_launch_flags;
 
 /* sparse = dense x dense: replaces _sparse_matmul._sdd_matmul + the SDD branch of the kernel

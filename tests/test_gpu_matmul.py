@@ -4,7 +4,7 @@ import torch
 
 import torch_blocksparse as tb
 from oracle import dense_oracle as D
-from helpers import assert_close, operand_shapes, random_layout, run_matmul_case as run_case
+from helpers import assert_close, guard_allocations, operand_shapes, random_layout, run_matmul_case as run_case
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda'
@@ -408,3 +408,35 @@ def test_wide_kernels_agree_with_the_general_ones(monkeypatch):
         for x, y in zip(*outs):
             tol = 4e-3 * (float(y.float().abs().max()) + 1e-6)
             assert float((x.float() - y.float()).abs().max()) <= tol
+
+
+@pytest.mark.parametrize('block,dtype', [(32, torch.float16), (32, torch.float32), (64, torch.bfloat16), (64, torch.float32), (128, torch.float16), (128, torch.float32)])
+@pytest.mark.parametrize('tokens', [1, 15, 17, 255, 257, 529, 720])
+def test_linear_with_a_number_of_tokens_that_divides_by_nothing(block, dtype, tokens):
+    # y, dx and dw without a padded copy of the operands, around the 16 rows of a step, the 256 columns of a wide tile and the
+    # reductions from which dw takes the kernels for long ones; nothing may be written around the outputs
+    torch.manual_seed(tokens)
+    lay = random_layout((1, 4, 5), 0.5, 3)
+    lin = tb.Linear(4 * block, 5 * block, block, lay).to(DEV).to(dtype)
+    x = torch.randn(tokens, 4 * block, device=DEV).to(dtype).requires_grad_(True)
+    dy = torch.randn(tokens, 5 * block, device=DEV).to(dtype)
+    with guard_allocations('linear'):
+        y = lin(x)
+        y.backward(dy)
+        torch.cuda.synchronize()
+    xd, dyd, w = x.detach().cpu().double(), dy.cpu().double(), D.sparse_to_dense(lin.weight.detach().cpu().double()[None], lay, block)[0, 0]
+
+    def close(got, a, b, what):
+        assert_close(got, (a @ b).float(), dtype, what, mag=(a.abs() @ b.abs()).float() if dtype == torch.float32 else None)
+
+    close(y, xd, w, 'y')
+    close(x.grad, dyd, w.t(), 'dx')
+    blocks = lambda t: D.dense_to_sparse(t[None, None], lay, block)[0]
+    assert_close(lin.weight.grad, blocks((xd.t() @ dyd).float()), dtype, 'dw', mag=blocks((xd.t().abs() @ dyd.abs()).float()) if dtype == torch.float32 else None)
+
+
+def test_a_reduction_that_is_no_multiple_of_16_stays_refused_elsewhere():
+    lay = torch.ones(1, 2, 2, dtype=torch.int64)
+    a, b = torch.randn(1, 1, 24, 64, device=DEV), torch.randn(1, 1, 24, 64, device=DEV)
+    with pytest.raises(ValueError):
+        tb.MatMul(lay, 32, 'sdd', trans_a=True, trans_b=False)(a, b)

@@ -9,6 +9,9 @@ namespace {
 bool no_groups(int flags) { return (flags & BSP_FLAG_NO_GROUPS) != 0; }
 bool general_only(int flags) { return (flags & BSP_FLAG_GENERAL_ONLY) != 0; }
 bool no_wide(int flags) { return (flags & (BSP_FLAG_NO_WIDE | BSP_FLAG_GENERAL_ONLY)) != 0; }
+// the reduction of an sdd product: a multiple of 16 (reference matmul.py:318-319), or any number of rows where both operands hold
+// it as rows and the caller says so (the general kernels then read row by row up to the last)
+bool sdd_k_ok(int K, int trans_a, int trans_b, int flags) { return K % 16 == 0 || ((flags & BSP_FLAG_ANY_K) && trans_a && !trans_b); }
 bool rowpair(int flags) { return (flags & BSP_FLAG_PLAN_ROWPAIR) != 0; }
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 bool block_ok(int block) { return block == 16 || block == 32 || block == 64 || block == 128; }
@@ -46,7 +49,7 @@ extern "C" int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, vo
     levels[i] = SddLevel{packs[i], d_luts[i], d_valids[i], n_groups[i]};
   }
   if (!block_ok(block)) return BSP_ERR_UNSUPPORTED;
-  if (K % 16) return BSP_ERR_K_MULTIPLE;   // reference matmul.py:318-319
+  if (!sdd_k_ok(K, trans_a, trans_b, flags)) return BSP_ERR_K_MULTIPLE;
   const int u = elems16(dtype);
   if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return BSP_ERR_ARG;
   if (a_stride_z % u || a_stride_h % u || lda % u || b_stride_z % u || b_stride_h % u || ldb % u || c_stride_z % u) return BSP_ERR_ARG;
@@ -61,7 +64,7 @@ extern "C" int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, vo
   // op(A)[m][k]: reduction contiguous unless A is read transposed; op(B)[k][n]: contiguous when B is read transposed
   const bool a_kc = !trans_a, b_kc = trans_b != 0;
   hipStream_t st = as_stream(stream);
-  int rc = general_only(flags) ? 0 : sdd_fast64(dtype, g, block, packs[0], a_kc, b_kc, st);
+  int rc = general_only(flags) || K % 16 ? 0 : sdd_fast64(dtype, g, block, packs[0], a_kc, b_kc, st);
   if (rc < 0) return rc;
   // (a kernel that works from the plan writes the whole layout; the one for a single level serves blocks of 64, which have no other)
   if (rc >= 1) { BSP_LAUNCH_CHECK(); return rc == 2 ? BSP_OK_WHOLE_LAYOUT : BSP_OK; }
@@ -192,7 +195,9 @@ extern "C" int bsp_dsd_matmul(int dtype, const void *a, const void *b, void *c, 
   if (!block_ok(block)) return BSP_ERR_UNSUPPORTED;
   const int u = elems16(dtype);
   if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return BSP_ERR_ARG;
-  if (N % u || a_stride_z % u || b_stride_z % u || b_stride_h % u || ldb % u || c_stride_z % u || c_stride_h % u || ldc % u) return BSP_ERR_ARG;
+  // (a free dimension whose elements are whole rows on both sides may have any size, one that lies along the rows is read and
+  // written in chunks of 16 bytes)
+  if ((N % u && !(trans_b && trans_c)) || a_stride_z % u || b_stride_z % u || b_stride_h % u || ldb % u || c_stride_z % u || c_stride_h % u || ldc % u) return BSP_ERR_ARG;
   XsdArgs g;
   g.sp = a; g.dn = b; g.out = c; g.Z = Z; g.NF = N;
   g.sp_sz = a_stride_z; g.dn_sz = b_stride_z; g.dn_sh = b_stride_h; g.ldd = ldb;
@@ -282,7 +287,7 @@ extern "C" int bsp_dds_matmul(int dtype, const void *a, const void *b, void *c, 
   if (!block_ok(block)) return BSP_ERR_UNSUPPORTED;
   const int u = elems16(dtype);
   if (!aligned16(a) || !aligned16(b) || !aligned16(c)) return BSP_ERR_ARG;
-  if (M % u || a_stride_z % u || a_stride_h % u || lda % u || b_stride_z % u || c_stride_z % u || c_stride_h % u || ldc % u) return BSP_ERR_ARG;
+  if ((M % u && (trans_a || trans_c)) || a_stride_z % u || a_stride_h % u || lda % u || b_stride_z % u || c_stride_z % u || c_stride_h % u || ldc % u) return BSP_ERR_ARG;
   XsdArgs g;
   g.sp = b; g.dn = a; g.out = c; g.Z = Z; g.NF = M;
   g.sp_sz = b_stride_z; g.dn_sz = a_stride_z; g.dn_sh = a_stride_h; g.ldd = lda;

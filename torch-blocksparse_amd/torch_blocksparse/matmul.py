@@ -271,6 +271,7 @@ class SddTables(list):
     build_long = None
     widths = None
     packs = None
+    any_k = False         # a reduction along the rows of both operands may have any length (the weight gradient of Linear)
 
     def materialize(self):
         if self.build is not None:
@@ -361,14 +362,20 @@ class _sparse_matmul(torch.autograd.Function):
         a, b = _prep(a), _prep(b)
         AS0 = a.size(0)
         AS3 = a.size(2 if trans_a else 3)
-        if AS3 % 16 != 0:
+        lazy = isinstance(luts, SddTables)
+        any_k = AS3 % 16 != 0 and lazy and luts.any_k and trans_a and not trans_b
+        if AS3 % 16 != 0 and not any_k:
             raise ValueError('Reduction size for SDD must be a multiple of 16')
         if b.size(0) != AS0 or b.size(1) != a.size(1) or b.size(3 if trans_b else 2) != AS3:
             raise ValueError('incompatible operand shapes for sdd: %s and %s' % (tuple(a.shape), tuple(b.shape)))
         _check_dense('a', a, spdims[0], block * spdims[1], None, trans_a)
         _check_dense('b', b, spdims[0], None, block * spdims[2], trans_b)
+        if lazy and luts.any_k and trans_a and not trans_b and AS3 % 32 and a.dtype != torch.float32 and (
+                block in (16, 32) and AS3 >= 256 or block == 128 and AS3 >= 512):
+            # the kernels for a long reduction take whole steps of 32 rows
+            a, b = _sparse_matmul._pad_free_dim(a, 2, 32), _sparse_matmul._pad_free_dim(b, 2, 32)
+            AS3, any_k = a.size(2), False
         lib = _lib.load()
-        lazy = isinstance(luts, SddTables)
         total_width = luts.nnz if lazy else sum(w * p * p for w, p in zip(widths, packs))
         c = torch.empty((AS0, total_width, block, block), dtype=a.dtype, device=a.device)
         timer = _Timer(bench, a.device)
@@ -379,6 +386,7 @@ class _sparse_matmul(torch.autograd.Function):
         # nothing was launched (NEEDS_TABLE), the tables are built and all pack levels go in one call, with the plan.
         gplan = GroupPlan.args(getattr(luts, 'gplan', None))
         rc = _lib.NEEDS_TABLE
+        flags = KERNEL_FLAGS | (_lib.FLAG_ANY_K if any_k else 0)
         long_k = (lazy and block in (16, 32) and AS3 >= 256 and AS3 % 32 == 0 and a.dtype != torch.float32
                   and getattr(luts, 'build_long', None) is not None)
         if long_k:
@@ -386,13 +394,12 @@ class _sparse_matmul(torch.autograd.Function):
             if luts.gplan_long is None:
                 luts.gplan_long = luts.build_long()
             lp = GroupPlan.args(luts.gplan_long)
-            flags = KERNEL_FLAGS | (_lib.FLAG_PLAN_ROWPAIR if luts.gplan_long.rowpair else 0)
             # (the largest group of the plan sizes the grid: workgroups for block-columns that no group reaches are not launched)
             rc = lib.bsp_sdd_matmul(*operands, 0, ctypes.c_void_p(0), ctypes.c_void_p(0), min(spdims[2], luts.gplan_long.max_entries()),
-                                    lp[0], lp[1], lp[2], flags, _lib.stream_ptr(a.device))
+                                    lp[0], lp[1], lp[2], flags | (_lib.FLAG_PLAN_ROWPAIR if luts.gplan_long.rowpair else 0), _lib.stream_ptr(a.device))
             if rc not in (_lib.OK_WHOLE_LAYOUT, _lib.NEEDS_TABLE):
                 _lib.check(rc, 'bsp_sdd_matmul')
-        elif lazy and luts.gplan is not None and luts.build is not None:
+        elif lazy and luts.gplan is not None and luts.build is not None and not any_k:
             rc = lib.bsp_sdd_matmul(*operands, 0, ctypes.c_void_p(0), ctypes.c_void_p(0), spdims[2], gplan[0], gplan[1], gplan[2],
                                     KERNEL_FLAGS, _lib.stream_ptr(a.device))
             if rc not in (_lib.OK_WHOLE_LAYOUT, _lib.NEEDS_TABLE):
@@ -407,7 +414,7 @@ class _sparse_matmul(torch.autograd.Function):
             if n:
                 rc = lib.bsp_sdd_matmul_levels(*operands, n, (ctypes.c_int * n)(*packs), (ctypes.c_void_p * n)(*[t.data_ptr() for t in luts]),
                                                (ctypes.c_void_p * n)(*[t.valid.data_ptr() if getattr(t, 'valid', None) is not None else None for t in luts]),
-                                               (ctypes.c_int64 * n)(*widths), gplan[0], gplan[1], gplan[2], KERNEL_FLAGS, _lib.stream_ptr(a.device))
+                                               (ctypes.c_int64 * n)(*widths), gplan[0], gplan[1], gplan[2], flags, _lib.stream_ptr(a.device))
                 if rc != _lib.OK_WHOLE_LAYOUT:
                     _lib.check(rc, 'bsp_sdd_matmul_levels')
         time[0] = timer.done()
@@ -516,7 +523,8 @@ class _sparse_matmul(torch.autograd.Function):
         _check_sparse('b', b, getattr(lut, 'nnz', None), block, a.size(0))
         _check_dense('a', a, spdims[0], None, block * spdims[2 if trans_b else 1], trans_a)
         AS2 = a.size(3 if trans_a else 2)                     # free dimension M (matmul.py:467)
-        a = _prep(_sparse_matmul._pad_free_dim(a, 3 if trans_a else 2, v))
+        # (a free dimension of whole rows on both sides needs no padding)
+        a = _prep(_sparse_matmul._pad_free_dim(a, 3 if trans_a else 2, v if trans_a or trans_c else 1))
         M = a.size(3 if trans_a else 2)
         b = b if b.is_contiguous() else b.contiguous()
         BS2 = block * spdims[1 if trans_b else 2]             # matmul.py:471
@@ -541,7 +549,7 @@ class _sparse_matmul(torch.autograd.Function):
         _check_sparse('a', a, getattr(lut, 'nnz', None), block, b.size(0))
         _check_dense('b', b, spdims[0], block * spdims[1 if trans_a else 2], None, trans_b)
         BS3 = b.size(2 if trans_b else 3)                     # free dimension N (matmul.py:518)
-        b = _prep(_sparse_matmul._pad_free_dim(b, 2 if trans_b else 3, v))
+        b = _prep(_sparse_matmul._pad_free_dim(b, 2 if trans_b else 3, 1 if trans_b and trans_c else v))
         N = b.size(2 if trans_b else 3)
         a = a if a.is_contiguous() else a.contiguous()
         AS1 = block * spdims[2 if trans_a else 1]             # matmul.py:513
@@ -608,6 +616,7 @@ class MatMul:
     mode 'sdd': C sparse, A and B dense; 'dsd': A sparse; 'dds': B sparse.  `layout` ([H, R, C], 0/1, on the CPU)
     always describes the sparse tensor as stored.
     """
+    any_k = False             # see SddTables
 
     def make_lut(self, dtype, device):
         key = (dtype, device)
@@ -616,7 +625,12 @@ class MatMul:
         layout, block = self.layout, self.block
         step = 8 if dtype == torch.float32 else 16             # matmul.py:617
         ctx = _LayoutOnDevice(layout, device)                  # one upload of the layout and one workspace for all tables
-        sdd = lambda: _sparse_matmul.make_sdd_lut(layout, block, dtype, device, ctx=ctx, lazy=True)
+
+        def sdd():
+            made = _sparse_matmul.make_sdd_lut(layout, block, dtype, device, ctx=ctx, lazy=True)
+            made[0].any_k = self.any_k
+            return made
+
         dxx = lambda trans: _sparse_matmul.make_dxx_lut(layout, block, step, trans, device, ctx=ctx)
         if self.mode == 'sdd':                                 # matmul.py:618-637
             c, da, db = sdd(), dxx(True), dxx(False)
@@ -690,10 +704,6 @@ class Linear(torch.nn.Module):
 
     def forward(self, input):
         shape = input.shape
-        x = input.reshape(1, 1, -1, shape[-1])
-        tokens = x.size(2)
-        pad = (-tokens) % 16     # the weight gradient is an sdd product reducing over the tokens (multiple of 16)
-        if pad:
-            x = torch.cat((x, x.new_zeros(1, 1, pad, shape[-1])), dim=2)
-        y = self.matmul(x, self.weight)[:, :, :tokens]
+        self.matmul.any_k = True     # the weight gradient is an sdd product that reduces over the tokens, however many there are
+        y = self.matmul(input.reshape(1, 1, -1, shape[-1]), self.weight)
         return y.reshape(shape[:-1] + (self.out_features,))

@@ -440,3 +440,12 @@ def test_a_reduction_that_is_no_multiple_of_16_stays_refused_elsewhere():
     a, b = torch.randn(1, 1, 24, 64, device=DEV), torch.randn(1, 1, 24, 64, device=DEV)
     with pytest.raises(ValueError):
         tb.MatMul(lay, 32, 'sdd', trans_a=True, trans_b=False)(a, b)
+
+
+def test_a_single_row_whose_stride_is_no_multiple_of_16_bytes():
+    # contiguous() returns such a tensor as it is: the row's stride of 1 means nothing, but the kernels look at it
+    lay = random_layout((1, 4, 5), 0.5, 3)
+    lin = tb.Linear(128, 160, 32, lay).to(DEV)
+    x = torch.randn(128, 1, device=DEV).t()
+    assert x.stride() == (1, 1) and x.is_contiguous()
+    assert torch.equal(lin(x), lin(x.clone(memory_format=torch.contiguous_format)))

@@ -60,8 +60,14 @@ class _LayoutOnDevice:
 def _prep(x):
     """Operands are read with 16-byte vector loads along a unit inner stride."""
     v = _vec(x.dtype)
-    ok = x.stride(-1) == 1 and x.data_ptr() % 16 == 0 and all(s % v == 0 for s in x.stride()[:-1])
-    return x if ok else x.contiguous()
+
+    def ok(t):
+        return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % v == 0 for s in t.stride()[:-1])
+
+    if ok(x):
+        return x
+    x = x.contiguous()           # (which returns a tensor with an odd stride of a dimension of size 1, or at an odd address, as it is)
+    return x if ok(x) else x.clone(memory_format=torch.contiguous_format)
 
 
 class _Timer:
@@ -207,14 +213,18 @@ class GroupPlan:
         split chains.  One buffer per plan: launches of one operator are assumed to be ordered on one stream.
         A launch that needs more than the buffer holds gets a larger one, and the smaller one stays allocated for the
         life of the plan: a captured HIP graph replays launches that carry its address."""
+        at, n = self.workspace_address(free_dim, Z)
+        return ctypes.c_void_p(at), n
+
+    def workspace_address(self, free_dim, Z):
         if self.n_split == 0:
-            return ctypes.c_void_p(0), 0
+            return 0, 0
         need = _lib.load().bsp_xsd_workspace_bytes(self.n_split, int(free_dim), int(Z))
         if self._ws is None or self._ws.numel() < need:
             if self._ws is not None:
                 self._ws_retired.append(self._ws)
             self._ws = torch.empty(need, dtype=torch.uint8, device=self.table.device)
-        return _lib.ptr(self._ws), self._ws.numel()
+        return self._ws.data_ptr(), self._ws.numel()
 
     @staticmethod
     def args(plan):
@@ -272,6 +282,18 @@ class SddTables(list):
     widths = None
     packs = None
     any_k = False         # a reduction along the rows of both operands may have any length (the weight gradient of Linear)
+
+    _splitk_ws = None
+
+    def splitk_workspace(self, need, device):
+        """address of a workspace of `need` bytes for the sdd in parts: it only grows, and one that a larger launch supersedes stays
+        allocated, because a captured graph may still use it"""
+        ws = self._splitk_ws
+        if ws is None or ws.numel() < need:
+            if ws is not None:
+                self._splitk_retired = getattr(self, '_splitk_retired', []) + [ws]
+            ws = self._splitk_ws = torch.empty(need, dtype=torch.uint8, device=device)
+        return ws.data_ptr()
 
     def materialize(self):
         if self.build is not None:
@@ -435,14 +457,10 @@ class _sparse_matmul(torch.autograd.Function):
             return False
         parts = max(1, min(_sparse_matmul.SPLITK_TARGET_WORKGROUPS // (n * Z), K // 256, 16))
         need = lib.bsp_sdd_splitk_workspace_bytes(Z, n, parts)
-        ws = getattr(luts, '_splitk_ws', None)
-        if need and (ws is None or ws.numel() < need):
-            if ws is not None:
-                luts._splitk_retired = getattr(luts, '_splitk_retired', []) + [ws]      # a captured graph may still use it
-            ws = luts._splitk_ws = torch.empty(need, dtype=torch.uint8, device=a.device)
+        ws = luts.splitk_workspace(need, a.device) if need else 0
         lut = luts[0]
         rc = lib.bsp_sdd_matmul_splitk(*operands, _lib.ptr(lut), _lib.ptr(getattr(lut, 'valid', None)), n, parts,
-                                       _lib.ptr(ws) if need else ctypes.c_void_p(0), ws.numel() if need else 0, KERNEL_FLAGS,
+                                       ctypes.c_void_p(ws), need, KERNEL_FLAGS,
                                        _lib.stream_ptr(a.device))
         if rc == _lib.ERR_UNSUPPORTED:
             return False
@@ -573,41 +591,90 @@ class _sparse_matmul(torch.autograd.Function):
           'dds': _dds_matmul.__get__(object)}
 
     @staticmethod
-    def forward(ctx, a, b, trans_a, trans_b, trans_c, mode, spdims, block,
-                c_lut, c_num_locks, c_width, c_packs, c_bench, c_time,
-                da_lut, da_num_locks, da_width, da_packs, da_bench, da_time,
-                db_lut, db_num_locks, db_width, db_packs, db_bench, db_time):
-        _lib.require_gpu_tensor(a, 'matmul operand a')
-        _lib.require_gpu_tensor(b, 'matmul operand b')
-        if a.dtype != b.dtype or a.dtype not in _lib.DTYPES:
-            raise ValueError('matmul operands must both be float16, bfloat16 or float32 (got %s, %s)' % (a.dtype, b.dtype))
-        c = _sparse_matmul.fn[mode](a, b, trans_a, trans_b, trans_c, spdims, block,
-                                    c_lut, c_num_locks, c_width, c_packs, c_bench, c_time)
+    def forward(ctx, a, b, product, times):
+        c = product.run(0, a, b, product.trans_a, product.trans_b, False, times)
         ctx.save_for_backward(a, b)
-        ctx.da = (da_lut, da_num_locks, da_width, da_packs, da_bench, da_time)
-        ctx.db = (db_lut, db_num_locks, db_width, db_packs, db_bench, db_time)
-        ctx.mode, ctx.spdims, ctx.block = mode, spdims, block
-        ctx.trans_a, ctx.trans_b = trans_a, trans_b
+        ctx.product, ctx.times = product, times
         return c
 
     @staticmethod
     def backward(ctx, dc):
         a, b = ctx.saved_tensors
-        mode = ctx.mode
+        p = ctx.product
         da = db = None
         # db before da: in an attention chain da of the dsd product (an sdd launch) is what the softmax backward
         # reads next, and da of the sdd product is what the caller's next op reads; measured 1 % faster per step.
         if ctx.needs_input_grad[1]:                        # matmul.py:598-601
-            mode_db = mode[2] + mode[1] + mode[0]
-            db = _sparse_matmul.fn[mode_db](a, dc, not ctx.trans_a, False, ctx.trans_b, ctx.spdims, ctx.block, *ctx.db)
+            db = p.run(2, a, dc, not p.trans_a, False, p.trans_b, ctx.times)
             if db.shape != b.shape:
                 db = db.reshape(b.shape) if db.numel() == b.numel() else db.sum(0).reshape(b.shape)
         if ctx.needs_input_grad[0]:                           # matmul.py:593-596
-            mode_da = mode[1] + mode[0] + mode[2]
-            da = _sparse_matmul.fn[mode_da](dc, b, False, not ctx.trans_b, ctx.trans_a, ctx.spdims, ctx.block, *ctx.da)
+            da = p.run(1, dc, b, False, not p.trans_b, p.trans_a, ctx.times)
             if da.shape != a.shape:
                 da = da.reshape(a.shape) if da.numel() == a.numel() else da.sum(0).reshape(a.shape)
-        return (da, db) + (None,) * 24
+        return da, db, None, None
+
+
+class _Product:
+    """A MatMul's product and its two gradients for one data type and device: the tables, and how the native launcher
+    (csrc/launch.cpp) wants them.  run() tries that one; what it leaves, the functions above do."""
+
+    def __init__(self, op, luts, dtype, device):
+        mode = op.mode
+        self.luts, self.bench, self.dtype, self.device = luts, op.bench, _lib.DTYPES.get(dtype, -1), device
+        self.trans_a, self.trans_b, self.spdims, self.block = op.trans_a, op.trans_b, op.spdims, op.block
+        self.modes = (mode, mode[1] + mode[0] + mode[2], mode[2] + mode[1] + mode[0])      # c, da, db (matmul.py:593-601)
+        self.native = [None, None, None]
+        self.built = [None, None, None]         # which of the tables made on demand were there
+
+    def run(self, which, a, b, trans_a, trans_b, trans_c, times):
+        mode = self.modes[which]
+        if not self.bench:
+            launch = _lib.native()
+            tables = self.native[which] or self._tables(which)
+            if tables is not None:
+                c = (launch.sdd(tables, a, b, trans_a, trans_b, trans_c, KERNEL_FLAGS) if mode == 'sdd' else
+                     launch.xsd(tables, mode == 'dds', a, b, trans_a, trans_b, trans_c, KERNEL_FLAGS))
+                if c is not None:
+                    return c
+        _lib.require_gpu_tensor(a, 'matmul operand a')
+        _lib.require_gpu_tensor(b, 'matmul operand b')
+        if a.dtype != b.dtype or a.dtype not in _lib.DTYPES:
+            raise ValueError('matmul operands must both be float16, bfloat16 or float32 (got %s, %s)' % (a.dtype, b.dtype))
+        c = _sparse_matmul.fn[mode](a, b, trans_a, trans_b, trans_c, self.spdims, self.block, *self.luts[4 * which:4 * which + 4], self.bench, times[which])
+        if self.built[which] != self._on_demand(which):
+            self.native[which] = None
+        return c
+
+    def _on_demand(self, which):
+        lut = self.luts[4 * which]
+        if self.modes[which] == 'sdd':
+            return lut.gplan_long is None, lut.build is None
+        return (lut.gplan_wide is None,)
+
+    def _tables(self, which):
+        """a capsule with the pointers and numbers of the tables as they are now, and the tensors behind them"""
+        if self.device.type != 'cuda' or self.dtype < 0:
+            return None
+        lut, _, width, _ = self.luts[4 * which:4 * which + 4]
+        H, R, C = [int(n) for n in self.spdims]
+        dev = self.device.index if self.device.index is not None else torch.cuda.current_device()
+        plan = lambda p: (0, 0, 0, 0) if p is None else (p.table.data_ptr(), p.n_groups, -p.lines if p.coarse else p.lines, p.n_split)
+        if self.modes[which] == 'sdd':
+            levels = None
+            if lut.build is None:
+                levels = tuple((p, t.data_ptr(), t.valid.data_ptr() if getattr(t, 'valid', None) is not None else 0, w)
+                               for t, w, p in zip(lut, lut.widths, lut.packs))
+            late = lut.gplan_long
+            made = _lib.native().make_sdd((lut, lut.gplan, late) + tuple(lut) + tuple(getattr(t, 'valid', None) for t in lut), self.block, self.dtype, dev, lut.nnz, H, R, C,
+                                          plan(lut.gplan), plan(late), 0 if lut.build_long is None else 1 if late is None else 2,
+                                          int(late is not None and late.rowpair), late.max_entries() if late is not None else 0, int(lut.any_k), levels)
+        else:
+            made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, lut.nnz, H, R, C,
+                                          plan(lut.gplan), plan(lut.gplan_wide),
+                                          2 if lut.gplan_wide is not None else int(getattr(lut, 'build_wide', None) is not None))
+        self.native[which], self.built[which] = made, self._on_demand(which)
+        return made
 
 
 class MatMul:
@@ -641,12 +708,27 @@ class MatMul:
         self.lut_cache[key] = c + da + db
         return self.lut_cache[key]
 
+    def _product(self, dtype, device):
+        luts = self.make_lut(dtype, device)
+        product = self._products.get((dtype, device))
+        if product is None or product.luts is not luts or product.bench != self.bench:
+            product = self._products[(dtype, device)] = _Product(self, luts, dtype, device)
+        return product
+
+    def __getstate__(self):
+        """a copy (of a module that holds the operator, say) makes its own products from its own tables"""
+        return {k: v for k, v in self.__dict__.items() if k != '_products'}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state, _products=dict())
+
     def __init__(self, layout, block, mode, trans_a=False, trans_b=False, bench=False):
         if mode not in ['sdd', 'dsd', 'dds']:
             raise NotImplementedError('Supported modes are: sdd, dsd, dds')
         if block not in (16, 32, 64, 128):
             raise ValueError('block must be 16, 32, 64 or 128')
         self.lut_cache = dict()
+        self._products = dict()
         self.trans_a = trans_a
         self.trans_b = trans_b
         self.mode = mode
@@ -660,6 +742,8 @@ class MatMul:
 
     @staticmethod
     def _pad_shape(x, is_sparse):
+        if x.dim() == 4:
+            return x
         max_dim = 3 if is_sparse else 4                        # matmul.py:663-668
         for _ in range(max_dim - x.dim()):
             x = x.unsqueeze(0)
@@ -667,15 +751,12 @@ class MatMul:
 
     def __call__(self, a, b):
         _lib.require_gpu_tensor(a, 'matmul operand a')
-        luts = self.make_lut(a.dtype, a.device)
-        time_c, time_da, time_db = [None], [None], [None]
+        product = self._product(a.dtype, a.device)
+        times = ([None], [None], [None])
         a = MatMul._pad_shape(a, self.mode == 'dsd')
         b = MatMul._pad_shape(b, self.mode == 'dds')
-        c = _sparse_matmul.apply(a, b, self.trans_a, self.trans_b, False, self.mode, self.spdims, self.block,
-                                 luts[0], luts[1], luts[2], luts[3], self.bench, time_c,
-                                 luts[4], luts[5], luts[6], luts[7], self.bench, time_da,
-                                 luts[8], luts[9], luts[10], luts[11], self.bench, time_db)
-        self.time_c, self.time_da, self.time_db = time_c[0], time_da[0], time_db[0]
+        c = _sparse_matmul.apply(a, b, product, times)
+        self.time_c, self.time_da, self.time_db = times[0][0], times[1][0], times[2][0]
         return c
 
 

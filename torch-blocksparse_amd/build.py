@@ -6,6 +6,7 @@ in parallel and linked into one shared library with a plain C ABI (include/bsp.h
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -69,9 +70,20 @@ def build(verbose=False, jobs=None, sources=None):
                 print(err)
     objs = [os.path.join(OBJDIR, os.path.splitext(s)[0] + '.o') for s in SOURCES]
     subprocess.check_call(['hipcc', '--offload-arch=gfx950', '-shared', '-fPIC', '-o', lib_path()] + objs)
+    build_launch()
     if sources is None:
         build_probe()
     return lib_path()
+
+
+def build_launch():
+    """The host side of the launches: a CPython extension beside the library, which it calls through the C ABI."""
+    out = os.path.join(LIBDIR, '_launch.so')
+    r = subprocess.run(['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-I' + sysconfig.get_paths()['include'], os.path.join(CSRC, 'launch.cpp'), '-o', out,
+                        '-L' + LIBDIR, '-lbsp_hip', '-Wl,-rpath,$ORIGIN'], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError('g++ failed on launch.cpp:\n%s' % r.stderr)
+    return out
 
 
 def build_probe():

@@ -5,12 +5,15 @@ been built, importing the package still works (so that layouts and configuration
 every operator raises at its first call.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), 'lib', 'libbsp_hip.so')
+NATIVE_PATH = os.path.join(os.path.dirname(_HERE), 'lib', '_launch.so')
 
 F16, BF16, F32 = 0, 1, 2
 DTYPES = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
@@ -111,6 +114,25 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_native = None
+
+
+def native():
+    """The extension module with the host side of a launch (csrc/launch.cpp), loaded once.  Like the HIP library it has no stand-in."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise BlocksparseLibraryError('torch_blocksparse: %s not found. Build it with `python torch-blocksparse_amd/build.py`.' % NATIVE_PATH)
+        from .matmul import _sparse_matmul
+        loader = importlib.machinery.ExtensionFileLoader('torch_blocksparse._launch', NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location('torch_blocksparse._launch', NATIVE_PATH, loader=loader))
+        loader.exec_module(module)
+        module.setup(torch, check, torch._C._cuda_getCurrentRawStream, torch.nn.Parameter, _sparse_matmul)
+        _native = module
+    return _native
 
 
 def strerror(code):

@@ -110,6 +110,18 @@ class _QuadTables:
         self.split = self.rows[info.split_offset:] if info.n_split else None
         self.lines, self.longest, self.columns = info.lines, info.longest_line, info.columns
         self.n_items, self.n_slots, self.n_split = info.n_items, info.n_slots, info.n_split
+        self.shape, self._native = (H, R, C, block), None
+
+    def __getstate__(self):
+        return dict(self.__dict__, _native=None)
+
+    def native(self):
+        """what the native launcher (csrc/launch.cpp) wants to know of the tables, made once"""
+        if self._native is None:
+            dev = self.rows.device.index if self.rows.device.index is not None else torch.cuda.current_device()
+            self._native = _lib.native().make_attn(self.rows, self.rows.data_ptr(), self.items.data_ptr(), 0 if self.split is None else self.split.data_ptr(), self.lines,
+                                                   self.columns, self.n_items, self.n_slots, self.n_split, dev, self.longest, *self.shape)
+        return self._native
 
 
 def _vec_ok(t):
@@ -184,6 +196,11 @@ class AttentionCore:
         raise the reference's errors.)"""
         if not FUSED or self.block not in (16, 32, 64) or dropout_p:
             return False
+        tables = self._tables.get(str(q.device)) if q.is_cuda else None
+        if tables is not None and tables[0] is not None:
+            usable = _lib.native().attn_usable(tables[0].native(), q, k, v)
+            if usable is not None:
+                return usable
         if not (q.is_cuda and q.dtype in (torch.float16, torch.bfloat16) and k.dtype == q.dtype and v.dtype == q.dtype):
             return False
         if q.dim() != 4 or k.dim() != 4 or v.dim() != 4 or q.size(3) not in (64, 128):
@@ -232,20 +249,20 @@ class _attention_quad(torch.autograd.Function):
         tables = core.quad(q.device)
         lines = tables.lines
         keep = grad_enabled and any(ctx.needs_input_grad[:3])
-        q, k, v = _near(q), _near(k), _near(v)
         kpm = None
         if key_padding_mask is not None:                   # element (z, c), softmax.py:60-62, 274
             kpm = _sparse_softmax._strided16(key_padding_mask, 'key_padding_mask')
             if keep and kpm.data_ptr() == key_padding_mask.data_ptr():
                 kpm = _packed(kpm[:, :k.size(2)])          # the backward pass reads it again, the caller may fill it with the next mask until then
         ctx.kpm_args = (kpm.stride(0) if kpm is not None and kpm.size(0) > 1 else 0, int(kp_mask_mode == 'mul'))
-        o = torch.empty((Z, H, R * core.block, D), dtype=q.dtype, device=q.device)
-        lse = torch.empty((Z, H, 2, lines * 64), dtype=torch.float32, device=q.device) if keep else None      # (and what its rounding left out)
-        rc = _lib.load().bsp_attention_rows_fwd(
-            _lib.DTYPES[q.dtype] | _lib.ROWS_WITH_REST, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse), Z, H, lines, k.size(2), D,
-            q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
-            o.stride(0), o.stride(1), o.stride(2), lines * 128, scale, _lib.ptr(tables.rows), _lib.ptr(kpm), *ctx.kpm_args, _lib.stream_ptr(q.device))
-        _lib.check(rc, 'bsp_attention_rows_fwd')
+        launch, native = _lib.native(), tables.native()
+        made = launch.attn_fwd(native, q, k, v, scale, kpm, *ctx.kpm_args, keep)
+        if made is None:                                   # operands that the kernels cannot address are copied to memory of their own
+            q, k, v = _near(q), _near(k), _near(v)
+            made = launch.attn_fwd(native, q, k, v, scale, kpm, *ctx.kpm_args, keep)
+            if made is None:
+                raise _lib.BlocksparseLibraryError('attention: operands %s, %s, %s do not fit the layout' % (tuple(q.shape), tuple(k.shape), tuple(v.shape)))
+        o, lse = made                                      # lse [Z, H, 2, rows]: and what its rounding left out
         fused_calls += 1
         if keep:
             ctx.save_for_backward(q, k, v, o, lse, kpm)
@@ -307,8 +324,12 @@ class _attention_quad(torch.autograd.Function):
     def backward(ctx, do):
         saved = ctx.saved_tensors                          # (unpacked once: non-reentrant checkpoints allow no more)
         q = saved[0]
-        do = _near(do)
         need_q, need_k, need_v = ctx.needs_input_grad[:3]
+        if FUSED_KV:
+            made = _lib.native().attn_bwd(ctx.tables.native(), do, *saved[:5], ctx.scale, saved[5], *ctx.kpm_args, need_q, need_k, need_v)
+            if made is not None:
+                return made + (None,) * 5
+        do = _near(do)
         dq = dk = dv = None
         rows = (q.size(0), q.size(1), 2, ctx.tables.lines * 64)      # (the rows of a head as far apart as those of lse; the second half is not used)
         delta = None

@@ -120,7 +120,13 @@ class _sparse_softmax(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, scale, rpe, key_padding_mask, attn_mask, kp_mask_mode, attn_mask_mode,
-                spdims, block, lut, maxlut, bench, time, dropout=None):
+                spdims, block, lut, maxlut, bench, time, dropout=None, tables=None):
+        ctx.tables = tables = None if bench or dropout is not None else tables
+        if tables is not None and _lib.native().softmax_fwd(tables, x, scale, rpe, key_padding_mask, attn_mask, kp_mask_mode == 'mul', attn_mask_mode == 'mul'):
+            ctx.mark_dirty(x)
+            ctx.save_for_backward(x, lut)
+            ctx.dropout, ctx.spdims, ctx.block, ctx.maxlut, ctx.scale = None, spdims, block, maxlut, scale
+            return x
         _lib.require_gpu_tensor(x, 'softmax input')
         if x.dtype not in _lib.DTYPES:
             raise ValueError('softmax input must be float16, bfloat16 or float32')
@@ -187,6 +193,8 @@ class _sparse_softmax(torch.autograd.Function):
         if dx.data_ptr() % 16 != 0 or not private:
             dx = torch.empty_like(dx).copy_(dx)
         _sparse_softmax.in_place_backwards += int(private)
+        if ctx.tables is not None and _lib.native().softmax_bwd(ctx.tables, x, dx, ctx.scale):
+            return (dx,) + (None,) * 14
         args = (_lib.DTYPES[x.dtype], _lib.ptr(x), _lib.ptr(dx), float(ctx.scale), _lib.ptr(lut), ctx.maxlut, x.size(0),
                 ctx.spdims[0], ctx.spdims[1], ctx.block, x.stride(0), dx.stride(0))
         if ctx.dropout is None:
@@ -200,7 +208,7 @@ class _sparse_softmax(torch.autograd.Function):
             rc = _lib.load().bsp_softmax_bwd(*(args[:2] + (_lib.ptr(extra),) + args[3:-1] + (extra.stride(0),)), _lib.stream_ptr(x.device))
             _lib.check(rc, 'bsp_softmax_bwd')
             dx = dx + extra
-        return (dx,) + (None,) * 13
+        return (dx,) + (None,) * 14
 
 
 class Softmax:
@@ -214,6 +222,21 @@ class Softmax:
             self.lut_cache[key] = _sparse_softmax.make_lut(self.layout, self.block, device)
         return self.lut_cache[key]
 
+    def _tables(self, device, lut, maxlut):
+        """what the native launcher (csrc/launch.cpp) wants to know of the table, made once per device"""
+        held = self._native.get(device)
+        if held is None or held[0] is not lut:
+            H, R, C = [int(n) for n in self.spdims]
+            dev = device.index if device.index is not None else torch.cuda.current_device()
+            held = self._native[device] = (lut, _lib.native().make_rows(lut, lut.data_ptr(), maxlut, dev, (lut.numel() - 2 * H * R) // 4, H, R, C, self.block))
+        return held[1]
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != '_native'}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state, _native=dict())
+
     def __init__(self, layout, block, bench=False):
         if block not in (16, 32, 64, 128):
             raise ValueError('block must be 16, 32, 64 or 128')
@@ -222,6 +245,7 @@ class Softmax:
         self.block = block
         self.bench = bench
         self.lut_cache = dict()
+        self._native = dict()
         self.time_y = None
 
     def __call__(self, x, scale=1., rpe=None, key_padding_mask=None, attn_mask=None,
@@ -246,6 +270,6 @@ class Softmax:
             seed = int(torch.randint(0, 2 ** 62, (1,)).item()) if dropout_seed is None else int(dropout_seed)
             dropout = (float(dropout_p), seed, int(dropout_offset))
         x = Softmax.sparse_softmax(x, scale, rpe, key_padding_mask, attn_mask, key_padding_mask_mode, attn_mask_mode,
-                                   self.spdims, self.block, lut, maxlut, self.bench, time_y, dropout)
+                                   self.spdims, self.block, lut, maxlut, self.bench, time_y, dropout, self._tables(x.device, lut, maxlut))
         self.time_y = time_y[0]
         return x if dropout is None else x[0]

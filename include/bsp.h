@@ -148,8 +148,9 @@ typedef enum {
                                  the layout with every two block-rows merged, entries widened to 13 ints: position, 4 member ids,
                                  then the ids of the two blocks of each member, -1 where absent); plan_lines counts the pairs.  Such a
                                  plan serves the long-reduction kernel (K >= 256, K % 32 == 0, 16-bit types) and nothing else */
-  BSP_FLAG_ANY_K = 16         /* bsp_sdd_matmul_levels with trans_a and not trans_b (the reduction runs along the rows of both operands): K need
+  BSP_FLAG_ANY_K = 16,        /* bsp_sdd_matmul_levels with trans_a and not trans_b (the reduction runs along the rows of both operands): K need
                                  not be a multiple of 16 */
+  BSP_FLAG_WHOLE_K = 32        /* bsp_sdd_parts: one part whatever the sizes (for cross-checks) */
 } bsp_launch_flags;
 
 /* sparse = dense x dense: replaces _sparse_matmul._sdd_matmul + the SDD branch of the kernel
@@ -180,7 +181,12 @@ int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, void *c, int 
                           int64_t a_stride_z, int64_t a_stride_h, int64_t lda, int64_t b_stride_z, int64_t b_stride_h,
                           int64_t ldb, int64_t c_stride_z, int block, int n_levels, const int *packs, const int32_t *const *d_luts,
                           const uint8_t *const *d_valids, const int64_t *n_groups, const int32_t *d_gplan, int n_plan_groups, int plan_lines,
-                          int flags, void *stream);
+                          int parts, int64_t n_blocks, void *d_ws, int64_t ws_bytes, int flags, void *stream);
+/* parts > 1: the reduction is cut into that many parts, which run side by side on the general kernels and leave fp32 blocks in d_ws
+ * (bsp_sdd_parts_workspace_bytes(block, n_blocks, Z, parts) bytes, 16-byte aligned, no initialisation needed; n_blocks: blocks of the
+ * layout); a second launch adds them in order.  bsp_sdd_parts says how many parts suit a product (1: leave it whole). */
+int bsp_sdd_parts(int dtype, int block, int n_levels, const int *packs, const int64_t *n_groups, int Z, int K, int flags);
+int64_t bsp_sdd_parts_workspace_bytes(int block, int64_t n_blocks, int Z, int parts);
 
 /* sparse = dense x dense over a long reduction into few blocks of 128, the reduction cut into `parts` parts that run side by
  * side: replaces _sparse_matmul._sdd_matmul (matmul.py:299-364) where the reference would have used the split-K lock path of

@@ -58,11 +58,63 @@ def test_one_call_for_all_levels_gives_the_bits_of_a_call_per_level(block):
     n = len(luts)
     arrays = ((ctypes.c_int * n)(*packs), (ctypes.c_void_p * n)(*[t.data_ptr() for t in luts]),
               (ctypes.c_void_p * n)(*[None if v is None else v.data_ptr() for v in valid]), (ctypes.c_int64 * n)(*widths))
-    assert lib.bsp_sdd_matmul_levels(*args(one), n, *arrays, null, 0, 0, 0, st) == _lib.OK
+    tail = (null, 0, 0, 1, 0, null, 0, 0, st)
+    assert lib.bsp_sdd_matmul_levels(*args(one), n, *arrays, *tail) == _lib.OK
     torch.cuda.synchronize()
     assert not bool(torch.isnan(one).any()) and torch.equal(one, many)
     # the same level twice, a level that the block size does not have, no level
     twice = (ctypes.c_int * n)(*([packs[0]] * n))
-    assert lib.bsp_sdd_matmul_levels(*args(one), n, twice, *arrays[1:], null, 0, 0, 0, st) == _lib.ERR_UNSUPPORTED
-    assert lib.bsp_sdd_matmul_levels(*args(one), 1, (ctypes.c_int * 1)(8), *arrays[1:], null, 0, 0, 0, st) == _lib.ERR_UNSUPPORTED
-    assert lib.bsp_sdd_matmul_levels(*args(one), 0, *arrays, null, 0, 0, 0, st) < 0
+    assert lib.bsp_sdd_matmul_levels(*args(one), n, twice, *arrays[1:], *tail) == _lib.ERR_UNSUPPORTED
+    assert lib.bsp_sdd_matmul_levels(*args(one), 1, (ctypes.c_int * 1)(8), *arrays[1:], *tail) == _lib.ERR_UNSUPPORTED
+    assert lib.bsp_sdd_matmul_levels(*args(one), 0, *arrays, *tail) < 0
+
+
+@pytest.mark.parametrize('block,dtype', [(16, torch.float32), (32, torch.float32), (32, torch.bfloat16), (64, torch.float32), (64, torch.float16), (128, torch.float32)])
+@pytest.mark.parametrize('K', [784, 1600, 3120])
+def test_few_blocks_over_a_long_reduction_run_in_parts(block, dtype, K):
+    # 784: the first reductions that are cut at fp32; 3120 = 97.5 steps of 32: the last part is shorter, and half a step is past the end
+    n = 4 if block < 128 else 2
+    lay = torch.zeros(2, n, n, dtype=torch.int64)
+    lay[0, :2, :2] = 1
+    lay[:, n - 1, 1] = 1
+    lay[1, 0, 0] = 1
+    lib = _lib.load()
+    for ta, tb_, Z in ((True, False, 1), (False, True, 2)):
+        for rep in range(2):
+            run_matmul_case('sdd', ta, tb_, block, dtype, Z=Z, H=2, M=n * block, N=n * block, K=K, layout=lay, dist='randn', scale=K ** -0.5, seed=K, backward=False)
+    packs, n_groups = (ctypes.c_int * 1)(1), (ctypes.c_int64 * 1)(7)
+    parts = lib.bsp_sdd_parts(_lib.DTYPES[dtype], block, 1, packs, n_groups, 1, K, 0)
+    steps = -(-K // (16 if dtype == torch.float32 else 32))
+    assert (parts > 1) == (steps >= (48 if dtype == torch.float32 else 96)) and (parts - 1) * -(-steps // parts) < steps
+    assert lib.bsp_sdd_parts(_lib.DTYPES[dtype], block, 1, packs, n_groups, 1, K, _lib.FLAG_WHOLE_K) == 1
+
+
+def test_parts_give_the_same_bits_every_time_and_refuse_a_small_workspace():
+    torch.manual_seed(3)
+    lay = _layout(32, 'all')
+    luts, _, widths, packs = _sparse_matmul.make_sdd_lut(lay, 32, torch.float32, torch.device(DEV))
+    K, nnz = 2000, int(lay.sum())
+    a, b = torch.randn(2, 2, K, 256, device=DEV), torch.randn(2, 2, K, 256, device=DEV)
+    lib, n, null, st = _lib.load(), len(luts), ctypes.c_void_p(0), _lib.stream_ptr(torch.device(DEV))
+    valid = [getattr(t, 'valid', None) for t in luts]
+    arrays = ((ctypes.c_int * n)(*packs), (ctypes.c_void_p * n)(*[t.data_ptr() for t in luts]),
+              (ctypes.c_void_p * n)(*[None if v is None else v.data_ptr() for v in valid]), (ctypes.c_int64 * n)(*widths))
+
+    def run(parts, ws_bytes=None):
+        c = torch.full((2, nnz, 32, 32), float('nan'), device=DEV)
+        need = lib.bsp_sdd_parts_workspace_bytes(32, nnz, 2, parts)
+        ws = torch.full((max(need, 16),), 255, dtype=torch.uint8, device=DEV)         # (not a number, read as floats)
+        rc = lib.bsp_sdd_matmul_levels(_lib.F32, _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), 1, 0, 2, K, a.stride(0), a.stride(1), 256, b.stride(0), b.stride(1), 256,
+                                       c.stride(0), 32, n, *arrays, null, 0, 0, parts, nnz, _lib.ptr(ws), need if ws_bytes is None else ws_bytes, 0, st)
+        torch.cuda.synchronize()
+        return rc, c
+
+    rc, one = run(1)
+    assert rc == _lib.OK
+    for parts in (2, 5, 16):
+        rc, c = run(parts)
+        again = run(parts)[1]
+        bound = 1e-5 * (a.abs().transpose(2, 3) @ b.abs()).max()
+        assert rc == _lib.OK and torch.equal(c, again) and float((c - one).abs().max()) <= float(bound)
+    assert run(4, 1024)[0] == _lib.ERR_CAPACITY
+    assert run(126)[0] < 0 and run(125)[0] == _lib.OK                                 # (125 steps: 126 parts would leave one empty)

@@ -37,11 +37,41 @@ extern "C" const char *bsp_strerror(int status) {
   }
 }
 
+// Into how many parts the reduction of an sdd product on the general kernels is cut: launches that do not fill the chip (three
+// workgroups a compute unit) and whose workgroups run many steps one after the other.  Whole / in parts, us, blocks as workgroups
+// (a block of 128 counts as four): fp32, 92 of them, 340 steps 136 / 54 (8 parts), 53 steps 24 / 20 (3); 197, 125 steps 53 / 48
+// (4); 407, 512 steps 345 / 269 (4); 24, 120 steps 53 / 15 (7); 28 + 2 of four blocks of 32, 60 steps 26 / 13 (3); 174, 44 steps 22 / 22;
+// 254, 32 steps 15.5 / 17.4; 24 steps and fewer: the second launch costs more than the parts gain.  16-bit types take twice the
+// elements a step and less time for it: 92, 170 steps 40 / 19 (8); 24, 32 steps 9.2 / 11.8; 407, 256 steps 73 / 77.
+extern "C" int bsp_sdd_parts(int dtype, int block, int n_levels, const int *packs, const int64_t *n_groups, int Z, int K, int flags) {
+  if (!block_ok(block) || n_levels < 1 || !packs || !n_groups || Z <= 0 || K <= 0 || (flags & BSP_FLAG_WHOLE_K)) return 1;
+  int64_t wgs = 0;
+  for (int i = 0; i < n_levels; i++) {
+    const int tile = block * packs[i];
+    wgs += tile >= 128 ? n_groups[i] * (n_groups[i] * Z < 512 ? 4 : 1) : tile < 32 ? (n_groups[i] + 3) / 4 : n_groups[i];
+  }
+  wgs *= Z;
+  const bool f32 = dtype == BSP_F32;
+  const int unit = f32 ? 16 : 32, steps = (K + unit - 1) / unit;
+  if (wgs <= 0 || wgs > (f32 ? 512 : 256) || steps < (f32 ? 48 : 96)) return 1;
+  int64_t parts = 800 / wgs;
+  if (f32 && parts < steps / 128) parts = steps / 128;
+  if (parts > steps / 16) parts = steps / 16;
+  if (parts > 16) parts = 16;
+  if (parts <= 1) return 1;
+  const int per = (int)((steps + parts - 1) / parts);
+  return (steps + per - 1) / per;                      // (no part is empty)
+}
+
+extern "C" int64_t bsp_sdd_parts_workspace_bytes(int block, int64_t n_blocks, int Z, int parts) {
+  return parts > 1 && n_blocks > 0 && Z > 0 ? (int64_t)parts * Z * n_blocks * block * block * (int64_t)sizeof(float) : 0;
+}
+
 extern "C" int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, void *c, int trans_a, int trans_b, int Z, int K,
                                      int64_t a_stride_z, int64_t a_stride_h, int64_t lda, int64_t b_stride_z, int64_t b_stride_h,
                                      int64_t ldb, int64_t c_stride_z, int block, int n_levels, const int *packs, const int32_t *const *d_luts,
                                      const uint8_t *const *d_valids, const int64_t *n_groups, const int32_t *d_gplan, int n_plan_groups,
-                                     int plan_lines, int flags, void *stream) {
+                                     int plan_lines, int parts, int64_t n_blocks, void *d_ws, int64_t ws_bytes, int flags, void *stream) {
   if (!a || !b || !c || Z <= 0 || K <= 0 || n_levels < 1 || n_levels > 3 || !packs || !d_luts || !d_valids || !n_groups) return BSP_ERR_ARG;
   SddLevel levels[3];
   for (int i = 0; i < n_levels; i++) {
@@ -64,7 +94,15 @@ extern "C" int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, vo
   // op(A)[m][k]: reduction contiguous unless A is read transposed; op(B)[k][n]: contiguous when B is read transposed
   const bool a_kc = !trans_a, b_kc = trans_b != 0;
   hipStream_t st = as_stream(stream);
-  int rc = general_only(flags) || K % 16 ? 0 : sdd_fast64(dtype, g, block, packs[0], a_kc, b_kc, st);
+  if (parts > 1) {
+    if (n_blocks <= 0 || !d_ws || !aligned16(d_ws) || c_stride_z < n_blocks * block * block) return BSP_ERR_ARG;
+    if (ws_bytes < bsp_sdd_parts_workspace_bytes(block, n_blocks, Z, parts)) return BSP_ERR_CAPACITY;
+    const int unit = dtype == BSP_F32 ? 16 : 32;       // whole reduction steps
+    g.parts = parts; g.n_blocks = n_blocks; g.ws = reinterpret_cast<float *>(d_ws);
+    g.part_k = ((K + unit - 1) / unit + parts - 1) / parts * unit;
+    if ((int64_t)g.part_k * (parts - 1) >= K) return BSP_ERR_ARG;   // (a part would be empty)
+  }
+  int rc = general_only(flags) || K % 16 || parts > 1 ? 0 : sdd_fast64(dtype, g, block, packs[0], a_kc, b_kc, st);
   if (rc < 0) return rc;
   // (a kernel that works from the plan writes the whole layout; the one for a single level serves blocks of 64, which have no other)
   if (rc >= 1) { BSP_LAUNCH_CHECK(); return rc == 2 ? BSP_OK_WHOLE_LAYOUT : BSP_OK; }
@@ -86,7 +124,7 @@ extern "C" int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, 
                               int plan_lines, int flags, void *stream) {
   if (d_lut)
     return bsp_sdd_matmul_levels(dtype, a, b, c, trans_a, trans_b, Z, K, a_stride_z, a_stride_h, lda, b_stride_z, b_stride_h, ldb, c_stride_z, block,
-                                 1, &pack, &d_lut, &d_valid, &n_groups, d_gplan, n_plan_groups, plan_lines, flags, stream);
+                                 1, &pack, &d_lut, &d_valid, &n_groups, d_gplan, n_plan_groups, plan_lines, 1, 0, nullptr, 0, flags, stream);
   if (!a || !b || !c || Z <= 0 || K <= 0 || n_groups < 0) return BSP_ERR_ARG;
   if (!d_gplan || no_groups(flags) || general_only(flags)) return d_gplan ? BSP_NEEDS_TABLE : BSP_ERR_ARG;
   if (!block_ok(block)) return BSP_ERR_UNSUPPORTED;

@@ -270,6 +270,13 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   return checked(rc, dds ? "bsp_dds_matmul" : "bsp_dsd_matmul") ? c.release() : nullptr;
 }
 
+// the workspace that is kept with the tables, `need` bytes of it; nullptr with the error set
+void *splitk_workspace(const Sdd *s, int64_t need, const Operand &like) {
+  Ref dev(PyObject_GetAttr(like.obj, s_device));
+  Ref at(dev.o ? PyObject_CallMethod(PyTuple_GET_ITEM(s->keep, 0), "splitk_workspace", "LO", (long long)need, dev.o) : nullptr);
+  return at.o ? PyLong_AsVoidPtr(at.o) : nullptr;
+}
+
 // sdd(tables, a, b, trans_a, trans_b, trans_c, flags): bsp_sdd_matmul with the plan alone where a kernel takes it, else all pack levels
 PyObject *sdd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != 7) { PyErr_SetString(PyExc_TypeError, "sdd takes 7 arguments"); return nullptr; }
@@ -321,16 +328,18 @@ PyObject *sdd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (s->n_levels < 0) Py_RETURN_NONE;                  // (nothing was launched)
   if (parts) {
     const int64_t need = bsp_sdd_splitk_workspace_bytes((int)Z, s->widths[0], parts);
-    if (need) {                                         // (kept with the tables)
-      Ref dev(PyObject_GetAttr(a.obj, s_device));
-      Ref at(dev.o ? PyObject_CallMethod(PyTuple_GET_ITEM(s->keep, 0), "splitk_workspace", "LO", (long long)need, dev.o) : nullptr);
-      if (!at.o || !(wsp = PyLong_AsVoidPtr(at.o))) return nullptr;
-    }
+    if (need && !(wsp = splitk_workspace(s, need, a))) return nullptr;
     rc = unlocked([&] { return bsp_sdd_matmul_splitk(BSP_OPERANDS, s->luts[0], s->valids[0], s->widths[0], parts, wsp, need, flags, st); });
     if (rc != BSP_ERR_UNSUPPORTED) return checked(rc, "bsp_sdd_matmul_splitk") ? c.release() : nullptr;
   }
   if (s->n_levels == 0) return c.release();
-  rc = unlocked([&] { return bsp_sdd_matmul_levels(BSP_OPERANDS, s->n_levels, s->packs, s->luts, s->valids, s->widths, s->ordinary.table, s->ordinary.n_groups, s->ordinary.lines, flags, st); });
+  parts = bsp_sdd_parts(s->dtype, s->block, s->n_levels, s->packs, s->widths, (int)Z, (int)K, flags);
+  const int64_t need = bsp_sdd_parts_workspace_bytes(s->block, s->nnz, (int)Z, parts);
+  if (need && !(wsp = splitk_workspace(s, need, a))) return nullptr;
+  rc = unlocked([&] {
+    return bsp_sdd_matmul_levels(BSP_OPERANDS, s->n_levels, s->packs, s->luts, s->valids, s->widths, s->ordinary.table, s->ordinary.n_groups, s->ordinary.lines, parts, s->nnz,
+                                 wsp, need, flags, st);
+  });
 #undef BSP_OPERANDS
   return rc == BSP_OK_WHOLE_LAYOUT || checked(rc, "bsp_sdd_matmul_levels") ? c.release() : nullptr;
 }

@@ -196,7 +196,8 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
   // ksteps = number of TK-wide reduction steps.  Store(m, n, vals): vals[4] run along n (OUT_NCONTIG) or m.
   // SUB > 0: the output consists of SUB x SUB blocks that are each contiguous in memory (the sparse result of sdd);
   // the epilogue then writes block by block.  SUB == 0: the output is a matrix with long rows.
-  template <int SUB = 0, class XView, class YView, class Store>
+  // PARTIAL: the result is a part of a sum; store takes the fp32 values (f32x4) as they are.
+  template <int SUB = 0, bool PARTIAL = false, class XView, class YView, class Store>
   static __device__ __forceinline__ void run(const XView &xv, const YView &yv, int ksteps, T *smem, const Store &store) {
     const int tid = threadIdx.x % NT, lane = tid & 63, wave = tid >> 6;   // (a workgroup may hold several products of one wavefront)
     const int wm = wave / WGN, wn = wave % WGN;
@@ -275,6 +276,18 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
     // time through its own piece of LDS (free after the last barrier) and writes whole 16-byte chunks, consecutive
     // lanes along a row.  store(r, c, chunk): r = row (m if OUT_NCONTIG, else n), c = first of VE consecutive columns.
     constexpr int VE = 16 / (int)sizeof(T);
+    if constexpr (PARTIAL) {
+      // (straight from the accumulators, 16 bytes a lane: parts are few, and what reads them next finds them in L2)
+      static_assert(OUT_NCONTIG, "parts are written along n");
+#pragma unroll
+      for (int i = 0; i < RM; i++)
+#pragma unroll
+        for (int j = 0; j < RN; j++)
+#pragma unroll
+          for (int g4 = 0; g4 < M::NACC / 4; g4++)
+            store((wm * RM + i) * MS + lane % MS, (wn * RN + j) * MS + (MS == 16 ? 4 * (lane >> 4) : 8 * g4 + 4 * (lane >> 5)),
+                  f32x4{acc[i][j][4 * g4], acc[i][j][4 * g4 + 1], acc[i][j][4 * g4 + 2], acc[i][j][4 * g4 + 3]});
+    } else {
     if constexpr (SUB > 0 && OUT_NCONTIG && TM * (TN + VE) * (int)sizeof(T) <= SMEM_BYTES) {
       // Blocked output: the whole TM x TN tile is staged (all wavefronts, two barriers) and then written block by
       // block, consecutive lanes on consecutive 16-byte chunks of one block: 512 contiguous bytes per 32 lanes at
@@ -349,6 +362,7 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
       }
       __builtin_amdgcn_wave_barrier();
     }
+    }
   }
 };
 
@@ -366,6 +380,10 @@ struct SddArgs {
   int64_t n_groups;
   const int32_t *gplan; int n_pgroups; int lines;   // optional group plan (by rows), its groups, block-rows per head
   int cols = 0;                                       // block-columns per head when known (a call with the plan alone), else 0
+  // the reduction cut into parts of part_k elements, whose fp32 sums go to ws [part][Z][n_blocks][block][block]
+  int parts = 1, part_k = 0;
+  int64_t n_blocks = 0;
+  float *ws = nullptr;
 };
 
 struct SddLevel { int pack; const int32_t *lut; const uint8_t *valid; int64_t n; };   // one pack level of the sdd table, n super-blocks
@@ -376,9 +394,10 @@ template <typename T, int BLOCK, int PACK, bool KCONTIG> struct SddView {
   typedef int idx_t __attribute__((ext_vector_type(PACK == 1 ? 2 : PACK)));
   const T *base; int64_t ld; int K; idx_t idx;   // base doubles as the dummy address of out-of-range chunks
   int off = 0;                                        // first row of the tile inside its block (tiles smaller than a block)
+  int first = 0;                                      // where the reduction starts (K: where it ends)
   static constexpr int NB = 1;
   struct Step { int k0; bool live[1]; int klim; };
-  __device__ __forceinline__ Step step(int k0) const { return Step{k0, {true}, K - k0}; }
+  __device__ __forceinline__ Step step(int k0) const { return Step{first + k0, {true}, K - first - k0}; }
   __device__ __forceinline__ int blk(int row) const {
     int r = idx[0];
 #pragma unroll
@@ -394,8 +413,8 @@ template <typename T, int BLOCK, int PACK, bool KCONTIG> struct SddView {
 template <int T_> struct SddShape { static constexpr int WG = T_ >= 32 ? 2 : 1; };
 
 // One super-block, by the SddShape<BLOCK * PACK>::WG squared wavefronts that call it together
-template <typename T, int BLOCK, int PACK, bool A_KCONTIG, bool B_KCONTIG>
-__device__ __forceinline__ void sdd_super_block(const SddArgs &g, const int32_t *lut, const uint8_t *all_valid, int z, int64_t grp, bool keep, unsigned char *smem) {
+template <typename T, int BLOCK, int PACK, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
+__device__ __forceinline__ void sdd_super_block(const SddArgs &g, const int32_t *lut, const uint8_t *all_valid, int part, int z, int64_t grp, bool keep, unsigned char *smem) {
   constexpr int TT = BLOCK * PACK, WG = SddShape<TT>::WG;
   typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
   const table_ptr e = as_table(lut) + grp * (PACK * PACK * 4);
@@ -409,6 +428,10 @@ __device__ __forceinline__ void sdd_super_block(const SddArgs &g, const int32_t 
     av.idx[p] = e[(p * PACK) * 4 + 1];   // block-row of entries (p, 0)
     bv.idx[p] = e[p * 4 + 2];            // block-col of entries (0, p)
   }
+  if constexpr (PARTS) {
+    av.first = bv.first = part * g.part_k;
+    if (av.first + g.part_k < g.K) av.K = bv.K = av.first + g.part_k;
+  }
   T *cz = reinterpret_cast<T *>(g.c) + z * g.c_sz;
   const uint8_t *valid = all_valid ? all_valid + grp * (PACK * PACK) : nullptr;
   // The entry differs from lane to lane here, so the output block is looked up through an ordinary pointer (a vector
@@ -421,15 +444,48 @@ __device__ __forceinline__ void sdd_super_block(const SddArgs &g, const int32_t 
     const int64_t bk = eg[ent * 4 + 3];
     *reinterpret_cast<u32x4 *>(cz + bk * (BLOCK * BLOCK) + (m % BLOCK) * BLOCK + n % BLOCK) = v;
   };
-  G::template run<BLOCK>(av, bv, (g.K + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem), store);
+  if constexpr (PARTS) {
+    float *ws = g.ws + ((int64_t)part * g.Z + z) * g.n_blocks * (BLOCK * BLOCK);
+    auto store_part = [&](int m, int n, f32x4 v) {
+      const int ent = (m / BLOCK) * PACK + n / BLOCK;
+      if (!keep || (valid && !valid[ent])) return;
+      *reinterpret_cast<f32x4 *>(ws + (int64_t)eg[ent * 4 + 3] * (BLOCK * BLOCK) + (m % BLOCK) * BLOCK + n % BLOCK) = v;
+    };
+    // (every part of every wavefront runs the same number of steps: those past the end of the reduction multiply zeros)
+    G::template run<BLOCK, true>(av, bv, (g.part_k + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem), store_part);
+  } else {
+    G::template run<BLOCK>(av, bv, (g.K + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem), store);
+  }
 }
 
-template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG>
+template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __global__ void __launch_bounds__(64 * SddShape<BLOCK>::WG * SddShape<BLOCK>::WG) k_sdd(SddArgs g) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int64_t n_wg = g.n_groups * g.Z;
-  const int64_t w = xcd_remap(blockIdx.x, n_wg);
-  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG>(g, g.lut, g.valid, (int)(w / g.n_groups), w % g.n_groups, true, smem_raw);
+  const int64_t w = xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg);
+  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG, PARTS>(g, g.lut, g.valid, PARTS ? (int)(w / n_wg) : 0, (int)(w % n_wg / g.n_groups), w % g.n_groups, true, smem_raw);
+}
+
+// The second pass of an sdd in parts: the parts of every block in order, rounded once
+template <typename T> __global__ void __launch_bounds__(256) k_sdd_parts_sum(SddArgs g, int64_t per_z) {   // per_z: groups of four values of a batch's blocks
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, all = per_z * g.Z;
+  if (i >= all) return;
+  const f32x4 *ws = reinterpret_cast<const f32x4 *>(g.ws) + i;
+  f32x4 sum = ws[0];
+  for (int p = 1; p < g.parts; p++) {
+    const f32x4 v = ws[p * all];
+#pragma unroll
+    for (int e = 0; e < 4; e++) sum[e] += v[e];
+  }
+  T *c = reinterpret_cast<T *>(g.c) + (i / per_z) * g.c_sz + (i % per_z) * 4;
+  if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<f32x4 *>(c) = sum;
+  } else {
+    union { u32x2 raw; T e[4]; } u;
+#pragma unroll
+    for (int e = 0; e < 4; e++) u.e[e] = from_float<T>(sum[e]);
+    *reinterpret_cast<u32x2 *>(c) = u.raw;
+  }
 }
 
 // Blocks of 16 and 32: every pack level of the table in one launch, the largest super-blocks first.  A launch per level
@@ -449,14 +505,15 @@ template <typename T, int BLOCK, bool AK, bool BK> struct SddLevelsShape {
   static constexpr int SMEM = max_of(max_of(G<PACK0>::SMEM_BYTES, G<PACK0 / 2>::SMEM_BYTES), LAST_PER_WG * G<1>::SMEM_BYTES);
 };
 
-template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG>
-__global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> lv) {
+template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
+__global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> lv, int64_t per_part) {
   typedef SddLevelsShape<T, BLOCK, A_KCONTIG, B_KCONTIG> S;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  int64_t w = blockIdx.x, n = lv.n[0] * g.Z;
+  const int part = PARTS ? (int)(blockIdx.x / per_part) : 0;
+  int64_t w = PARTS ? blockIdx.x % per_part : blockIdx.x, n = lv.n[0] * g.Z;
   if (w < n) {
     w = xcd_remap(w, n);
-    sdd_super_block<T, BLOCK, S::PACK0, A_KCONTIG, B_KCONTIG>(g, lv.lut[0], lv.valid[0], (int)(w / lv.n[0]), w % lv.n[0], true, smem_raw);
+    sdd_super_block<T, BLOCK, S::PACK0, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[0], lv.valid[0], part, (int)(w / lv.n[0]), w % lv.n[0], true, smem_raw);
     return;
   }
   w -= n;
@@ -464,7 +521,7 @@ __global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> 
     n = lv.n[1] * g.Z;
     if (w < n) {
       w = xcd_remap(w, n);
-      sdd_super_block<T, 16, 2, A_KCONTIG, B_KCONTIG>(g, lv.lut[1], lv.valid[1], (int)(w / lv.n[1]), w % lv.n[1], true, smem_raw);
+      sdd_super_block<T, 16, 2, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[1], lv.valid[1], part, (int)(w / lv.n[1]), w % lv.n[1], true, smem_raw);
       return;
     }
     w -= n;
@@ -472,24 +529,24 @@ __global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> 
   constexpr int LAST = SddLevels<BLOCK>::N - 1, PER = S::LAST_PER_WG;
   const int64_t last = lv.n[LAST] * g.Z;
   w = xcd_remap(w, (last + PER - 1) / PER);
-  const int part = PER == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t i = w * PER + part, j = i < last ? i : last - 1;
-  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG>(g, lv.lut[LAST], lv.valid[LAST], (int)(j / lv.n[LAST]), j % lv.n[LAST], i < last,
-                                                     smem_raw + part * S::template G<1>::SMEM_BYTES);
+  const int own = PER == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t i = w * PER + own, j = i < last ? i : last - 1;
+  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[LAST], lv.valid[LAST], part, (int)(j / lv.n[LAST]), j % lv.n[LAST], i < last,
+                                                            smem_raw + own * S::template G<1>::SMEM_BYTES);
 }
 
 // sdd with SPLIT x SPLIT workgroups per block (pack 1): for layouts with so few blocks that one workgroup per block
 // would leave most of the chip idle (a 10 % dense 32 x 32 layout of 128-blocks has 100 blocks for 256 CUs).  The
 // sub-tiles of a block are neighbours in the grid, so that they meet their shared operand rows in L2.
-template <typename T, int BLOCK, int SPLIT, bool A_KCONTIG, bool B_KCONTIG>
+template <typename T, int BLOCK, int SPLIT, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __global__ void __launch_bounds__(64 * SddShape<BLOCK / SPLIT>::WG * SddShape<BLOCK / SPLIT>::WG) k_sdd_split(SddArgs g) {
   constexpr int TT = BLOCK / SPLIT, WG = SddShape<TT>::WG;
   typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int64_t n_wg = g.n_groups * g.Z * (SPLIT * SPLIT);
-  const int64_t w = xcd_remap(blockIdx.x, n_wg);
-  const int sub = (int)(w % (SPLIT * SPLIT));
-  const int z = (int)(w / (SPLIT * SPLIT) / g.n_groups);
+  const int64_t w = xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg);
+  const int sub = (int)(w % (SPLIT * SPLIT)), part = PARTS ? (int)(w / n_wg) : 0;
+  const int z = (int)(w % n_wg / (SPLIT * SPLIT) / g.n_groups);
   const int64_t grp = w / (SPLIT * SPLIT) % g.n_groups;
   const table_ptr e = as_table(g.lut) + grp * 4;
   if (g.valid && !g.valid[grp]) return;
@@ -499,6 +556,13 @@ __global__ void __launch_bounds__(64 * SddShape<BLOCK / SPLIT>::WG * SddShape<BL
   bv.base = reinterpret_cast<const T *>(g.b) + z * g.b_sz + e[0] * g.b_sh; bv.ld = g.ldb; bv.K = g.K;
   av.idx[0] = e[1]; av.off = (sub / SPLIT) * TT;
   bv.idx[0] = e[2]; bv.off = (sub % SPLIT) * TT;
+  if constexpr (PARTS) {
+    av.first = bv.first = part * g.part_k;
+    if (av.first + g.part_k < g.K) av.K = bv.K = av.first + g.part_k;
+    float *ws = g.ws + (((int64_t)part * g.Z + z) * g.n_blocks + e[3]) * (BLOCK * BLOCK) + av.off * BLOCK + bv.off;
+    G::template run<0, true>(av, bv, (g.part_k + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem_raw), [&](int m, int n, f32x4 v) { *reinterpret_cast<f32x4 *>(ws + m * BLOCK + n) = v; });
+    return;
+  }
   T *cb = reinterpret_cast<T *>(g.c) + z * g.c_sz + (int64_t)e[3] * (BLOCK * BLOCK) + av.off * BLOCK + bv.off;
   auto store = [&](int m, int n, u32x4 v) { *reinterpret_cast<u32x4 *>(cb + m * BLOCK + n) = v; };
   G::run(av, bv, (g.K + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem_raw), store);
@@ -665,13 +729,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 // ---------------------------------------------------------------------------------------------------------
 template <typename T, int BLOCK> int launch_sdd_b(const SddArgs &g, bool a_kc, bool b_kc, hipStream_t st) {
   constexpr int WG = SddShape<BLOCK>::WG;
-  const int64_t n_wg = g.n_groups * g.Z;
+  const int64_t n_wg = g.n_groups * g.Z * g.parts;
   if (n_wg <= 0) return BSP_OK;
   if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
-  hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK>), grid, blockdim,                                                 \
-                     (TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true>::SMEM_BYTES), st, g)
+  do {                                                                                                           \
+    constexpr int SMEM = TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true>::SMEM_BYTES;                            \
+    if (g.parts > 1) hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, true>), grid, blockdim, SMEM, st, g);           \
+    else hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, false>), grid, blockdim, SMEM, st, g);                      \
+  } while (0)
   if (a_kc && b_kc) BSP_SDD_LAUNCH(true, true);
   else if (a_kc && !b_kc) BSP_SDD_LAUNCH(true, false);
   else if (!a_kc && b_kc) BSP_SDD_LAUNCH(false, true);
@@ -692,9 +759,14 @@ template <typename T, int BLOCK> int launch_sdd_levels(const SddArgs &g, const S
     n_wg += (levels[i].n * g.Z + per - 1) / per;
   }
   if (n_wg <= 0) return BSP_OK;
-  if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
-  dim3 grid((unsigned)n_wg), blockdim(256);
-#define BSP_SDD_LAUNCH(AK, BK) hipLaunchKernelGGL((k_sdd_levels<T, BLOCK, AK, BK>), grid, blockdim, (SddLevelsShape<T, BLOCK, AK, BK>::SMEM), st, g, lv)
+  if (n_wg * g.parts >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
+  dim3 grid((unsigned)(n_wg * g.parts)), blockdim(256);
+#define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
+  do {                                                                                                           \
+    constexpr int SMEM = SddLevelsShape<T, BLOCK, AK, BK>::SMEM;                                                 \
+    if (g.parts > 1) hipLaunchKernelGGL((k_sdd_levels<T, BLOCK, AK, BK, true>), grid, blockdim, SMEM, st, g, lv, n_wg); \
+    else hipLaunchKernelGGL((k_sdd_levels<T, BLOCK, AK, BK, false>), grid, blockdim, SMEM, st, g, lv, n_wg);     \
+  } while (0)
   if (a_kc && b_kc) BSP_SDD_LAUNCH(true, true);
   else if (a_kc && !b_kc) BSP_SDD_LAUNCH(true, false);
   else if (!a_kc && b_kc) BSP_SDD_LAUNCH(false, true);
@@ -705,12 +777,16 @@ template <typename T, int BLOCK> int launch_sdd_levels(const SddArgs &g, const S
 
 template <typename T, int BLOCK, int SPLIT> int launch_sdd_split(const SddArgs &g, bool a_kc, bool b_kc, hipStream_t st) {
   constexpr int TT = BLOCK / SPLIT, WG = SddShape<TT>::WG;
-  const int64_t n_wg = g.n_groups * g.Z * (SPLIT * SPLIT);
+  const int64_t n_wg = g.n_groups * g.Z * (SPLIT * SPLIT) * g.parts;
   if (n_wg <= 0) return BSP_OK;
+  if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
-  hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK>), grid, blockdim,                                    \
-                     (TileGemm<T, TT, TT, WG, WG, AK, BK, true>::SMEM_BYTES), st, g)
+  do {                                                                                                           \
+    constexpr int SMEM = TileGemm<T, TT, TT, WG, WG, AK, BK, true>::SMEM_BYTES;                                  \
+    if (g.parts > 1) hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, true>), grid, blockdim, SMEM, st, g); \
+    else hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, false>), grid, blockdim, SMEM, st, g);         \
+  } while (0)
   if (a_kc && b_kc) BSP_SDD_LAUNCH(true, true);
   else if (a_kc && !b_kc) BSP_SDD_LAUNCH(true, false);
   else if (!a_kc && b_kc) BSP_SDD_LAUNCH(false, true);
@@ -719,7 +795,7 @@ template <typename T, int BLOCK, int SPLIT> int launch_sdd_split(const SddArgs &
   return BSP_OK;
 }
 
-template <typename T> int launch_sdd(const SddArgs &g0, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st) {
+template <typename T> int launch_sdd_whole(const SddArgs &g0, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st) {
   if (block == 16) return launch_sdd_levels<T, 16>(g0, levels, n_levels, a_kc, b_kc, st);
   if (block == 32) return launch_sdd_levels<T, 32>(g0, levels, n_levels, a_kc, b_kc, st);
   if (n_levels != 1 || levels[0].pack != 1) return BSP_ERR_UNSUPPORTED;
@@ -730,6 +806,14 @@ template <typename T> int launch_sdd(const SddArgs &g0, int block, const SddLeve
   if (block == 64) return launch_sdd_b<T, 64>(g, a_kc, b_kc, st);
   if (block == 128) return launch_sdd_b<T, 128>(g, a_kc, b_kc, st);
   return BSP_ERR_UNSUPPORTED;
+}
+
+template <typename T> int launch_sdd(const SddArgs &g, int block, const SddLevel *levels, int n_levels, bool a_kc, bool b_kc, hipStream_t st) {
+  const int rc = launch_sdd_whole<T>(g, block, levels, n_levels, a_kc, b_kc, st);
+  if (rc != BSP_OK || g.parts <= 1) return rc;
+  const int64_t per_z = g.n_blocks * (block * block / 4);
+  hipLaunchKernelGGL((k_sdd_parts_sum<T>), dim3((unsigned)((per_z * g.Z + 255) / 256)), dim3(256), 0, st, g, per_z);
+  return BSP_OK;
 }
 
 template <typename T, int BLOCK, bool WIDE> int launch_xsd_bw(const XsdArgs &g0, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {

@@ -434,9 +434,13 @@ class _sparse_matmul(torch.autograd.Function):
                 return c
             n = len(luts)
             if n:
-                rc = lib.bsp_sdd_matmul_levels(*operands, n, (ctypes.c_int * n)(*packs), (ctypes.c_void_p * n)(*[t.data_ptr() for t in luts]),
+                c_packs, c_widths = (ctypes.c_int * n)(*packs), (ctypes.c_int64 * n)(*widths)
+                parts = lib.bsp_sdd_parts(operands[0], block, n, c_packs, c_widths, AS0, AS3, flags) if lazy else 1
+                need = lib.bsp_sdd_parts_workspace_bytes(block, total_width, AS0, parts)
+                rc = lib.bsp_sdd_matmul_levels(*operands, n, c_packs, (ctypes.c_void_p * n)(*[t.data_ptr() for t in luts]),
                                                (ctypes.c_void_p * n)(*[t.valid.data_ptr() if getattr(t, 'valid', None) is not None else None for t in luts]),
-                                               (ctypes.c_int64 * n)(*widths), gplan[0], gplan[1], gplan[2], flags, _lib.stream_ptr(a.device))
+                                               c_widths, gplan[0], gplan[1], gplan[2], parts, total_width,
+                                               ctypes.c_void_p(luts.splitk_workspace(need, a.device) if need else 0), need, flags, _lib.stream_ptr(a.device))
                 if rc != _lib.OK_WHOLE_LAYOUT:
                     _lib.check(rc, 'bsp_sdd_matmul_levels')
         time[0] = timer.done()

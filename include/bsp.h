@@ -150,7 +150,7 @@ typedef enum {
                                  plan serves the long-reduction kernel (K >= 256, K % 32 == 0, 16-bit types) and nothing else */
   BSP_FLAG_ANY_K = 16,        /* bsp_sdd_matmul_levels with trans_a and not trans_b (the reduction runs along the rows of both operands): K need
                                  not be a multiple of 16 */
-  BSP_FLAG_WHOLE_K = 32        /* bsp_sdd_parts: one part whatever the sizes (for cross-checks) */
+  BSP_FLAG_WHOLE_K = 32        /* bsp_sdd_parts, bsp_xsd_parts: one part whatever the sizes (for cross-checks) */
 } bsp_launch_flags;
 
 /* sparse = dense x dense: replaces _sparse_matmul._sdd_matmul + the SDD branch of the kernel
@@ -246,6 +246,18 @@ int bsp_dds_matmul(int dtype, const void *a, const void *b, void *c, int trans_a
                    int64_t c_stride_z, int64_t c_stride_h, int64_t ldc, int block, const int32_t *d_lut,
                    const int32_t *d_plan, int width, const int32_t *d_gplan, int n_plan_groups, int plan_lines,
                    int n_split, void *d_ws, int64_t ws_bytes, int flags, void *stream);
+
+/* dsd (is_dds = 0) or dds products in fp32 whose long segments run in parts: a segment of more than part_blocks blocks is taken by
+ * several workgroups, which leave fp32 tiles in d_ws (bsp_xsd_parts_workspace_bytes bytes, 16-byte aligned, no initialisation needed); a
+ * second launch adds them in order.  sp: the sparse operand, dn: the dense one, trans_a / trans_b / trans_c as in bsp_dsd_matmul resp.
+ * bsp_dds_matmul, tables as there.  bsp_xsd_parts: how many parts the longest segment (of `longest` blocks; nnz blocks in all) should
+ * make and how many blocks each takes; 1: none is worth cutting, call the ordinary entry point. */
+int bsp_xsd_parts(int dtype, int block, int width, int longest, int64_t nnz, int free_dim, int Z, int flags, int *part_blocks);
+int64_t bsp_xsd_parts_workspace_bytes(int block, int width, int free_dim, int Z, int parts);
+int bsp_xsd_matmul_parts(int is_dds, int dtype, const void *sp, const void *dn, void *c, int trans_a, int trans_b, int trans_c, int Z, int free_dim,
+                         int64_t sp_stride_z, int64_t dn_stride_z, int64_t dn_stride_h, int64_t ldd, int64_t c_stride_z, int64_t c_stride_h,
+                         int64_t ldc, int block, const int32_t *d_lut, const int32_t *d_plan, int width, int parts, int part_blocks, void *d_ws,
+                         int64_t ws_bytes, void *stream);
 
 /* ---------------------------------------------------------------------------------------------------
  * Softmax launchers: replace softmax_fwd / softmax_bwd and their dispatch (softmax.py:7-138, 144-194,

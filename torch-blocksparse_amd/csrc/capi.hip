@@ -250,6 +250,66 @@ extern "C" int bsp_dsd_matmul(int dtype, const void *a, const void *b, void *c, 
   return xsd_dispatch(dtype, g, block, trans_a != 0, trans_b != 0, !trans_c, flags, stream);
 }
 
+// Segments of how many blocks a dsd / dds product of the general kernels takes whole; returns how many parts the longest one makes (1:
+// all are taken whole).  fp32 only: the 16-bit kernels have plans of their own for long lines.  A launch ends with its longest
+// segments, which run alone: a global column of an attention layout is 64 blocks where the others are 4.  Whole / in parts, us, the
+// transposed product of 'fixed' layouts with a head dimension of 64 (longest segment, average): block 32, 64 of 19 blocks 62 / 53,
+// 61 of 10 59 / 39, 121 of 12 85 / 45; block 64, 16 of 7 30 / 21; block 16, 125 of 18 48 / 39, but 128 of 35 51 / 55 (its parts are read
+// and written as often as the blocks, so the line lies higher).  Launches that do not fill the chip: 27 segments of up to 54 blocks of
+// 64 107 / 27, 64 of up to 64 blocks of 32 115 / 38.  With equal segments, or more
+// workgroups than the chip holds, parts only cost (19 of 19 36 / 42; 14 of 5, 1161 workgroups 79 / 83).
+extern "C" int bsp_xsd_parts(int dtype, int block, int width, int longest, int64_t nnz, int free_dim, int Z, int flags, int *part_blocks) {
+  *part_blocks = 0;
+  if (dtype != BSP_F32 || !block_ok(block) || width <= 0 || free_dim <= 0 || Z <= 0 || longest <= 0 || (flags & BSP_FLAG_WHOLE_K)) return 1;
+  const int tile = xsd_tile(block, free_dim);
+  const int64_t wgs = (int64_t)width * ((free_dim + tile - 1) / tile) * Z;
+  const int steps = longest * (block / 16);
+  if (wgs > 1024 || steps < 48) return 1;
+  int64_t parts = 1;
+  if ((int64_t)longest * width >= (block == 16 ? 4 : 2) * nnz) parts = steps / (block == 16 ? 32 : 16);
+  if (wgs <= 384 && parts < 800 / wgs) parts = 800 / wgs < steps / 16 ? 800 / wgs : steps / 16;
+  if (parts > 8) parts = 8;
+  if (parts <= 1) return 1;
+  const int per = (longest + (int)parts - 1) / (int)parts;
+  if (bsp_xsd_parts_workspace_bytes(block, width, free_dim, Z, (longest + per - 1) / per) > ((int64_t)256 << 20)) return 1;
+  *part_blocks = per;
+  return (longest + per - 1) / per;
+}
+
+extern "C" int64_t bsp_xsd_parts_workspace_bytes(int block, int width, int free_dim, int Z, int parts) {
+  if (parts <= 1) return 0;
+  const int tile = xsd_tile(block, free_dim);
+  return (int64_t)parts * Z * width * ((free_dim + tile - 1) / tile) * block * tile * (int64_t)sizeof(float);
+}
+
+extern "C" int bsp_xsd_matmul_parts(int is_dds, int dtype, const void *sp, const void *dn, void *c, int trans_a, int trans_b, int trans_c, int Z, int free_dim,
+                                    int64_t sp_stride_z, int64_t dn_stride_z, int64_t dn_stride_h, int64_t ldd, int64_t c_stride_z, int64_t c_stride_h,
+                                    int64_t ldc, int block, const int32_t *d_lut, const int32_t *d_plan, int width, int parts, int part_blocks, void *d_ws,
+                                    int64_t ws_bytes, void *stream) {
+  if (!sp || !dn || !c || !d_lut || !d_plan || Z <= 0 || free_dim <= 0 || width < 0 || parts < 2 || part_blocks < 1 || !d_ws) return BSP_ERR_ARG;
+  if (!block_ok(block) || dtype != BSP_F32) return BSP_ERR_UNSUPPORTED;
+  if (!aligned16(sp) || !aligned16(dn) || !aligned16(c) || !aligned16(d_ws)) return BSP_ERR_ARG;
+  if (sp_stride_z % 4 || dn_stride_z % 4 || dn_stride_h % 4 || ldd % 4 || c_stride_z % 4 || c_stride_h % 4 || ldc % 4) return BSP_ERR_ARG;
+  const bool whole_rows = is_dds ? !trans_a && !trans_c : trans_b && trans_c;
+  if (free_dim % 4 && !whole_rows) return BSP_ERR_ARG;
+  if (ws_bytes < bsp_xsd_parts_workspace_bytes(block, width, free_dim, Z, parts)) return BSP_ERR_CAPACITY;
+  XsdArgs g;
+  g.sp = sp; g.dn = dn; g.out = c; g.Z = Z; g.NF = free_dim;
+  g.sp_sz = sp_stride_z; g.dn_sz = dn_stride_z; g.dn_sh = dn_stride_h; g.ldd = ldd;
+  g.out_sz = c_stride_z; g.out_sh = c_stride_h; g.ldo = ldc;
+  g.lut = d_lut; g.order = d_plan; g.plan = d_plan + bsp_dxx_plan_pairs_offset(width); g.width = width;
+  g.div2 = 2 * (block / 8);
+  g.n_tiles = (free_dim + 63) / 64;
+  g.gplan = nullptr; g.n_pgroups = 0; g.lines = 0;
+  g.parts = parts; g.part_blocks = part_blocks; g.partials = reinterpret_cast<float *>(d_ws);
+  // (orientations as in bsp_dsd_matmul and bsp_dds_matmul)
+  const int rc = is_dds ? xsd_generic_f32(g, block, trans_b == 0, trans_a == 0, trans_c != 0, as_stream(stream))
+                        : xsd_generic_f32(g, block, trans_a != 0, trans_b != 0, trans_c == 0, as_stream(stream));
+  if (rc != BSP_OK) return rc;
+  BSP_LAUNCH_CHECK();
+  return BSP_OK;
+}
+
 // Whether a dsd launch with these properties is taken by a kernel that runs split chains and so uses the workspace:
 // the row-group kernels on 64 x 64 tiles (block 64, or block 16 with a plan over tiles: negative line count), 16-bit
 // types, dense operand not reduction-contiguous, output rows contiguous, whole 64-wide tiles of the free dimension,

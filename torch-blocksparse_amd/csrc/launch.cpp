@@ -17,7 +17,7 @@
 namespace {
 
 PyObject *g_torch, *g_check, *g_raw_stream, *g_tensor, *g_parameter, *g_dtypes[3], *g_matmul_class;   // (borrowed for the life of the process)
-PyObject *s_shape, *s_stride, *s_data_ptr, *s_dtype, *s_device, *s_get_device, *s_empty, *s_float32, *s_target;
+PyObject *s_shape, *s_stride, *s_data_ptr, *s_dtype, *s_device, *s_get_device, *s_empty, *s_uint8, *s_float32, *s_target;
 PyObject *k_dtype_device;                               // ('dtype', 'device')
 
 struct Ref {                                            // an owned reference
@@ -90,6 +90,10 @@ PyObject *empty(const int64_t *size, int n, PyObject *dtype, PyObject *like) {
   return PyObject_Vectorcall(fn.o, args, 1, k_dtype_device);
 }
 PyObject *empty_like_type(const int64_t *size, int n, const Operand &like) { return empty(size, n, g_dtypes[like.dtype], like.obj); }
+PyObject *empty_bytes(int64_t n, PyObject *like) {
+  Ref dt(PyObject_GetAttr(g_torch, s_uint8));
+  return dt.o ? empty(&n, 1, dt.o, like) : nullptr;
+}
 PyObject *empty_floats(const int64_t *size, int n, PyObject *like) {
   Ref dt(PyObject_GetAttr(g_torch, s_float32));
   return dt.o ? empty(size, n, dt.o, like) : nullptr;
@@ -128,7 +132,7 @@ struct Plan { const int32_t *table; int n_groups, lines, n_split; };
 struct Xsd {
   PyObject *keep;                                       // a tuple, the ordinary plan its second, the wide one its third member
   const int32_t *lut, *plan;
-  int width, block, dtype, dev;
+  int width, block, dtype, dev, longest;
   int64_t nnz, H, R, C;
   Plan ordinary, wide;
   int wide_state;                                       // 0: there is none, 1: not built yet, 2: built
@@ -171,7 +175,7 @@ const char *kXsd = "torch_blocksparse.xsd", *kSdd = "torch_blocksparse.sdd", *kR
 PyObject *make_xsd(PyObject *, PyObject *args) {
   Xsd s{};
   unsigned long long lut, planbuf, gp, wp;
-  if (!PyArg_ParseTuple(args, "OKKiiiiLLLL(Kiii)(Kiii)i", &s.keep, &lut, &planbuf, &s.width, &s.block, &s.dtype, &s.dev, &s.nnz, &s.H, &s.R, &s.C, &gp,
+  if (!PyArg_ParseTuple(args, "OKKiiiiiLLLL(Kiii)(Kiii)i", &s.keep, &lut, &planbuf, &s.width, &s.block, &s.dtype, &s.dev, &s.longest, &s.nnz, &s.H, &s.R, &s.C, &gp,
                         &s.ordinary.n_groups, &s.ordinary.lines, &s.ordinary.n_split, &wp, &s.wide.n_groups, &s.wide.lines, &s.wide.n_split, &s.wide_state))
     return nullptr;
   s.lut = reinterpret_cast<const int32_t *>(lut); s.plan = reinterpret_cast<const int32_t *>(planbuf);
@@ -263,6 +267,18 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     wsp = reinterpret_cast<void *>(at);
   }
   const int64_t sp_sz = sp.dim == 4 && sp.size[0] > 1 ? sp.stride[0] : 0, ldc = shape[3], c_sh = shape[2] * shape[3], c_sz = s->H * c_sh;
+  int part_blocks = 0;
+  const int parts = bsp_xsd_parts(s->dtype, s->block, s->width, s->longest, s->nnz, (int)free_dim, (int)Z, flags, &part_blocks);
+  if (parts > 1) {
+    const int64_t need = bsp_xsd_parts_workspace_bytes(s->block, s->width, (int)free_dim, (int)Z, parts);
+    Ref ws(empty_bytes(need, dn.obj));
+    if (!ws.o || !pointer(ws.o, &wsp)) return nullptr;
+    const int rc = unlocked([&] {
+      return bsp_xsd_matmul_parts(dds, s->dtype, sp.data(), dn.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, sp_sz, dn.stride[0], dn.stride[1], dn.stride[2], c_sz, c_sh, ldc,
+                                  s->block, s->lut, s->plan, s->width, parts, part_blocks, wsp, need, st);
+    });
+    return checked(rc, "bsp_xsd_matmul_parts") ? c.release() : nullptr;
+  }
   const int rc = unlocked([&] { return dds ? bsp_dds_matmul(s->dtype, dn.data(), sp.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, dn.stride[0], dn.stride[1], dn.stride[2], sp_sz, c_sz, c_sh, ldc,
                                       s->block, s->lut, s->plan, s->width, plan.table, plan.n_groups, plan.lines, plan.n_split, wsp, ws_bytes, flags, st)
                      : bsp_dsd_matmul(s->dtype, sp.data(), dn.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, sp_sz, dn.stride[0], dn.stride[1], dn.stride[2], c_sz, c_sh, ldc,
@@ -536,7 +552,7 @@ static_assert(BSP_F16 == 0 && BSP_BF16 == 1 && BSP_F32 == 2, "the order of the t
 
 PyMODINIT_FUNC PyInit__launch(void) {
   struct { PyObject **at; const char *name; } names[] = {{&s_shape, "shape"}, {&s_stride, "stride"}, {&s_data_ptr, "data_ptr"}, {&s_dtype, "dtype"}, {&s_device, "device"},
-                                                         {&s_get_device, "get_device"}, {&s_empty, "empty"}, {&s_float32, "float32"},
+                                                         {&s_get_device, "get_device"}, {&s_empty, "empty"}, {&s_uint8, "uint8"}, {&s_float32, "float32"},
                                                          {&s_target, "SPLITK_TARGET_WORKGROUPS"}};
   for (auto &e : names) if (!(*e.at = PyUnicode_InternFromString(e.name))) return nullptr;
   if (!(k_dtype_device = PyTuple_Pack(2, s_dtype, s_device))) return nullptr;

@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   const int n_tiles = (g.NF + kTN - 1) / kTN;
   int z, nt, seg0;
-  xsd_work_item(g, n_tiles, z, nt, seg0);
+  xsd_work_item(g, n_tiles, blockIdx.x, z, nt, seg0);
   const int seg = g.order ? as_table(g.order)[seg0] : seg0;
   const table_ptr hd = as_table(g.lut) + 6 * (int64_t)seg;
   const int offset = hd[0], seglen = hd[1], column = hd[2], depth = hd[3];

@@ -278,15 +278,16 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
     constexpr int VE = 16 / (int)sizeof(T);
     if constexpr (PARTIAL) {
       // (straight from the accumulators, 16 bytes a lane: parts are few, and what reads them next finds them in L2)
-      static_assert(OUT_NCONTIG, "parts are written along n");
 #pragma unroll
       for (int i = 0; i < RM; i++)
 #pragma unroll
         for (int j = 0; j < RN; j++)
 #pragma unroll
-          for (int g4 = 0; g4 < M::NACC / 4; g4++)
-            store((wm * RM + i) * MS + lane % MS, (wn * RN + j) * MS + (MS == 16 ? 4 * (lane >> 4) : 8 * g4 + 4 * (lane >> 5)),
+          for (int g4 = 0; g4 < M::NACC / 4; g4++) {
+            const int m0 = (wm * RM + i) * MS, nn0 = (wn * RN + j) * MS, along = MS == 16 ? 4 * (lane >> 4) : 8 * g4 + 4 * (lane >> 5);
+            store(lane % MS + (OUT_NCONTIG ? m0 : nn0), along + (OUT_NCONTIG ? nn0 : m0),
                   f32x4{acc[i][j][4 * g4], acc[i][j][4 * g4 + 1], acc[i][j][4 * g4 + 2], acc[i][j][4 * g4 + 3]});
+          }
     } else {
     if constexpr (SUB > 0 && OUT_NCONTIG && TM * (TN + VE) * (int)sizeof(T) <= SMEM_BYTES) {
       // Blocked output: the whole TM x TN tile is staged (all wavefronts, two barriers) and then written block by
@@ -584,6 +585,9 @@ struct XsdArgs {
   const int32_t *gplan; int n_pgroups; int lines;   // optional group plan, its groups, lines (block-rows or -columns) per head
   int n_split = 0;                      // split chains of the plan; their fp32 partial tiles (caller's workspace)
   float *partials = nullptr;
+  // general kernels: segments of more than part_blocks blocks run in parts of that many (at most `parts` of them), whose fp32 tiles
+  // go to partials [part][Z][width][tiles]
+  int parts = 1, part_blocks = 0;
 };
 
 // A reduction step of TK elements lies inside one block (BLOCK >= TK) or covers TK / BLOCK whole blocks.
@@ -638,15 +642,16 @@ template <typename T, int BLOCK> struct DenseView {                   // element
   __device__ __forceinline__ int64_t scalar_r(const Step &st, int i) const { return ((int64_t)st.pos[i] + st.kin) * ld; }
 };
 
-template <int BLOCK, bool WIDE> struct XsdShape {
-  // Tile of the dense free dimension.  Wide tiles for block 32 and 128: a wavefront then reuses each fragment of the
-  // sparse block for two or four MFMAs (LDS reads per MFMA are what bounds these kernels); measured +13 % at block 32.
-  // The narrow shape serves free dimensions up to 64 (the head dimension of an attention product), where a wide
-  // tile would be mostly padding.
-  static constexpr int TN = !WIDE ? 64 : BLOCK == 64 ? 128 : BLOCK >= 32 ? 256 : 64;
-  // wide: 32 -> 1x4 wavefronts of 32x64; 64 -> 2x2 of 32x64; 128 -> 2x2 of 64x128.  narrow: 16 -> 1x4 of 16x16;
+// Tile of the dense free dimension, TN: 64, 128 or 256 wide.  Wide tiles for blocks of 32 and 128: a wavefront then reuses each fragment
+// of the sparse block for two or four MFMAs (LDS reads per MFMA are what bounds these kernels); measured +13 % at block 32.  A free
+// dimension up to 64 or 128 (the head dimension of an attention product) takes a tile that it fills: fp32, block 32, 18 blocks a row, 128
+// wide, 52 us on tiles of 256, half of them padding.
+constexpr int xsd_tile(int block, int free_dim) { return free_dim <= 64 || block == 16 ? 64 : block == 64 || free_dim <= 128 ? 128 : 256; }
+template <int BLOCK, int TN_> struct XsdShape {
+  static constexpr int TN = TN_;
+  // wider than 64: 32 -> 1x4 wavefronts of 32x32 / 32x64; 64 -> 2x2 of 32x64; 128 -> 2x2 of 64x64 / 64x128.  64: 16 -> 1x4 of 16x16;
   // 32 -> 2x2 of 16x32; 64 -> 2x2 of 32x32; 128 -> 2x2 of 64x32
-  static constexpr int WGM = (WIDE ? BLOCK >= 64 : BLOCK >= 32) ? 2 : 1;
+  static constexpr int WGM = (TN > 64 ? BLOCK >= 64 : BLOCK >= 32) ? 2 : 1;
   static constexpr int WGN = 4 / WGM;
 };
 
@@ -657,9 +662,9 @@ template <int BLOCK, bool WIDE> struct XsdShape {
 // eighth of the launch, so inside its eighth the position in the order is the slow index and the tile the fast one.
 // One batch with a number of tiles that divides by 8: every XCD gets all segments for its own tiles; a batch that
 // divides by 8: every XCD gets whole batches.
-__device__ __forceinline__ void xsd_work_item(const XsdArgs &g, int n_tiles, int &z, int &nt, int &seg0) {
+__device__ __forceinline__ void xsd_work_item(const XsdArgs &g, int n_tiles, int64_t wg, int &z, int &nt, int &seg0) {
   const int64_t per_z = (int64_t)g.width * n_tiles, total = per_z * g.Z;
-  const int64_t w = xcd_remap(blockIdx.x, total);
+  const int64_t w = xcd_remap(wg, total);
   z = (int)(w / per_z);
   nt = (int)((w % per_z) / g.width);
   seg0 = (int)((w % per_z) % g.width);
@@ -680,24 +685,32 @@ __device__ __forceinline__ void xsd_work_item(const XsdArgs &g, int n_tiles, int
 }
 
 // (at least two wavefronts per SIMD: the 128 x 256 tile of block 128 would otherwise take 266 registers and run alone)
-template <typename T, int BLOCK, bool WIDE, bool SP_TRANS, bool DN_KCONTIG, bool OUT_NCONTIG>
+template <typename T, int BLOCK, int TN_, bool SP_TRANS, bool DN_KCONTIG, bool OUT_NCONTIG, bool PARTS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_xsd(XsdArgs g) {
-  typedef XsdShape<BLOCK, WIDE> S;
+  typedef XsdShape<BLOCK, TN_> S;
   typedef TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !SP_TRANS, DN_KCONTIG, OUT_NCONTIG> G;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int n_tiles = (g.NF + S::TN - 1) / S::TN;
+  const int64_t n_wg = (int64_t)g.width * n_tiles * g.Z;
+  const int part = PARTS ? (int)(blockIdx.x / n_wg) : 0;
   int z, nt, seg0;
-  xsd_work_item(g, n_tiles, z, nt, seg0);
+  xsd_work_item(g, n_tiles, PARTS ? blockIdx.x % n_wg : blockIdx.x, z, nt, seg0);
   const int seg = g.order ? as_table(g.order)[seg0] : seg0;   // longest first only where the launch is short (see the dispatcher)
   const table_ptr hd = as_table(g.lut) + 6 * (int64_t)seg;
   const int offset = hd[0], seglen = hd[1], column = hd[2], depth = hd[3];
-  const int nblk = seglen / BLOCK;
+  const int whole = seglen / BLOCK;
+  int nblk = whole;
+  if constexpr (PARTS) {
+    nblk = whole - part * g.part_blocks;
+    if (part > 0 && nblk <= 0) return;
+    if (nblk > g.part_blocks) nblk = g.part_blocks;
+  }
   if (nblk == 0) {
     // The table carries zero-length segments.  One that stands alone is an empty row/column of the layout and
     // must zero-fill its output tile; one that follows a real segment of the same row/column must not touch it.
     if (seg > 0 && hd[-6 + 2] == column && hd[-6 + 3] == depth) return;
   }
-  const int t0 = (offset - 6 * g.width) / g.div2;   // first block of the segment in table order
+  const int t0 = (offset - 6 * g.width) / g.div2 + part * g.part_blocks;   // first block of the segment (the part) in table order
   SparseView<T, BLOCK, SP_TRANS> sv;
   sv.base = reinterpret_cast<const T *>(g.sp) + z * g.sp_sz; sv.plan = as_table(g.plan) + 2 * (int64_t)t0; sv.nblk = nblk;
   DenseView<T, BLOCK> dv;
@@ -721,7 +734,47 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
     for (int i = threadIdx.x; i < BLOCK * S::TN / VE; i += 256) store(i / (CW / VE), (i % (CW / VE)) * VE, zero);
     return;
   }
+  if constexpr (PARTS) {
+    if (whole > g.part_blocks) {
+      constexpr int CW = OUT_NCONTIG ? S::TN : BLOCK;
+      float *ws = g.partials + ((((int64_t)part * g.Z + z) * g.width + seg) * n_tiles + nt) * (BLOCK * S::TN);
+      G::template run<0, true>(sv, dv, (nblk * BLOCK + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem_raw), [&](int r, int c, f32x4 v) { *reinterpret_cast<f32x4 *>(ws + r * CW + c) = v; });
+      return;
+    }
+  }
   G::run(sv, dv, (nblk * BLOCK + G::TK - 1) / G::TK, reinterpret_cast<T *>(smem_raw), store);
+}
+
+// The second pass of segments in parts: a workgroup per segment, tile and batch adds the parts in order
+template <typename T, int BLOCK, int TN, bool OUT_NCONTIG> __global__ void __launch_bounds__(256) k_xsd_parts_sum(XsdArgs g) {
+  constexpr int CW = OUT_NCONTIG ? TN : BLOCK;
+  const int n_tiles = (g.NF + TN - 1) / TN;
+  const int seg = blockIdx.x % g.width, nt = (blockIdx.x / g.width) % n_tiles, z = blockIdx.x / g.width / n_tiles;
+  const table_ptr hd = as_table(g.lut) + 6 * (int64_t)seg;
+  const int nblk = hd[1] / BLOCK, column = hd[2], depth = hd[3];
+  if (nblk <= g.part_blocks) return;
+  const int parts = (nblk + g.part_blocks - 1) / g.part_blocks;
+  const int64_t stride = (int64_t)g.Z * g.width * n_tiles * (BLOCK * TN);
+  const float *ws = g.partials + (((int64_t)z * g.width + seg) * n_tiles + nt) * (BLOCK * TN);
+  T *oz = reinterpret_cast<T *>(g.out) + z * g.out_sz + depth * g.out_sh;
+  for (int i = threadIdx.x * 4; i < BLOCK * TN; i += 1024) {
+    const int r = i / CW, c = i % CW;
+    if (nt * TN + (OUT_NCONTIG ? c : r) >= g.NF) continue;
+    f32x4 sum = *reinterpret_cast<const f32x4 *>(ws + i);
+    for (int p = 1; p < parts; p++) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(ws + p * stride + i);
+#pragma unroll
+      for (int e = 0; e < 4; e++) sum[e] += v[e];
+    }
+    T *dst = OUT_NCONTIG ? oz + ((int64_t)column * BLOCK + r) * g.ldo + nt * TN + c : oz + (int64_t)(nt * TN + r) * g.ldo + column * BLOCK + c;
+    if constexpr (sizeof(T) == 4) *reinterpret_cast<f32x4 *>(dst) = sum;
+    else {
+      union { u32x2 raw; T e[4]; } u;
+#pragma unroll
+      for (int e = 0; e < 4; e++) u.e[e] = from_float<T>(sum[e]);
+      *reinterpret_cast<u32x2 *>(dst) = u.raw;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -816,21 +869,29 @@ template <typename T> int launch_sdd(const SddArgs &g, int block, const SddLevel
   return BSP_OK;
 }
 
-template <typename T, int BLOCK, bool WIDE> int launch_xsd_bw(const XsdArgs &g0, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
-  typedef XsdShape<BLOCK, WIDE> S;
+template <typename T, int BLOCK, int TN_> int launch_xsd_bw(const XsdArgs &g0, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
+  typedef XsdShape<BLOCK, TN_> S;
   const int64_t n_wg = (int64_t)g0.width * ((g0.NF + S::TN - 1) / S::TN) * g0.Z;
   if (n_wg <= 0) return BSP_OK;
-  if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
+  if (n_wg * g0.parts >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
   // Longest segments first only in short launches (a few workgroups per CU), where the last workgroups to start
   // decide when the launch ends: 7 % on an 8192 x 4096 x 4096 linear layer at block 128 and 10 % density (1024
   // workgroups).  A long launch balances by itself and reads the sparse blocks in storage order without it (1 %
   // faster at 65536 workgroups).
   XsdArgs g = g0;
   if (n_wg > 16 * 256) g.order = nullptr;
-  dim3 grid((unsigned)n_wg), blockdim(256);
+  dim3 grid((unsigned)(n_wg * g.parts)), blockdim(256);
 #define BSP_XSD_LAUNCH(ST, DK, ON)                                                                               \
-  hipLaunchKernelGGL((k_xsd<T, BLOCK, WIDE, ST, DK, ON>), grid, blockdim,                                       \
-                     (TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON>::SMEM_BYTES), st, g)
+  do {                                                                                                           \
+    constexpr int SMEM = TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON>::SMEM_BYTES;                     \
+    if constexpr (sizeof(T) == 4)                                                                                \
+      if (g.parts > 1) {                                                                                         \
+        hipLaunchKernelGGL((k_xsd<T, BLOCK, TN_, ST, DK, ON, true>), grid, blockdim, SMEM, st, g);              \
+        hipLaunchKernelGGL((k_xsd_parts_sum<T, BLOCK, TN_, ON>), dim3((unsigned)n_wg), blockdim, 0, st, g);     \
+        break;                                                                                                   \
+      }                                                                                                          \
+    hipLaunchKernelGGL((k_xsd<T, BLOCK, TN_, ST, DK, ON, false>), grid, blockdim, SMEM, st, g);                 \
+  } while (0)
   const int key = (sp_trans ? 4 : 0) | (dn_kc ? 2 : 0) | (out_nc ? 1 : 0);
   switch (key) {
     case 0: BSP_XSD_LAUNCH(false, false, false); break;
@@ -847,8 +908,12 @@ template <typename T, int BLOCK, bool WIDE> int launch_xsd_bw(const XsdArgs &g0,
 }
 
 template <typename T, int BLOCK> int launch_xsd_b(const XsdArgs &g, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
-  if (g.NF > 64 && XsdShape<BLOCK, true>::TN > 64) return launch_xsd_bw<T, BLOCK, true>(g, sp_trans, dn_kc, out_nc, st);
-  return launch_xsd_bw<T, BLOCK, false>(g, sp_trans, dn_kc, out_nc, st);
+  const int tile = xsd_tile(BLOCK, g.NF);
+  if constexpr (BLOCK == 32 || BLOCK == 128)
+    if (tile == 256) return launch_xsd_bw<T, BLOCK, 256>(g, sp_trans, dn_kc, out_nc, st);
+  if constexpr (BLOCK != 16)
+    if (tile == 128) return launch_xsd_bw<T, BLOCK, 128>(g, sp_trans, dn_kc, out_nc, st);
+  return launch_xsd_bw<T, BLOCK, 64>(g, sp_trans, dn_kc, out_nc, st);
 }
 
 template <typename T> int launch_xsd(const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {

@@ -67,6 +67,9 @@ SIGNATURES = {
                             _i, _vp, _i, _i, _i, _vp, _i64, _i, _vp]),
     'bsp_dsd_matmul_noalloc': (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _vp, _vp,
                                     _i, _vp, _i, _i, _i, _i, _vp]),
+    'bsp_xsd_parts': (_i, [_i, _i, _i, _i, _i64, _i, _i, _i, _vp]),
+    'bsp_xsd_parts_workspace_bytes': (_i64, [_i, _i, _i, _i, _i]),
+    'bsp_xsd_matmul_parts': (_i, [_i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _vp, _vp, _i, _i, _i, _vp, _i64, _vp]),
     'bsp_dds_matmul': (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _vp, _vp,
                             _i, _vp, _i, _i, _i, _vp, _i64, _i, _vp]),
     'bsp_softmax_fwd': (_i, [_i, _vp, _f, _vp, _i, _vp, _i64, _i64, _i64, _vp, _i64, _i, _vp, _i64, _i, _i, _i, _i, _i,

@@ -503,6 +503,7 @@ class _sparse_matmul(torch.autograd.Function):
         lut.planbuf = planbuf
         lut.plan = planbuf[first:first + 2 * nnz].view(nnz, 2)
         lut.nnz = nnz
+        lut.longest = int((layout != 0).sum(2 if trans else 1).max())     # blocks of the longest segment
         lut.spdims = tuple(layout.shape)
         lut.gplan = GroupPlan.build_coarse(layout, block, trans, dev, ctx=ctx) if block == 16 else None
         if lut.gplan is None and block in (16, 32, 64):
@@ -515,6 +516,22 @@ class _sparse_matmul(torch.autograd.Function):
         if block == 32:
             lut.build_wide = lambda: GroupPlan.build(layout, trans, dev, thin_min=0, order_buckets=1, ctx=ctx)
         return lut, num_locks.value, width.value, None
+
+    @staticmethod
+    def _in_parts(is_dds, sp, dn, c, trans_a, trans_b, trans_c, Z, free_dim, sp_sz, block, lut, width):
+        """the product with its long segments in parts, where bsp_xsd_parts asks for that: whether it was launched"""
+        lib, part_blocks = _lib.load(), ctypes.c_int(0)
+        dtype = _lib.DTYPES[dn.dtype]
+        parts = lib.bsp_xsd_parts(dtype, block, width, getattr(lut, 'longest', 0), getattr(lut, 'nnz', 0), free_dim, Z, KERNEL_FLAGS, ctypes.byref(part_blocks))
+        if parts <= 1:
+            return False
+        need = lib.bsp_xsd_parts_workspace_bytes(block, width, free_dim, Z, parts)
+        ws = torch.empty(need, dtype=torch.uint8, device=dn.device)
+        rc = lib.bsp_xsd_matmul_parts(int(is_dds), dtype, _lib.ptr(sp), _lib.ptr(dn), _lib.ptr(c), int(trans_a), int(trans_b), int(trans_c), Z, free_dim, sp_sz,
+                                      dn.stride(0), dn.stride(1), dn.stride(2), c.stride(0), c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf),
+                                      width, parts, part_blocks.value, _lib.ptr(ws), need, _lib.stream_ptr(dn.device))
+        _lib.check(rc, 'bsp_xsd_matmul_parts')
+        return True
 
     @staticmethod
     def _plan_for(lut, block, free_dim, dtype, width, batch):
@@ -554,7 +571,7 @@ class _sparse_matmul(torch.autograd.Function):
         c = torch.empty((a.size(0), a.size(1), CS2, CS3), dtype=a.dtype, device=a.device)
         b_sz = b.stride(0) if (b.dim() == 4 and b.size(0) > 1) else 0   # a 3-D (or batch-1) sparse operand is shared by the batch
         timer = _Timer(bench, a.device)
-        rc = _lib.load().bsp_dds_matmul(_lib.DTYPES[a.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
+        rc = _lib.OK if _sparse_matmul._in_parts(True, b, a, c, trans_a, trans_b, trans_c, a.size(0), M, b_sz, block, lut, width) else _lib.load().bsp_dds_matmul(_lib.DTYPES[a.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
                                         int(trans_c), a.size(0), M, a.stride(0), a.stride(1), a.stride(2), b_sz, c.stride(0),
                                         c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
                                         *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, M, a.dtype, width, a.size(0)), M, a.size(0)), KERNEL_FLAGS,
@@ -579,7 +596,7 @@ class _sparse_matmul(torch.autograd.Function):
         c = torch.empty((b.size(0), b.size(1), CS2, CS3), dtype=b.dtype, device=b.device)
         a_sz = a.stride(0) if (a.dim() == 4 and a.size(0) > 1) else 0
         timer = _Timer(bench, b.device)
-        rc = _lib.load().bsp_dsd_matmul(_lib.DTYPES[b.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
+        rc = _lib.OK if _sparse_matmul._in_parts(False, a, b, c, trans_a, trans_b, trans_c, b.size(0), N, a_sz, block, lut, width) else _lib.load().bsp_dsd_matmul(_lib.DTYPES[b.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
                                         int(trans_c), b.size(0), N, a_sz, b.stride(0), b.stride(1), b.stride(2), c.stride(0),
                                         c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
                                         *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, N, b.dtype, width, b.size(0)), N, b.size(0)), KERNEL_FLAGS,
@@ -674,7 +691,7 @@ class _Product:
                                           plan(lut.gplan), plan(late), 0 if lut.build_long is None else 1 if late is None else 2,
                                           int(late is not None and late.rowpair), late.max_entries() if late is not None else 0, int(lut.any_k), levels)
         else:
-            made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, lut.nnz, H, R, C,
+            made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, lut.longest, lut.nnz, H, R, C,
                                           plan(lut.gplan), plan(lut.gplan_wide),
                                           2 if lut.gplan_wide is not None else int(getattr(lut, 'build_wide', None) is not None))
         self.native[which], self.built[which] = made, self._on_demand(which)

@@ -150,7 +150,9 @@ typedef enum {
                                  plan serves the long-reduction kernel (K >= 256, K % 32 == 0, 16-bit types) and nothing else */
   BSP_FLAG_ANY_K = 16,        /* bsp_sdd_matmul_levels with trans_a and not trans_b (the reduction runs along the rows of both operands): K need
                                  not be a multiple of 16 */
-  BSP_FLAG_WHOLE_K = 32        /* bsp_sdd_parts, bsp_xsd_parts: one part whatever the sizes (for cross-checks) */
+  BSP_FLAG_WHOLE_K = 32,       /* bsp_sdd_parts, bsp_xsd_parts: one part whatever the sizes (for cross-checks) */
+  BSP_FLAG_PLAN_TILES = 64     /* bsp_sdd_matmul without a table: d_gplan holds n_plan_groups tiles of bsp_sdd_tiles_build, plan_lines and n_groups the
+                                  block-rows and block-columns of a head; blocks of 32, K >= 256, K % 32 == 0, 16-bit types */
 } bsp_launch_flags;
 
 /* sparse = dense x dense: replaces _sparse_matmul._sdd_matmul + the SDD branch of the kernel
@@ -173,6 +175,11 @@ int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, int trans_a
                    int64_t ldb, int64_t c_stride_z, int block, int pack, const int32_t *d_lut,
                    const uint8_t *d_valid, int64_t n_groups, const int32_t *d_gplan, int n_plan_groups, int plan_lines, int flags,
                    void *stream);
+
+/* The tiles of BSP_FLAG_PLAN_TILES, on the host: layout H x R x C bytes (0: no block), out: *n_tiles tiles of 148 ints each, in the order of
+ * the heads and block-rows (BSP_ERR_CAPACITY with *n_tiles set when cap ints do not hold them).  A tile is sixteen consecutive block-rows by
+ * up to sixteen block-columns that hold at most 64 blocks there. */
+int bsp_sdd_tiles_build(const uint8_t *layout, int H, int R, int C, int32_t *out, int64_t cap, int64_t *n_tiles);
 
 /* ... all pack levels of the table (n_levels <= 3, each pack width at most once) in one call: packs, d_luts, d_valids (entries may
  * be NULL) and n_groups are host arrays with what a call of bsp_sdd_matmul per level would get.  Blocks of 16 and 32, which are

@@ -142,10 +142,11 @@ extern "C" int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, 
   g.gplan = d_gplan; g.n_pgroups = n_plan_groups; g.lines = plan_lines;
   const bool a_kc = !trans_a, b_kc = trans_b != 0;
   hipStream_t st = as_stream(stream);
-  int rc = no_wide(flags) ? 0 : sdd_dl(dtype, g, block, rowpair(flags), a_kc, b_kc, st);
+  const bool tiles = (flags & BSP_FLAG_PLAN_TILES) != 0;
+  int rc = no_wide(flags) ? 0 : tiles ? sdd_list(dtype, g, block, a_kc, b_kc, st) : sdd_dl(dtype, g, block, rowpair(flags), a_kc, b_kc, st);
   if (rc < 0) return rc;
   if (rc == 2) { BSP_LAUNCH_CHECK(); return BSP_OK_WHOLE_LAYOUT; }
-  if (rowpair(flags)) return BSP_NEEDS_TABLE;      // a plan over pairs of block-rows serves the long-reduction kernel only
+  if (rowpair(flags) || tiles) return BSP_NEEDS_TABLE;      // a plan over pairs of block-rows serves the long-reduction kernel only
   rc = sdd_fast64(dtype, g, block, pack, a_kc, b_kc, st);
   if (rc < 0) return rc;
   if (rc >= 1) { BSP_LAUNCH_CHECK(); return rc == 2 ? BSP_OK_WHOLE_LAYOUT : BSP_OK; }

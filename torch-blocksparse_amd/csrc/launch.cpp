@@ -141,7 +141,8 @@ struct Sdd {
   PyObject *keep;                                       // a tuple, the SddTables first
   int block, dtype, dev;
   int64_t nnz, H, R, C;
-  Plan ordinary, longk;
+  Plan ordinary, longk, tiles;
+  int tiles_state, tiles_launch, tile_blocks;           // as wide_state; SddTables.TILES_LAUNCH, TILE_BLOCKS
   int long_state, long_rowpair, long_entries;           // as wide_state
   int n_levels, any_k;                                  // n_levels -1: the tables are not built yet
   int packs[3];
@@ -186,12 +187,13 @@ PyObject *make_xsd(PyObject *, PyObject *args) {
 
 PyObject *make_sdd(PyObject *, PyObject *args) {
   Sdd s{};
-  unsigned long long gp, lp;
+  unsigned long long gp, lp, tp;
   PyObject *levels;
-  if (!PyArg_ParseTuple(args, "OiiiLLLL(Kiii)(Kiii)iiiiO", &s.keep, &s.block, &s.dtype, &s.dev, &s.nnz, &s.H, &s.R, &s.C, &gp, &s.ordinary.n_groups,
+  if (!PyArg_ParseTuple(args, "OiiiLLLL(Kiii)(Kiii)iiii(Kiii)iiiO", &s.keep, &s.block, &s.dtype, &s.dev, &s.nnz, &s.H, &s.R, &s.C, &gp, &s.ordinary.n_groups,
                         &s.ordinary.lines, &s.ordinary.n_split, &lp, &s.longk.n_groups, &s.longk.lines, &s.longk.n_split, &s.long_state, &s.long_rowpair,
-                        &s.long_entries, &s.any_k, &levels))
+                        &s.long_entries, &s.any_k, &tp, &s.tiles.n_groups, &s.tiles.lines, &s.tiles.n_split, &s.tiles_state, &s.tiles_launch, &s.tile_blocks, &levels))
     return nullptr;
+  s.tiles.table = reinterpret_cast<const int32_t *>(tp);
   s.ordinary.table = reinterpret_cast<const int32_t *>(gp); s.longk.table = reinterpret_cast<const int32_t *>(lp);
   s.n_levels = -1;
   if (levels != Py_None) {
@@ -316,6 +318,9 @@ PyObject *sdd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (any_k) flags |= BSP_FLAG_ANY_K;
   const bool long_k = (s->block == 16 || s->block == 32) && K >= 256 && K % 32 == 0 && !f32 && s->long_state;
   if ((long_k && s->long_state != 2) || (s->n_levels < 0 && (any_k || (!long_k && !s->ordinary.table)))) Py_RETURN_NONE;
+  bool tiles = long_k && s->tiles_state && s->nnz * Z >= (int64_t)s->tiles_launch * s->tile_blocks;       // SddTables.tiles_for
+  if (tiles && s->tiles_state != 2) Py_RETURN_NONE;
+  tiles = tiles && (int64_t)s->tiles.n_groups * Z >= s->tiles_launch && s->nnz >= (int64_t)s->tile_blocks * s->tiles.n_groups;
   int parts = 0;
   if (s->n_levels == 1 && s->block == 128 && !f32 && K % 32 == 0 && K >= 512 && s->packs[0] == 1 && !(flags & (BSP_FLAG_GENERAL_ONLY | BSP_FLAG_NO_WIDE))) {
     Ref t(PyObject_GetAttr(g_matmul_class, s_target));  // _sdd_splitk in matmul.py
@@ -334,7 +339,12 @@ PyObject *sdd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!c.o || !pointer(c.o, &cp) || !stream_of(a.dev, &st)) return nullptr;
 #define BSP_OPERANDS s->dtype, a.data(), b.data(), cp, ta, tb, (int)Z, (int)K, a.stride[0], a.stride[1], a.stride[2], b.stride[0], b.stride[1], b.stride[2], c_sz, s->block
   int rc = BSP_NEEDS_TABLE;
-  if (long_k)
+  if (tiles)
+    rc = unlocked([&] {
+      return bsp_sdd_matmul(BSP_OPERANDS, 0, nullptr, nullptr, s->C, s->tiles.table, s->tiles.n_groups, s->tiles.lines, flags | BSP_FLAG_PLAN_TILES, st);
+    });
+  if (rc != BSP_NEEDS_TABLE) {
+  } else if (long_k)
     rc = unlocked([&] { return bsp_sdd_matmul(BSP_OPERANDS, 0, nullptr, nullptr, s->long_entries < s->C ? s->long_entries : s->C, s->longk.table, s->longk.n_groups, s->longk.lines,
                         flags | (s->long_rowpair ? BSP_FLAG_PLAN_ROWPAIR : 0), st); });
   else if (s->n_levels < 0)

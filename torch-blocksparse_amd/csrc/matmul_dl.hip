@@ -23,7 +23,9 @@
 // A standalone dense probe of this pipeline (128 x 256 x 32 tiles) reaches 0.9 PFLOP/s on an 8192 x 4096 x 4096
 // product where the register-staged general kernel reaches 0.75.
 #include "matmul_generic.h"
+#include <algorithm>
 #include <atomic>
+#include <vector>
 
 namespace bsp {
 namespace {
@@ -722,6 +724,182 @@ template <typename T, int BLOCK> int launch_sdd_rg_dl(const SddArgs &g, bool a_k
 }
 
 // ---------------------------------------------------------------------------------------------------------
+// sdd with a long reduction, blocks of 32, fp16 / bf16, layouts that hold a fair share of their blocks: a workgroup of eight
+// wavefronts takes sixteen consecutive block-rows (512 rows of A) and up to sixteen block-columns gathered so that at most 64 blocks
+// lie in them (512 rows of B), and computes those blocks and no others: each wavefront eight of them, from a list, in registers over
+// the whole reduction.  What bounds k_sdd_rg_dl at these layouts is work and feed for absent blocks: it multiplies its whole 128 x 256
+// tile, of which a quarter to a third of the blocks exist.  Here a step's 64 KiB at most serve up to 64 blocks, all of them wanted, and
+// what bounds it is that feed and the LDS reads: a wavefront reads both fragments of every block (2 KiB a matrix instruction), so that
+// nothing in a step depends on the list but the addresses, which are computed once.  128 KiB of LDS: one workgroup a compute unit.
+// 16 heads of 64 x 64 blocks, a quarter of them there, batch 8, reduction 2048, fp16: 1594 -> 1071 us (513 TFLOP/s), 1668 -> 965 with
+// A transposed.
+// Tiles (bsp_sdd_tiles_build), kTileInts ints each: head, first block-row, block-columns n, blocks m, the 16 block-columns (the last
+// repeated), per block its id, per block its row in the tile + 256 * its column in the tile (the first repeated past m).
+// ---------------------------------------------------------------------------------------------------------
+constexpr int kTileRows = 16, kTileCols = 16, kTileBlocks = 64, kTileInts = 4 + kTileCols + 2 * kTileBlocks;
+
+template <typename T, bool A_KC, bool B_KC>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) k_sdd_list_dl(SddArgs g) {
+  typedef Mma<T, 32> M;
+  typedef typename M::frag_t frag_t;
+  constexpr int TM = kTileRows * 32, TN = kTileCols * 32, PER = kTileBlocks / 8;
+  typedef DlTile<T, TM, A_KC> XT;
+  typedef DlTile<T, TN, B_KC> YT;
+  constexpr int STAGE = XT::BYTES + YT::BYTES;
+  constexpr int XL = XT::LOADS / 8, YL = YT::LOADS / 8;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t w = xcd_remap(blockIdx.x, (int64_t)g.n_pgroups * g.Z);
+  const int z = (int)(w / g.n_pgroups);
+  const table_ptr tile = as_table(g.gplan) + (int64_t)kTileInts * (w % g.n_pgroups);
+  const int h = tile[0], row0 = tile[1] * 32, n_cols = tile[2], m = tile[3];
+  const table_ptr cols = tile + 4, where = tile + 4 + kTileCols + kTileBlocks;
+  const int rows_a = g.lines * 32;                    // rows of op(A) per head
+  const int64_t lda = g.lda, ldb = g.ldb;
+  const T *pa = reinterpret_cast<const T *>(g.a) + z * g.a_sz + h * g.a_sh + (int64_t)row0 * (A_KC ? lda : 1);
+  const T *pb = reinterpret_cast<const T *>(g.b) + z * g.b_sz + h * g.b_sh;
+  // Loop-invariant part of every load address, as in k_sdd_rg_dl: rows past the end of A read its last rows
+  uint32_t xoff[XL], yoff[YL];
+#pragma unroll
+  for (int i = 0; i < XL; i++) {
+    const int ld = wave * XL + i;
+    if constexpr (A_KC) {
+      const int row = ld * 16 + (lane >> 2), chunk16 = (lane & 3) ^ kc_swz(row);
+      const int r = row0 + row < rows_a ? row : rows_a - 1 - row0;
+      xoff[i] = (uint32_t)(r * lda + chunk16 * 8) * 2u;
+    } else {
+      constexpr int CPR = TM / 8;
+      const int j = ld * 64 + lane, k = j / CPR, slot = j % CPR;
+      const int c = (((slot >> 1) ^ ks_swz<TM>(k)) << 1) | (slot & 1);
+      const int r = row0 + c * 8 < rows_a ? c * 8 : rows_a - 8 - row0;
+      xoff[i] = (uint32_t)(k * lda + r) * 2u;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < YL; i++) {
+    const int ld = wave * YL + i;
+    if constexpr (B_KC) {
+      const int row = ld * 16 + (lane >> 2), chunk16 = (lane & 3) ^ kc_swz(row);
+      yoff[i] = (uint32_t)(((int64_t)cols[ld / 2] * 32 + (row & 31)) * ldb + chunk16 * 8) * 2u;
+    } else {
+      constexpr int CPR = TN / 8;
+      const int j = ld * 64 + lane, k = j / CPR, slot = j % CPR;
+      const int c = (((slot >> 1) ^ ks_swz<TN>(k)) << 1) | (slot & 1);
+      const int32_t *vcols = g.gplan + (int64_t)kTileInts * (w % g.n_pgroups) + 4;     // (the column differs from lane to lane)
+      yoff[i] = (uint32_t)(k * ldb + (int64_t)vcols[c >> 2] * 32 + (c & 3) * 8) * 2u;
+    }
+  }
+  // The wavefront's blocks: an equal share of the list, in its order (by rows).  LDS byte addresses of their fragments of the first
+  // stage; a row or column of blocks further is 2 KiB where the reduction is contiguous, 64 bytes (under the swizzle, so an
+  // exclusive-or) where it is strided.
+  const int first = wave * m / 8, count = (wave + 1) * m / 8 - first;
+  const uint32_t base = (uint32_t)(uintptr_t)((const void __attribute__((address_space(3))) *)smem);
+  const uint32_t xlane = A_KC ? (uint32_t)kc_offset(lane & 31, lane >> 5) : (uint32_t)ks_offset<TM>(8 * (lane >> 5) + ((lane & 15) >> 2), 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+  const uint32_t ylane = B_KC ? (uint32_t)kc_offset(lane & 31, lane >> 5) : (uint32_t)ks_offset<TN>(8 * (lane >> 5) + ((lane & 15) >> 2), 16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+  uint32_t xa[PER], ya[PER];
+#pragma unroll
+  for (int i = 0; i < PER; i++) {
+    const int rc = where[i < count ? first + i : first < m ? first : 0];
+    xa[i] = base + (A_KC ? xlane + (uint32_t)(rc & 255) * 2048u : xlane ^ ((uint32_t)(rc & 255) * 64u));
+    ya[i] = base + XT::BYTES + (B_KC ? ylane + (uint32_t)(rc >> 8) * 2048u : ylane ^ ((uint32_t)(rc >> 8) * 64u));
+  }
+  typename M::acc_t acc[PER];
+#pragma unroll
+  for (int i = 0; i < PER; i++)
+#pragma unroll
+    for (int v = 0; v < M::NACC; v++) acc[i][v] = 0.f;
+  const int ksteps = g.K / kTK;
+  auto issue = [&](int s, const unsigned char *st) {
+    const int64_t k0 = (int64_t)s * kTK;
+    const T *xb = pa + (A_KC ? k0 : k0 * lda);
+    const T *yb = pb + (B_KC ? k0 : k0 * ldb);
+#pragma unroll
+    for (int i = 0; i < XL; i++) load_lds16(xb, xoff[i], st + (wave * XL + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < YL; i++)
+      if (!B_KC || (wave * YL + i) / 2 < n_cols) load_lds16(yb, yoff[i], st + XT::BYTES + (wave * YL + i) * 1024);
+  };
+  // the fragment of reduction indices 16 kk .. at the address of indices 0 ..
+  auto fragment = [&](auto kcontig, auto rows, uint32_t at, int kk) {
+    typedef typename Mma<T, 32>::frag_t __attribute__((address_space(3))) * frag_ptr;
+    typedef s16x4 __attribute__((address_space(3))) * tr_ptr;
+    if constexpr (decltype(kcontig)::value) {
+      return *(frag_ptr)(uintptr_t)(at ^ (uint32_t)(kk << 5));
+    } else {
+      constexpr int ROW = decltype(rows)::value * 2;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)(at + kk * 16 * ROW)), hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)(at + (kk * 16 + 4) * ROW));
+      typedef short s16x8 __attribute__((ext_vector_type(8)));
+      return __builtin_bit_cast(frag_t, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+  };
+  issue(0, smem);
+  for (int s = 0; s < ksteps; s++) {
+    BSP_WAIT_VM(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + 1 < ksteps) issue(s + 1, smem + ((s + 1) & 1) * STAGE);
+    const uint32_t at = (uint32_t)(s & 1) * STAGE;
+#pragma unroll
+    for (int kk = 0; kk < kTK / 16; kk++)
+#pragma unroll
+      for (int i0 = 0; i0 < PER; i0 += 4) {
+        frag_t xf[4], yf[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          xf[i] = fragment(Const<A_KC>{}, Const<TM>{}, xa[i0 + i] + at, kk);
+          yf[i] = fragment(Const<B_KC>{}, Const<TN>{}, ya[i0 + i] + at, kk);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i0 + i] = M::run(yf[i], xf[i], acc[i0 + i]);     // 4 consecutive values run along the block's columns
+      }
+  }
+  BSP_WAIT_VM(0);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  // each block through the wavefront's piece of LDS to 2 KiB of consecutive addresses
+  constexpr int LDR = 40;
+  T *stage = reinterpret_cast<T *>(smem) + wave * 32 * LDR;
+  T *pc = reinterpret_cast<T *>(g.c) + z * g.c_sz;
+#pragma unroll
+  for (int i = 0; i < PER; i++)
+    if (i < count) {
+#pragma unroll
+      for (int g4 = 0; g4 < 4; g4++) {
+        union { u32x2 raw; T e[4]; } u;
+#pragma unroll
+        for (int e = 0; e < 4; e++) u.e[e] = from_float<T>(acc[i][4 * g4 + e]);
+        *reinterpret_cast<u32x2 *>(stage + (lane & 31) * LDR + 8 * g4 + 4 * (lane >> 5)) = u.raw;
+      }
+      __builtin_amdgcn_wave_barrier();                 // (the LDS operations of one wavefront complete in order)
+      T *dst = pc + (int64_t)tile[4 + kTileCols + first + i] * 1024;
+#pragma unroll
+      for (int c = lane; c < 128; c += 64) *reinterpret_cast<u32x4 *>(dst + c * 8) = *reinterpret_cast<const u32x4 *>(stage + (c >> 2) * LDR + (c & 3) * 8);
+      __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <typename T> int launch_sdd_list_dl(const SddArgs &g, bool a_kc, bool b_kc, hipStream_t st) {
+  constexpr int SMEM = 2 * (kTileRows + kTileCols) * 32 * kTK * 2;
+  const int64_t n_wg = (int64_t)g.n_pgroups * g.Z;
+  if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
+  dim3 grid((unsigned)n_wg), wg(512);
+#define BSP_SDD_LIST_LAUNCH(AK, BK)                                                                                     \
+  do {                                                                                                                  \
+    static std::atomic<uint64_t> done{0};                                                                               \
+    if (!raise_lds_limit((const void *)k_sdd_list_dl<T, AK, BK>, SMEM, done)) return BSP_ERR_HIP;                       \
+    hipLaunchKernelGGL((k_sdd_list_dl<T, AK, BK>), grid, wg, SMEM, st, g);                                              \
+  } while (0)
+  if (a_kc && b_kc) BSP_SDD_LIST_LAUNCH(true, true);
+  else if (a_kc) BSP_SDD_LIST_LAUNCH(true, false);
+  else if (b_kc) BSP_SDD_LIST_LAUNCH(false, true);
+  else BSP_SDD_LIST_LAUNCH(false, false);
+#undef BSP_SDD_LIST_LAUNCH
+  return BSP_OK;
+}
+
+// ---------------------------------------------------------------------------------------------------------
 // sdd over a long reduction into few blocks of 128 (the weight gradient of a block-sparse linear layer: 102 blocks,
 // reduction over 8192 tokens).  One workgroup per block leaves most of the chip idle, four 64 x 64 workgroups per block
 // fetch every operand row twice.  Here a workgroup computes a whole 128 x 128 block over a PART of the reduction with
@@ -976,6 +1154,15 @@ int sdd128_splitk(int dtype, const SddArgs &g, int parts, float *ws, bool a_kc, 
   return dtype == BSP_F16 ? launch_sdd128_splitk<f16>(g, sk, a_kc, b_kc, st) : launch_sdd128_splitk<bf16>(g, sk, a_kc, b_kc, st);
 }
 
+// The same from the tiles of bsp_sdd_tiles_build (g.gplan, g.n_pgroups of them; g.lines: block-rows, g.cols: block-columns of a head):
+// 2 = launched, every block of the layout written; 0 = not applicable, < 0 = error
+int sdd_list(int dtype, const SddArgs &g, int block, bool a_kc, bool b_kc, hipStream_t st) {
+  if (dtype == BSP_F32 || block != 32 || !g.gplan || g.n_pgroups <= 0 || g.lines <= 0 || g.cols <= 0) return 0;
+  if (g.K < 256 || g.K % kTK || !near_rows(kTileRows * 32, g.lda) || !near_rows(b_kc ? (int64_t)g.cols * 32 : kTK, g.ldb)) return 0;
+  const int rc = dtype == BSP_F16 ? launch_sdd_list_dl<f16>(g, a_kc, b_kc, st) : launch_sdd_list_dl<bf16>(g, a_kc, b_kc, st);
+  return rc == BSP_OK ? 2 : rc;
+}
+
 // sdd with a long reduction at blocks of 32 from the group plan alone: 2 = launched (every block of the layout is
 // written), 0 = not applicable, < 0 = error
 int sdd_dl(int dtype, const SddArgs &g, int block, bool rowpair_plan, bool a_kc, bool b_kc, hipStream_t st) {
@@ -989,3 +1176,65 @@ int sdd_dl(int dtype, const SddArgs &g, int block, bool rowpair_plan, bool a_kc,
 }
 
 }  // namespace bsp
+
+extern "C" int bsp_sdd_tiles_build(const uint8_t *layout, int H, int R, int C, int32_t *out, int64_t cap, int64_t *n_tiles) {
+  using namespace bsp;
+  if (!layout || !n_tiles || H <= 0 || R <= 0 || C <= 0 || cap < 0 || (cap > 0 && !out)) return BSP_ERR_ARG;
+  int64_t n = 0, blocks_before = 0;
+  std::vector<int64_t> row_first(R + 1);               // id of the first block of a block-row
+  for (int h = 0; h < H; h++) {
+    const uint8_t *lay = layout + (int64_t)h * R * C;
+    row_first[0] = blocks_before;
+    for (int r = 0; r < R; r++) row_first[r + 1] = row_first[r] + std::count_if(lay + (int64_t)r * C, lay + (int64_t)(r + 1) * C, [](uint8_t v) { return v != 0; });
+    blocks_before = row_first[R];
+    for (int r0 = 0; r0 < R; r0 += kTileRows) {
+      const int rows = R - r0 < kTileRows ? R - r0 : kTileRows;
+      // a tile's blocks: those of whole columns, except that its first column may lack its first rows and its last one its last rows,
+      // which the tile before and the next one have (64 x 64 blocks a head, 90 % of them there: tiles of whole columns 3147 us, these 2555)
+      int cols[kTileCols], n_cols = 0, m = 0, from = 0, upto = rows;
+      int64_t next[kTileRows];                         // id of the row's next block
+      for (int r = 0; r < rows; r++) next[r] = row_first[r0 + r];
+      auto flush = [&]() {
+        if (m && (n + 1) * kTileInts <= cap) {
+          int32_t *t = out + n * kTileInts, at = 0;
+          t[0] = h; t[1] = r0; t[2] = n_cols; t[3] = m;
+          for (int c = 0; c < kTileCols; c++) t[4 + c] = cols[c < n_cols ? c : n_cols - 1];
+          for (int r = 0; r < rows; r++)
+            for (int c = 0; c < n_cols; c++)
+              if (lay[(int64_t)(r0 + r) * C + cols[c]] && (c > 0 || r >= from) && (c < n_cols - 1 || r < upto)) {
+                t[4 + kTileCols + at] = (int32_t)next[r]++;
+                t[4 + kTileCols + kTileBlocks + at++] = r | c << 8;
+              }
+          for (; at < kTileBlocks; at++) t[4 + kTileCols + at] = -1, t[4 + kTileCols + kTileBlocks + at] = t[4 + kTileCols + kTileBlocks];
+        }
+        if (m) n++;
+        n_cols = m = 0;
+        from = 0;
+        upto = rows;
+      };
+      for (int c = 0; c < C; c++) {
+        int here = 0;
+        for (int r = 0; r < rows; r++) here += lay[(int64_t)(r0 + r) * C + c] != 0;
+        if (!here) continue;
+        if (n_cols == kTileCols || m == kTileBlocks) flush();
+        cols[n_cols++] = c;
+        if (m + here <= kTileBlocks) {
+          m += here;
+          continue;
+        }
+        int r = 0, left = kTileBlocks - m;             // the rows before r fill the tile
+        for (; left > 0; r++) left -= lay[(int64_t)(r0 + r) * C + c] != 0;
+        here -= kTileBlocks - m;
+        m = kTileBlocks;
+        upto = r;
+        flush();
+        cols[n_cols++] = c;
+        m = here;
+        from = r;
+      }
+      flush();
+    }
+  }
+  *n_tiles = n;
+  return n * kTileInts > cap ? BSP_ERR_CAPACITY : BSP_OK;
+}

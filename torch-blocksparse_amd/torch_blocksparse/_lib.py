@@ -19,7 +19,7 @@ F16, BF16, F32 = 0, 1, 2
 DTYPES = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
 
 ROWS_WITH_REST = 256  # BSP_ROWS_WITH_REST
-FLAG_GENERAL_ONLY, FLAG_NO_GROUPS, FLAG_NO_WIDE, FLAG_PLAN_ROWPAIR, FLAG_ANY_K, FLAG_WHOLE_K = 1, 2, 4, 8, 16, 32   # bsp_launch_flags
+FLAG_GENERAL_ONLY, FLAG_NO_GROUPS, FLAG_NO_WIDE, FLAG_PLAN_ROWPAIR, FLAG_ANY_K, FLAG_WHOLE_K, FLAG_PLAN_TILES = 1, 2, 4, 8, 16, 32, 64   # bsp_launch_flags
 
 OK = 0
 OK_WHOLE_LAYOUT = 1   # bsp_sdd_matmul: the group plan was used, every block of the layout is written
@@ -58,6 +58,7 @@ SIGNATURES = {
                             _i64, _vp, _i, _i, _i, _vp]),
     'bsp_sdd_matmul_levels': (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _i, _vp, _vp, _vp, _vp,
                                    _vp, _i, _i, _i, _i64, _vp, _i64, _i, _vp]),
+    'bsp_sdd_tiles_build': (_i, [_vp, _i, _i, _i, _vp, _i64, _vp]),
     'bsp_sdd_parts': (_i, [_i, _i, _i, _vp, _vp, _i, _i, _i]),
     'bsp_sdd_parts_workspace_bytes': (_i64, [_i, _i64, _i, _i]),
     'bsp_sdd_splitk_workspace_bytes': (_i64, [_i, _i64, _i]),

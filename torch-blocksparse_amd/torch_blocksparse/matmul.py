@@ -201,6 +201,17 @@ class GroupPlan:
         out.rowpair = True
         return out
 
+    @staticmethod
+    def build_sdd_tiles(layout, device):
+        """The tiles of the sdd kernel for long reductions at block 32 (bsp_sdd_tiles_build), made on the host"""
+        lay = (layout != 0).to(torch.uint8).cpu().contiguous()
+        H, R, C = lay.shape
+        n, lib = ctypes.c_int64(0), _lib.load()
+        cap = 148 * (int(lay.sum()) // 16 + H * (-(-R // 16)) * (C // 16 + 1))
+        host = torch.empty(cap, dtype=torch.int32)
+        _lib.check(lib.bsp_sdd_tiles_build(_lib.ptr(lay), H, R, C, _lib.ptr(host), cap, ctypes.byref(n)), 'bsp_sdd_tiles_build')
+        return GroupPlan(host[:148 * n.value].to(device), n.value, R)
+
     def max_entries(self):
         """The largest number of entries of any group of the plan (read back from the device once and kept)."""
         if self._max_entries is None:
@@ -283,7 +294,29 @@ class SddTables(list):
     packs = None
     any_k = False         # a reduction along the rows of both operands may have any length (the weight gradient of Linear)
 
+    tiles = None          # block 32: the tiles of bsp_sdd_tiles_build, built by build_tiles on demand
+    build_tiles = None
     _splitk_ws = None
+
+    # Long reductions at block 32 run from the tiles (k_sdd_list_dl) rather than from the groups of block-rows (k_sdd_rg_dl) where a launch
+    # has TILES_LAUNCH tiles, they hold TILE_BLOCKS blocks on average and the layout at most TILES_DENSITY of its blocks.  Measured on
+    # 64 x 64 blocks a head, fp16, reduction 2048, us from groups / tiles:  16 heads, batch 8:  density .05 (18 blocks a tile) 620 / 670,
+    # .075 (24) 1087 / 790, .1 (26) 1062 / 877, .25 (52) 1582 / 1071, .5 (60) 2088 / 1658, .7 2307 / 2173, .9 2475 / 2555;
+    # density .25, 312 tiles 224 / 186, 157 tiles 107 / 88;  other layouts, 132 tiles of 55 blocks 31 / 33, 132 of 46 blocks 57 / 44.
+    TILES_LAUNCH, TILE_BLOCKS, TILES_DENSITY = 150, 22, .75
+
+    def tiles_apply(self):
+        """whether the layout is one for the tiles at all (a batch may still be too small)"""
+        return self.build_tiles is not None and self.spdims is not None and self.nnz <= self.TILES_DENSITY * math.prod(self.spdims)
+
+    def tiles_for(self, Z):
+        """the tiles, where this batch should run on them (fp16 / bf16, a reduction for long ones)"""
+        if not self.tiles_apply() or self.nnz * Z < self.TILES_LAUNCH * self.TILE_BLOCKS:
+            return None
+        if self.tiles is None and not torch.cuda.is_current_stream_capturing():
+            self.tiles = self.build_tiles()
+        t = self.tiles
+        return t if t is not None and t.n_groups * Z >= self.TILES_LAUNCH and self.nnz >= self.TILE_BLOCKS * t.n_groups else None
 
     def splitk_workspace(self, need, device):
         """address of a workspace of `need` bytes for the sdd in parts: it only grows, and one that a larger launch supersedes stays
@@ -368,6 +401,7 @@ class _sparse_matmul(torch.autograd.Function):
         luts.gplan_long = None
         if block == 32:
             luts.build_long = lambda: GroupPlan.build(layout, True, dev, thin_min=0, order_buckets=1, ctx=ctx)
+            luts.build_tiles = lambda: GroupPlan.build_sdd_tiles(layout, dev)
         elif block == 16 and R % 2 == 0:
             # blocks of 16: the same kernel on pairs of block-rows (a plan and a flag of its own)
             luts.build_long = lambda: GroupPlan.build_rowpair(layout, dev, ctx=ctx)
@@ -416,9 +450,16 @@ class _sparse_matmul(torch.autograd.Function):
             if luts.gplan_long is None:
                 luts.gplan_long = luts.build_long()
             lp = GroupPlan.args(luts.gplan_long)
+            tiles = luts.tiles_for(AS0)
+            if tiles is not None:
+                rc = lib.bsp_sdd_matmul(*operands, 0, ctypes.c_void_p(0), ctypes.c_void_p(0), spdims[2], _lib.ptr(tiles.table), tiles.n_groups, tiles.lines,
+                                        flags | _lib.FLAG_PLAN_TILES, _lib.stream_ptr(a.device))
+                if rc not in (_lib.OK_WHOLE_LAYOUT, _lib.NEEDS_TABLE):
+                    _lib.check(rc, 'bsp_sdd_matmul')
             # (the largest group of the plan sizes the grid: workgroups for block-columns that no group reaches are not launched)
-            rc = lib.bsp_sdd_matmul(*operands, 0, ctypes.c_void_p(0), ctypes.c_void_p(0), min(spdims[2], luts.gplan_long.max_entries()),
-                                    lp[0], lp[1], lp[2], flags | (_lib.FLAG_PLAN_ROWPAIR if luts.gplan_long.rowpair else 0), _lib.stream_ptr(a.device))
+            if rc == _lib.NEEDS_TABLE:
+                rc = lib.bsp_sdd_matmul(*operands, 0, ctypes.c_void_p(0), ctypes.c_void_p(0), min(spdims[2], luts.gplan_long.max_entries()),
+                                        lp[0], lp[1], lp[2], flags | (_lib.FLAG_PLAN_ROWPAIR if luts.gplan_long.rowpair else 0), _lib.stream_ptr(a.device))
             if rc not in (_lib.OK_WHOLE_LAYOUT, _lib.NEEDS_TABLE):
                 _lib.check(rc, 'bsp_sdd_matmul')
         elif lazy and luts.gplan is not None and luts.build is not None and not any_k:
@@ -670,7 +711,7 @@ class _Product:
     def _on_demand(self, which):
         lut = self.luts[4 * which]
         if self.modes[which] == 'sdd':
-            return lut.gplan_long is None, lut.build is None
+            return lut.gplan_long is None, lut.build is None, lut.tiles is None
         return (lut.gplan_wide is None,)
 
     def _tables(self, which):
@@ -687,9 +728,12 @@ class _Product:
                 levels = tuple((p, t.data_ptr(), t.valid.data_ptr() if getattr(t, 'valid', None) is not None else 0, w)
                                for t, w, p in zip(lut, lut.widths, lut.packs))
             late = lut.gplan_long
-            made = _lib.native().make_sdd((lut, lut.gplan, late) + tuple(lut) + tuple(getattr(t, 'valid', None) for t in lut), self.block, self.dtype, dev, lut.nnz, H, R, C,
+            tiles = lut.tiles
+            made = _lib.native().make_sdd((lut, lut.gplan, late, tiles) + tuple(lut) + tuple(getattr(t, 'valid', None) for t in lut), self.block, self.dtype, dev, lut.nnz, H, R, C,
                                           plan(lut.gplan), plan(late), 0 if lut.build_long is None else 1 if late is None else 2,
-                                          int(late is not None and late.rowpair), late.max_entries() if late is not None else 0, int(lut.any_k), levels)
+                                          int(late is not None and late.rowpair), late.max_entries() if late is not None else 0, int(lut.any_k),
+                                          plan(tiles), (1 if tiles is None else 2) if lut.tiles_apply() else 0,
+                                          lut.TILES_LAUNCH, lut.TILE_BLOCKS, levels)
         else:
             made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, lut.longest, lut.nnz, H, R, C,
                                           plan(lut.gplan), plan(lut.gplan_wide),

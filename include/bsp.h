@@ -151,7 +151,7 @@ typedef enum {
   BSP_FLAG_ANY_K = 16,        /* bsp_sdd_matmul_levels with trans_a and not trans_b (the reduction runs along the rows of both operands): K need
                                  not be a multiple of 16 */
   BSP_FLAG_WHOLE_K = 32,       /* bsp_sdd_parts, bsp_xsd_parts: one part whatever the sizes (for cross-checks) */
-  BSP_FLAG_PLAN_TILES = 64     /* bsp_sdd_matmul without a table: d_gplan holds n_plan_groups tiles of bsp_sdd_tiles_build, plan_lines and n_groups the
+  BSP_FLAG_PLAN_TILES = 64     /* bsp_dsd_matmul, bsp_dds_matmul: see bsp_xsd_chunks_build.  bsp_sdd_matmul without a table: d_gplan holds n_plan_groups tiles of bsp_sdd_tiles_build, plan_lines and n_groups the
                                   block-rows and block-columns of a head; blocks of 32, K >= 256, K % 32 == 0, 16-bit types */
 } bsp_launch_flags;
 
@@ -180,6 +180,12 @@ int bsp_sdd_matmul(int dtype, const void *a, const void *b, void *c, int trans_a
  * the heads and block-rows (BSP_ERR_CAPACITY with *n_tiles set when cap ints do not hold them).  A tile is sixteen consecutive block-rows by
  * up to sixteen block-columns that hold at most 64 blocks there. */
 int bsp_sdd_tiles_build(const uint8_t *layout, int H, int R, int C, int32_t *out, int64_t cap, int64_t *n_tiles);
+
+/* The same for dsd and dds: with BSP_FLAG_PLAN_TILES d_gplan holds the ints of bsp_xsd_chunks_build, n_plan_groups its groups, plan_lines the
+ * lines of a head (block-rows with rows != 0, else block-columns; what the product's table has as its lines).  They serve blocks of 32 of
+ * 16-bit types with a free dimension of 128 or more; another product runs from its table alone.  *n_ints ints: per sixteen consecutive lines (*n_groups of those) four,
+ * then records of 32, each up to four reduction blocks in which the lines have at most 24 blocks. */
+int bsp_xsd_chunks_build(const uint8_t *layout, int H, int R, int C, int rows, int32_t *out, int64_t cap, int *n_groups, int64_t *n_ints);
 
 /* ... all pack levels of the table (n_levels <= 3, each pack width at most once) in one call: packs, d_luts, d_valids (entries may
  * be NULL) and n_groups are host arrays with what a call of bsp_sdd_matmul per level would get.  Blocks of 16 and 32, which are

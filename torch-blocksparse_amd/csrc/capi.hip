@@ -204,12 +204,14 @@ static int xsd_workspace(XsdArgs &g, int n_split, int free_dim, void *d_ws, int6
   return BSP_OK;
 }
 
-static int xsd_dispatch(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, int flags, void *stream) {
+static int xsd_dispatch(int dtype, XsdArgs g, int block, bool sp_trans, bool dn_kc, bool out_nc, int flags, void *stream) {
   hipStream_t st = as_stream(stream);
   // a wide free dimension at blocks 64 / 128: the kernels bound by the matrix cores and the feed from L2
-  int rc = no_wide(flags) ? 0 : xsd_dl(dtype, g, block, sp_trans, dn_kc, out_nc, st);
+  const bool chunks = (flags & BSP_FLAG_PLAN_TILES) != 0;
+  int rc = no_wide(flags) ? 0 : chunks ? xsd_list(dtype, g, block, sp_trans, dn_kc, out_nc, st) : xsd_dl(dtype, g, block, sp_trans, dn_kc, out_nc, st);
   if (rc < 0) return rc;
   if (rc == 1) { BSP_LAUNCH_CHECK(); return BSP_OK; }
+  if (chunks) g.gplan = nullptr;                       // (the chunks serve no other kernel)
   rc = general_only(flags) ? 0 : xsd_fast64(dtype, g, block, sp_trans, dn_kc, out_nc, st);
   if (rc < 0) return rc;
   if (rc == 1) { BSP_LAUNCH_CHECK(); return BSP_OK; }

@@ -135,6 +135,7 @@ struct Xsd {
   int width, block, dtype, dev, longest;
   int64_t nnz, H, R, C;
   Plan ordinary, wide;
+  int wide_flags;                                       // that go with the wide plan
   int wide_state;                                       // 0: there is none, 1: not built yet, 2: built
 };
 struct Sdd {
@@ -176,8 +177,8 @@ const char *kXsd = "torch_blocksparse.xsd", *kSdd = "torch_blocksparse.sdd", *kR
 PyObject *make_xsd(PyObject *, PyObject *args) {
   Xsd s{};
   unsigned long long lut, planbuf, gp, wp;
-  if (!PyArg_ParseTuple(args, "OKKiiiiiLLLL(Kiii)(Kiii)i", &s.keep, &lut, &planbuf, &s.width, &s.block, &s.dtype, &s.dev, &s.longest, &s.nnz, &s.H, &s.R, &s.C, &gp,
-                        &s.ordinary.n_groups, &s.ordinary.lines, &s.ordinary.n_split, &wp, &s.wide.n_groups, &s.wide.lines, &s.wide.n_split, &s.wide_state))
+  if (!PyArg_ParseTuple(args, "OKKiiiiiLLLL(Kiii)(Kiii)ii", &s.keep, &lut, &planbuf, &s.width, &s.block, &s.dtype, &s.dev, &s.longest, &s.nnz, &s.H, &s.R, &s.C, &gp,
+                        &s.ordinary.n_groups, &s.ordinary.lines, &s.ordinary.n_split, &wp, &s.wide.n_groups, &s.wide.lines, &s.wide.n_split, &s.wide_flags, &s.wide_state))
     return nullptr;
   s.lut = reinterpret_cast<const int32_t *>(lut); s.plan = reinterpret_cast<const int32_t *>(planbuf);
   s.ordinary.table = reinterpret_cast<const int32_t *>(gp); s.wide.table = reinterpret_cast<const int32_t *>(wp);
@@ -237,7 +238,7 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const Xsd *s = static_cast<const Xsd *>(PyCapsule_GetPointer(args[0], kXsd));
   if (!s) return nullptr;
   const bool dds = truth(args[1]), ta = truth(args[4]), tb = truth(args[5]), tc = truth(args[6]);
-  const int flags = (int)PyLong_AsLong(args[7]);
+  int flags = (int)PyLong_AsLong(args[7]);
   Operand sp, dn;
   if (!sp.read(args[dds ? 3 : 2]) || !dn.read(args[dds ? 2 : 3])) Py_RETURN_NONE;
   if (dn.dtype != s->dtype || sp.dtype != s->dtype || dn.dev != s->dev || sp.dev != s->dev || dn.dim != 4 || sp.dim < 3) Py_RETURN_NONE;
@@ -255,6 +256,7 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (block == 32 && free_dim >= 256 && s->dtype != BSP_F32 && s->wide_state && (int64_t)(s->width + 3) / 4 * ((free_dim + 255) / 256) * Z >= 384) {   // _plan_for in matmul.py
     if (s->wide_state != 2) Py_RETURN_NONE;
     plan = s->wide;
+    flags |= s->wide_flags;
   }
   const bool out_free_last = dds ? tc : !tc;            // the result's free dimension is its last one
   const int64_t shape[4] = {Z, s->H, out_free_last ? out_sp : free_dim, out_free_last ? free_dim : out_sp};

@@ -511,6 +511,266 @@ template <typename T> int launch_rg_dl(const XsdArgs &g, bool sp_trans, bool dn_
 }
 
 // ---------------------------------------------------------------------------------------------------------
+// ... and from chunks with lists of blocks: a workgroup of eight wavefronts takes sixteen consecutive lines and 128 columns of the free
+// dimension (512 x 128 of the result, 128 accumulators a lane) and walks chunks of up to four reduction blocks in which the lines have
+// at most 24 blocks together.  k_xsd_rg_dl feeds 16 KiB of the dense operand for the 1.5 blocks that four lines have in a reduction
+// block at a quarter density, 40 flops a byte, and the feed from L2 bounds it; here 8 KiB serve the four of sixteen lines: 64 flops a
+// byte.  A wavefront has 32 columns and eight of the lines, so the two wavefronts of a SIMD share the lines of the same columns and
+// every SIMD has all the blocks of a chunk to multiply, however they fall.  The dense operands of a chunk stay in registers
+// for all of its lines; a block is 2 LDS reads and 2 matrix instructions behind a bit of the chunk's mask.  Two stages of 80 KiB: one
+// workgroup a compute unit, which stays for many tiles, so that the next chunk is in flight while this one is multiplied, also where it
+// is the first of the next tile, during this one's stores.  What bounds it now is LDS (192 KiB read and 64 written for a chunk of 16
+// blocks) and the stores, which wait together.
+// 16 heads of 64 x 64 blocks, a quarter of them there, batch 8, free dimension 2048, fp16: 1175 -> 1054 us (519 TFLOP/s), with the dense
+// operand's reduction contiguous 1500 -> 1045.  A workgroup a tile with the whole tile staged in LDS at its end: 1277; the results
+// stored from registers: 1105.
+// Chunk records (bsp_xsd_chunks_build), kChunkInts ints: reduction blocks n, blocks m, the mask (two ints, bit 4 line + block of the
+// chunk), the n positions, the m ids in the order of the mask's bits.  Before them per group: head, first line, first chunk, chunks (a
+// group without blocks has a chunk without any).
+// ---------------------------------------------------------------------------------------------------------
+constexpr int kChunkLines = 16, kChunkCols = 4, kChunkBlocks = 24, kChunkInts = 8 + kChunkBlocks, kChunkN = 128;
+
+// Tiles lo, lo + stride ... below hi of a workgroup: the tiles are dealt to the XCDs in contiguous ranges, and an XCD's to its workgroups
+struct TileRange { uint32_t at, end, stride; };
+__device__ __forceinline__ TileRange tile_range(uint32_t n) {
+  const uint32_t v = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+  if (gridDim.x % 8) return {v, n, gridDim.x};
+  const uint32_t per = gridDim.x / 8, x = v / per;
+  return {(uint32_t)((uint64_t)n * x / 8) + v % per, (uint32_t)((uint64_t)n * (x + 1) / 8), per};
+}
+
+template <typename T, bool SP_TRANS, bool DN_KC, bool OUT_NC>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) k_xsd_list_dl(XsdArgs g) {
+  typedef Mma<T, 32> M;
+  typedef typename M::frag_t frag_t;
+  constexpr int B = 32, HALF = kChunkLines / 2;
+  typedef DlTile<T, B, !SP_TRANS> XT;                 // a block: 2 KiB
+  typedef DlTile<T, kChunkN, DN_KC> YT;               // 32 reduction indices of the dense tile: 8 KiB
+  static_assert(YT::LOADS == 8 && XT::LOADS == 2 && kChunkCols == 4 && kChunkBlocks % 8 == 0, "two wavefronts load a dense tile, each every eighth block");
+  constexpr int XBYTES = kChunkBlocks * XT::BYTES, STAGE = XBYTES + kChunkCols * YT::BYTES;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = wave >> 2, wn = wave & 3;          // wavefronts w and w + 4 run on one SIMD
+  // tiles in the order batch, head, columns, group: neighbours share the dense operand and the blocks in L2
+  const uint32_t n_tiles = (g.NF + kChunkN - 1) / kChunkN, per_head = (g.lines + kChunkLines - 1) / kChunkLines, heads = g.n_pgroups / per_head;
+  const TileRange tiles = tile_range((uint32_t)g.n_pgroups * n_tiles * (uint32_t)g.Z);
+  if (tiles.at >= tiles.end) return;
+  const int NF = g.NF;
+  const int64_t ldd = g.ldd, ldo = g.ldo;
+  const int32_t *records = g.gplan + 4 * (int64_t)g.n_pgroups;
+  struct Place { uint32_t group, nt, z; };             // of a tile: group of lines (of all heads), columns, batch
+  auto place = [&](uint32_t w) {
+    const uint32_t a = w / per_head, b = a / n_tiles, z = b / heads;
+    return Place{(b - z * heads) * per_head + (w - a * per_head), a - b * n_tiles, z};
+  };
+
+  // the tile being loaded
+  const int ycol = wave >> 1;                         // the wavefront loads one half of the dense tile of this reduction block
+  uint32_t xoff[2], yoff[4];
+  const T *sp = nullptr, *dn = nullptr;
+#pragma unroll
+  for (int i = 0; i < 2; i++) xoff[i] = SP_TRANS ? XT::lane_offset(i, lane, 1, B) : XT::lane_offset(i, lane, B, 1);
+  auto load_from = [&](Place p, int depth) {
+    const int n0 = (int)p.nt * kChunkN;
+    sp = reinterpret_cast<const T *>(g.sp) + p.z * g.sp_sz;
+    dn = reinterpret_cast<const T *>(g.dn) + p.z * g.dn_sz + depth * g.dn_sh + (DN_KC ? n0 * ldd : n0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int ld = (wave & 1) * 4 + i;
+      if constexpr (DN_KC) {
+        const int row = ld * 16 + (lane >> 2), chunk = (lane & 3) ^ kc_swz(row);
+        const int n = n0 + row < NF ? row : NF - 1 - n0;
+        yoff[i] = (uint32_t)(n * ldd + chunk * 8) * 2u;
+      } else {
+        constexpr int CPR = kChunkN / 8;
+        const int j = ld * 64 + lane, k = j / CPR, slot = j % CPR;
+        const int chunk = (((slot >> 1) ^ ks_swz<kChunkN>(k)) << 1) | (slot & 1);
+        const int n = n0 + chunk * 8 < NF ? chunk * 8 : NF - 8 - n0;   // whole chunks: NF is a multiple of 8
+        yoff[i] = (uint32_t)(k * ldd + n) * 2u;
+      }
+    }
+  };
+  auto issue = [&](int rec, unsigned char *st) {       // rec: the chunk's record, int l in lane l
+    const int cols = __builtin_amdgcn_readlane(rec, 0), blocks = __builtin_amdgcn_readlane(rec, 1);
+    if (ycol < cols) {
+      const int64_t pos = (int64_t)__builtin_amdgcn_readlane(rec, 4 + ycol) * B;
+      const T *yb = dn + (DN_KC ? pos : pos * ldd);
+#pragma unroll
+      for (int i = 0; i < 4; i++) load_lds16(yb, yoff[i], st + XBYTES + ycol * YT::BYTES + ((wave & 1) * 4 + i) * 1024);
+    }
+#pragma unroll
+    for (int b0 = 0; b0 < kChunkBlocks; b0 += 8) {
+      const int b = b0 + wave;
+      if (b < blocks) {
+        const T *xb = sp + (int64_t)__builtin_amdgcn_readlane(rec, 8 + b) * (B * B);
+#pragma unroll
+        for (int i = 0; i < 2; i++) load_lds16(xb, xoff[i], st + b * XT::BYTES + i * 1024);
+      }
+    }
+  };
+  typename M::acc_t acc[HALF];
+#pragma unroll
+  for (int m = 0; m < HALF; m++)
+#pragma unroll
+    for (int v = 0; v < M::NACC; v++) acc[m][v] = 0.f;
+
+  const int at = lane & (kChunkInts - 1);
+  uint32_t w = tiles.at;
+  Place here = place(w);
+  int depth, line0, chunk0, chunks;                    // of the tile at w, then of the one after it
+  auto header = [&](uint32_t group) {
+    const table_ptr hd = as_table(g.gplan) + 4 * (int64_t)group;
+    depth = hd[0]; line0 = hd[1]; chunk0 = hd[2]; chunks = hd[3];
+  };
+  header(here.group);
+  int rec = records[(int64_t)kChunkInts * chunk0 + at], next = records[(int64_t)kChunkInts * (chunk0 + (chunks > 1)) + at];
+  load_from(here, depth);
+  asm volatile("" : "+v"(rec), "+v"(next));
+  unsigned stage = 0;
+  issue(rec, smem);
+  BSP_WAIT_VM(0);
+  for (;;) {
+    const bool more = w + tiles.stride < tiles.end;
+    const int depth_here = depth, line_here = line0, chunk_here = chunk0, n_chunks = chunks;
+    Place then = here;
+    // the next tile's place and first records
+    int rec_after = 0, next_after = 0;
+    if (more) {
+      then = place(w + tiles.stride);
+      header(then.group);
+      rec_after = records[(int64_t)kChunkInts * chunk0 + at];
+      next_after = records[(int64_t)kChunkInts * (chunk0 + (chunks > 1)) + at];
+    }
+    for (int s = 0;; s++) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();                    // everybody's loads of the chunk have landed, and everybody is done reading the one before
+      asm volatile("" ::: "memory");
+      const unsigned low = __builtin_amdgcn_readlane(rec, 2), mask = half ? __builtin_amdgcn_readlane(rec, 3) : low;
+      const unsigned char *st = smem + stage * STAGE;
+      stage ^= 1;
+      if (s + 1 < n_chunks) {
+        issue(next, smem + stage * STAGE);
+        rec = next;
+        if (s + 2 < n_chunks) next = records[(int64_t)kChunkInts * (chunk_here + s + 2) + at];
+      } else if (more) {
+        load_from(then, depth);
+        issue(rec_after, smem + stage * STAGE);
+        rec = rec_after;
+        next = next_after;
+      }
+      const unsigned char *xs = st + (half ? __builtin_popcount(low) : 0) * XT::BYTES;
+      frag_t yf[kChunkCols][kTK / 16];
+#pragma unroll
+      for (int c = 0; c < kChunkCols; c++)
+#pragma unroll
+        for (int kk = 0; kk < kTK / 16; kk++) yf[c][kk] = YT::frag(st + XBYTES + c * YT::BYTES, wn * 32, kk, lane);   // (past the chunk's reduction blocks: never used)
+#pragma unroll
+      for (int m = 0; m < HALF; m++)
+#pragma unroll
+        for (int c = 0; c < kChunkCols; c++)
+          if ((mask >> (m * kChunkCols + c)) & 1) {
+            // (their latency is the other wavefront's time: read a block ahead, which takes moving them, the kernel was 2 % slower)
+            frag_t xf[kTK / 16];
+#pragma unroll
+            for (int kk = 0; kk < kTK / 16; kk++) xf[kk] = XT::frag(xs, 0, kk, lane);
+#pragma unroll
+            for (int kk = 0; kk < kTK / 16; kk++) {
+              if constexpr (OUT_NC) acc[m] = M::run(yf[c][kk], xf[kk], acc[m]);
+              else acc[m] = M::run(xf[kk], yf[c][kk], acc[m]);
+            }
+            xs += XT::BYTES;
+          }
+      if (s + 1 >= n_chunks) break;
+      BSP_WAIT_VM(0);                                  // this wavefront's loads of the next chunk, and the record after it
+      asm volatile("" : "+v"(next), "+v"(rec_after), "+v"(next_after) : : "memory");
+    }
+    // the results, one half of the lines at a time, through the stage just read (the next tile's first chunk is on its way to the other
+    // one), so that whole rows of them are stored: from registers it would be 64 bytes of a row at a time
+    const int n0 = (int)here.nt * kChunkN;
+    T *oz = reinterpret_cast<T *>(g.out) + here.z * g.out_sz + depth_here * g.out_sh;
+    constexpr int TM = HALF * B, CW = OUT_NC ? kChunkN : TM, NR = OUT_NC ? TM : kChunkN, LDR = CW + 8;
+    static_assert(NR * LDR * 2 <= STAGE && NR * CW / 8 == 512 * HALF, "half a tile fits into a stage, eight stores a lane");
+    T *buf = reinterpret_cast<T *>(smem + (stage ^ 1) * STAGE);
+    auto store = [&](auto whole) {
+#pragma unroll
+      for (int hh = 0; hh < 2; hh++) {
+        BSP_WAIT_VM(63);                               // (LDS only)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (half == hh) {
+#pragma unroll
+          for (int m = 0; m < HALF; m++)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; g4++) {
+              const int fast = 8 * g4 + 4 * (lane >> 5), slow = lane & 31;
+              const int row = OUT_NC ? m * B + slow : wn * 32 + slow, col = OUT_NC ? wn * 32 + fast : m * B + fast;
+              union { u32x2 raw; T e[4]; } u;
+#pragma unroll
+              for (int e = 0; e < 4; e++) u.e[e] = from_float<T>(acc[m][4 * g4 + e]);
+              *reinterpret_cast<u32x2 *>(buf + row * LDR + col) = u.raw;
+            }
+        }
+        BSP_WAIT_VM(63);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int m0 = (line_here + hh * HALF) * B, rows = g.lines * B - m0;      // first row of the half; how many there are
+#pragma unroll
+        for (int i = 0; i < HALF; i++) {
+          const int c = tid + i * 512, row = c / (CW / 8), col = (c % (CW / 8)) * 8;
+          const u32x4 v = *reinterpret_cast<const u32x4 *>(buf + row * LDR + col);
+          T *dst = OUT_NC ? oz + (int64_t)(m0 + row) * ldo + n0 + col : oz + (int64_t)(n0 + row) * ldo + m0 + col;
+          if (decltype(whole)::value || (OUT_NC ? row < rows && n0 + col < NF : col < rows && n0 + row < NF)) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(dst));
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < HALF; m++)
+#pragma unroll
+        for (int v = 0; v < M::NACC; v++) acc[m][v] = 0.f;
+    };
+    // the next tile's first chunk was asked for before the stores of this one, which need not be waited for where their number is known
+    if (line_here + kChunkLines <= g.lines && n0 + kChunkN <= NF) {
+      store(Const<1>{});
+      if (!more) break;
+      BSP_WAIT_VM(2 * HALF);
+    } else {
+      store(Const<0>{});
+      if (!more) break;
+      BSP_WAIT_VM(0);
+    }
+    w += tiles.stride;
+    here = then;
+  }
+}
+
+template <typename T> int launch_xsd_list_dl(const XsdArgs &g, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
+  const int64_t n_wg = (int64_t)g.n_pgroups * ((g.NF + kChunkN - 1) / kChunkN) * g.Z;
+  if (n_wg >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
+  constexpr int SMEM = 2 * (kChunkCols * kChunkN + kChunkBlocks * 32) * kTK * 2;
+  dim3 grid((unsigned)(n_wg < 256 ? n_wg : 256)), wg(512);
+#define BSP_XSD_LIST_LAUNCH(ST, DK, ON)                                                                                 \
+  do {                                                                                                                  \
+    static std::atomic<uint64_t> done{0};                                                                               \
+    if (!raise_lds_limit((const void *)k_xsd_list_dl<T, ST, DK, ON>, SMEM, done)) return BSP_ERR_HIP;                   \
+    hipLaunchKernelGGL((k_xsd_list_dl<T, ST, DK, ON>), grid, wg, SMEM, st, g);                                          \
+  } while (0)
+  const int key = (sp_trans ? 4 : 0) | (dn_kc ? 2 : 0) | (out_nc ? 1 : 0);
+  switch (key) {
+    case 0: BSP_XSD_LIST_LAUNCH(false, false, false); break;
+    case 1: BSP_XSD_LIST_LAUNCH(false, false, true); break;
+    case 2: BSP_XSD_LIST_LAUNCH(false, true, false); break;
+    case 3: BSP_XSD_LIST_LAUNCH(false, true, true); break;
+    case 4: BSP_XSD_LIST_LAUNCH(true, false, false); break;
+    case 5: BSP_XSD_LIST_LAUNCH(true, false, true); break;
+    case 6: BSP_XSD_LIST_LAUNCH(true, true, false); break;
+    default: BSP_XSD_LIST_LAUNCH(true, true, true); break;
+  }
+#undef BSP_XSD_LIST_LAUNCH
+  return BSP_OK;
+}
+
+// ---------------------------------------------------------------------------------------------------------
 // sdd with a long reduction (hundreds of elements or more), blocks of 32, fp16 / bf16.  One output block is a 32 x 32
 // product: a workgroup per block (or per 2 x 2 pack of the reference's table) fetches 2 + 2 KiB per 65 kflop and is bound
 // by the feed from L2 at a thirteenth of the matrix peak.  Here a workgroup takes a group of four consecutive block-rows
@@ -1144,6 +1404,14 @@ int xsd_dl(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bo
   return rc == BSP_OK ? 1 : rc;
 }
 
+// The same from the chunks of bsp_xsd_chunks_build (g.gplan, g.n_pgroups groups of them)
+int xsd_list(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
+  if (dtype == BSP_F32 || block != 32 || !g.gplan || g.n_pgroups <= 0 || g.lines <= 0 || g.NF < kChunkN || !near_rows(kTN, g.ldd)) return 0;
+  if (g.n_pgroups % ((g.lines + kChunkLines - 1) / kChunkLines)) return BSP_ERR_ARG;
+  const int rc = dtype == BSP_F16 ? launch_xsd_list_dl<f16>(g, sp_trans, dn_kc, out_nc, st) : launch_xsd_list_dl<bf16>(g, sp_trans, dn_kc, out_nc, st);
+  return rc == BSP_OK ? 1 : rc;
+}
+
 // sdd at blocks of 128 over a reduction cut into `parts` parts (pack-1 table rows; ws: parts fp32 blocks per table row and
 // batch, may be null when parts == 1): BSP_OK = launched, BSP_ERR_UNSUPPORTED = not this kernel's case
 int sdd128_splitk(int dtype, const SddArgs &g, int parts, float *ws, bool a_kc, bool b_kc, hipStream_t st) {
@@ -1237,4 +1505,60 @@ extern "C" int bsp_sdd_tiles_build(const uint8_t *layout, int H, int R, int C, i
   }
   *n_tiles = n;
   return n * kTileInts > cap ? BSP_ERR_CAPACITY : BSP_OK;
+}
+
+extern "C" int bsp_xsd_chunks_build(const uint8_t *layout, int H, int R, int C, int rows, int32_t *out, int64_t cap, int *n_groups, int64_t *n_ints) {
+  using namespace bsp;
+  if (!layout || !n_groups || !n_ints || H <= 0 || R <= 0 || C <= 0 || cap < 0 || (cap > 0 && !out)) return BSP_ERR_ARG;
+  const int L = rows ? R : C, K = rows ? C : R, per_head = (L + kChunkLines - 1) / kChunkLines;
+  const int64_t first = 4 * (int64_t)H * per_head;     // the records start behind the groups
+  int64_t n = 0, blocks_before = 0, group = 0;
+  std::vector<int32_t> id((int64_t)R * C);             // of the head's blocks, -1: none
+  for (int h = 0; h < H; h++) {
+    for (int64_t i = 0; i < (int64_t)R * C; i++) id[i] = layout[h * (int64_t)R * C + i] ? (int32_t)blocks_before++ : -1;
+    for (int l0 = 0; l0 < L; l0 += kChunkLines, group++) {
+      const int lines = L - l0 < kChunkLines ? L - l0 : kChunkLines;
+      const int64_t before = n;
+      int cols[kChunkCols], n_cols = 0, m = 0;
+      auto block_at = [&](int l, int k) { return rows ? id[(int64_t)(l0 + l) * C + k] : id[(int64_t)k * C + l0 + l]; };
+      auto flush = [&]() {
+        if (m && first + (n + 1) * kChunkInts <= cap) {
+          int32_t *r = out + first + n * kChunkInts;
+          std::fill(r, r + kChunkInts, 0);
+          r[0] = n_cols; r[1] = m;
+          int at = 0;
+          for (int c = 0; c < n_cols; c++) r[4 + c] = cols[c];
+          for (int l = 0; l < lines; l++)
+            for (int c = 0; c < n_cols; c++)
+              if (const int32_t b = block_at(l, cols[c]); b >= 0) {
+                const int bit = l * kChunkCols + c;
+                r[2 + bit / 32] = (int32_t)((uint32_t)r[2 + bit / 32] | 1u << bit % 32);
+                r[8 + at++] = b;
+              }
+        }
+        if (m) n++;
+        n_cols = m = 0;
+      };
+      for (int k = 0; k < K; k++) {
+        int here = 0;
+        for (int l = 0; l < lines; l++) here += block_at(l, k) >= 0;
+        if (!here) continue;
+        if (n_cols == kChunkCols || m + here > kChunkBlocks) flush();
+        cols[n_cols++] = k;
+        m += here;
+      }
+      flush();
+      if (n == before) {                               // no block: one record without any
+        if (first + (n + 1) * kChunkInts <= cap) std::fill(out + first + n * kChunkInts, out + first + (n + 1) * kChunkInts, 0);
+        n++;
+      }
+      if (4 * (group + 1) <= cap) {
+        int32_t *g = out + 4 * group;
+        g[0] = h; g[1] = l0; g[2] = (int32_t)before; g[3] = (int32_t)(n - before);
+      }
+    }
+  }
+  *n_groups = H * per_head;
+  *n_ints = first + n * kChunkInts;
+  return *n_ints > cap ? BSP_ERR_CAPACITY : BSP_OK;
 }

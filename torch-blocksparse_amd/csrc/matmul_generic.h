@@ -940,6 +940,7 @@ int sdd_fast64(int dtype, const SddArgs &g, int block, int pack, bool a_kc, bool
 int xsd_fast64(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st);
 // dsd / dds for a wide free dimension at blocks 64 / 128, 16-bit (matmul_dl.hip): same return convention
 int xsd_dl(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st);
+int xsd_list(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st);
 // sdd with a long reduction at blocks of 32, from the group plan alone (matmul_dl.hip): 2 = launched and every block written
 int sdd_dl(int dtype, const SddArgs &g, int block, bool rowpair_plan, bool a_kc, bool b_kc, hipStream_t st);
 int sdd_list(int dtype, const SddArgs &g, int block, bool a_kc, bool b_kc, hipStream_t st);   // ... from the tiles of bsp_sdd_tiles_build

@@ -97,6 +97,7 @@ class GroupPlan:
         self.table, self.n_groups, self.lines, self.n_split = table, n_groups, lines, n_split
         self.coarse = False
         self.rowpair = False
+        self.flags = 0        # launch flags that go with the plan
         self._max_entries = None
         self._ws = None
         self._ws_retired = []
@@ -211,6 +212,30 @@ class GroupPlan:
         host = torch.empty(cap, dtype=torch.int32)
         _lib.check(lib.bsp_sdd_tiles_build(_lib.ptr(lay), H, R, C, _lib.ptr(host), cap, ctypes.byref(n)), 'bsp_sdd_tiles_build')
         return GroupPlan(host[:148 * n.value].to(device), n.value, R)
+
+    @staticmethod
+    def build_xsd_chunks(layout, rows, device, always=False):
+        """The chunks of the dsd / dds kernel that works from lists of blocks (bsp_xsd_chunks_build), made on the host; None where the
+        kernel on groups of four lines (k_xsd_rg_dl) should run instead, unless `always`.
+        Measured on 16 heads of 64 x 64 blocks, batch 4, fp16, free dimension 1024, us from groups / chunks, dense reduction strided
+        (contiguous): density .1 (8 blocks a chunk) 166 / 183 (189 / 199), .125 (9) 187 / 195 (218 / 220), .15 (10) 210 / 211 (240 / 233),
+        .175 (11) 228 / 224 (262 / 244), .25 with batch 8 and 2048: 1175 / 1054 (1500 / 1045), .4 (20) 384 / 365 (434 / 373), .5 428 / 439
+        (498 / 448), .7 501 / 564 (582 / 587).  Groups of nine lines, density .4: 68 / 75."""
+        lay = (layout != 0).to(torch.uint8).cpu().contiguous()
+        H, R, C = lay.shape
+        n, groups, lib = ctypes.c_int64(0), ctypes.c_int(0), _lib.load()
+        L, K = (R, C) if rows else (C, R)
+        nnz = int(lay.sum())
+        if not always and (L * 8 < -(-L // 16) * 16 * 7 or nnz > .45 * H * R * C):
+            return None
+        cap = H * -(-L // 16) * (36 + 32 * -(-K // 4)) + 32 * (nnz // 9)      # a chunk has four reduction blocks, or nine blocks of the layout
+        host = torch.empty(cap, dtype=torch.int32)
+        _lib.check(lib.bsp_xsd_chunks_build(_lib.ptr(lay), H, R, C, int(rows), _lib.ptr(host), cap, ctypes.byref(groups), ctypes.byref(n)), 'bsp_xsd_chunks_build')
+        if not always and nnz < 11 * ((n.value - 4 * groups.value) // 32):
+            return None
+        out = GroupPlan(host[:n.value].to(device), groups.value, L)
+        out.flags = _lib.FLAG_PLAN_TILES
+        return out
 
     def max_entries(self):
         """The largest number of entries of any group of the plan (read back from the device once and kept)."""
@@ -555,7 +580,7 @@ class _sparse_matmul(torch.autograd.Function):
         # group): its plan has no chains and runs head by head; built when such a product first comes
         lut.gplan_wide = None
         if block == 32:
-            lut.build_wide = lambda: GroupPlan.build(layout, trans, dev, thin_min=0, order_buckets=1, ctx=ctx)
+            lut.build_wide = lambda: GroupPlan.build_xsd_chunks(layout, trans, dev) or GroupPlan.build(layout, trans, dev, thin_min=0, order_buckets=1, ctx=ctx)
         return lut, num_locks.value, width.value, None
 
     @staticmethod
@@ -576,7 +601,7 @@ class _sparse_matmul(torch.autograd.Function):
 
     @staticmethod
     def _plan_for(lut, block, free_dim, dtype, width, batch):
-        """The group plan that goes with a dsd / dds launch: the wide-free-dimension plan for blocks of 32 (16-bit types,
+        """The group plan that goes with a dsd / dds launch: the wide-free-dimension plan (chunks or groups) for blocks of 32 (16-bit types,
         256 dense rows or more, a launch of 384 workgroups or more of the wide kernel, which measures by the same rule),
         else the table's ordinary plan."""
         if (block == 32 and free_dim >= 256 and dtype != torch.float32
@@ -611,11 +636,12 @@ class _sparse_matmul(torch.autograd.Function):
         CS2, CS3 = (BS2, M) if trans_c else (M, BS2)
         c = torch.empty((a.size(0), a.size(1), CS2, CS3), dtype=a.dtype, device=a.device)
         b_sz = b.stride(0) if (b.dim() == 4 and b.size(0) > 1) else 0   # a 3-D (or batch-1) sparse operand is shared by the batch
+        plan = _sparse_matmul._plan_for(lut, block, M, a.dtype, width, a.size(0))
         timer = _Timer(bench, a.device)
         rc = _lib.OK if _sparse_matmul._in_parts(True, b, a, c, trans_a, trans_b, trans_c, a.size(0), M, b_sz, block, lut, width) else _lib.load().bsp_dds_matmul(_lib.DTYPES[a.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
                                         int(trans_c), a.size(0), M, a.stride(0), a.stride(1), a.stride(2), b_sz, c.stride(0),
                                         c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
-                                        *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, M, a.dtype, width, a.size(0)), M, a.size(0)), KERNEL_FLAGS,
+                                        *GroupPlan.xsd_args(plan, M, a.size(0)), KERNEL_FLAGS | (plan.flags if plan is not None else 0),
                                         _lib.stream_ptr(a.device))
         _lib.check(rc, 'bsp_dds_matmul')
         time[0] = timer.done()
@@ -636,11 +662,12 @@ class _sparse_matmul(torch.autograd.Function):
         CS2, CS3 = (N, AS1) if trans_c else (AS1, N)
         c = torch.empty((b.size(0), b.size(1), CS2, CS3), dtype=b.dtype, device=b.device)
         a_sz = a.stride(0) if (a.dim() == 4 and a.size(0) > 1) else 0
+        plan = _sparse_matmul._plan_for(lut, block, N, b.dtype, width, b.size(0))
         timer = _Timer(bench, b.device)
         rc = _lib.OK if _sparse_matmul._in_parts(False, a, b, c, trans_a, trans_b, trans_c, b.size(0), N, a_sz, block, lut, width) else _lib.load().bsp_dsd_matmul(_lib.DTYPES[b.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
                                         int(trans_c), b.size(0), N, a_sz, b.stride(0), b.stride(1), b.stride(2), c.stride(0),
                                         c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
-                                        *GroupPlan.xsd_args(_sparse_matmul._plan_for(lut, block, N, b.dtype, width, b.size(0)), N, b.size(0)), KERNEL_FLAGS,
+                                        *GroupPlan.xsd_args(plan, N, b.size(0)), KERNEL_FLAGS | (plan.flags if plan is not None else 0),
                                         _lib.stream_ptr(b.device))
         _lib.check(rc, 'bsp_dsd_matmul')
         time[0] = timer.done()
@@ -736,7 +763,7 @@ class _Product:
                                           lut.TILES_LAUNCH, lut.TILE_BLOCKS, levels)
         else:
             made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, lut.longest, lut.nnz, H, R, C,
-                                          plan(lut.gplan), plan(lut.gplan_wide),
+                                          plan(lut.gplan), plan(lut.gplan_wide), lut.gplan_wide.flags if lut.gplan_wide is not None else 0,
                                           2 if lut.gplan_wide is not None else int(getattr(lut, 'build_wide', None) is not None))
         self.native[which], self.built[which] = made, self._on_demand(which)
         return made

@@ -463,8 +463,9 @@ template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __global__ void __launch_bounds__(64 * SddShape<BLOCK>::WG * SddShape<BLOCK>::WG) k_sdd(SddArgs g) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int64_t n_wg = g.n_groups * g.Z;
-  const int64_t w = xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg);
-  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG, PARTS>(g, g.lut, g.valid, PARTS ? (int)(w / n_wg) : 0, (int)(w % n_wg / g.n_groups), w % g.n_groups, true, smem_raw);
+  const uint32_t w = (uint32_t)xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg), part = PARTS ? w / (uint32_t)n_wg : 0;
+  const Quotient z((PARTS ? w - part * (uint32_t)n_wg : w), (uint32_t)g.n_groups);
+  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG, PARTS>(g, g.lut, g.valid, (int)part, (int)z.q, z.r, true, smem_raw);
 }
 
 // The second pass of an sdd in parts: the parts of every block in order, rounded once
@@ -510,19 +511,19 @@ template <typename T, int BLOCK, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> lv, int64_t per_part) {
   typedef SddLevelsShape<T, BLOCK, A_KCONTIG, B_KCONTIG> S;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  const int part = PARTS ? (int)(blockIdx.x / per_part) : 0;
-  int64_t w = PARTS ? blockIdx.x % per_part : blockIdx.x, n = lv.n[0] * g.Z;
+  const int part = PARTS ? (int)(blockIdx.x / (uint32_t)per_part) : 0;
+  int64_t w = PARTS ? blockIdx.x % (uint32_t)per_part : blockIdx.x, n = lv.n[0] * g.Z;
   if (w < n) {
-    w = xcd_remap(w, n);
-    sdd_super_block<T, BLOCK, S::PACK0, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[0], lv.valid[0], part, (int)(w / lv.n[0]), w % lv.n[0], true, smem_raw);
+    const Quotient z((uint32_t)xcd_remap(w, n), (uint32_t)lv.n[0]);
+    sdd_super_block<T, BLOCK, S::PACK0, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[0], lv.valid[0], part, (int)z.q, z.r, true, smem_raw);
     return;
   }
   w -= n;
   if constexpr (BLOCK == 16) {
     n = lv.n[1] * g.Z;
     if (w < n) {
-      w = xcd_remap(w, n);
-      sdd_super_block<T, 16, 2, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[1], lv.valid[1], part, (int)(w / lv.n[1]), w % lv.n[1], true, smem_raw);
+      const Quotient z((uint32_t)xcd_remap(w, n), (uint32_t)lv.n[1]);
+      sdd_super_block<T, 16, 2, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[1], lv.valid[1], part, (int)z.q, z.r, true, smem_raw);
       return;
     }
     w -= n;
@@ -532,7 +533,8 @@ __global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> 
   w = xcd_remap(w, (last + PER - 1) / PER);
   const int own = PER == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t i = w * PER + own, j = i < last ? i : last - 1;
-  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[LAST], lv.valid[LAST], part, (int)(j / lv.n[LAST]), j % lv.n[LAST], i < last,
+  const Quotient z((uint32_t)j, (uint32_t)lv.n[LAST]);
+  sdd_super_block<T, BLOCK, 1, A_KCONTIG, B_KCONTIG, PARTS>(g, lv.lut[LAST], lv.valid[LAST], part, (int)z.q, z.r, i < last,
                                                             smem_raw + own * S::template G<1>::SMEM_BYTES);
 }
 
@@ -545,10 +547,11 @@ __global__ void __launch_bounds__(64 * SddShape<BLOCK / SPLIT>::WG * SddShape<BL
   typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int64_t n_wg = g.n_groups * g.Z * (SPLIT * SPLIT);
-  const int64_t w = xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg);
-  const int sub = (int)(w % (SPLIT * SPLIT)), part = PARTS ? (int)(w / n_wg) : 0;
-  const int z = (int)(w % n_wg / (SPLIT * SPLIT) / g.n_groups);
-  const int64_t grp = w / (SPLIT * SPLIT) % g.n_groups;
+  const uint32_t w = (uint32_t)xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg);
+  const int sub = (int)(w % (SPLIT * SPLIT)), part = PARTS ? (int)(w / (uint32_t)n_wg) : 0;
+  const Quotient batch((PARTS ? w - part * (uint32_t)n_wg : w) / (SPLIT * SPLIT), (uint32_t)g.n_groups);
+  const int z = (int)batch.q;
+  const int64_t grp = batch.r;
   const table_ptr e = as_table(g.lut) + grp * 4;
   if (g.valid && !g.valid[grp]) return;
   SddView<T, BLOCK, 1, A_KCONTIG> av;
@@ -662,26 +665,28 @@ template <int BLOCK, int TN_> struct XsdShape {
 // eighth of the launch, so inside its eighth the position in the order is the slow index and the tile the fast one.
 // One batch with a number of tiles that divides by 8: every XCD gets all segments for its own tiles; a batch that
 // divides by 8: every XCD gets whole batches.
-__device__ __forceinline__ void xsd_work_item(const XsdArgs &g, int n_tiles, int64_t wg, int &z, int &nt, int &seg0) {
-  const int64_t per_z = (int64_t)g.width * n_tiles, total = per_z * g.Z;
-  const int64_t w = xcd_remap(wg, total);
-  z = (int)(w / per_z);
-  nt = (int)((w % per_z) / g.width);
-  seg0 = (int)((w % per_z) % g.width);
-  if (g.order && total % 8 == 0) {
-    const int64_t chunk = total / 8, p = w % chunk;
-    const int x = (int)(w / chunk);
-    if (g.Z == 1 && n_tiles % 8 == 0) {
-      const int tpx = n_tiles / 8;
-      seg0 = (int)(p / tpx);
-      nt = x * tpx + (int)(p % tpx);
-    } else if (g.Z % 8 == 0) {
-      const int64_t q = p % per_z;
-      z = x * (g.Z / 8) + (int)(p / per_z);
-      seg0 = (int)(q / n_tiles);
-      nt = (int)(q % n_tiles);
+__device__ __forceinline__ void xsd_work_item(const XsdArgs &g, int n_tiles, uint32_t wg, int &z, int &nt, int &seg0) {
+  const uint32_t per_z = (uint32_t)g.width * n_tiles, total = per_z * (uint32_t)g.Z;   // (a launch has fewer than 2^31 workgroups)
+  const uint32_t w = (uint32_t)xcd_remap(wg, total);
+  if (g.order && total % 8 == 0 && ((g.Z == 1 && n_tiles % 8 == 0) || g.Z % 8 == 0)) {
+    const Quotient x(w, total / 8);
+    if (g.Z % 8) {
+      const Quotient s(x.r, (uint32_t)n_tiles / 8);
+      z = 0;
+      seg0 = (int)s.q;
+      nt = (int)(x.q * (n_tiles / 8) + s.r);
+    } else {
+      const Quotient b(x.r, per_z), s(b.r, (uint32_t)n_tiles);
+      z = (int)(x.q * (g.Z / 8) + b.q);
+      seg0 = (int)s.q;
+      nt = (int)s.r;
     }
+    return;
   }
+  const Quotient b(w, per_z), t(b.r, (uint32_t)g.width);
+  z = (int)b.q;
+  nt = (int)t.q;
+  seg0 = (int)t.r;
 }
 
 // (at least two wavefronts per SIMD: the 128 x 256 tile of block 128 would otherwise take 266 registers and run alone)
@@ -692,9 +697,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int n_tiles = (g.NF + S::TN - 1) / S::TN;
   const int64_t n_wg = (int64_t)g.width * n_tiles * g.Z;
-  const int part = PARTS ? (int)(blockIdx.x / n_wg) : 0;
+  const int part = PARTS ? (int)(blockIdx.x / (uint32_t)n_wg) : 0;
   int z, nt, seg0;
-  xsd_work_item(g, n_tiles, PARTS ? blockIdx.x % n_wg : blockIdx.x, z, nt, seg0);
+  xsd_work_item(g, n_tiles, PARTS ? blockIdx.x % (uint32_t)n_wg : blockIdx.x, z, nt, seg0);
   const int seg = g.order ? as_table(g.order)[seg0] : seg0;   // longest first only where the launch is short (see the dispatcher)
   const table_ptr hd = as_table(g.lut) + 6 * (int64_t)seg;
   const int offset = hd[0], seglen = hd[1], column = hd[2], depth = hd[3];

@@ -614,6 +614,11 @@ def other_config(config, steps, warmup):
             kernel = xsd_kernel_name(block, bits, N, ta, tb_, H * M // block, Z)
         else:                    # dds = dsd on the transposed problem
             kernel = xsd_kernel_name(block, bits, M, not tb_, not ta, H * N // block, Z)
+        lut = op.make_lut(dtype, dev)[0]          # (with the plans that the launches built)
+        if kernel == 'k_sdd_rg_dl' and lut.tiles_for(Z) is not None:
+            kernel = 'k_sdd_list_dl'
+        elif kernel == 'k_xsd_rg_dl' and lut.gplan_wide.flags:
+            kernel = 'k_xsd_list_dl'
         out.append({'launch': name, 'ms': round(ms, 4), 'TFLOP/s': round(fl / ms * 1e-9, 2), 'mfma_frac': round(fl / ms * 1e-9 / peak, 4),
                     'GB/s': round(nbytes / ms * 1e-6, 1), 'hbm_frac': round(nbytes / ms * 1e-6 / HBM_PEAK_GBS, 4),
                     'roofline': launch_roofline(kernel, fl, nbytes, ms, peak)})

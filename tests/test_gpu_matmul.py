@@ -226,8 +226,8 @@ def test_sparse_linear_layer_config_reduced():
 
 @pytest.mark.parametrize('tokens', [(5, 7), (3, 16)])
 def test_linear_module(tokens):
-    # y, dx and the weight gradient against dense fp32; 35 tokens are padded to a multiple of 16 inside the module (the
-    # weight gradient is an sdd product over the tokens), 48 are not
+    # y, dx and the weight gradient against dense fp32; 35 tokens are no multiple of 16 (the weight gradient is an sdd product
+    # over the tokens), 48 are
     torch.manual_seed(3)
     lay = random_layout((1, 4, 6), 0.5, 3)
     lin = tb.Linear(256, 384, 64, lay).to(DEV).half()

@@ -519,8 +519,8 @@ template <typename T> int launch_rg_dl(const XsdArgs &g, bool sp_trans, bool dn_
 // every SIMD has all the blocks of a chunk to multiply, however they fall.  The dense operands of a chunk stay in registers
 // for all of its lines; a block is 2 LDS reads and 2 matrix instructions behind a bit of the chunk's mask.  Two stages of 80 KiB: one
 // workgroup a compute unit, which stays for many tiles, so that the next chunk is in flight while this one is multiplied, also where it
-// is the first of the next tile, during this one's stores.  What bounds it now is LDS (192 KiB read and 64 written for a chunk of 16
-// blocks) and the stores, which wait together.
+// is the first of the next tile, during this one's stores.  What bounds it now is latency, of the chunk's loads, of the LDS reads
+// behind the branches and at the tile's end: matrix units busy 22 % of the cycles, LDS 20 %, a feed of 7.8 TB/s where 11.6 were reached.
 // 16 heads of 64 x 64 blocks, a quarter of them there, batch 8, free dimension 2048, fp16: 1175 -> 1054 us (519 TFLOP/s), with the dense
 // operand's reduction contiguous 1500 -> 1045.  A workgroup a tile with the whole tile staged in LDS at its end: 1277; the results
 // stored from registers: 1105.
@@ -989,8 +989,9 @@ template <typename T, int BLOCK> int launch_sdd_rg_dl(const SddArgs &g, bool a_k
 // lie in them (512 rows of B), and computes those blocks and no others: each wavefront eight of them, from a list, in registers over
 // the whole reduction.  What bounds k_sdd_rg_dl at these layouts is work and feed for absent blocks: it multiplies its whole 128 x 256
 // tile, of which a quarter to a third of the blocks exist.  Here a step's 64 KiB at most serve up to 64 blocks, all of them wanted, and
-// what bounds it is that feed and the LDS reads: a wavefront reads both fragments of every block (2 KiB a matrix instruction), so that
-// nothing in a step depends on the list but the addresses, which are computed once.  128 KiB of LDS: one workgroup a compute unit.
+// a wavefront reads both fragments of every block (2 KiB a matrix instruction), so that nothing in a step depends on the list but the
+// addresses, which are computed once.  128 KiB of LDS: one workgroup a compute unit.  What bounds it is the feed and the step's barrier:
+// 10 TB/s from L2, matrix units busy 32 % of the cycles, LDS 33 %.
 // 16 heads of 64 x 64 blocks, a quarter of them there, batch 8, reduction 2048, fp16: 1594 -> 1071 us (513 TFLOP/s), 1668 -> 965 with
 // A transposed.
 // Tiles (bsp_sdd_tiles_build), kTileInts ints each: head, first block-row, block-columns n, blocks m, the 16 block-columns (the last

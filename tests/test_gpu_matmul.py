@@ -3,6 +3,7 @@ import pytest
 import torch
 
 import torch_blocksparse as tb
+from torch_blocksparse import _lib, matmul
 from oracle import dense_oracle as D
 from helpers import assert_close, guard_allocations, operand_shapes, random_layout, run_matmul_case as run_case
 
@@ -449,3 +450,24 @@ def test_a_single_row_whose_stride_is_no_multiple_of_16_bytes():
     x = torch.randn(128, 1, device=DEV).t()
     assert x.stride() == (1, 1) and x.is_contiguous()
     assert torch.equal(lin(x), lin(x.clone(memory_format=torch.contiguous_format)))
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize('mode,trans', [('dsd', False), ('dsd', True), ('dds', False), ('dds', True)])
+@pytest.mark.parametrize('free', [136, 264, 392])
+def test_narrow_tiles_of_a_launch_that_does_not_fill_the_chip(mode, trans, free, dtype, monkeypatch):
+    # 16-bit, blocks of 32: below 512 workgroups the general kernel takes tiles of 128.  The same product in a batch that has more of
+    # them adds the same terms in the same order on tiles of 256, so the results are equal.
+    monkeypatch.setattr(matmul, 'KERNEL_FLAGS', _lib.FLAG_NO_WIDE)
+    lay = random_layout((2, 5, 9), 0.5, 3)
+    torch.manual_seed(free)
+    Z = 128                                               # 10 lines or more, at least 1280 workgroups
+    sp = torch.randn(1, int(lay.sum()), 32, 32, device=DEV).to(dtype).expand(Z, -1, -1, -1).contiguous()
+    red = 32 * (lay.shape[1] if (mode == 'dsd') == trans else lay.shape[2])
+    dn = torch.randn((1, 2) + ((red, free) if mode == 'dsd' else (free, red)), device=DEV).to(dtype).expand(Z, -1, -1, -1).contiguous()
+    op = tb.MatMul(lay, 32, mode, trans_a=trans) if mode == 'dsd' else tb.MatMul(lay, 32, mode, trans_b=trans)
+    args = lambda z: (sp[:z], dn[:z]) if mode == 'dsd' else (dn[:z], sp[:z])
+    with guard_allocations('narrow tiles'):
+        one = op(*args(1))
+        many = op(*args(Z))
+    assert torch.equal(many, one.expand_as(many)) and bool(torch.isfinite(one).all())

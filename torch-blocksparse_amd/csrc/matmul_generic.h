@@ -913,7 +913,11 @@ template <typename T, int BLOCK, int TN_> int launch_xsd_bw(const XsdArgs &g0, b
 }
 
 template <typename T, int BLOCK> int launch_xsd_b(const XsdArgs &g, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
-  const int tile = xsd_tile(BLOCK, g.NF);
+  int tile = xsd_tile(BLOCK, g.NF);
+  // 16-bit, blocks of 32: a launch on tiles of 256 has two workgroups a compute unit from 512 on; fewer leave the chip waiting for the few
+  // steps in flight, and tiles of 128 are twice as many.  Tiles of 256 / 128, us, of the launches on 256: 128 of them 20.7 / 16.3 (31 blocks
+  // a line) and 7.9 / 6.3 (8), 256 20.1 / 17.2, 384 25.7 / 23.4; 512 10.6 / 10.9, 14.3 / 14.3, 17.6 / 20.3; 768 18.2 / 19.1, 25.2 / 27.6.
+  if (sizeof(T) == 2 && BLOCK == 32 && tile == 256 && (int64_t)g.width * ((g.NF + 255) / 256) * g.Z < 512) tile = 128;
   if constexpr (BLOCK == 32 || BLOCK == 128)
     if (tile == 256) return launch_xsd_bw<T, BLOCK, 256>(g, sp_trans, dn_kc, out_nc, st);
   if constexpr (BLOCK != 16)

@@ -197,7 +197,8 @@ int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, void *c, int 
                           int parts, int64_t n_blocks, void *d_ws, int64_t ws_bytes, int flags, void *stream);
 /* parts > 1: the reduction is cut into that many parts, which run side by side on the general kernels and leave fp32 blocks in d_ws
  * (bsp_sdd_parts_workspace_bytes(block, n_blocks, Z, parts) bytes, 16-byte aligned, no initialisation needed; n_blocks: blocks of the
- * layout); a second launch adds them in order.  bsp_sdd_parts says how many parts suit a product (1: leave it whole). */
+ * layout); a second launch adds them in order.  Calls that overlap (on several streams, or made by several threads) need a d_ws each;
+ * that holds for every entry point here that takes one.  bsp_sdd_parts says how many parts suit a product (1: leave it whole). */
 int bsp_sdd_parts(int dtype, int block, int n_levels, const int *packs, const int64_t *n_groups, int Z, int K, int flags);
 int64_t bsp_sdd_parts_workspace_bytes(int block, int64_t n_blocks, int Z, int parts);
 

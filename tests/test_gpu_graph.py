@@ -159,7 +159,7 @@ def test_split_chains_captured_then_a_larger_eager_call_between_replays():
 
 def test_sparse_linear_layer_captured_and_replayed():
     # A block-128 sparse linear layer, forward and backward: the wide dds kernels and the weight gradient as an sdd
-    # in parts (fp32 partial blocks in a workspace of the operator, allocated by the warm-up step).  Replays must equal
+    # in parts (fp32 partial blocks in memory of the call's own, here the graph's).  Replays must equal
     # the eager run bit for bit, with eager work and a larger eager call in between.
     torch.manual_seed(21)
     block, tokens, feat = 128, 1024, 512

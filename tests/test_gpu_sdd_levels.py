@@ -2,6 +2,7 @@
 last level whose super-blocks do not fill its workgroups, reductions around the depth of the register ring, every
 orientation; and the C entry point against one call per level, bit for bit."""
 import ctypes
+import threading
 
 import pytest
 import torch
@@ -118,3 +119,48 @@ def test_parts_give_the_same_bits_every_time_and_refuse_a_small_workspace():
         assert rc == _lib.OK and torch.equal(c, again) and float((c - one).abs().max()) <= float(bound)
     assert run(4, 1024)[0] == _lib.ERR_CAPACITY
     assert run(126)[0] < 0 and run(125)[0] == _lib.OK                                 # (125 steps: 126 parts would leave one empty)
+
+
+@pytest.mark.parametrize('block,dtype', [(32, torch.float32), (64, torch.float16), (128, torch.float16)])
+@pytest.mark.parametrize('threads', [False, True])
+def test_one_operator_on_two_streams_and_in_two_threads(block, dtype, threads):
+    # products in parts, with nothing between the streams (threads: two of them on one stream): the bits of one call after the other
+    lay = torch.zeros(1, 4, 4, dtype=torch.int64)
+    lay[0, :2, :2] = lay[0, 3, 1:] = 1
+    K, reps = 4096, 40
+    torch.manual_seed(block)
+    op = tb.MatMul(lay, block, 'sdd', trans_a=True)
+    sets = [[torch.randn(1, 1, K, 4 * block, device=DEV).to(dtype) for _ in range(2)] for _ in range(2)]
+    want = [op(*s) for s in sets]
+    assert not torch.equal(*want)
+    torch.cuda.synchronize()
+    got = [[], []]
+    if threads:
+        def work(i):
+            got[i] = [op(*sets[i]) for _ in range(reps)]
+        both = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in both:
+            t.start()
+        for t in both:
+            t.join()
+    else:
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        for _ in range(reps):
+            for i in range(2):
+                with torch.cuda.stream(streams[i]):
+                    got[i].append(op(*sets[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == reps and all(torch.equal(c, want[i]) for c in got[i])
+
+
+def test_a_longer_reduction_leaves_no_memory_behind():
+    lin = tb.Linear(1280, 1280, 64, torch.ones(1, 20, 20, dtype=torch.int64)).to(DEV)
+    held = []
+    for tokens in (768, 1536, 6144, 24576):
+        x = torch.randn(tokens, 1280, device=DEV, requires_grad=True)
+        dw = torch.autograd.grad(lin(x), lin.weight, torch.ones(tokens, 1280, device=DEV))[0]
+        del x, dw
+        torch.cuda.synchronize()
+        held.append(torch.cuda.memory_allocated())
+    assert held == held[:1] * len(held)

@@ -1,0 +1,107 @@
+"""The host side of the launches without a GPU: what a call allocates, keeps and passes on.  Tensors are stand-ins, and every call of
+the library below is one that it refuses, or that a stand-in takes, before anything is launched."""
+import ctypes
+import threading
+import types
+
+import pytest
+import torch
+
+from torch_blocksparse import _lib, matmul
+from torch_blocksparse.matmul import SddTables, _sparse_matmul
+
+
+class FakeTensor:
+    """what csrc/launch.cpp asks of a tensor"""
+
+    def __init__(self, shape, dtype, ptr=1 << 20, device='cuda:0'):
+        self.shape, self.dtype, self.device, self._ptr = tuple(shape), dtype, device, ptr
+
+    def get_device(self):
+        return 0
+
+    def stride(self):
+        out = [1]
+        for n in self.shape[:0:-1]:
+            out.insert(0, out[0] * n)
+        return tuple(out)
+
+    def data_ptr(self):
+        return self._ptr
+
+
+@pytest.fixture
+def launcher():
+    """csrc/launch.cpp on stand-ins: the module, what it allocated, and the statuses of the library that it raised"""
+    module, made, raised = _lib.native(), [], []
+
+    def empty(shape, dtype, device):
+        # (memory for parts at an odd address: the library refuses such a call before it launches anything)
+        made.append((shape, dtype))
+        return FakeTensor(shape, dtype, 1 << 20 | (8 if dtype == 'uint8' else 0))
+
+    def check(code, what):
+        raised.append((what, code))
+        raise ValueError(what)
+
+    fake = types.SimpleNamespace(Tensor=FakeTensor, float16='float16', bfloat16='bfloat16', float32='float32', uint8='uint8', empty=empty)
+    module.setup(fake, check, lambda dev: 0, FakeTensor, _sparse_matmul)
+    yield types.SimpleNamespace(module=module, made=made, raised=raised)
+    _lib._native = None                                    # (the next caller sets it up again)
+
+
+def _sdd_tables(launch, block, dtype, n):
+    """tables of n single blocks, the first of 4 x 4"""
+    at = 1 << 21
+    return launch.make_sdd((None,), block, dtype, 0, n, 1, 4, 4, (0, 0, 0, 0), (0, 0, 0, 0), 0, 0, 0, 0, (0, 0, 0, 0), 0, 150, 22, ((1, at, 0, n),))
+
+
+@pytest.mark.parametrize('block,dtype,name', [(32, _lib.F32, 'float32'), (64, _lib.F16, 'float16'), (128, _lib.F16, 'float16')])
+def test_every_sdd_in_parts_has_memory_of_its_own(launcher, block, dtype, name):
+    lib, n, K = _lib.load(), 7, 4096
+    tables = _sdd_tables(launcher.module, block, dtype, n)
+    a = FakeTensor((1, 1, K, 4 * block), name)
+    if block == 128:
+        need = lib.bsp_sdd_splitk_workspace_bytes(1, n, 16)
+    else:
+        parts = lib.bsp_sdd_parts(dtype, block, 1, (ctypes.c_int * 1)(1), (ctypes.c_int64 * 1)(n), 1, K, 0)
+        assert parts > 1
+        need = lib.bsp_sdd_parts_workspace_bytes(block, n, 1, parts)
+    assert need > 0
+    for call in range(2):
+        with pytest.raises(ValueError):
+            launcher.module.sdd(tables, a, a, True, False, False, 0)
+    assert launcher.made == [((1, n, block, block), name), ((need,), 'uint8')] * 2
+    assert [code for _, code in launcher.raised] == [-1, -1]
+
+
+@pytest.mark.parametrize('block,dtype', [(32, torch.float32), (128, torch.float16)])
+def test_calls_that_overlap_share_no_memory(block, dtype, monkeypatch):
+    # the general host side: a second thread's call while the first one is between its two launches
+    real, K, nnz = _lib.load(), 4096, 3
+    places, inner = [], []
+
+    def launch(*args):
+        ws, need = [(a.value, n) for a, n in zip(args, args[1:]) if hasattr(a, 'value') and a.value and isinstance(n, int) and n > 4096][-1]
+        places.append((ws, need))
+        if len(places) == 1:
+            t = threading.Thread(target=lambda: inner.append(product()))
+            t.start()
+            t.join(60)
+        return _lib.OK
+
+    class Library:
+        bsp_sdd_matmul_levels = bsp_sdd_matmul_splitk = staticmethod(launch)
+
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+    monkeypatch.setattr(_lib, 'load', lambda: Library())
+    monkeypatch.setattr(_lib, 'stream_ptr', lambda device: None)
+    tables = SddTables([torch.zeros(4 * nnz, dtype=torch.int32)])
+    tables.nnz, tables.spdims, tables.widths, tables.packs = nnz, (1, 4, 4), [nnz], [1]
+    a = torch.zeros(1, 1, K, 4 * block, dtype=dtype)
+    product = lambda: _sparse_matmul._sdd_matmul(a, a, True, False, False, (1, 4, 4), block, tables, None, None, None, False, [None])
+    product()
+    (one, need), (two, again) = places
+    assert inner and need == again and (one + need <= two or two + need <= one)

@@ -104,6 +104,11 @@ bool pointer(PyObject *t, void **out) {
   *out = PyLong_AsVoidPtr(p.o);
   return !PyErr_Occurred();
 }
+// memory for the fp32 parts of one call, which has it to itself until its launches are made (_scratch in matmul.py)
+bool scratch(int64_t n, PyObject *like, Ref &held, void **out) {
+  Py_XSETREF(held.o, empty_bytes(n, like));
+  return held.o && pointer(held.o, out);
+}
 bool stream_of(int dev, void **out) {
   Ref d(PyLong_FromLong(dev));
   Ref s(d.o ? PyObject_CallOneArg(g_raw_stream, d.o) : nullptr);
@@ -275,8 +280,8 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const int parts = bsp_xsd_parts(s->dtype, s->block, s->width, s->longest, s->nnz, (int)free_dim, (int)Z, flags, &part_blocks);
   if (parts > 1) {
     const int64_t need = bsp_xsd_parts_workspace_bytes(s->block, s->width, (int)free_dim, (int)Z, parts);
-    Ref ws(empty_bytes(need, dn.obj));
-    if (!ws.o || !pointer(ws.o, &wsp)) return nullptr;
+    Ref ws;
+    if (!scratch(need, dn.obj, ws, &wsp)) return nullptr;
     const int rc = unlocked([&] {
       return bsp_xsd_matmul_parts(dds, s->dtype, sp.data(), dn.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, sp_sz, dn.stride[0], dn.stride[1], dn.stride[2], c_sz, c_sh, ldc,
                                   s->block, s->lut, s->plan, s->width, parts, part_blocks, wsp, need, st);
@@ -288,13 +293,6 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
                      : bsp_dsd_matmul(s->dtype, sp.data(), dn.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, sp_sz, dn.stride[0], dn.stride[1], dn.stride[2], c_sz, c_sh, ldc,
                                       s->block, s->lut, s->plan, s->width, plan.table, plan.n_groups, plan.lines, plan.n_split, wsp, ws_bytes, flags, st); });
   return checked(rc, dds ? "bsp_dds_matmul" : "bsp_dsd_matmul") ? c.release() : nullptr;
-}
-
-// the workspace that is kept with the tables, `need` bytes of it; nullptr with the error set
-void *splitk_workspace(const Sdd *s, int64_t need, const Operand &like) {
-  Ref dev(PyObject_GetAttr(like.obj, s_device));
-  Ref at(dev.o ? PyObject_CallMethod(PyTuple_GET_ITEM(s->keep, 0), "splitk_workspace", "LO", (long long)need, dev.o) : nullptr);
-  return at.o ? PyLong_AsVoidPtr(at.o) : nullptr;
 }
 
 // sdd(tables, a, b, trans_a, trans_b, trans_c, flags): bsp_sdd_matmul with the plan alone where a kernel takes it, else all pack levels
@@ -336,7 +334,7 @@ PyObject *sdd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
   }
   const int64_t shape[4] = {Z, s->nnz, s->block, s->block}, c_sz = s->nnz * s->block * s->block;
-  Ref c(empty_like_type(shape, 4, a));
+  Ref c(empty_like_type(shape, 4, a)), ws;
   void *cp, *wsp = nullptr, *st;
   if (!c.o || !pointer(c.o, &cp) || !stream_of(a.dev, &st)) return nullptr;
 #define BSP_OPERANDS s->dtype, a.data(), b.data(), cp, ta, tb, (int)Z, (int)K, a.stride[0], a.stride[1], a.stride[2], b.stride[0], b.stride[1], b.stride[2], c_sz, s->block
@@ -356,14 +354,14 @@ PyObject *sdd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (s->n_levels < 0) Py_RETURN_NONE;                  // (nothing was launched)
   if (parts) {
     const int64_t need = bsp_sdd_splitk_workspace_bytes((int)Z, s->widths[0], parts);
-    if (need && !(wsp = splitk_workspace(s, need, a))) return nullptr;
+    if (need && !scratch(need, a.obj, ws, &wsp)) return nullptr;
     rc = unlocked([&] { return bsp_sdd_matmul_splitk(BSP_OPERANDS, s->luts[0], s->valids[0], s->widths[0], parts, wsp, need, flags, st); });
     if (rc != BSP_ERR_UNSUPPORTED) return checked(rc, "bsp_sdd_matmul_splitk") ? c.release() : nullptr;
   }
   if (s->n_levels == 0) return c.release();
   parts = bsp_sdd_parts(s->dtype, s->block, s->n_levels, s->packs, s->widths, (int)Z, (int)K, flags);
   const int64_t need = bsp_sdd_parts_workspace_bytes(s->block, s->nnz, (int)Z, parts);
-  if (need && !(wsp = splitk_workspace(s, need, a))) return nullptr;
+  if (need && !scratch(need, a.obj, ws, &wsp)) return nullptr;
   rc = unlocked([&] {
     return bsp_sdd_matmul_levels(BSP_OPERANDS, s->n_levels, s->packs, s->luts, s->valids, s->widths, s->ordinary.table, s->ordinary.n_groups, s->ordinary.lines, parts, s->nnz,
                                  wsp, need, flags, st);

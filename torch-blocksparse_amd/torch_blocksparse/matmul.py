@@ -70,6 +70,12 @@ def _prep(x):
     return x if ok(x) else x.clone(memory_format=torch.contiguous_format)
 
 
+def _scratch(nbytes, device):
+    """Memory for the fp32 parts of one call, None where it has none.  Every call has its own: one operator may run on several streams and
+    threads at once, and the parts lie there between the product's two launches."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+
+
 class _Timer:
     """Event timing of one launch when bench=True (milliseconds); the reference stores the JIT's own timing."""
 
@@ -321,7 +327,6 @@ class SddTables(list):
 
     tiles = None          # block 32: the tiles of bsp_sdd_tiles_build, built by build_tiles on demand
     build_tiles = None
-    _splitk_ws = None
 
     # Long reductions at block 32 run from the tiles (k_sdd_list_dl) rather than from the groups of block-rows (k_sdd_rg_dl) where a launch
     # has TILES_LAUNCH tiles, they hold TILE_BLOCKS blocks on average and the layout at most TILES_DENSITY of its blocks.  Measured on
@@ -342,16 +347,6 @@ class SddTables(list):
             self.tiles = self.build_tiles()
         t = self.tiles
         return t if t is not None and t.n_groups * Z >= self.TILES_LAUNCH and self.nnz >= self.TILE_BLOCKS * t.n_groups else None
-
-    def splitk_workspace(self, need, device):
-        """address of a workspace of `need` bytes for the sdd in parts: it only grows, and one that a larger launch supersedes stays
-        allocated, because a captured graph may still use it"""
-        ws = self._splitk_ws
-        if ws is None or ws.numel() < need:
-            if ws is not None:
-                self._splitk_retired = getattr(self, '_splitk_retired', []) + [ws]
-            ws = self._splitk_ws = torch.empty(need, dtype=torch.uint8, device=device)
-        return ws.data_ptr()
 
     def materialize(self):
         if self.build is not None:
@@ -503,10 +498,11 @@ class _sparse_matmul(torch.autograd.Function):
                 c_packs, c_widths = (ctypes.c_int * n)(*packs), (ctypes.c_int64 * n)(*widths)
                 parts = lib.bsp_sdd_parts(operands[0], block, n, c_packs, c_widths, AS0, AS3, flags) if lazy else 1
                 need = lib.bsp_sdd_parts_workspace_bytes(block, total_width, AS0, parts)
+                ws = _scratch(need, a.device)
                 rc = lib.bsp_sdd_matmul_levels(*operands, n, c_packs, (ctypes.c_void_p * n)(*[t.data_ptr() for t in luts]),
                                                (ctypes.c_void_p * n)(*[t.valid.data_ptr() if getattr(t, 'valid', None) is not None else None for t in luts]),
                                                c_widths, gplan[0], gplan[1], gplan[2], parts, total_width,
-                                               ctypes.c_void_p(luts.splitk_workspace(need, a.device) if need else 0), need, flags, _lib.stream_ptr(a.device))
+                                               _lib.ptr(ws), need, flags, _lib.stream_ptr(a.device))
                 if rc != _lib.OK_WHOLE_LAYOUT:
                     _lib.check(rc, 'bsp_sdd_matmul_levels')
         time[0] = timer.done()
@@ -527,11 +523,10 @@ class _sparse_matmul(torch.autograd.Function):
             return False
         parts = max(1, min(_sparse_matmul.SPLITK_TARGET_WORKGROUPS // (n * Z), K // 256, 16))
         need = lib.bsp_sdd_splitk_workspace_bytes(Z, n, parts)
-        ws = luts.splitk_workspace(need, a.device) if need else 0
+        ws = _scratch(need, a.device)
         lut = luts[0]
         rc = lib.bsp_sdd_matmul_splitk(*operands, _lib.ptr(lut), _lib.ptr(getattr(lut, 'valid', None)), n, parts,
-                                       ctypes.c_void_p(ws), need, KERNEL_FLAGS,
-                                       _lib.stream_ptr(a.device))
+                                       _lib.ptr(ws), need, KERNEL_FLAGS, _lib.stream_ptr(a.device))
         if rc == _lib.ERR_UNSUPPORTED:
             return False
         _lib.check(rc, 'bsp_sdd_matmul_splitk')
@@ -592,7 +587,7 @@ class _sparse_matmul(torch.autograd.Function):
         if parts <= 1:
             return False
         need = lib.bsp_xsd_parts_workspace_bytes(block, width, free_dim, Z, parts)
-        ws = torch.empty(need, dtype=torch.uint8, device=dn.device)
+        ws = _scratch(need, dn.device)
         rc = lib.bsp_xsd_matmul_parts(int(is_dds), dtype, _lib.ptr(sp), _lib.ptr(dn), _lib.ptr(c), int(trans_a), int(trans_b), int(trans_c), Z, free_dim, sp_sz,
                                       dn.stride(0), dn.stride(1), dn.stride(2), c.stride(0), c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf),
                                       width, parts, part_blocks.value, _lib.ptr(ws), need, _lib.stream_ptr(dn.device))

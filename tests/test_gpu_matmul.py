@@ -1,4 +1,6 @@
 """GPU: block-sparse matmul sdd / dsd / dds, forward and backward, against the fp32 dense-masked oracle."""
+import copy
+
 import pytest
 import torch
 
@@ -434,6 +436,25 @@ def test_linear_with_a_number_of_tokens_that_divides_by_nothing(block, dtype, to
     close(x.grad, dyd, w.t(), 'dx')
     blocks = lambda t: D.dense_to_sparse(t[None, None], lay, block)[0]
     assert_close(lin.weight.grad, blocks((xd.t() @ dyd).float()), dtype, 'dw', mag=blocks((xd.t().abs() @ dyd.abs()).float()) if dtype == torch.float32 else None)
+
+
+@pytest.mark.parametrize('ahead', ['tables', 'product'])
+def test_linear_whose_tables_were_built_before_its_first_call(ahead):
+    lay = random_layout((1, 4, 5), 0.5, 3)
+    lin = tb.Linear(128, 160, 32, lay).to(DEV).half()
+    if ahead == 'tables':
+        lin.matmul.make_lut(torch.float16, lin.weight.device)
+    else:
+        x = torch.randn(1, 1, 64, 128, device=DEV, dtype=torch.float16, requires_grad=True)
+        lin.matmul(x, lin.weight).sum().backward()
+        lin.weight.grad = None
+    x = torch.randn(999, 128, device=DEV, dtype=torch.float16)
+    lin(x).backward(torch.ones(999, 160, device=DEV, dtype=torch.float16))
+    other = copy.deepcopy(lin)
+    other.matmul.lut_cache.clear()
+    other.weight.grad = None
+    other(x).backward(torch.ones(999, 160, device=DEV, dtype=torch.float16))
+    assert torch.equal(lin.weight.grad, other.weight.grad)
 
 
 def test_a_reduction_that_is_no_multiple_of_16_stays_refused_elsewhere():

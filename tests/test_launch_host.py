@@ -105,3 +105,23 @@ def test_calls_that_overlap_share_no_memory(block, dtype, monkeypatch):
     product()
     (one, need), (two, again) = places
     assert inner and need == again and (one + need <= two or two + need <= one)
+
+
+def test_a_linear_layer_takes_any_number_of_tokens_whenever_its_tables_were_built(monkeypatch):
+    # made ahead (make_lut), or by a call of the product itself, which reduces over multiples of 16 only
+    lin = matmul.Linear(64, 96, 32, torch.ones(1, 2, 3, dtype=torch.int64))
+    key = (torch.float32, torch.device('cpu'))
+    tables = SddTables()
+    lin.matmul.lut_cache[key] = (None,) * 8 + (tables, None, None, None)
+    first = lin.matmul._product(*key)
+    assert lin.matmul._product(*key) is first and not tables.any_k
+    seen = []
+
+    def call(op, a, b):
+        product = op._product(*key)
+        seen.append((product.luts[8].any_k, op._product(*key) is product))
+        return a.new_zeros(1, 1, a.size(2), 96)
+
+    monkeypatch.setattr(matmul.MatMul, '__call__', call)
+    lin(torch.zeros(7, 64))
+    assert seen == [(True, True)]

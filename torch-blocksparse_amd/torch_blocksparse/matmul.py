@@ -708,6 +708,9 @@ class _Product:
         self.luts, self.bench, self.dtype, self.device = luts, op.bench, _lib.DTYPES.get(dtype, -1), device
         self.trans_a, self.trans_b, self.spdims, self.block = op.trans_a, op.trans_b, op.spdims, op.block
         self.modes = (mode, mode[1] + mode[0] + mode[2], mode[2] + mode[1] + mode[0])      # c, da, db (matmul.py:593-601)
+        self.any_k = op.any_k
+        if self.any_k:                          # (the tables may have been built for other calls of the operator)
+            luts[4 * self.modes.index('sdd')].any_k = True
         self.native = [None, None, None]
         self.built = [None, None, None]         # which of the tables made on demand were there
 
@@ -779,12 +782,7 @@ class MatMul:
         layout, block = self.layout, self.block
         step = 8 if dtype == torch.float32 else 16             # matmul.py:617
         ctx = _LayoutOnDevice(layout, device)                  # one upload of the layout and one workspace for all tables
-
-        def sdd():
-            made = _sparse_matmul.make_sdd_lut(layout, block, dtype, device, ctx=ctx, lazy=True)
-            made[0].any_k = self.any_k
-            return made
-
+        sdd = lambda: _sparse_matmul.make_sdd_lut(layout, block, dtype, device, ctx=ctx, lazy=True)
         dxx = lambda trans: _sparse_matmul.make_dxx_lut(layout, block, step, trans, device, ctx=ctx)
         if self.mode == 'sdd':                                 # matmul.py:618-637
             c, da, db = sdd(), dxx(True), dxx(False)
@@ -798,7 +796,7 @@ class MatMul:
     def _product(self, dtype, device):
         luts = self.make_lut(dtype, device)
         product = self._products.get((dtype, device))
-        if product is None or product.luts is not luts or product.bench != self.bench:
+        if product is None or product.luts is not luts or product.bench != self.bench or product.any_k != self.any_k:
             product = self._products[(dtype, device)] = _Product(self, luts, dtype, device)
         return product
 

@@ -200,6 +200,9 @@ int bsp_sdd_matmul_levels(int dtype, const void *a, const void *b, void *c, int 
  * layout); a second launch adds them in order.  Calls that overlap (on several streams, or made by several threads) need a d_ws each;
  * that holds for every entry point here that takes one.  bsp_sdd_parts says how many parts suit a product (1: leave it whole). */
 int bsp_sdd_parts(int dtype, int block, int n_levels, const int *packs, const int64_t *n_groups, int Z, int K, int flags);
+/* Whether an sdd product over K rows (BSP_FLAG_ANY_K) into n_blocks blocks of a rows x cols matrix is better given copies of its operands
+ * with rows of zeros up to a multiple of 32, which the kernels for long reductions take (1), or taken as it is (0). */
+int bsp_sdd_whole_steps(int dtype, int block, int64_t n_blocks, int64_t rows, int64_t cols, int K);
 int64_t bsp_sdd_parts_workspace_bytes(int block, int64_t n_blocks, int Z, int parts);
 
 /* sparse = dense x dense over a long reduction into few blocks of 128, the reduction cut into `parts` parts that run side by

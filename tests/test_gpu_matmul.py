@@ -6,6 +6,7 @@ import torch
 
 import torch_blocksparse as tb
 from torch_blocksparse import _lib, matmul
+from torch_blocksparse.matmul import _sparse_matmul
 from oracle import dense_oracle as D
 from helpers import assert_close, guard_allocations, operand_shapes, random_layout, run_matmul_case as run_case
 
@@ -455,6 +456,54 @@ def test_linear_whose_tables_were_built_before_its_first_call(ahead):
     other.weight.grad = None
     other(x).backward(torch.ones(999, 160, device=DEV, dtype=torch.float16))
     assert torch.equal(lin.weight.grad, other.weight.grad)
+
+
+def _weight_gradient(lin, x, dy):
+    return torch.autograd.grad(lin(x), lin.weight, dy)[0]
+
+
+@pytest.mark.parametrize('block,R,C,tokens,copies', [(16, 64, 64, 2095, False), (16, 64, 64, 2101, True), (32, 64, 64, 1427, False), (32, 64, 64, 1433, True),
+                                                     (128, 3, 2, 2863, False)])
+def test_weight_gradient_over_a_ragged_reduction_on_both_sides_of_the_rule(block, R, C, tokens, copies, monkeypatch):
+    # with copies of whole steps and as it is
+    assert bool(_lib.load().bsp_sdd_whole_steps(_lib.F16, block, R * C, R * block, C * block, tokens)) == copies
+    torch.manual_seed(tokens)
+    lin = tb.Linear(R * block, C * block, block, torch.ones(1, R, C, dtype=torch.int64)).to(DEV).half()
+    x, dy = torch.randn(tokens, R * block, device=DEV).half(), torch.randn(tokens, C * block, device=DEV).half()
+    made = []
+    pad = _sparse_matmul._pad_free_dim
+    monkeypatch.setattr(_sparse_matmul, '_pad_free_dim', staticmethod(lambda t, dim, v: (v == 32 and made.append(t), pad(t, dim, v))[1]))
+    with guard_allocations('dw'):
+        got, again = _weight_gradient(lin, x, dy), _weight_gradient(lin, x, dy)
+    assert len(made) == (4 if copies else 0) and torch.equal(got, again)
+    blocks = lambda t: t.reshape(R, block, C, block).transpose(1, 2).reshape(R * C, block, block)
+    want, terms = blocks(x.double().t() @ dy.double()), blocks(x.double().abs().t() @ dy.double().abs())
+    # half a unit of the 16-bit result, and an fp32 sum of the terms
+    assert bool(((got.double() - want).abs() <= 2. ** -11 * want.abs() + tokens * 2. ** -24 * terms + 2. ** -24).all())
+
+
+def test_ragged_weight_gradient_under_capture_where_only_the_long_plan_is_built():
+    lin = tb.Linear(128, 128, 32, torch.ones(1, 4, 4, dtype=torch.int64)).to(DEV).half()
+    make = lambda tokens: (torch.randn(tokens, 128, device=DEV).half(), torch.randn(tokens, 128, device=DEV).half())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _weight_gradient(lin, *make(512))                 # whole steps: the table is not needed
+        x, dy = make(500)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    assert lin.matmul.make_lut(torch.float16, x.device)[8].build is not None
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = _weight_gradient(lin, x, dy)
+    for _ in range(3):
+        for t, fresh in zip((x, dy), make(500)):
+            t.copy_(fresh)
+        graph.replay()
+        want = _weight_gradient(lin, x, dy).double()
+        # another order of the fp32 sums: a unit of the 16-bit result, and two sums of the terms
+        bound = 2. ** -10 * want.abs() + 2 * 500 * 2. ** -24 * (x.double().abs().t() @ dy.double().abs()).max() + 2. ** -24
+        assert bool(((got.double() - want).abs() <= bound).all())
 
 
 def test_a_reduction_that_is_no_multiple_of_16_stays_refused_elsewhere():

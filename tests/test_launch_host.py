@@ -125,3 +125,12 @@ def test_a_linear_layer_takes_any_number_of_tokens_whenever_its_tables_were_buil
     monkeypatch.setattr(matmul.MatMul, '__call__', call)
     lin(torch.zeros(7, 64))
     assert seen == [(True, True)]
+
+
+def test_copies_of_ragged_operands_only_where_they_pay():
+    whole = _lib.load().bsp_sdd_whole_steps
+    for dtype, block, side, density, K, copies in (
+            (_lib.F16, 128, 4096, .5, 8176, 0), (_lib.BF16, 64, 4096, .5, 8176, 0), (_lib.F32, 32, 4096, .5, 8176, 0), (_lib.F16, 32, 4096, .5, 8192, 0),
+            (_lib.F16, 32, 4096, .1, 8176, 0), (_lib.F16, 32, 4096, .25, 8176, 1), (_lib.F16, 32, 4096, .25, 1040, 0), (_lib.F16, 32, 1024, .5, 8176, 0), (_lib.F16, 32, 2048, .5, 8176, 0),
+            (_lib.F16, 16, 4096, .1, 2032, 1), (_lib.F16, 16, 4096, .1, 1040, 0), (_lib.F16, 16, 1024, .5, 8176, 0), (_lib.F16, 16, 65536, .5, 255, 0)):
+        assert whole(dtype, block, int(density * (side // block) ** 2), side, side, K) == copies, (dtype, block, side, density, K)

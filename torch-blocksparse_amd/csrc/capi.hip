@@ -63,6 +63,22 @@ extern "C" int bsp_sdd_parts(int dtype, int block, int n_levels, const int *pack
   return (steps + per - 1) / per;                      // (no part is empty)
 }
 
+// Blocks of 16 and 32, 16-bit, a reduction that is no multiple of 32: as it is on the general kernel, or as copies with whole steps on
+// k_sdd_rg_dl.  The copies take 10 to 100 us, and that kernel is the faster one only with a large result (with a small one it has too few
+// workgroups for its long chains of steps), so they need many elements, many of them per row copied, and much work.  As it is / with
+// copies, us, fp16, the density and in brackets the rows of the reduction.
+// Block 32, 4096 x 4096: .1 257 / 281 (8170); .25 47 / 59 (1000), 103 / 89 (2041), 548 / 295 (8170); .5 41 / 46 (531), 80 / 60 (1000),
+// 963 / 309 (8170).  2048 x 2048: .5 91 / 127 (4090), 206 / 233 (8170).  1024 x 1024: .5 74 / 210 (8170).
+// Block 16, 4096 x 4096: .1 52 / 59 (1000), 133 / 89 (2041), 746 / 319 (8170); .25 29 / 33 (271), 56 / 46 (531); .5 54 / 35 (271).
+// 2048 x 2048: .25 66 / 74 (2041), 147 / 125 (4090), 352 / 231 (8170).  1024 x 1024: .5 126 / 206 (8170).
+// Block 128, whose kernel for whole steps is k_sdd128_splitk: as it is everywhere, 4096 x 4096, .1 8 / 34 (531), 75 / 158 (8170), .5
+// 23 / 39 (531), 224 / 294 (8170).
+extern "C" int bsp_sdd_whole_steps(int dtype, int block, int64_t n_blocks, int64_t rows, int64_t cols, int K) {
+  if (dtype == BSP_F32 || (block != 16 && block != 32) || K < 256 || K % 32 == 0 || n_blocks <= 0) return 0;
+  const int64_t elems = n_blocks * block * block, few = block == 16 ? 1000000 : 3000000, work = block == 16 ? 2200000000 : 6000000000;
+  return elems >= few && elems >= 8 * block * (rows + cols) && elems * K >= work;
+}
+
 extern "C" int64_t bsp_sdd_parts_workspace_bytes(int block, int64_t n_blocks, int Z, int parts) {
   return parts > 1 && n_blocks > 0 && Z > 0 ? (int64_t)parts * Z * n_blocks * block * block * (int64_t)sizeof(float) : 0;
 }

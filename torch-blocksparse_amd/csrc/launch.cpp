@@ -312,7 +312,7 @@ PyObject *sdd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (Z <= 0 || K <= 0 || K > INT32_MAX || b.size[0] != Z || a.size[1] != s->H || b.size[1] != s->H || b.size[tb ? 3 : 2] != K) Py_RETURN_NONE;
   if (a.size[ta ? 3 : 2] != s->block * s->R || b.size[tb ? 2 : 3] != s->block * s->C) Py_RETURN_NONE;
   const bool by_rows = s->any_k && ta && !tb;
-  if (by_rows && K % 32 && !f32 && (((s->block == 16 || s->block == 32) && K >= 256) || (s->block == 128 && K >= 512))) Py_RETURN_NONE;   // (padded to whole steps)
+  if (by_rows && s->long_state && bsp_sdd_whole_steps(s->dtype, s->block, s->nnz, s->block * s->R, s->block * s->C, (int)K)) Py_RETURN_NONE;   // (copied)
   const bool any_k = K % 16 != 0;
   if (any_k && !by_rows) Py_RETURN_NONE;
   if (any_k) flags |= BSP_FLAG_ANY_K;

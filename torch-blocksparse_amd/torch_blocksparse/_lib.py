@@ -61,6 +61,7 @@ SIGNATURES = {
     'bsp_sdd_tiles_build': (_i, [_vp, _i, _i, _i, _vp, _i64, _vp]),
     'bsp_xsd_chunks_build': (_i, [_vp, _i, _i, _i, _i, _vp, _i64, _vp, _vp]),
     'bsp_sdd_parts': (_i, [_i, _i, _i, _vp, _vp, _i, _i, _i]),
+    'bsp_sdd_whole_steps': (_i, [_i, _i, _i64, _i64, _i64, _i]),
     'bsp_sdd_parts_workspace_bytes': (_i64, [_i, _i64, _i, _i]),
     'bsp_sdd_splitk_workspace_bytes': (_i64, [_i, _i64, _i]),
     'bsp_sdd_matmul_splitk': (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i, _vp, _vp,

@@ -446,12 +446,14 @@ class _sparse_matmul(torch.autograd.Function):
             raise ValueError('incompatible operand shapes for sdd: %s and %s' % (tuple(a.shape), tuple(b.shape)))
         _check_dense('a', a, spdims[0], block * spdims[1], None, trans_a)
         _check_dense('b', b, spdims[0], None, block * spdims[2], trans_b)
-        if lazy and luts.any_k and trans_a and not trans_b and AS3 % 32 and a.dtype != torch.float32 and (
-                block in (16, 32) and AS3 >= 256 or block == 128 and AS3 >= 512):
-            # the kernels for a long reduction take whole steps of 32 rows
-            a, b = _sparse_matmul._pad_free_dim(a, 2, 32), _sparse_matmul._pad_free_dim(b, 2, 32)
-            AS3, any_k = a.size(2), False
         lib = _lib.load()
+        if lazy and luts.any_k and trans_a and not trans_b and AS3 % 32 and luts.build_long is not None:
+            whole_steps = lib.bsp_sdd_whole_steps(_lib.DTYPES[a.dtype], block, luts.nnz, block * spdims[1], block * spdims[2], AS3)
+            # (the table of the general kernel cannot be built under capture: the plan of the kernel for long reductions may be there)
+            if whole_steps or (luts.build is not None and luts.gplan_long is not None and a.dtype != torch.float32 and AS3 >= 256
+                               and torch.cuda.is_current_stream_capturing()):
+                a, b = _sparse_matmul._pad_free_dim(a, 2, 32), _sparse_matmul._pad_free_dim(b, 2, 32)
+                AS3, any_k = a.size(2), False
         total_width = luts.nnz if lazy else sum(w * p * p for w, p in zip(widths, packs))
         c = torch.empty((AS0, total_width, block, block), dtype=a.dtype, device=a.device)
         timer = _Timer(bench, a.device)

@@ -75,6 +75,18 @@ def test_every_sdd_in_parts_has_memory_of_its_own(launcher, block, dtype, name):
     assert [code for _, code in launcher.raised] == [-1, -1]
 
 
+@pytest.mark.parametrize('need', [(True, True, True), (True, False, False), (False, True, True)])
+def test_attention_backward_allocates_in_front_of_each_launch(launcher, need):
+    # delta and dq, then the row kernel (refused here: no lse), then dk, dv and the parts of long columns for the column kernel
+    H, L, D, lines = 2, 256, 64, 4
+    tables = launcher.module.make_attn((), 1 << 21, 1 << 21, 1 << 21, lines, 4, 8, 3, 1, 0, 4, H, 4, 4, 64)
+    t = FakeTensor((3, H, L, D), 'float16')
+    with pytest.raises(ValueError):
+        launcher.module.attn_bwd(tables, t, t, t, t, t, FakeTensor((3, H, 2, 64 * lines), 'float32', 0), 1., None, 0, 0, *need)
+    assert launcher.raised == [('bsp_attention_rows_bwd', -1)]
+    assert launcher.made == [((3, H, 2, 64 * lines), 'float32')] * need[1] + [((3, H, L, D), 'float16')]
+
+
 @pytest.mark.parametrize('block,dtype', [(32, torch.float32), (128, torch.float16)])
 def test_calls_that_overlap_share_no_memory(block, dtype, monkeypatch):
     # the general host side: a second thread's call while the first one is between its two launches

@@ -1,6 +1,9 @@
 """The host side of the launches without a GPU: what a call allocates, keeps and passes on.  Tensors are stand-ins, and every call of
 the library below is one that it refuses, or that a stand-in takes, before anything is launched."""
 import ctypes
+import os
+import subprocess
+import sys
 import threading
 import types
 
@@ -85,6 +88,45 @@ def test_attention_backward_allocates_in_front_of_each_launch(launcher, need):
         launcher.module.attn_bwd(tables, t, t, t, t, t, FakeTensor((3, H, 2, 64 * lines), 'float32', 0), 1., None, 0, 0, *need)
     assert launcher.raised == [('bsp_attention_rows_bwd', -1)]
     assert launcher.made == [((3, H, 2, 64 * lines), 'float32')] * need[1] + [((3, H, L, D), 'float16')]
+
+
+def _softmax_flags():
+    """flags that run Python code when they are asked (as the results of an overloaded comparison may): in a process of its own"""
+    asked = []
+
+    class Flag:
+        def __bool__(self):
+            asked.append(sys._getframe(1).f_code.co_name)
+            return True
+
+    class NoFlag:
+        def __bool__(self):
+            raise KeyError('no flag')
+
+    module, raised = _lib.native(), []
+    fake = types.SimpleNamespace(Tensor=FakeTensor, float16='float16', bfloat16='bfloat16', float32='float32')
+
+    def check(code, what):
+        raised.append(code)
+        raise ValueError(what)
+
+    module.setup(fake, check, lambda dev: 0, FakeTensor, _sparse_matmul)
+    rows = module.make_rows((), 0, 2, 0, 4, 1, 2, 2, 32)          # (no table: the library refuses the call)
+    x = FakeTensor((1, 4, 32, 32), 'float16')
+    for flags, error in (((Flag(), Flag()), ValueError), ((True, False), ValueError), ((NoFlag(), True), KeyError)):
+        try:
+            module.softmax_fwd(rows, x, 1., None, None, None, *flags)
+        except error:
+            continue
+        raise AssertionError(flags)
+    assert asked == ['_softmax_flags'] * 2 and raised == [-1, -1]
+
+
+def test_the_softmax_reads_its_flags_with_the_lock_held():
+    here = os.path.dirname(os.path.abspath(__file__))
+    done = subprocess.run([sys.executable, '-c', 'import test_launch_host as t; t._softmax_flags()'], cwd=here, env=dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path)),
+                          capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, (done.returncode, done.stderr[-2000:])
 
 
 @pytest.mark.parametrize('block,dtype', [(32, torch.float32), (128, torch.float16)])

@@ -124,7 +124,7 @@ bool checked(int rc, const char *what) {                // true, or false with t
   return false;
 }
 
-// An entry point without the interpreter's lock: a launch waits where the queue is full
+// An entry point without the interpreter's lock: a launch waits where the queue is full.  (f touches no Python object.)
 template <class F> int unlocked(F &&f) {
   PyThreadState *t = PyEval_SaveThread();
   const int rc = f();
@@ -409,11 +409,15 @@ PyObject *softmax_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
       r[0] = rpe.t.size[0] == 1 ? 0 : rpe.t.stride[0];
     }
   }
+  const int kpm_mul = truth(args[6]), att_mul = truth(args[7]);
+  const int64_t kpm_sz = kpm.given && kpm.t.size[0] > 1 ? kpm.t.stride[0] : 0, att_ld = att.given ? att.t.stride[0] : 0;
   void *st;
-  if (!stream_of(x.dev, &st)) return nullptr;
-  const int rc = unlocked([&] { return bsp_softmax_fwd(x.dtype, x.data(), (float)scale, s->lut, s->maxlut, rpe.given ? rpe.t.data() : nullptr, r[0], r[1], r[2], kpm.given ? kpm.t.data() : nullptr,
-                                 kpm.given && kpm.t.size[0] > 1 ? kpm.t.stride[0] : 0, truth(args[6]), att.given ? att.t.data() : nullptr, att.given ? att.t.stride[0] : 0,
-                                 truth(args[7]), (int)Z, (int)s->H, (int)s->R, (int)s->block, s->nnz * s->block * s->block, st); });
+  if (PyErr_Occurred() || !stream_of(x.dev, &st)) return nullptr;
+  const int rc = unlocked([&] {
+    return bsp_softmax_fwd(x.dtype, x.data(), (float)scale, s->lut, s->maxlut, rpe.given ? rpe.t.data() : nullptr, r[0], r[1], r[2],
+                           kpm.given ? kpm.t.data() : nullptr, kpm_sz, kpm_mul, att.given ? att.t.data() : nullptr, att_ld, att_mul,
+                           (int)Z, (int)s->H, (int)s->R, (int)s->block, s->nnz * s->block * s->block, st);
+  });
   if (!checked(rc, "bsp_softmax_fwd")) return nullptr;
   Py_RETURN_TRUE;
 }

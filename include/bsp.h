@@ -27,7 +27,7 @@ typedef enum {
   BSP_OK_WHOLE_LAYOUT = 1,   /* bsp_sdd_matmul only: the group plan was used, every block of the layout is written */
   BSP_NEEDS_TABLE = 2,       /* bsp_sdd_matmul called with the plan alone: nothing launched, call again with the sdd table */
   BSP_ERR_ARG = -1,          /* null pointer, bad size, misaligned operand */
-  BSP_ERR_UNSUPPORTED = -2,  /* block size / dtype / mode not built */
+  BSP_ERR_UNSUPPORTED = -2,  /* block size / dtype / mode not built; a builder that runs on the host: not enough memory for its lists */
   BSP_ERR_CAPACITY = -3,     /* caller-provided table or workspace too small */
   BSP_ERR_EMPTY_HEAD = -4,   /* a head of the layout has no nonzero block (the reference raises here) */
   BSP_ERR_HIP = -5,          /* a HIP runtime call failed */

@@ -2,6 +2,7 @@
 the library below is one that it refuses, or that a stand-in takes, before anything is launched."""
 import ctypes
 import os
+import resource
 import subprocess
 import sys
 import threading
@@ -122,11 +123,16 @@ def _softmax_flags():
     assert asked == ['_softmax_flags'] * 2 and raised == [-1, -1]
 
 
-def test_the_softmax_reads_its_flags_with_the_lock_held():
+def _alone(name):
+    """a function of this file in a process of its own, which it may end"""
     here = os.path.dirname(os.path.abspath(__file__))
-    done = subprocess.run([sys.executable, '-c', 'import test_launch_host as t; t._softmax_flags()'], cwd=here, env=dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path)),
+    done = subprocess.run([sys.executable, '-c', 'import test_launch_host as t; t.%s()' % name], cwd=here, env=dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path)),
                           capture_output=True, text=True, timeout=300)
     assert done.returncode == 0, (done.returncode, done.stderr[-2000:])
+
+
+def test_the_softmax_reads_its_flags_with_the_lock_held():
+    _alone('_softmax_flags')
 
 
 @pytest.mark.parametrize('block,dtype', [(32, torch.float32), (128, torch.float16)])
@@ -188,3 +194,22 @@ def test_copies_of_ragged_operands_only_where_they_pay():
             (_lib.F16, 32, 4096, .1, 8176, 0), (_lib.F16, 32, 4096, .25, 8176, 1), (_lib.F16, 32, 4096, .25, 1040, 0), (_lib.F16, 32, 1024, .5, 8176, 0), (_lib.F16, 32, 2048, .5, 8176, 0),
             (_lib.F16, 16, 4096, .1, 2032, 1), (_lib.F16, 16, 4096, .1, 1040, 0), (_lib.F16, 16, 1024, .5, 8176, 0), (_lib.F16, 16, 65536, .5, 255, 0)):
         assert whole(dtype, block, int(density * (side // block) ** 2), side, side, K) == copies, (dtype, block, side, density, K)
+
+
+def _builders_without_memory():
+    """the builders of tables on the host with no memory left for their lists: in a process of its own"""
+    lib = _lib.load()
+    wide = ctypes.create_string_buffer(1 << 24)            # 16 Mi cells of a layout, none there
+    out, n, m, info = (ctypes.c_int32 * 1024)(), ctypes.c_int64(0), ctypes.c_int(0), _lib.AttentionTables()
+    with open('/proc/self/statm') as f:
+        used = int(f.read().split()[0]) * resource.getpagesize()
+    resource.setrlimit(resource.RLIMIT_AS, (used + (24 << 20),) * 2)
+    assert lib.bsp_sdd_tiles_build(wide, 1, 1 << 24, 1, out, 1024, ctypes.byref(n)) == _lib.ERR_UNSUPPORTED
+    assert lib.bsp_xsd_chunks_build(wide, 1, 4096, 4096, 1, out, 1024, ctypes.byref(m), ctypes.byref(n)) == _lib.ERR_UNSUPPORTED
+    assert lib.bsp_attention_tables_build(wide, 1, 1, 1 << 24, 64, out, 1024, ctypes.byref(info)) == _lib.ERR_UNSUPPORTED
+    assert lib.bsp_attention_stored_tables_build(wide, None, 1, 1, 1 << 24, 64, 0, out, 1024, ctypes.byref(info)) == _lib.ERR_UNSUPPORTED
+    assert lib.bsp_sdd_tiles_build(wide, 1, 64, 64, out, 1024, ctypes.byref(n)) == _lib.OK and n.value == 0
+
+
+def test_builders_report_that_memory_is_short():
+    _alone('_builders_without_memory')

@@ -166,8 +166,8 @@ void indices(const int *at, int S, int32_t *out) {
 
 using namespace bsp;
 
-extern "C" int bsp_attention_tables_build(const uint8_t *h_layout, int H, int R, int C, int block, int32_t *h_tables,
-                                          int64_t cap, bsp_attention_tables *info) {
+static int attention_tables_build(const uint8_t *h_layout, int H, int R, int C, int block, int32_t *h_tables,
+                                  int64_t cap, bsp_attention_tables *info) {
   if (!h_layout || !info || H <= 0 || R <= 0 || C <= 0 || (cap > 0 && !h_tables)) return BSP_ERR_ARG;
   if (block != 16 && block != 32 && block != 64) return BSP_ERR_UNSUPPORTED;
   const int S = 64 / block;
@@ -250,9 +250,13 @@ extern "C" int bsp_attention_tables_build(const uint8_t *h_layout, int H, int R,
   }
   return BSP_OK;
 }
+extern "C" int bsp_attention_tables_build(const uint8_t *h_layout, int H, int R, int C, int block, int32_t *h_tables,
+                                          int64_t cap, bsp_attention_tables *info) {
+  return no_throw([&] { return attention_tables_build(h_layout, H, R, C, block, h_tables, cap, info); });
+}
 
-extern "C" int bsp_attention_stored_tables_build(const uint8_t *h_layout, const int32_t *h_ids, int H, int R, int C, int block, int part,
-                                                 int32_t *h_tables, int64_t cap, bsp_attention_tables *info) {
+static int attention_stored_tables_build(const uint8_t *h_layout, const int32_t *h_ids, int H, int R, int C, int block, int part,
+                                         int32_t *h_tables, int64_t cap, bsp_attention_tables *info) {
   if (!h_layout || !info || H <= 0 || R <= 0 || C <= 0 || part < 0 || (cap > 0 && !h_tables)) return BSP_ERR_ARG;
   if (block != 16 && block != 32 && block != 64) return BSP_ERR_UNSUPPORTED;
   const int S = 64 / block, ints = S == 1 ? 4 : 8 + S * S;   // ints per entry
@@ -347,4 +351,8 @@ extern "C" int bsp_attention_stored_tables_build(const uint8_t *h_layout, const 
     indices(&keys[(size_t)splits[i].col * S], S, e + 4);
   }
   return BSP_OK;
+}
+extern "C" int bsp_attention_stored_tables_build(const uint8_t *h_layout, const int32_t *h_ids, int H, int R, int C, int block, int part,
+                                                 int32_t *h_tables, int64_t cap, bsp_attention_tables *info) {
+  return no_throw([&] { return attention_stored_tables_build(h_layout, h_ids, H, R, C, block, part, h_tables, cap, info); });
 }

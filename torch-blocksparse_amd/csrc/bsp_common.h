@@ -18,6 +18,15 @@
 
 namespace bsp {
 
+// A builder that allocates host memory, behind its C entry point: no exception may leave that
+template <class F> int no_throw(F &&build) {
+  try {
+    return build();
+  } catch (...) {
+    return BSP_ERR_UNSUPPORTED;
+  }
+}
+
 typedef _Float16 f16;
 typedef __bf16 bf16;
 

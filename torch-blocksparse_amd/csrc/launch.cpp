@@ -12,6 +12,7 @@
 #include <Python.h>
 #include <cstdint>
 #include <initializer_list>
+#include <new>
 #include "../../include/bsp.h"
 
 namespace {
@@ -172,7 +173,10 @@ template <class S> void drop(PyObject *cap) {
   S *s = static_cast<S *>(PyCapsule_GetPointer(cap, PyCapsule_GetName(cap)));
   if (s) { Py_XDECREF(s->keep); delete s; }
 }
-template <class S> PyObject *capsule(S *s, const char *name) {
+template <class S> PyObject *capsule(const S &tables, const char *name) {
+  S *s = new (std::nothrow) S(tables);
+  if (!s) return PyErr_NoMemory();
+  Py_INCREF(s->keep);
   PyObject *c = PyCapsule_New(s, name, drop<S>);
   if (!c) { Py_XDECREF(s->keep); delete s; }
   return c;
@@ -187,8 +191,7 @@ PyObject *make_xsd(PyObject *, PyObject *args) {
     return nullptr;
   s.lut = reinterpret_cast<const int32_t *>(lut); s.plan = reinterpret_cast<const int32_t *>(planbuf);
   s.ordinary.table = reinterpret_cast<const int32_t *>(gp); s.wide.table = reinterpret_cast<const int32_t *>(wp);
-  Py_INCREF(s.keep);
-  return capsule(new Xsd(s), kXsd);
+  return capsule(s, kXsd);
 }
 
 PyObject *make_sdd(PyObject *, PyObject *args) {
@@ -212,8 +215,7 @@ PyObject *make_sdd(PyObject *, PyObject *args) {
       s.luts[i] = reinterpret_cast<const int32_t *>(l); s.valids[i] = reinterpret_cast<const uint8_t *>(v); s.widths[i] = w;
     }
   }
-  Py_INCREF(s.keep);
-  return capsule(new Sdd(s), kSdd);
+  return capsule(s, kSdd);
 }
 
 PyObject *make_rows(PyObject *, PyObject *args) {
@@ -221,8 +223,7 @@ PyObject *make_rows(PyObject *, PyObject *args) {
   unsigned long long lut;
   if (!PyArg_ParseTuple(args, "OKiiLLLLL", &s.keep, &lut, &s.maxlut, &s.dev, &s.nnz, &s.H, &s.R, &s.C, &s.block)) return nullptr;
   s.lut = reinterpret_cast<const int32_t *>(lut);
-  Py_INCREF(s.keep);
-  return capsule(new Rows(s), kRows);
+  return capsule(s, kRows);
 }
 
 PyObject *make_attn(PyObject *, PyObject *args) {
@@ -232,8 +233,7 @@ PyObject *make_attn(PyObject *, PyObject *args) {
                         &s.block))
     return nullptr;
   s.rows = reinterpret_cast<const int32_t *>(r); s.items = reinterpret_cast<const int32_t *>(i); s.split = reinterpret_cast<const int32_t *>(p);
-  Py_INCREF(s.keep);
-  return capsule(new Attn(s), kAttn);
+  return capsule(s, kAttn);
 }
 
 // ---- products ----

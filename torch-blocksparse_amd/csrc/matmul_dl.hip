@@ -1446,11 +1446,11 @@ int sdd_dl(int dtype, const SddArgs &g, int block, bool rowpair_plan, bool a_kc,
 
 }  // namespace bsp
 
-extern "C" int bsp_sdd_tiles_build(const uint8_t *layout, int H, int R, int C, int32_t *out, int64_t cap, int64_t *n_tiles) {
+static int sdd_tiles_build(const uint8_t *layout, int H, int R, int C, int32_t *out, int64_t cap, int64_t *n_tiles) {
   using namespace bsp;
   if (!layout || !n_tiles || H <= 0 || R <= 0 || C <= 0 || cap < 0 || (cap > 0 && !out)) return BSP_ERR_ARG;
   int64_t n = 0, blocks_before = 0;
-  std::vector<int64_t> row_first(R + 1);               // id of the first block of a block-row
+  std::vector<int64_t> row_first((size_t)R + 1);             // id of the first block of a block-row
   for (int h = 0; h < H; h++) {
     const uint8_t *lay = layout + (int64_t)h * R * C;
     row_first[0] = blocks_before;
@@ -1507,8 +1507,11 @@ extern "C" int bsp_sdd_tiles_build(const uint8_t *layout, int H, int R, int C, i
   *n_tiles = n;
   return n * kTileInts > cap ? BSP_ERR_CAPACITY : BSP_OK;
 }
+extern "C" int bsp_sdd_tiles_build(const uint8_t *layout, int H, int R, int C, int32_t *out, int64_t cap, int64_t *n_tiles) {
+  return bsp::no_throw([&] { return sdd_tiles_build(layout, H, R, C, out, cap, n_tiles); });
+}
 
-extern "C" int bsp_xsd_chunks_build(const uint8_t *layout, int H, int R, int C, int rows, int32_t *out, int64_t cap, int *n_groups, int64_t *n_ints) {
+static int xsd_chunks_build(const uint8_t *layout, int H, int R, int C, int rows, int32_t *out, int64_t cap, int *n_groups, int64_t *n_ints) {
   using namespace bsp;
   if (!layout || !n_groups || !n_ints || H <= 0 || R <= 0 || C <= 0 || cap < 0 || (cap > 0 && !out)) return BSP_ERR_ARG;
   const int L = rows ? R : C, K = rows ? C : R, per_head = (L + kChunkLines - 1) / kChunkLines;
@@ -1562,4 +1565,7 @@ extern "C" int bsp_xsd_chunks_build(const uint8_t *layout, int H, int R, int C, 
   *n_groups = H * per_head;
   *n_ints = first + n * kChunkInts;
   return *n_ints > cap ? BSP_ERR_CAPACITY : BSP_OK;
+}
+extern "C" int bsp_xsd_chunks_build(const uint8_t *layout, int H, int R, int C, int rows, int32_t *out, int64_t cap, int *n_groups, int64_t *n_ints) {
+  return bsp::no_throw([&] { return xsd_chunks_build(layout, H, R, C, rows, out, cap, n_groups, n_ints); });
 }

@@ -213,3 +213,16 @@ def _builders_without_memory():
 
 def test_builders_report_that_memory_is_short():
     _alone('_builders_without_memory')
+
+
+def test_a_product_follows_the_operator_as_it_is_at_the_call():
+    op = matmul.MatMul(torch.ones(1, 2, 2, dtype=torch.int64), 32, 'dds')
+    key = (torch.float32, torch.device('cpu'))
+    op.lut_cache[key] = (None,) * 8 + (SddTables(), None, None, None)
+    first = op._product(*key)
+    assert op._product(*key) is first
+    op.trans_a = True                                      # (the tables of dds do not depend on it)
+    turned = op._product(*key)
+    assert turned.trans_a and not first.trans_a
+    op.trans_a, op.bench = False, True
+    assert op._product(*key).bench and not op._product(*key).trans_a

@@ -707,14 +707,19 @@ class _Product:
 
     def __init__(self, op, luts, dtype, device):
         mode = op.mode
-        self.luts, self.bench, self.dtype, self.device = luts, op.bench, _lib.DTYPES.get(dtype, -1), device
-        self.trans_a, self.trans_b, self.spdims, self.block = op.trans_a, op.trans_b, op.spdims, op.block
+        self.asked = _Product.asked_of(op)
+        self.trans_a, self.trans_b, self.bench, self.any_k = self.asked
+        self.luts, self.dtype, self.device, self.spdims, self.block = luts, _lib.DTYPES.get(dtype, -1), device, op.spdims, op.block
         self.modes = (mode, mode[1] + mode[0] + mode[2], mode[2] + mode[1] + mode[0])      # c, da, db (matmul.py:593-601)
-        self.any_k = op.any_k
         if self.any_k:                          # (the tables may have been built for other calls of the operator)
             luts[4 * self.modes.index('sdd')].any_k = True
         self.native = [None, None, None]
         self.built = [None, None, None]         # which of the tables made on demand were there
+
+    @staticmethod
+    def asked_of(op):
+        """what a call takes from the operator as it is then, beside its tables"""
+        return op.trans_a, op.trans_b, op.bench, op.any_k
 
     def run(self, which, a, b, trans_a, trans_b, trans_c, times):
         mode = self.modes[which]
@@ -798,7 +803,7 @@ class MatMul:
     def _product(self, dtype, device):
         luts = self.make_lut(dtype, device)
         product = self._products.get((dtype, device))
-        if product is None or product.luts is not luts or product.bench != self.bench or product.any_k != self.any_k:
+        if product is None or product.luts is not luts or product.asked != _Product.asked_of(self):
             product = self._products[(dtype, device)] = _Product(self, luts, dtype, device)
         return product
 

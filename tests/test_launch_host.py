@@ -2,6 +2,7 @@
 the library below is one that it refuses, or that a stand-in takes, before anything is launched."""
 import ctypes
 import os
+import pickle
 import resource
 import subprocess
 import sys
@@ -12,7 +13,8 @@ import pytest
 import torch
 
 from torch_blocksparse import _lib, matmul
-from torch_blocksparse.matmul import SddTables, _sparse_matmul
+from torch_blocksparse.attention_core import AttentionCore
+from torch_blocksparse.matmul import GroupPlan, SddTables, _sparse_matmul
 
 
 class FakeTensor:
@@ -226,3 +228,23 @@ def test_a_product_follows_the_operator_as_it_is_at_the_call():
     assert turned.trans_a and not first.trans_a
     op.trans_a, op.bench = False, True
     assert op._product(*key).bench and not op._product(*key).trans_a
+
+
+def test_operators_saved_without_what_the_native_launches_keep_can_be_loaded():
+    core = AttentionCore(torch.ones(1, 2, 2, dtype=torch.int64), 64)
+    quad = core._made(torch.device('cpu'))[0]
+    shape = quad.__dict__.pop('shape')
+    loaded = pickle.loads(pickle.dumps(core))
+    got = loaded._tables['cpu'][0]
+    assert got.shape == shape == (1, 2, 2, 64) and got._native is None and torch.equal(got.rows, quad.rows)
+    # a product's tables: no length of the longest segment, plans without flags
+    plan = GroupPlan(torch.zeros(8, dtype=torch.int32), 1, 2)
+    plan.__dict__.pop('flags', None)
+    lut = torch.zeros(64, dtype=torch.int32)
+    lut.planbuf, lut.nnz, lut.gplan, lut.gplan_wide = torch.zeros(64, dtype=torch.int32), 4, plan, None
+    lut, plan = pickle.loads(pickle.dumps((lut, plan)))
+    assert lut.gplan.flags == plan.flags == 0
+    op = matmul.MatMul(torch.ones(1, 2, 2, dtype=torch.int64), 64, 'dsd')
+    op.lut_cache[torch.float32, torch.device('cuda', 0)] = (lut, 0, 2, None) + (SddTables(), None, None, None) + (lut, 0, 2, None)
+    product = op._product(torch.float32, torch.device('cuda', 0))
+    assert product._tables(0) is not None and product._tables(2) is not None

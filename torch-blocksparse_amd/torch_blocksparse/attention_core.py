@@ -95,6 +95,7 @@ class _ColumnTable:
 class _QuadTables:
     """The tables of the kernels without sparse tensors (bsp_attention_tables_build), made on the host in one call and copied
     to `device` in one piece: rows (forward and row kernel), items and split (column kernel), and their sizes."""
+    _native = None
 
     def __init__(self, layout, block, device):
         lay = (layout != 0).cpu().contiguous()
@@ -110,10 +111,10 @@ class _QuadTables:
         self.split = self.rows[info.split_offset:] if info.n_split else None
         self.lines, self.longest, self.columns = info.lines, info.longest_line, info.columns
         self.n_items, self.n_slots, self.n_split = info.n_items, info.n_slots, info.n_split
-        self.shape, self._native = (H, R, C, block), None
+        self.shape = (H, R, C, block)
 
     def __getstate__(self):
-        return dict(self.__dict__, _native=None)
+        return {k: v for k, v in self.__dict__.items() if k != '_native'}
 
     def native(self):
         """what the native launcher (csrc/launch.cpp) wants to know of the tables, made once"""
@@ -157,6 +158,12 @@ class AttentionCore:
         self.dsd_tn = MatMul(layout, block, 'dsd', trans_a=True, trans_b=False)
         self.nnz = None
         self._tables = dict()
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        for quad, _ in self._tables.values():              # (saved before the tables kept their shape)
+            if quad is not None and not hasattr(quad, 'shape'):
+                quad.shape = tuple(int(n) for n in self.spdims) + (self.block,)
 
     def blocks(self):
         if self.nnz is None:

@@ -99,11 +99,12 @@ class GroupPlan:
     """Work list of the row-group kernels (see bsp_group_plan_build): device table, number of header rows, lines per
     head, number of split chains (their fp32 partial tiles live in `workspace`)."""
 
+    flags = 0             # launch flags that go with the plan
+
     def __init__(self, table, n_groups, lines, n_split=0):
         self.table, self.n_groups, self.lines, self.n_split = table, n_groups, lines, n_split
         self.coarse = False
         self.rowpair = False
-        self.flags = 0        # launch flags that go with the plan
         self._max_entries = None
         self._ws = None
         self._ws_retired = []
@@ -767,7 +768,7 @@ class _Product:
                                           plan(tiles), (1 if tiles is None else 2) if lut.tiles_apply() else 0,
                                           lut.TILES_LAUNCH, lut.TILE_BLOCKS, levels)
         else:
-            made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, lut.longest, lut.nnz, H, R, C,
+            made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, getattr(lut, 'longest', 0), lut.nnz, H, R, C,
                                           plan(lut.gplan), plan(lut.gplan_wide), lut.gplan_wide.flags if lut.gplan_wide is not None else 0,
                                           2 if lut.gplan_wide is not None else int(getattr(lut, 'build_wide', None) is not None))
         self.native[which], self.built[which] = made, self._on_demand(which)

@@ -1,9 +1,11 @@
 """GPU: the wide dsd / dds kernels at the edges of their three-stage ring and of the 64-entry windows in which they hold the
-table: lines of 1, 2, 3, 4, 63, 64, 65 and 66 blocks."""
+table: lines of 1, 2, 3, 4, 63, 64, 65 and 66 blocks; blocks of 32 also on the kernel that works from lists."""
 import pytest
 import torch
 
 import torch_blocksparse as tb
+from torch_blocksparse import _lib
+from torch_blocksparse.matmul import GroupPlan
 
 pytestmark = pytest.mark.gpu
 
@@ -16,11 +18,13 @@ def _lines():
     return lines
 
 
-@pytest.mark.parametrize('block,Z', [(32, 12), (64, 5)])      # launches large enough for the wide kernels in every orientation
+# launches large enough for the wide kernels in every orientation; blocks of 32: the kernel on lists of blocks, which this layout takes, and
+# the one on groups of four lines, whose ring and windows these are
+@pytest.mark.parametrize('block,Z,lists', [(32, 12, True), (32, 12, False), (64, 5, None)])
 @pytest.mark.parametrize('mode', ['dsd', 'dds'])
 @pytest.mark.parametrize('trans_a', [False, True])
 @pytest.mark.parametrize('trans_b', [False, True])
-def test_ring_and_table_windows(mode, block, Z, trans_a, trans_b):
+def test_ring_and_table_windows(mode, block, Z, lists, trans_a, trans_b, monkeypatch):
     dtype = torch.float16 if trans_a == trans_b else torch.bfloat16
     lines, free = _lines(), 2048 - 24                          # (the last tile of the free dimension is not full)
     K = 66 * block
@@ -34,8 +38,12 @@ def test_ring_and_table_windows(mode, block, Z, trans_a, trans_b):
     dense_trans = trans_b if mode == 'dsd' else trans_a
     shape = (Z, 1, K, free) if (mode == 'dsd') != dense_trans else (Z, 1, free, K)
     dn = torch.randn(shape, generator=g, device='cuda').to(dtype)
+    if lists is False:
+        monkeypatch.setattr(GroupPlan, 'build_xsd_chunks', staticmethod(lambda *args, **kw: None))
     dot = tb.MatMul(lay, block, mode, trans_a=trans_a, trans_b=trans_b)
     got = (dot(sp, dn) if mode == 'dsd' else dot(dn, sp)).float()
+    if block == 32:
+        assert dot.make_lut(dtype, sp.device)[0].gplan_wide.flags == (_lib.FLAG_PLAN_TILES if lists else 0)
     full = torch.zeros((Z, 1, lay.size(1), lay.size(2), block, block), device='cuda')
     h, r, c = lay.nonzero().unbind(1)
     full[:, h, r, c] = sp.float()

@@ -1,15 +1,13 @@
 """GPU: the dsd / dds kernel that works from chunks with lists of blocks (block 32, fp16 / bf16): against the general kernel in every
 orientation, lines that do not fill a group, empty lines and groups, chunks of one block and of 24, ragged free dimensions; and the rule
 that brings it into a product."""
-import ctypes
-
 import pytest
 import torch
 
 import torch_blocksparse as tb
 from torch_blocksparse import _lib, matmul
 from torch_blocksparse.matmul import GroupPlan, _sparse_matmul
-from helpers import assert_close, guard_allocations, random_layout
+from helpers import Guarded, assert_close, guard_allocations, random_layout
 
 DEV = 'cuda'
 
@@ -53,13 +51,10 @@ def test_chunks_hold_the_layout(kind, rows):
     assert torch.equal(seen, ids)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize('kind', ['one block', 'full', 'ragged'])
-@pytest.mark.parametrize('dtype,N', [(torch.float16, 256), (torch.bfloat16, 136), (torch.float16, 392)])
-def test_chunks_against_the_general_kernel(kind, dtype, N):
-    lay = _layout(kind)
+def _against_the_general_kernel(lay, dtype, N, Z, once=False):
+    """every orientation from chunks, between guard bands, against the general kernel"""
     H, R, C = lay.shape
-    dev, Z, nnz = torch.device(DEV), 2, int(lay.sum())
+    dev, nnz = torch.device(DEV), int(lay.sum())
     lib, st = _lib.load(), _lib.stream_ptr(dev)
     torch.manual_seed(N)
     sp = torch.randn(Z, nnz, 32, 32, device=DEV).to(dtype)
@@ -73,9 +68,13 @@ def test_chunks_against_the_general_kernel(kind, dtype, N):
                 for tc in (0, 1):
                     # dense operand: dsd K x N, dds N x K
                     flip = bool(tdn) != dds
-                    dn = torch.randn((Z, H) + ((N, K * 32) if flip else (K * 32, N)), device=DEV).to(dtype) * K ** -0.5
                     out_n_last = bool(tc) == dds
-                    ref, got = [torch.full((Z, H) + ((L * 32, N) if out_n_last else (N, L * 32)), float('nan'), device=DEV, dtype=dtype) for _ in range(2)]
+                    if N % 8 and (not flip or out_n_last):  # (such a free dimension lies along whole rows on both sides)
+                        continue
+                    dn = torch.randn((Z, H) + ((N, K * 32) if flip else (K * 32, N)), device=DEV).to(dtype) * K ** -0.5
+                    shape = (Z, H) + ((L * 32, N) if out_n_last else (N, L * 32))
+                    ref, out = torch.full(shape, float('nan'), device=DEV, dtype=dtype), Guarded(shape, dtype, fill=float('nan'))
+                    got, what = out.t, 'chunks dds=%d tsp=%d tdn=%d tc=%d' % (dds, tsp, tdn, tc)
 
                     def call(c, plan, flags):
                         strides = (dn.stride(0), dn.stride(1), dn.stride(2))
@@ -87,12 +86,60 @@ def test_chunks_against_the_general_kernel(kind, dtype, N):
 
                     assert call(ref, None, _lib.FLAG_GENERAL_ONLY) == _lib.OK
                     assert call(got, chunks, _lib.FLAG_PLAN_TILES) == _lib.OK
-                    torch.cuda.synchronize()
-                    assert_close(got, ref, dtype, 'chunks %s dds=%d tsp=%d tdn=%d tc=%d' % (kind, dds, tsp, tdn, tc))
+                    out.check(what)
+                    assert_close(got, ref, dtype, what)
+                    if once:
+                        continue
                     got.fill_(float('nan'))               # a product that they do not serve runs from its table
                     assert call(got, chunks, _lib.FLAG_PLAN_TILES | _lib.FLAG_GENERAL_ONLY) == _lib.OK
-                    torch.cuda.synchronize()
+                    out.check(what)
                     assert torch.equal(got, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind', ['one block', 'full', 'ragged'])
+@pytest.mark.parametrize('dtype,N', [(torch.float16, 256), (torch.bfloat16, 136), (torch.float16, 392), (torch.float16, 257), (torch.bfloat16, 999)])
+def test_chunks_against_the_general_kernel(kind, dtype, N):
+    _against_the_general_kernel(_layout(kind), dtype, N, Z=2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind,Z', [('one block', 300), ('ragged', 75)])
+@pytest.mark.parametrize('dtype,N', [(torch.float16, 256), (torch.bfloat16, 256), (torch.bfloat16, 136), (torch.float16, 257)])
+def test_workgroups_that_take_several_tiles(kind, Z, dtype, N):
+    # 600 tiles and more for 256 workgroups: a tile's first chunk is on its way during the stores of the one before; whole tiles and partial
+    # ones (lines and columns past the end), tiles of one chunk, tiles without blocks between others
+    lay = _layout(kind)
+    assert lay.shape[0] * -(-min(lay.shape[1:]) // 16) * -(-N // 128) * Z >= 600
+    _against_the_general_kernel(lay, dtype, N, Z, once=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('lists', [True, False])
+@pytest.mark.parametrize('M,Z', [(257, 16), (999, 8)])
+def test_rows_that_divide_by_nothing_on_the_wide_kernels(M, Z, lists, monkeypatch):
+    # y = x W and dx = dy W^T with M rows, from chunks and from groups of four lines
+    if not lists:
+        monkeypatch.setattr(GroupPlan, 'build_xsd_chunks', staticmethod(lambda *args, **kw: None))
+    lay = random_layout((1, 48, 48), 0.3, 3)
+    assert 48 // 4 * -(-M // 256) * Z >= 384                 # the launches that take the wide kernels
+    op = tb.MatMul(lay, 32, 'dds')
+    torch.manual_seed(M)
+    x, dy = [torch.randn(Z, 1, M, 48 * 32, device=DEV).half() for _ in range(2)]
+    w = torch.randn(Z, int(lay.sum()), 32, 32, device=DEV).half() / 16
+    x.requires_grad_(True)
+
+    def both():
+        y = op(x, w)
+        return y.detach(), torch.autograd.grad(y, x, dy)[0]
+
+    with guard_allocations('wide'):
+        got = both()
+    luts = op.make_lut(torch.float16, x.device)
+    assert [t.gplan_wide.flags for t in (luts[0], luts[4])] == [_lib.FLAG_PLAN_TILES if lists else 0] * 2
+    monkeypatch.setattr(matmul, 'KERNEL_FLAGS', _lib.FLAG_GENERAL_ONLY)
+    for one, two, what in zip(got, both(), ('y', 'dx')):
+        assert_close(one, two, torch.float16, what)
 
 
 @pytest.mark.gpu

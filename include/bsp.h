@@ -151,8 +151,9 @@ typedef enum {
   BSP_FLAG_ANY_K = 16,        /* bsp_sdd_matmul_levels with trans_a and not trans_b (the reduction runs along the rows of both operands): K need
                                  not be a multiple of 16 */
   BSP_FLAG_WHOLE_K = 32,       /* bsp_sdd_parts, bsp_xsd_parts: one part whatever the sizes (for cross-checks) */
-  BSP_FLAG_PLAN_TILES = 64     /* bsp_dsd_matmul, bsp_dds_matmul: see bsp_xsd_chunks_build.  bsp_sdd_matmul without a table: d_gplan holds n_plan_groups tiles of bsp_sdd_tiles_build, plan_lines and n_groups the
-                                  block-rows and block-columns of a head; blocks of 32, K >= 256, K % 32 == 0, 16-bit types */
+  BSP_FLAG_PLAN_TILES = 64     /* bsp_dsd_matmul, bsp_dds_matmul: see bsp_xsd_chunks_build.  bsp_sdd_matmul without a table: d_gplan holds
+                                  n_plan_groups tiles of bsp_sdd_tiles_build, plan_lines and n_groups the block-rows and block-columns of a
+                                  head; blocks of 32, K >= 256, K % 32 == 0, 16-bit types */
 } bsp_launch_flags;
 
 /* sparse = dense x dense: replaces _sparse_matmul._sdd_matmul + the SDD branch of the kernel

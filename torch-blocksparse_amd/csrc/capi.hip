@@ -275,8 +275,8 @@ extern "C" int bsp_dsd_matmul(int dtype, const void *a, const void *b, void *c, 
 // transposed product of 'fixed' layouts with a head dimension of 64 (longest segment, average): block 32, 64 of 19 blocks 62 / 53,
 // 61 of 10 59 / 39, 121 of 12 85 / 45; block 64, 16 of 7 30 / 21; block 16, 125 of 18 48 / 39, but 128 of 35 51 / 55 (its parts are read
 // and written as often as the blocks, so the line lies higher).  Launches that do not fill the chip: 27 segments of up to 54 blocks of
-// 64 107 / 27, 64 of up to 64 blocks of 32 115 / 38.  With equal segments, or more
-// workgroups than the chip holds, parts only cost (19 of 19 36 / 42; 14 of 5, 1161 workgroups 79 / 83).
+// 64 107 / 27, 64 of up to 64 blocks of 32 115 / 38.  With equal segments, or more workgroups than the chip holds, parts only cost (19 of
+// 19 36 / 42; 14 of 5, 1161 workgroups 79 / 83).
 extern "C" int bsp_xsd_parts(int dtype, int block, int width, int longest, int64_t nnz, int free_dim, int Z, int flags, int *part_blocks) {
   *part_blocks = 0;
   if (dtype != BSP_F32 || !block_ok(block) || width <= 0 || free_dim <= 0 || Z <= 0 || longest <= 0 || (flags & BSP_FLAG_WHOLE_K)) return 1;

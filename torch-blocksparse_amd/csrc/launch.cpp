@@ -258,7 +258,8 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const bool whole_rows = dds ? !ta && !tc : tb && tc;  // the free dimension lies along whole rows on both sides
   if ((free_dim % dn.vec() && !whole_rows) || free_dim > INT32_MAX) Py_RETURN_NONE;
   Plan plan = s->ordinary;
-  if (block == 32 && free_dim >= 256 && s->dtype != BSP_F32 && s->wide_state && (int64_t)(s->width + 3) / 4 * ((free_dim + 255) / 256) * Z >= 384) {   // _plan_for in matmul.py
+  // (_plan_for in matmul.py)
+  if (block == 32 && free_dim >= 256 && s->dtype != BSP_F32 && s->wide_state && (int64_t)(s->width + 3) / 4 * ((free_dim + 255) / 256) * Z >= 384) {
     if (s->wide_state != 2) Py_RETURN_NONE;
     plan = s->wide;
     flags |= s->wide_flags;
@@ -288,10 +289,14 @@ PyObject *xsd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
     return checked(rc, "bsp_xsd_matmul_parts") ? c.release() : nullptr;
   }
-  const int rc = unlocked([&] { return dds ? bsp_dds_matmul(s->dtype, dn.data(), sp.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, dn.stride[0], dn.stride[1], dn.stride[2], sp_sz, c_sz, c_sh, ldc,
-                                      s->block, s->lut, s->plan, s->width, plan.table, plan.n_groups, plan.lines, plan.n_split, wsp, ws_bytes, flags, st)
-                     : bsp_dsd_matmul(s->dtype, sp.data(), dn.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, sp_sz, dn.stride[0], dn.stride[1], dn.stride[2], c_sz, c_sh, ldc,
-                                      s->block, s->lut, s->plan, s->width, plan.table, plan.n_groups, plan.lines, plan.n_split, wsp, ws_bytes, flags, st); });
+  const int rc = unlocked([&] {
+    return dds ? bsp_dds_matmul(s->dtype, dn.data(), sp.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, dn.stride[0], dn.stride[1], dn.stride[2], sp_sz,
+                                c_sz, c_sh, ldc, s->block, s->lut, s->plan, s->width, plan.table, plan.n_groups, plan.lines, plan.n_split, wsp, ws_bytes,
+                                flags, st)
+               : bsp_dsd_matmul(s->dtype, sp.data(), dn.data(), cp, ta, tb, tc, (int)Z, (int)free_dim, sp_sz, dn.stride[0], dn.stride[1], dn.stride[2],
+                                c_sz, c_sh, ldc, s->block, s->lut, s->plan, s->width, plan.table, plan.n_groups, plan.lines, plan.n_split, wsp, ws_bytes,
+                                flags, st);
+  });
   return checked(rc, dds ? "bsp_dds_matmul" : "bsp_dsd_matmul") ? c.release() : nullptr;
 }
 

@@ -492,8 +492,9 @@ template <typename T> __global__ void __launch_bounds__(256) k_sdd_parts_sum(Sdd
 
 // Blocks of 16 and 32: every pack level of the table in one launch, the largest super-blocks first.  A launch per level
 // leaves the chip idle between them and at the end of each: fp32, block 16, 256 x 512 x 384 in 8 heads and batches, half of
-// the blocks, takes 11.3 + 9.5 us in two launches and 14.7 in one, beside the launch that the host does not make.  The last level of block 16 has super-blocks of one wavefront; four of them share a workgroup: they run the same
-// number of steps and so of barriers, the ones past the end of the level repeat its last super-block and keep nothing.
+// the blocks, takes 11.3 + 9.5 us in two launches and 14.7 in one.  The host makes one launch less, too.
+// The last level of block 16 has super-blocks of one wavefront, four of which share a workgroup: they run the same number of steps and
+// so of barriers, and the ones past the end of the level repeat its last super-block and keep nothing.
 template <int BLOCK> struct SddLevels {
   static constexpr int N = BLOCK == 16 ? 3 : 2;
   const int32_t *lut[N];                 // by pack: 64 / BLOCK, half of that, ..., 1

@@ -636,12 +636,13 @@ class _sparse_matmul(torch.autograd.Function):
         b_sz = b.stride(0) if (b.dim() == 4 and b.size(0) > 1) else 0   # a 3-D (or batch-1) sparse operand is shared by the batch
         plan = _sparse_matmul._plan_for(lut, block, M, a.dtype, width, a.size(0))
         timer = _Timer(bench, a.device)
-        rc = _lib.OK if _sparse_matmul._in_parts(True, b, a, c, trans_a, trans_b, trans_c, a.size(0), M, b_sz, block, lut, width) else _lib.load().bsp_dds_matmul(_lib.DTYPES[a.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
-                                        int(trans_c), a.size(0), M, a.stride(0), a.stride(1), a.stride(2), b_sz, c.stride(0),
-                                        c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
-                                        *GroupPlan.xsd_args(plan, M, a.size(0)), KERNEL_FLAGS | (plan.flags if plan is not None else 0),
-                                        _lib.stream_ptr(a.device))
-        _lib.check(rc, 'bsp_dds_matmul')
+        if not _sparse_matmul._in_parts(True, b, a, c, trans_a, trans_b, trans_c, a.size(0), M, b_sz, block, lut, width):
+            rc = _lib.load().bsp_dds_matmul(_lib.DTYPES[a.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
+                                            int(trans_c), a.size(0), M, a.stride(0), a.stride(1), a.stride(2), b_sz, c.stride(0),
+                                            c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
+                                            *GroupPlan.xsd_args(plan, M, a.size(0)), KERNEL_FLAGS | (plan.flags if plan is not None else 0),
+                                            _lib.stream_ptr(a.device))
+            _lib.check(rc, 'bsp_dds_matmul')
         time[0] = timer.done()
         if M != AS2:
             c = c[:, :, :, :AS2] if trans_c else c[:, :, :AS2, :]
@@ -662,12 +663,13 @@ class _sparse_matmul(torch.autograd.Function):
         a_sz = a.stride(0) if (a.dim() == 4 and a.size(0) > 1) else 0
         plan = _sparse_matmul._plan_for(lut, block, N, b.dtype, width, b.size(0))
         timer = _Timer(bench, b.device)
-        rc = _lib.OK if _sparse_matmul._in_parts(False, a, b, c, trans_a, trans_b, trans_c, b.size(0), N, a_sz, block, lut, width) else _lib.load().bsp_dsd_matmul(_lib.DTYPES[b.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
-                                        int(trans_c), b.size(0), N, a_sz, b.stride(0), b.stride(1), b.stride(2), c.stride(0),
-                                        c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
-                                        *GroupPlan.xsd_args(plan, N, b.size(0)), KERNEL_FLAGS | (plan.flags if plan is not None else 0),
-                                        _lib.stream_ptr(b.device))
-        _lib.check(rc, 'bsp_dsd_matmul')
+        if not _sparse_matmul._in_parts(False, a, b, c, trans_a, trans_b, trans_c, b.size(0), N, a_sz, block, lut, width):
+            rc = _lib.load().bsp_dsd_matmul(_lib.DTYPES[b.dtype], _lib.ptr(a), _lib.ptr(b), _lib.ptr(c), int(trans_a), int(trans_b),
+                                            int(trans_c), b.size(0), N, a_sz, b.stride(0), b.stride(1), b.stride(2), c.stride(0),
+                                            c.stride(1), c.stride(2), block, _lib.ptr(lut), _lib.ptr(lut.planbuf), width,
+                                            *GroupPlan.xsd_args(plan, N, b.size(0)), KERNEL_FLAGS | (plan.flags if plan is not None else 0),
+                                            _lib.stream_ptr(b.device))
+            _lib.check(rc, 'bsp_dsd_matmul')
         time[0] = timer.done()
         if N != BS3:
             c = c[:, :, :BS3, :] if trans_c else c[:, :, :, :BS3]
@@ -708,19 +710,13 @@ class _Product:
 
     def __init__(self, op, luts, dtype, device):
         mode = op.mode
-        self.asked = _Product.asked_of(op)
-        self.trans_a, self.trans_b, self.bench, self.any_k = self.asked
+        self.trans_a, self.trans_b, self.bench, self.any_k = op.trans_a, op.trans_b, op.bench, op.any_k
         self.luts, self.dtype, self.device, self.spdims, self.block = luts, _lib.DTYPES.get(dtype, -1), device, op.spdims, op.block
         self.modes = (mode, mode[1] + mode[0] + mode[2], mode[2] + mode[1] + mode[0])      # c, da, db (matmul.py:593-601)
         if self.any_k:                          # (the tables may have been built for other calls of the operator)
             luts[4 * self.modes.index('sdd')].any_k = True
         self.native = [None, None, None]
         self.built = [None, None, None]         # which of the tables made on demand were there
-
-    @staticmethod
-    def asked_of(op):
-        """what a call takes from the operator as it is then, beside its tables"""
-        return op.trans_a, op.trans_b, op.bench, op.any_k
 
     def run(self, which, a, b, trans_a, trans_b, trans_c, times):
         mode = self.modes[which]
@@ -762,13 +758,15 @@ class _Product:
                                for t, w, p in zip(lut, lut.widths, lut.packs))
             late = lut.gplan_long
             tiles = lut.tiles
-            made = _lib.native().make_sdd((lut, lut.gplan, late, tiles) + tuple(lut) + tuple(getattr(t, 'valid', None) for t in lut), self.block, self.dtype, dev, lut.nnz, H, R, C,
+            made = _lib.native().make_sdd((lut, lut.gplan, late, tiles) + tuple(lut) + tuple(getattr(t, 'valid', None) for t in lut),
+                                          self.block, self.dtype, dev, lut.nnz, H, R, C,
                                           plan(lut.gplan), plan(late), 0 if lut.build_long is None else 1 if late is None else 2,
                                           int(late is not None and late.rowpair), late.max_entries() if late is not None else 0, int(lut.any_k),
                                           plan(tiles), (1 if tiles is None else 2) if lut.tiles_apply() else 0,
                                           lut.TILES_LAUNCH, lut.TILE_BLOCKS, levels)
         else:
-            made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype, dev, getattr(lut, 'longest', 0), lut.nnz, H, R, C,
+            made = _lib.native().make_xsd((lut, lut.gplan, lut.gplan_wide), lut.data_ptr(), lut.planbuf.data_ptr(), width, self.block, self.dtype,
+                                          dev, getattr(lut, 'longest', 0), lut.nnz, H, R, C,
                                           plan(lut.gplan), plan(lut.gplan_wide), lut.gplan_wide.flags if lut.gplan_wide is not None else 0,
                                           2 if lut.gplan_wide is not None else int(getattr(lut, 'build_wide', None) is not None))
         self.native[which], self.built[which] = made, self._on_demand(which)
@@ -802,10 +800,12 @@ class MatMul:
         return self.lut_cache[key]
 
     def _product(self, dtype, device):
-        luts = self.make_lut(dtype, device)
-        product = self._products.get((dtype, device))
-        if product is None or product.luts is not luts or product.asked != _Product.asked_of(self):
-            product = self._products[(dtype, device)] = _Product(self, luts, dtype, device)
+        key = (dtype, device)
+        luts, product = self.lut_cache.get(key) or self.make_lut(dtype, device), self._products.get(key)
+        # (the flags are those of the operator as it is now)
+        if (product is None or product.luts is not luts or product.trans_a is not self.trans_a or product.trans_b is not self.trans_b or
+                product.bench is not self.bench or product.any_k is not self.any_k):
+            product = self._products[key] = _Product(self, luts, dtype, device)
         return product
 
     def __getstate__(self):

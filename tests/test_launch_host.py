@@ -248,3 +248,22 @@ def test_operators_saved_without_what_the_native_launches_keep_can_be_loaded():
     op.lut_cache[torch.float32, torch.device('cuda', 0)] = (lut, 0, 2, None) + (SddTables(), None, None, None) + (lut, 0, 2, None)
     product = op._product(torch.float32, torch.device('cuda', 0))
     assert product._tables(0) is not None and product._tables(2) is not None
+
+
+def test_tables_that_another_thread_builds_meanwhile_are_seen_by_the_next_call(monkeypatch):
+    lut = torch.zeros(64, dtype=torch.int32)
+    lut.planbuf, lut.nnz, lut.longest, lut.gplan, lut.gplan_wide = torch.zeros(64, dtype=torch.int32), 4, 2, None, None
+    lut.build_wide = lambda: None
+    op = matmul.MatMul(torch.ones(1, 2, 2, dtype=torch.int64), 32, 'dsd')
+    key = (torch.float16, torch.device('cuda', 0))
+    op.lut_cache[key] = (lut, 0, 2, None) + (SddTables(), None, None, None) + (lut, 0, 2, None)
+    real = _lib.native()
+
+    def make_xsd(*args):
+        made = real.make_xsd(*args)
+        lut.gplan_wide = GroupPlan(torch.zeros(8, dtype=torch.int32), 1, 2)      # the other thread
+        return made
+
+    monkeypatch.setattr(_lib, 'native', lambda: types.SimpleNamespace(make_xsd=make_xsd))
+    product = op._product(*key)
+    assert product._tables(0) is not None and product.built[0] != product._on_demand(0)

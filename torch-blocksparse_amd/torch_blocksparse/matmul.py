@@ -747,6 +747,7 @@ class _Product:
         """a capsule with the pointers and numbers of the tables as they are now, and the tensors behind them"""
         if self.device.type != 'cuda' or self.dtype < 0:
             return None
+        built = self._on_demand(which)          # (first: another thread may build more of them meanwhile)
         lut, _, width, _ = self.luts[4 * which:4 * which + 4]
         H, R, C = [int(n) for n in self.spdims]
         dev = self.device.index if self.device.index is not None else torch.cuda.current_device()
@@ -769,7 +770,7 @@ class _Product:
                                           dev, getattr(lut, 'longest', 0), lut.nnz, H, R, C,
                                           plan(lut.gplan), plan(lut.gplan_wide), lut.gplan_wide.flags if lut.gplan_wide is not None else 0,
                                           2 if lut.gplan_wide is not None else int(getattr(lut, 'build_wide', None) is not None))
-        self.native[which], self.built[which] = made, self._on_demand(which)
+        self.native[which], self.built[which] = made, built
         return made
 
 

@@ -453,6 +453,37 @@ int bsp_attention_cols_bwd(int dtype, const void *d_o, const void *q, const void
                            const int32_t *d_items, int n_items, float *partial, int n_slots, const int32_t *d_split, int n_split,
                            const void *kpm, int64_t kpm_stride_z, int kpm_mul, void *stream);
 
+/* The same chain in fp32, D = 64 or 128, with the tables of bsp_attention_tables_build.  The operands are kept as three bfloat16 parts
+ * each, whose products add up to fp32 products (heads that hold a value of 2^30 or more, an infinity or a NaN are computed on the
+ * fp32 matrix units instead).
+ * Z, H, R: batches, heads, lines of 64 rows; keys: positions of k and v (a multiple of 64).  strides: of batch, head and row, in
+ * elements, three per tensor in the order of the call's tensor arguments (fwd: q, k, v, o; bwd: d_o, o, dq, dk, dv); multiples of 4,
+ * unit inner stride, 16-byte aligned pointers.  kpm: element (z, key) at kpm[z * kpm_stride_z + key], or NULL.
+ * planes: bsp_attention_f32_bytes(Z, H, 64 R, keys, D) bytes (rows 0 where stats is NULL), written by fwd and read by bwd.  stats:
+ * [Z][H][2][64 R] floats, written by fwd (NULL: no backward pass to follow) and read by bwd: the reference of the row's exponentials (log2
+ * domain), one over their sum.
+ * bwd: do_planes: bsp_attention_f32_bytes(Z, H, 64 R, 0, D) bytes of scratch; neg_delta: [Z][H][64 R] floats of scratch.  dk and dv are
+ * computed together; without them (both NULL) do_planes, neg_delta and what follows may be NULL and 0.  d_items .. n_split: as for
+ * bsp_attention_cols_bwd; partial: bsp_attention_f32_slots(Z, n_slots) slots of 2 x 64 x D floats. */
+typedef struct {
+  int Z, H, R, D;
+  int64_t keys;
+  int64_t strides[15];
+  const int32_t *d_rows;
+  const float *kpm;
+  int64_t kpm_stride_z;
+  void *planes;
+  float *stats;
+  float scale;
+  int kpm_mul;
+} bsp_attention_f32_call;
+int64_t bsp_attention_f32_bytes(int Z, int H, int64_t rows, int64_t keys, int D);
+int64_t bsp_attention_f32_slots(int Z, int n_slots);
+int bsp_attention_f32_fwd(const bsp_attention_f32_call *call, const float *q, const float *k, const float *v, float *o, void *stream);
+int bsp_attention_f32_bwd(const bsp_attention_f32_call *call, const float *d_o, const float *o, float *dq, float *dk, float *dv, void *do_planes,
+                          float *neg_delta, const int32_t *d_items, int n_items, float *partial, int n_slots, const int32_t *d_split,
+                          int n_split, void *stream);
+
 /* ---------------------------------------------------------------------------------------------------
  * Dense utility ops of the reference package.
  * ReLU: replaces the relu_y / relu_dxdsdbdres kernels and their launches (relu.py:8-91).  All tensors hold n

@@ -1,0 +1,147 @@
+"""GPU: the attention chain in fp32 on the bfloat16 matrix units (bsp_attention_f32_fwd / _bwd behind attention_chain) against dense 64-bit
+arithmetic and against the three operators, which compute on the fp32 units.
+
+Tolerance: a product keeps what counts in 24 bits and is rounded less often than on the fp32 units, so every result is at least as
+close to 64 bits as the operators' one, give or take a unit of 2^-23 for the softmax (relative 2-norm)."""
+import pytest
+import torch
+
+import torch_blocksparse as tb
+from torch_blocksparse import attention_core as ac
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+
+def _ops(lay, block):
+    return tb.MatMul(lay, block, 'sdd', trans_b=True), tb.Softmax(lay, block), tb.MatMul(lay, block, 'dsd')
+
+
+def _run(ops, q, k, v, do, fused, **kw):
+    xs = [t.detach().clone().requires_grad_() for t in (q, k, v)]
+    before, was = ac.fused_f32_calls, ac.FUSED
+    ac.FUSED = fused
+    try:
+        o = ac.attention_chain(*ops, *xs, **kw)
+        grads = torch.autograd.grad(o, xs, do)
+    finally:
+        ac.FUSED = was
+    assert ac.fused_f32_calls - before == int(fused)
+    return (o.detach(),) + grads
+
+
+def _dense(q, k, v, do, lay, block, scale, kpm=None):
+    xs = [t.detach().double().requires_grad_() for t in (q, k, v)]
+    m = lay.to(DEV).repeat_interleave(block, 1).repeat_interleave(block, 2).bool()
+    s = xs[0] @ xs[1].transpose(-1, -2) * scale
+    if kpm is not None:
+        s = s + kpm.double()[:, None, None, :]
+    s = s.masked_fill(~m, float('-inf'))
+    p = torch.where(m.any(-1, keepdim=True), torch.softmax(s, -1), torch.zeros((), dtype=torch.float64, device=DEV))
+    o = p @ xs[2]
+    return (o.detach(),) + torch.autograd.grad(o, xs, do.double())
+
+
+def _layout(H, R, C, kind):
+    g = torch.Generator().manual_seed(R * 131 + C)
+    if kind == 'dense':
+        return torch.ones(H, R, C, dtype=torch.int64)
+    lay = (torch.rand((H, R, C), generator=g) < 0.3).long()
+    lay[:, :, 0] = 1                                                      # a long column (in parts where it is long enough), no row without keys
+    if kind == 'holes':                                                   # rows without any block beside one that has some
+        lay[:, 4:8] = 0
+        lay[:, 5, min(3, C - 1)] = 1
+    return lay
+
+
+# one tile; a tile of remainders; lines and columns of one to many tiles; parts of long columns in 4, 2 and 1 pieces (1, 66 and 512 batches x
+# heads of one 40-tile column in three parts, 2 of 64); from 32 heads on another order of the workgroups
+@pytest.mark.parametrize('Z,H,R,C,block,D,kind,padded', [
+    (1, 1, 1, 1, 64, 64, 'dense', False),
+    (2, 1, 4, 4, 16, 128, 'random', True),
+    (1, 2, 2, 10, 32, 64, 'random', True),
+    (2, 2, 16, 24, 32, 64, 'holes', True),
+    (1, 2, 12, 8, 16, 64, 'holes', False),
+    (1, 3, 40, 6, 64, 64, 'random', False),
+    (11, 6, 80, 8, 32, 64, 'random', False),
+    (2, 32, 40, 4, 64, 128, 'random', True),
+    (64, 8, 40, 2, 64, 64, 'random', False),
+    (1, 2, 32, 32, 64, 128, 'dense', False),
+])
+def test_against_64_bits(Z, H, R, C, block, D, kind, padded):
+    torch.manual_seed(R + C + D)
+    lay = _layout(H, R, C, kind)
+    q, do = [torch.randn(Z, H, R * block, D, device=DEV) for _ in range(2)]
+    k, v = [torch.randn(Z, H, C * block, D, device=DEV) for _ in range(2)]
+    kw = dict(scale=D ** -0.5)
+    if padded:
+        kpm = torch.zeros(Z, C * block, device=DEV)
+        kpm[0, block:block + 9] = float('-inf')
+        kpm[-1, block + 5:] = -2.
+        kw['key_padding_mask'] = kpm
+    ref = _dense(q, k, v, do, lay, block, D ** -0.5, kw.get('key_padding_mask'))
+    ops = _ops(lay, block)
+    got, other = [_run(ops, q, k, v, do, fused, **kw) for fused in (True, False)]
+    for name, g, c, r in zip(('o', 'dq', 'dk', 'dv'), got, other, ref):
+        assert bool(torch.isfinite(g).all()), name
+        err, bound = [float((x.double() - r).norm() / r.norm()) for x in (g, c)]
+        assert err <= bound + 2 ** -23, (name, err, bound)
+    again = _run(ops, q, k, v, do, True, **kw)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+# Values that have no bfloat16 parts, or whose products fp32 does not hold, in one row of one head: what is and what is not finite comes out
+# as it does on the fp32 units, also for rows whose tiles hold the value in a block that they do not have.
+@pytest.mark.parametrize('where,value', [('q', float('inf')), ('k', float('-inf')), ('v', float('inf')), ('v', float('nan')), ('do', float('-inf')), ('k', 1e20), ('k', 3.4e38), ('q', 1e10)])
+@pytest.mark.parametrize('block,D', [(32, 64), (16, 128)])
+def test_values_without_parts(where, value, block, D):
+    torch.manual_seed(block)
+    n = 256 // block
+    lay = _layout(2, n, n, 'random')
+    x = {t: torch.randn(2, 2, 256, D, device=DEV) for t in ('q', 'k', 'v', 'do')}
+    x[where][0, 1, 37, 5] = value
+    ops = _ops(lay, block)
+    got, other = [_run(ops, x['q'], x['k'], x['v'], x['do'], fused, scale=D ** -0.5) for fused in (True, False)]
+    for name, g, c in zip(('o', 'dq', 'dk', 'dv'), got, other):
+        assert bool((torch.isfinite(g) == torch.isfinite(c)).all()), name
+        # (an infinite do gives infinities of both signs, whose sum over a row the operators form and these kernels do not)
+        assert where == 'do' or bool((torch.isnan(g) == torch.isnan(c)).all()), name
+    # the other batch and head are as if nothing had been there (a few 2^-24 of two correct results)
+    for g, c in zip(got, other):
+        assert float((g[1, 0] - c[1, 0]).norm() / c[1, 0].norm()) < 2e-6
+
+
+def test_padding_values_that_leave_no_score():
+    """The lowest finite value (and -1e9) on every key of a sequence: fp32 rounds the scores away beside it and every key gets the same
+    share, as from the operators; -inf on every key gives NaN for that sequence alone."""
+    torch.manual_seed(3)
+    lay = _layout(2, 4, 4, 'random')
+    ops = _ops(lay, 64)
+    q, k, v, do = [torch.randn(2, 2, 256, 64, device=DEV) for _ in range(4)]
+    for value in (-1e9, torch.finfo(torch.float32).min, float('-inf')):
+        kpm = torch.zeros(2, 256, device=DEV)
+        kpm[0] = value
+        got, other = [_run(ops, q, k, v, do, fused, scale=0.125, key_padding_mask=kpm) for fused in (True, False)]
+        for g, c in zip(got, other):
+            assert bool((torch.isnan(g) == torch.isnan(c)).all())
+            assert float((g[1] - c[1]).norm() / c[1].norm()) < 2e-6
+        if value != float('-inf'):
+            assert float((got[0][0] - other[0][0]).norm() / other[0][0].norm()) < 2e-6
+
+
+def test_operands_that_are_copied_and_inference():
+    """Odd strides, an expanded gradient, gradients of some operands only, and a forward pass alone (which keeps no parts of q)."""
+    torch.manual_seed(4)
+    lay = _layout(2, 8, 8, 'random')
+    ops = _ops(lay, 32)
+    q, k, v = [torch.randn(2, 2, 256, 64, device=DEV) for _ in range(3)]
+    want = _run(ops, q, k, v, torch.ones(2, 2, 256, 64, device=DEV), True, scale=0.125)
+    odd = torch.empty(2, 2, 256, 66, device=DEV)[..., 1:65].copy_(k)
+    got = _run(ops, q.transpose(1, 2).contiguous().transpose(1, 2), odd, v, torch.ones(1, 1, 1, 1, device=DEV).expand(2, 2, 256, 64), True, scale=0.125)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+    for i in range(3):
+        xs = [t.clone().requires_grad_(i == j) for j, t in enumerate((q, k, v))]
+        (grad,) = torch.autograd.grad(ac.attention_chain(*ops, *xs, scale=0.125).sum(), xs[i])
+        assert torch.equal(grad, want[1 + i])
+    with torch.no_grad():
+        assert torch.equal(ac.attention_chain(*ops, q, k, v, scale=0.125), want[0])

@@ -15,7 +15,7 @@ LIBDIR = os.path.join(HERE, 'lib')
 OBJDIR = os.path.join(HERE, 'build')
 LIBNAME = 'libbsp_hip.so'
 PROBE_LIBNAME = 'libbsp_probe.so'
-SOURCES = ['lut.hip', 'layout.hip', 'softmax.hip', 'softmax_row.hip', 'attention_core.hip', 'attention_long.hip', 'attention_kv.hip', 'attention_fwd.hip', 'attention_bwd.hip', 'attention_tables.hip', 'matmul_f16.hip', 'matmul_bf16.hip', 'matmul_f32.hip', 'matmul_fast64.hip', 'matmul_dl.hip', 'elementwise.hip', 'capi.hip']
+SOURCES = ['lut.hip', 'layout.hip', 'softmax.hip', 'softmax_row.hip', 'attention_core.hip', 'attention_long.hip', 'attention_kv.hip', 'attention_fwd.hip', 'attention_bwd.hip', 'attention_f32.hip', 'attention_tables.hip', 'matmul_f16.hip', 'matmul_bf16.hip', 'matmul_f32.hip', 'matmul_fast64.hip', 'matmul_dl.hip', 'elementwise.hip', 'capi.hip']
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-fno-gpu-rdc', '-Wall', '-Wno-unused-function',
          # packed-fp32 instruction selection is switched off on purpose
          '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops']
@@ -28,7 +28,7 @@ def lib_path():
 # Kernels that count their own outstanding vector-memory operations (s_waitcnt vmcnt(n) in front of the barriers of an
 # LDS ring of direct global -> LDS loads).  A register spill adds scratch loads and stores to that count and the waits
 # would then let a tile be read before it has landed: the build refuses such a kernel.
-COUNTED_WAITS = {'attention_core.hip': 'k_attn64', 'attention_long.hip': 'k_attn64', 'attention_kv.hip': 'k_attn64', 'attention_fwd.hip': 'k_attn', 'attention_bwd.hip': 'k_attn', 'matmul_dl.hip': 'k_'}
+COUNTED_WAITS = {'attention_core.hip': 'k_attn64', 'attention_long.hip': 'k_attn64', 'attention_kv.hip': 'k_attn64', 'attention_fwd.hip': 'k_attn', 'attention_bwd.hip': 'k_attn', 'attention_f32.hip': 'k_attn32', 'matmul_dl.hip': 'k_'}
 
 
 def _spilled_kernels(remarks, prefix):

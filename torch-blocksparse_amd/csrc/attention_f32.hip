@@ -1,0 +1,1010 @@
+// The attention chain without sparse tensors in fp32 (head dimension 64 or 128; calls without relative position embedding and attention
+// mask): what attention_fwd.hip and attention_bwd.hip do for 16-bit tensors, in single precision and on the bfloat16 matrix units.
+//
+// Products.  A number of 24 bits is the sum of three bfloat16 numbers, each rounded to nearest: x = x0 + x1 + x2 (exactly, down
+// to 2^-110).  A product is the sum of the six products of such parts that count in 24 bits, smallest first, in one fp32
+// accumulator: x2 y0 + x1 y1 + x0 y2 + x1 y0 + x0 y1 + x0 y0.  Six MFMAs of bfloat16 do in 6 x 32 cycles what eight of fp32 do in
+// 8 x 64, and round less often (once a step of sixteen instead of two).  Error against 64 bits of 32 x 32 products of N(0, 1) operands, relative 2-norm, this /
+// fp32 MFMA: 64 terms 1.1e-7 / 1.5e-7, 512 terms 3.4e-7 / 4.0e-7, 4096 terms 9.9e-7 / 1.15e-6; uniform operands 0.9e-7 / 1.2e-7, 2.4e-7 /
+// 2.9e-7, 5.2e-7 / 8.3e-7.  (Parts cut off instead of rounded: 1e-5 for 4096 uniform terms, their sums being one-sided.)
+// Infinities have no such parts, and their products with zero parts would be NaN: where a head's operands hold a value of 2^30 or
+// more, an infinity or a NaN (a flag per 64 rows, made beside the parts), the kernels compute its products from the whole
+// values on the fp32 units, as the operators do.  Below 2^30 no product overflows.
+//
+// Launches.  k_attn32_planes writes the three parts of q, k and v (backward: do) as planes, [row][part][D], so that the other
+// kernels fetch them tile by tile straight into LDS.  Those walk the same tables and 64 x 64 tiles as the 16-bit kernels; a
+// workgroup is four wavefronts, one per 32 x 32 quadrant, since a line is few tiles and 64 rows with two wavefronts would leave
+// half of the SIMDs of a launch of a few hundred lines without any.  The quadrants of the same rows add up at the end through LDS.
+// A tile's operands come in two pieces (k, v; columns: q, do) of 64 rows x 3 parts, 24 KiB at head dimension 64; the ring has
+// three slots of a piece, so two workgroups share a CU: while a piece is used the next is on its way, and the one after that
+// where a slot is free.
+#include "attention_quad.h"
+#include <atomic>
+
+// (a multiplication and the subtraction behind it stay two roundings: see pad_term)
+#pragma clang fp contract(off)
+
+namespace bsp {
+namespace {
+
+struct F32Args : QuadArgs {            // k, v: the planes; q: forward q itself, backward the planes; d_o: row kernel do itself, column kernel
+                                       // the planes; lse: per row the reference m of its exponentials, rest floats on 1 / l
+  bf16 *planes_out;                    // forward: planes of q (NULL: no backward pass to follow); row kernel: planes of do
+  int32_t *flags_out;                  // ... and their flags
+  const int32_t *fq, *fk, *fv, *fdo;   // flags [Z][H]: of 32 rows each (q, do) or 64 (k, v)
+  int64_t rows, keys;
+  int sub;                             // column kernel: pieces that a part of a long column is cut into
+};
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+struct Parts { bf16x8 p[3]; };
+constexpr float kLargest = 1073741824.f;               // 2^30
+
+// the parts of eight values; WHOLE: also of those that are not below kLargest (infinities and NaN in the first part alone)
+template <bool WHOLE> __device__ __forceinline__ Parts split8(const float (&v)[8]) {
+  union { bf16x2 two[4]; bf16x8 all; } h, m, l;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const f32x2 x = {v[2 * i], v[2 * i + 1]};
+    h.two[i] = __builtin_convertvector(x, bf16x2);
+    const f32x2 r = x - __builtin_convertvector(h.two[i], f32x2);
+    m.two[i] = __builtin_convertvector(r, bf16x2);
+    l.two[i] = __builtin_convertvector(r - __builtin_convertvector(m.two[i], f32x2), bf16x2);
+  }
+  if constexpr (WHOLE) {
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      if (!(fabsf(v[i]) < kLargest)) {
+        const bool finite = fabsf(v[i]) < INFINITY;
+        const float a = finite ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i]) & 0xffff0000u) : v[i], r = finite ? v[i] - a : 0.f;
+        const float b = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xffff0000u);
+        h.all[i] = (bf16)a; m.all[i] = (bf16)b; l.all[i] = (bf16)(r - b);
+      }
+  }
+  Parts s;
+  s.p[0] = h.all; s.p[1] = m.all; s.p[2] = l.all;
+  return s;
+}
+
+__device__ __forceinline__ f32x16 mma(const bf16x8 &a, const bf16x8 &b, const f32x16 &c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+// value i of eight that are held as parts
+__device__ __forceinline__ float whole(const u32x4 (&v)[3], int i) {
+  auto part = [&](int p) { return __builtin_bit_cast(float, i & 1 ? v[p][i >> 1] & 0xffff0000u : v[p][i >> 1] << 16); };
+  return part(0) + part(1) + part(2);
+}
+// acc += a . b over sixteen indices from the whole values, on the fp32 units.  (The empty assembly keeps whole values from being held
+// beside the parts, the barrier keeps the next operands from being fetched ahead: this way is about registers, not time.)
+template <class F> __device__ __forceinline__ f32x16 whole_product(const Parts &a, F &&b, f32x16 acc) {
+  u32x4 x[3];
+#pragma unroll
+  for (int p = 0; p < 3; p++) {
+    x[p] = __builtin_bit_cast(u32x4, a.p[p]);
+    asm volatile("" : "+v"(x[p]));
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(whole(x, i), b(i), acc, 0, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  return acc;
+}
+__device__ __forceinline__ f32x16 whole_parts_product(const Parts &a, const Parts &b, f32x16 acc) {
+  u32x4 y[3];
+#pragma unroll
+  for (int p = 0; p < 3; p++) {
+    y[p] = __builtin_bit_cast(u32x4, b.p[p]);
+    asm volatile("" : "+v"(y[p]));
+  }
+  return whole_product(a, [&](int i) { return whole(y, i); }, acc);
+}
+
+template <int D> struct Ring {
+  static constexpr int PLANE = 64 * D * 2, PIECE = 3 * PLANE, SIDE = 4 * 512;   // SIDE: two words a lane for each wavefront, beside a piece
+  static constexpr int BYTES = 3 * (PIECE + SIDE);
+};
+
+// acc[i] += (32 rows of the piece, dealt by deal_row) . b, as in attention_quad.h
+// The scores come out the same, bit for bit, with the rows of q or those of k in LDS (SWAP: the parts of b are taken as the first factor's), so
+// that the backward pass has the forward pass's probabilities however large the scores are.
+// (WHOLE: b is fetched again for each product, from its planes or as it is, which leaves its registers to the fp32 units' way of working)
+template <bool WHOLE, bool SWAP, int D, typename S>
+__device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const RowReads<D, true> &reads, const Parts (&b)[D / 16], const S *b_row, f32x16 acc) {
+  uint32_t at[D / 16];
+  reads.get(at);
+#pragma unroll
+  for (int s = 0; s < D / 16; s++) {
+    Parts f;
+#pragma unroll
+    for (int p = 0; p < 3; p++) f.p[p] = *reinterpret_cast<const bf16x8 *>(piece + p * Ring<D>::PLANE + at[s]);
+    if constexpr (WHOLE) {
+      asm volatile("" : "+v"(b_row));
+      if constexpr (sizeof(S) == 4) {
+        const f32x4 lo = *reinterpret_cast<const f32x4 *>(b_row + 16 * s), hi = *reinterpret_cast<const f32x4 *>(b_row + 16 * s + 4);
+        acc = whole_product(f, [&](int i) { return i < 4 ? lo[i & 3] : hi[i & 3]; }, acc);
+      } else {
+        Parts mine;
+#pragma unroll
+        for (int p = 0; p < 3; p++) mine.p[p] = *reinterpret_cast<const bf16x8 *>(b_row + p * D + 16 * s);
+        acc = whole_parts_product(f, mine, acc);
+      }
+    } else {
+      const Parts &x = SWAP ? b[s] : f, &y = SWAP ? f : b[s];
+      auto term = [&](int i, int j) { acc = SWAP ? mma(y.p[j], x.p[i], acc) : mma(x.p[i], y.p[j], acc); };
+      term(2, 0); term(0, 2); term(1, 1); term(0, 1); term(1, 0); term(0, 0);
+    }
+  }
+  return acc;
+}
+// acc[mt] += (32 rows of the piece, transposed) . b; WHOLE: only where here0 / here1, the first / second sixteen rows have a block (nothing of the
+// rows of a block that does not exist may reach the sums, and an infinity among them would).  Two chains of products at a time: two groups
+// of columns, each step's 32 terms added up first; TIGHT (where registers are short): one group, the smaller products of a step and the others.
+template <bool WHOLE, bool TIGHT, int D>
+__device__ __forceinline__ void columns_times(f32x16 (&acc)[D / 32], uint32_t piece, const TrReads<D, true> &reads, const Parts (&b)[2], bool here0, bool here1) {
+  uint32_t lo[D / 32], hi[D / 32];
+  reads.get(lo, hi);
+  auto fetch = [&](int mt, int ks) {
+    Parts f;
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+      f.p[p] = tr_fragment<bf16>(lo[mt] + piece + p * Ring<D>::PLANE + ks * (16 * 2 * D), hi[mt] + piece + p * Ring<D>::PLANE + ks * (16 * 2 * D) + 4 * 2 * D);
+    return f;
+  };
+  auto none = [] {
+    f32x16 v;
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = 0.f;
+    return v;
+  };
+  if constexpr (WHOLE) {
+#pragma unroll
+    for (int mt = 0; mt < D / 32; mt++)
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        const f32x16 sum = whole_parts_product(fetch(mt, ks), b[ks], acc[mt]);
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[mt][i] = (ks ? here1 : here0) ? sum[i] : acc[mt][i];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  } else if constexpr (TIGHT) {
+#pragma unroll
+    for (int mt = 0; mt < D / 32; mt++) {
+      f32x16 small = none();
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        const Parts f = fetch(mt, ks);
+        small = mma(f.p[2], b[ks].p[0], small);
+        acc[mt] = mma(f.p[0], b[ks].p[1], acc[mt]);
+        small = mma(f.p[1], b[ks].p[1], small);
+        acc[mt] = mma(f.p[0], b[ks].p[0], acc[mt]);
+        small = mma(f.p[0], b[ks].p[2], small);
+        small = mma(f.p[1], b[ks].p[0], small);
+        __builtin_amdgcn_sched_barrier(0);              // (nothing is fetched further ahead)
+      }
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[mt][i] += small[i];
+    }
+  } else {
+#pragma unroll
+    for (int mt = 0; mt < D / 32; mt += 2) {
+      f32x16 sum[2] = {none(), none()};
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        const Parts f[2] = {fetch(mt, ks), fetch(mt + 1, ks)};
+#pragma unroll
+        for (int t = 0; t < 6; t++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) sum[j] = mma(f[j].p[t == 0 ? 2 : t == 1 || t == 3 ? 1 : 0], b[ks].p[t == 1 || t == 4 ? 1 : t == 2 ? 2 : 0], sum[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[mt + j][i] += sum[j][i];
+    }
+  }
+}
+
+// key-padding value -> addend of the logits (softmax.py:104-106, 122-124), which are in the log2 domain and rounded to fp32 before the row's
+// reference m is taken off, as the softmax operator does it (so that a padding value of -1e9 leaves nothing of a score).
+// (Finite values stay finite: the lowest one is a usual padding value, and a row of nothing else has equal shares.)
+__device__ __forceinline__ float pad_term(float v, int mul) {
+  const float t = v * kLog2e;
+  return mul ? (v == 0.f ? -INFINITY : 0.f) : fabsf(v) < INFINITY && fabsf(t) == INFINITY ? copysignf(3.402823466e38f, v) : t;
+}
+// The work of a workgroup.  The tables have the long lines (columns) of four heads at a time first; from eight such groups on each XCD takes
+// its own ones, so that their rows meet in its L2.  Fewer groups would leave the XCDs that begin in the middle of one with its short lines alone: they
+// are dealt in turn.
+__device__ __forceinline__ int64_t place(const F32Args &a, int64_t n) {
+  return a.Z * a.H >= 8 * kHeadsTogether ? xcd_remap(blockIdx.x, n) : (int64_t)blockIdx.x;
+}
+
+// the flags of a head: is one of n set?  (in this lane; its first one is fetched before any is looked at)
+__device__ __forceinline__ int32_t flags_of(const int32_t *f, int64_t zh, int64_t n, int lane) {
+  int32_t set = f[zh * n + (lane < n ? lane : 0)];
+  for (int64_t i = lane + 64; i < n; i += 64) set |= f[zh * n + i];
+  return set;
+}
+
+// the wavefront's sixteen rows of a piece (its group), three planes
+template <int D> struct PieceLoad {
+  static constexpr int COUNT = 3 * GroupLoad<D>::LW;
+  GroupLoad<D> g;
+  __device__ __forceinline__ void init(int lane) { g.init(3 * D, lane); }
+  __device__ __forceinline__ void issue(const char *planes, int pos, uint32_t lds, int wave) const {
+#pragma unroll
+    for (int p = 0; p < 3; p++) g.issue(planes + p * (D * 2), (uint32_t)pos, 3 * D * 2, lds + p * Ring<D>::PLANE + wave * (16 * D * 2));
+  }
+};
+
+template <int N> __device__ __forceinline__ void wait_barrier() {
+  BSP_WAIT_VM(N);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The walk over the tiles of a line.  Each tile is two pieces, used one after the other: first(slot, n) with x in LDS, then second(slot, n) with
+// y.  Piece after piece goes round the three slots, so that two are on their way while one is used.  issue_x / issue_y(n, slot) ask for them
+// (NX / NY vector-memory operations a wavefront); those of the first tile (slots 0 and 1) are on their way when the walk begins.
+template <int NX, int NY, class IX, class IY, class F1, class F2> __device__ __forceinline__ void walk(int tiles, IX &&issue_x, IY &&issue_y, F1 &&first, F2 &&second) {
+  int a = 0, b = 1, c = 2;                              // the slots of this piece, the next and the one after it
+  for (int n = 0; n < tiles; n++) {
+    wait_barrier<NY>();                                 // x is here, and everybody is done with the piece before it
+    if (n + 1 < tiles) issue_x(n + 1, c);
+    first(a, n);
+    if (n + 1 < tiles) wait_barrier<NX>();
+    else wait_barrier<0>();
+    if (n + 1 < tiles) issue_y(n + 1, a);
+    second(b, n);
+    const int was = b;
+    b = a; a = c; c = was;
+  }
+}
+// ... where x is used again beside y: y can only be asked for when its tile begins (and only x of the first tile is on its way)
+template <int NX, class IX, class IY, class F1, class F2> __device__ __forceinline__ void walk_x_twice(int tiles, IX &&issue_x, IY &&issue_y, F1 &&first, F2 &&second) {
+  int x = 0, y = 1, free = 2;
+  for (int n = 0; n < tiles; n++) {
+    wait_barrier<0>();                                  // x of this tile is here; everybody is done with the tile before
+    issue_y(n, y);
+    if (n + 1 < tiles) issue_x(n + 1, free);
+    first(x, n);
+    if (n + 1 < tiles) wait_barrier<NX>();
+    else wait_barrier<0>();
+    second(x, y, n);
+    const int was = x;
+    x = free; free = y; y = was;
+  }
+}
+
+// 32 rows of D sums (as store_32_rows) to LDS rows of D + 4 and from there to whole rows in memory, the first sixteen from lo on, the others from hi
+template <int D> __device__ __forceinline__ void store_32_f32(float *stage, float *lo, float *hi, int64_t ld, const f32x16 (&acc)[D / 32], int lane) {
+#pragma unroll
+  for (int mt = 0; mt < D / 32; mt++)
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      *reinterpret_cast<f32x4 *>(stage + (lane & 31) * (D + 4) + 32 * mt + 8 * g + 4 * (lane >> 5)) = f32x4{acc[mt][4 * g], acc[mt][4 * g + 1], acc[mt][4 * g + 2], acc[mt][4 * g + 3]};
+  __builtin_amdgcn_wave_barrier();                      // (the LDS operations of one wavefront complete in order)
+  constexpr int CPR = D / 4, RPS = 64 / CPR;
+#pragma unroll
+  for (int i = 0; i < 32 / RPS; i++) {
+    const int r = i * RPS + lane / CPR, c = 4 * (lane % CPR);
+    float *dst = (i * RPS < 16 ? lo + (int64_t)r * ld : hi + (int64_t)(r - 16) * ld) + c;
+    *reinterpret_cast<f32x4 *>(dst) = *reinterpret_cast<const f32x4 *>(stage + r * (D + 4) + c);
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+// sums of one wavefront to another through LDS: lane by lane
+template <int D> __device__ __forceinline__ void put_sums(float *to, const f32x16 (&acc)[D / 32], int lane) {
+#pragma unroll
+  for (int mt = 0; mt < D / 32; mt++)
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      *reinterpret_cast<f32x4 *>(to + ((mt * 4 + g) * 64 + lane) * 4) = f32x4{acc[mt][4 * g], acc[mt][4 * g + 1], acc[mt][4 * g + 2], acc[mt][4 * g + 3]};
+}
+template <int D, class F> __device__ __forceinline__ void take_sums(const float *from, f32x16 (&acc)[D / 32], int lane, F &&add) {
+#pragma unroll
+  for (int mt = 0; mt < D / 32; mt++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(from + ((mt * 4 + g) * 64 + lane) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[mt][4 * g + e] = add(acc[mt][4 * g + e], v[e]);
+    }
+}
+
+// the lane's row of an operand that stays in registers, from the planes
+template <int D> __device__ __forceinline__ void load_parts(Parts (&f)[D / 16], const bf16 *row) {
+#pragma unroll
+  for (int s = 0; s < D / 16; s++)
+#pragma unroll
+    for (int p = 0; p < 3; p++) f[s].p[p] = *reinterpret_cast<const bf16x8 *>(row + p * D + 16 * s);
+}
+
+// ... from a piece in LDS: its row r
+template <int D> __device__ __forceinline__ void own_parts(Parts (&f)[D / 16], const unsigned char *piece, int r, int half) {
+#pragma unroll
+  for (int s = 0; s < D / 16; s++)
+#pragma unroll
+    for (int p = 0; p < 3; p++) f[s].p[p] = *reinterpret_cast<const bf16x8 *>(piece + p * Ring<D>::PLANE + quad_offset<D>(r, 2 * s + half));
+}
+// ... from the operand itself, fp32
+template <int D> __device__ __forceinline__ void fetch_row(f32x4 (&v)[D / 8], const float *row) {
+#pragma unroll
+  for (int s = 0; s < D / 16; s++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) v[2 * s + j] = *reinterpret_cast<const f32x4 *>(row + 16 * s + 4 * j);
+}
+// its parts; those of the steps s that are `mine` also to the planes row `out` unless NULL.  -> does it (in this lane) hold a value that is
+// not below kLargest?
+template <int D> __device__ __forceinline__ int take_parts(Parts (&f)[D / 16], const f32x4 (&v)[D / 8], bf16 *out, int mine) {
+  int large = 0;
+#pragma unroll
+  for (int s = 0; s < D / 16; s++) {
+    float e[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      e[j] = v[2 * s + (j >> 2)][j & 3];
+      large |= !(fabsf(e[j]) < kLargest);
+    }
+    f[s] = split8<true>(e);
+    if (out != nullptr && (s & 1) == mine) {
+#pragma unroll
+      for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8 *>(out + p * D + 16 * s) = f[s].p[p];
+    }
+  }
+  return large;
+}
+
+// ---- planes ----
+struct PlaneArgs {
+  const float *x[2];
+  bf16 *planes[2];
+  int32_t *flags[2];
+  int64_t sz[2], sh[2], ld[2];
+  int chunks, H;                       // pieces of 64 rows of a head; heads of a batch
+  uint32_t per_tensor;                 // workgroups
+};
+template <int D> __global__ void __launch_bounds__(256) k_attn32_planes(PlaneArgs a) {
+  const int t = blockIdx.x >= a.per_tensor;
+  const uint32_t wg = blockIdx.x - t * a.per_tensor;
+  const Quotient head(wg, a.chunks), zh(head.q, a.H);
+  const float *x = a.x[t] + zh.q * a.sz[t] + zh.r * a.sh[t] + (int64_t)head.r * 64 * a.ld[t];
+  bf16 *to = a.planes[t] + (int64_t)wg * (64 * 3 * D);
+  int large = 0;
+  constexpr int PER = 64 * D / 8 / 256;
+  f32x4 v[PER][2];
+#pragma unroll
+  for (int i = 0; i < PER; i++) {
+    const int c = threadIdx.x + 256 * i, row = c / (D / 8), col = 8 * (c % (D / 8));
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(x + row * a.ld[t] + col);
+    v[i][0] = src[0]; v[i][1] = src[1];
+  }
+#pragma unroll
+  for (int i = 0; i < PER; i++) {
+    const int c = threadIdx.x + 256 * i, row = c / (D / 8), col = 8 * (c % (D / 8));
+    float e[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      e[j] = v[i][j >> 2][j & 3];
+      large |= !(fabsf(e[j]) < kLargest);
+    }
+    const Parts s = split8<true>(e);
+#pragma unroll
+    for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8 *>(to + row * (3 * D) + p * D + col) = s.p[p];
+  }
+  const int any = __syncthreads_or(large);
+  if (threadIdx.x == 0) a.flags[t][wg] = any;
+}
+
+// ---- forward ----
+template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) k_attn32_fwd(F32Args a) {
+  typedef Ring<D> R;
+  constexpr int MT = D / 32, NK = PieceLoad<D>::COUNT + (KPM ? 1 : 0);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  float *side = reinterpret_cast<float *>(smem + 3 * R::PIECE);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, half = lane >> 5, rh = wave & 1, kh = wave >> 1;       // the wavefront's rows and columns of a tile
+  const int64_t wg = place(a, (int64_t)a.Z * a.H * a.R);
+  int line, zh;
+  line_of(wg, a, line, zh);
+  const int h = zh % a.H, z = zh / a.H;
+  const table_ptr lut = as_table(a.lut);
+  const int tiles = lut[2 * (h * a.R + line)];
+  const table_ptr core = lut + lut[2 * (h * a.R + line) + 1];
+  const int64_t row = (int64_t)line * 64 + 32 * rh + l32;
+  f32x16 o[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) o[mt][i] = 0.f;
+  float m = -INFINITY, l = 0.f;
+  int rows_seen = 0;
+  bf16 *q_out = a.planes_out ? a.planes_out + (zh * a.rows + row) * (3 * D) + 8 * half : nullptr;
+  auto put_flag = [&](int large) {
+    const bool any = __builtin_amdgcn_ballot_w64(large != 0);
+    if (q_out != nullptr && kh == 0 && lane == 0) a.flags_out[(zh * a.rows + row) / 32] = any;
+  };
+
+  if (tiles > 0) {
+    Parts xq[D / 16];
+    const float *q_row = reinterpret_cast<const float *>(a.q) + z * a.q_sz + h * a.q_sh + row * a.q_ld + 8 * half;
+    const float sc = a.scale * kLog2e;
+    const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D));
+    const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D));
+    const char *pkpm = reinterpret_cast<const char *>(reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz);
+    PieceLoad<D> load;
+    load.init(lane);
+    RowReads<D, true> rows_k;
+    TrReads<D, true> tr_v;
+    rows_k.init(32 * kh, lane);
+    tr_v.init(lds_address(smem), 32 * kh, lane);
+    const float *kp_lane = side + (2 * kh + ((lane >> 3) & 1)) * 128 + 8 * half + (lane & 7);   // value i of the lane comes from lane i of each sixteen
+    // the table runs a tile ahead of the loads
+    int pos_next = core[wave], pos = 0, bits_next = 0;
+    auto issue_k = [&](int n, int slot) {
+      pos = pos_next;
+      load.issue(pk, pos, lds_address(smem) + slot * R::PIECE, wave);
+      if constexpr (KPM) load_to_lds<4>(pkpm, (uint32_t)(pos + (lane & 15)) * 4u, 0, lds_address(side) + slot * R::SIDE + wave * 512);
+      pos_next = core[kEntry * (n + 1 < tiles ? n + 1 : n) + wave];
+    };
+    auto issue_v = [&](int n, int slot) {
+      load.issue(pv, pos, lds_address(smem) + slot * R::PIECE, wave);
+      bits_next = core[kEntry * n + 4];
+    };
+    float e[16];
+    auto run = [&](auto whole) {
+      constexpr bool W = decltype(whole)::value;
+      int here = 0;
+      walk<NK, PieceLoad<D>::COUNT>(tiles, issue_k, issue_v,
+        [&](int x, int) {
+          f32x16 s;
+#pragma unroll
+          for (int i = 0; i < 16; i++) s[i] = 0.f;
+          s = rows_times<W, false, D>(smem + x * R::PIECE, rows_k, xq, q_row, s);
+          here = bits_next >> (8 * rh + 2 * kh);
+          rows_seen |= here & 0x33;
+          const float kp = KPM ? pad_term(kp_lane[x * (R::SIDE / 4)], a.kpm_mul) : 0.f;
+          const int mine = here >> ((lane >> 4) & 1) * 4;
+          const bool here0 = mine & 1, here1 = mine & 2;        // pieces without a block take no part in the row
+          for_16<0>([&](auto ic) { s[decltype(ic)::value] = KPM ? fmaf(s[decltype(ic)::value], sc, row_bcast<decltype(ic)::value>(kp)) : s[decltype(ic)::value] * sc; });
+          float sum;
+          auto exponentials = [&]() {
+            const float ms = m == -INFINITY ? 0.f : m, off[2] = {here0 ? ms : INFINITY, here1 ? ms : INFINITY};
+            sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+              e[i] = __builtin_amdgcn_exp2f(s[i] - off[i >> 3]);
+              if constexpr (W) e[i] = (i < 8 ? here0 : here1) ? e[i] : 0.f;            // (the score may be anything there)
+              sum += e[i];
+            }
+          };
+          exponentials();
+          if (__builtin_amdgcn_ballot_w64(!(sum <= 8192.f) || m == -INFINITY)) {      // (also where an exponential overflowed)
+            float top = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 16; i++) top = fmaxf(top, (i < 8 ? here0 : here1) ? s[i] : -INFINITY);
+            const float mn = fmaxf(m, fmaxf(top, swap32(top))), f = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+            l *= f;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+              for (int i = 0; i < 16; i++) o[mt][i] *= f;
+            m = mn;
+            exponentials();
+          }
+          l += sum;
+        },
+        [&](int y, int) {
+          const Parts pf[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(e[0])), split8<W>(reinterpret_cast<const float (&)[8]>(e[8]))};
+          const int mine = here >> ((lane >> 4) & 1) * 4;
+          columns_times<W, false, D>(o, y * R::PIECE, tr_v, pf, mine & 1, mine & 2);
+        });
+    };
+    issue_k(0, 0);
+    issue_v(0, 1);
+    f32x4 q[D / 8];
+    fetch_row<D>(q, q_row);
+    int large = flags_of(a.fk, zh, a.keys / 64, lane) | flags_of(a.fv, zh, a.keys / 64, lane);
+    const int mine = take_parts<D>(xq, q, q_out, kh);
+    put_flag(mine);
+    large |= mine;
+    if (__builtin_amdgcn_ballot_w64(large != 0)) run(Const<1>{});
+    else run(Const<0>{});
+  } else if (q_out != nullptr) {                        // (the column kernel multiplies nothing of these rows, but takes the head's flags)
+    Parts none[D / 16];
+    f32x4 q[D / 8];
+    fetch_row<D>(q, reinterpret_cast<const float *>(a.q) + z * a.q_sz + h * a.q_sh + row * a.q_ld + 8 * half);
+    put_flag(take_parts<D>(none, q, q_out, kh));
+  }
+
+  // the two halves of the columns, each with its own reference m
+  l += swap32(l);
+  float *other = reinterpret_cast<float *>(smem) + rh * (16 * MT * 64 + 256);
+  wait_barrier<0>();                                    // the ring is free
+  if (kh) {
+    put_sums<D>(other, o, lane);
+    other[16 * MT * 64 + lane] = m;
+    other[16 * MT * 64 + 64 + lane] = l;
+    reinterpret_cast<int *>(other)[16 * MT * 64 + 128 + lane] = rows_seen;
+  }
+  wait_barrier<0>();
+  if (!kh) {
+    const float m1 = other[16 * MT * 64 + lane], l1 = other[16 * MT * 64 + 64 + lane];
+    rows_seen |= reinterpret_cast<const int *>(other)[16 * MT * 64 + 128 + lane];
+    const float top = fmaxf(m, m1), ms = top == -INFINITY ? 0.f : top, f0 = __builtin_amdgcn_exp2f(m - ms), f1 = __builtin_amdgcn_exp2f(m1 - ms);
+    const float sum = l * f0 + l1 * f1;
+    const bool any_block = (rows_seen >> 4 * ((lane >> 4) & 1)) & 15;
+    const float inv = any_block ? 1.f / sum : 0.f;      // masked everywhere: 0 * inf = NaN, as the softmax operator gives; no block at all: zeros
+    take_sums<D>(other, o, lane, [&](float a0, float a1) { return (a0 * f0 + a1 * f1) * inv; });
+    if (a.lse != nullptr && half == 0) {
+      float *to = a.lse + zh * a.row_sh + row;
+      to[0] = ms;
+      to[a.rest] = inv;
+    }
+  }
+  wait_barrier<0>();
+  if (!kh) {
+    float *po = reinterpret_cast<float *>(a.o) + z * a.o_sz + h * a.o_sh + ((int64_t)line * 64 + 32 * rh) * a.o_ld;
+    store_32_f32<D>(reinterpret_cast<float *>(smem) + rh * 32 * (D + 4), po, po + 16 * a.o_ld, a.o_ld, o, lane);
+  }
+}
+
+// ---- backward, rows: dq and -delta ----
+template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) k_attn32_bwd_rows(F32Args a) {
+  typedef Ring<D> R;
+  constexpr int MT = D / 32, NK = PieceLoad<D>::COUNT + (KPM ? 1 : 0);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  float *side = reinterpret_cast<float *>(smem + 3 * R::PIECE);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, half = lane >> 5, rh = wave & 1, kh = wave >> 1;
+  const int64_t wg = place(a, (int64_t)a.Z * a.H * a.R);
+  int line, zh;
+  line_of(wg, a, line, zh);
+  const int h = zh % a.H, z = zh / a.H;
+  const table_ptr lut = as_table(a.lut);
+  const int tiles = lut[2 * (h * a.R + line)];
+  const table_ptr core = lut + lut[2 * (h * a.R + line) + 1];
+  const int64_t row = (int64_t)line * 64 + 32 * rh + l32;
+  f32x16 dq[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) dq[mt][i] = 0.f;
+  // the rows' do: its parts, also for the column kernel, and delta
+  const float *do_row = reinterpret_cast<const float *>(a.d_o) + z * a.do_sz + h * a.do_sh + row * a.do_ld + 8 * half;
+  const float *o_row = reinterpret_cast<const float *>(a.o_in) + z * a.oin_sz + h * a.oin_sh + row * a.oin_ld + 8 * half;
+  auto sums = [&](const f32x4 (&d)[D / 8], const f32x4 (&o)[D / 8]) {
+    float delta = 0.f;
+#pragma unroll
+    for (int s = 0; s < D / 8; s++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) delta = fmaf(d[s][i], o[s][i], delta);
+    delta += swap32(delta);
+    if (a.delta != nullptr && half == 0 && kh == 0) a.delta[zh * a.rows + row] = -delta;
+    return delta;
+  };
+  bf16 *do_out = a.planes_out ? a.planes_out + (zh * a.rows + row) * (3 * D) + 8 * half : nullptr;
+  auto put_flag = [&](int large) {
+    const bool any = __builtin_amdgcn_ballot_w64(large != 0);
+    if (do_out != nullptr && kh == 0 && lane == 0) a.flags_out[(zh * a.rows + row) / 32] = any;
+  };
+  if (tiles == 0) {
+    Parts none[D / 16];
+    f32x4 g[D / 8], o[D / 8];
+    fetch_row<D>(g, do_row);
+    fetch_row<D>(o, o_row);
+    sums(g, o);
+    put_flag(take_parts<D>(none, g, do_out, kh));
+  }
+
+  if (tiles > 0) {
+    Parts xq[D / 16], xo[D / 16];
+    const bf16 *q_row = reinterpret_cast<const bf16 *>(a.q) + (zh * a.rows + row) * (3 * D) + 8 * half;
+    const float sc = a.scale * kLog2e, m = a.lse[zh * a.row_sh + row];
+    const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D));
+    const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D));
+    const char *pkpm = reinterpret_cast<const char *>(reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz);
+    PieceLoad<D> load;
+    load.init(lane);
+    RowReads<D, true> rows;
+    TrReads<D, true> tr;
+    rows.init(32 * kh, lane);
+    tr.init(lds_address(smem), 32 * kh, lane);
+    const float *kp_lane = side + (2 * kh + ((lane >> 3) & 1)) * 128 + 8 * half + (lane & 7);
+    int pos_next = core[wave], pos = 0, bits_next = 0;   // (as in the forward kernel)
+    auto issue_v = [&](int n, int slot) {
+      pos = pos_next;
+      load.issue(pv, pos, lds_address(smem) + slot * R::PIECE, wave);
+      pos_next = core[kEntry * (n + 1 < tiles ? n + 1 : n) + wave];
+    };
+    auto issue_k = [&](int n, int slot) {
+      load.issue(pk, pos, lds_address(smem) + slot * R::PIECE, wave);
+      if constexpr (KPM) load_to_lds<4>(pkpm, (uint32_t)(pos + (lane & 15)) * 4u, 0, lds_address(side) + slot * R::SIDE + wave * 512);
+      bits_next = core[kEntry * n + 4];
+    };
+    issue_v(0, 0);
+    issue_k(0, 1);
+    f32x4 g[D / 8], o[D / 8];
+    fetch_row<D>(g, do_row);
+    fetch_row<D>(o, o_row);
+    load_parts<D>(xq, q_row);
+    int large = a.fq[(zh * a.rows + row) / 32] | flags_of(a.fk, zh, a.keys / 64, lane) | flags_of(a.fv, zh, a.keys / 64, lane);
+    const float delta = sums(g, o);
+    const int mine = take_parts<D>(xo, g, do_out, kh);
+    put_flag(mine);
+    large |= mine;
+    f32x16 dp;
+    auto run = [&](auto whole) {
+      constexpr bool W = decltype(whole)::value;
+      int here = 0;
+      walk<PieceLoad<D>::COUNT, NK>(tiles, issue_v, issue_k,
+        [&](int x, int) {
+          here = bits_next >> (8 * rh + 2 * kh);
+#pragma unroll
+          for (int i = 0; i < 16; i++) dp[i] = 0.f;
+          dp = rows_times<W, false, D>(smem + x * R::PIECE, rows, xo, do_row, dp);
+        },
+        [&](int y, int) {
+          f32x16 s;
+#pragma unroll
+          for (int i = 0; i < 16; i++) s[i] = 0.f;
+          s = rows_times<W, false, D>(smem + y * R::PIECE, rows, xq, q_row, s);
+          const float kp = KPM ? pad_term(kp_lane[y * (R::SIDE / 4)], a.kpm_mul) : 0.f;
+          const int mine = here >> ((lane >> 4) & 1) * 4;
+          float e[16];                                  // (1 / l of the row comes last, on dq)
+          for_16<0>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            e[i] = __builtin_amdgcn_exp2f((KPM ? fmaf(s[i], sc, row_bcast<i>(kp)) : s[i] * sc) - m) * (dp[i] - delta);
+          });
+          if ((here & 0x33) != 0x33) {                  // pieces without a block
+#pragma unroll
+            for (int i = 0; i < 16; i++) e[i] = mine >> (i >> 3) & 1 ? e[i] : 0.f;
+          }
+          const Parts df[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(e[0])), split8<W>(reinterpret_cast<const float (&)[8]>(e[8]))};
+          columns_times<W, false, D>(dq, y * R::PIECE, tr, df, mine & 1, mine & 2);
+        });
+    };
+    if (__builtin_amdgcn_ballot_w64(large != 0)) run(Const<1>{});
+    else run(Const<0>{});
+  }
+  float *other = reinterpret_cast<float *>(smem) + rh * (16 * MT * 64);
+  wait_barrier<0>();
+  if (kh) put_sums<D>(other, dq, lane);
+  wait_barrier<0>();
+  if (!kh) {
+    const float last = a.lse[zh * a.row_sh + a.rest + row] * a.scale;
+    take_sums<D>(other, dq, lane, [&](float a0, float a1) { return (a0 + a1) * last; });
+  }
+  wait_barrier<0>();
+  if (!kh) {
+    float *po = reinterpret_cast<float *>(a.o) + z * a.o_sz + h * a.o_sh + ((int64_t)line * 64 + 32 * rh) * a.o_ld;
+    store_32_f32<D>(reinterpret_cast<float *>(smem) + rh * 32 * (D + 4), po, po + 16 * a.o_ld, a.o_ld, dq, lane);
+  }
+}
+
+// ---- backward, columns: dk and dv (work items as in attention_bwd.hip) ----
+template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) k_attn32_bwd_cols(F32Args a) {
+  typedef Ring<D> R;
+  constexpr int MT = D / 32, NX = PieceLoad<D>::COUNT + 2;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  float *side = reinterpret_cast<float *>(smem + 3 * R::PIECE);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, half = lane >> 5, kh = wave & 1, rh = wave >> 1;       // the wavefront's keys and rows of a tile
+  const int64_t work = place(a, (int64_t)a.Z * a.R * a.sub), wg = work / a.sub;     // the pieces of an item side by side
+  const bool in_turn = a.Z * a.H < 8 * kHeadsTogether;  // (then the long items of all batches come first)
+  const int item = (int)(in_turn ? wg / a.Z : wg % a.R), z = (int)(in_turn ? wg % a.Z : wg / a.R);
+  const table_ptr lut = as_table(a.lut), head = lut + 12 * item;
+  int tiles = head[0], slot_no = head[4];
+  const int h = head[2];
+  table_ptr core = lut + head[1];
+  if (a.sub > 1) {
+    const int piece = (int)(work % a.sub);
+    if (slot_no < 0) {                                  // not a part of a long column: one piece
+      if (piece) return;
+    } else {
+      const int from = (int)((int64_t)tiles * piece / a.sub), upto = (int)((int64_t)tiles * (piece + 1) / a.sub);
+      core += kEntry * from;
+      tiles = upto - from;
+      slot_no = slot_no * a.sub + piece;
+    }
+  }
+  const int64_t key_lo = head[8 + 2 * kh], key_hi = head[8 + 2 * kh + 1], zh = (int64_t)z * a.H + h;
+  f32x16 dk[MT], dv[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) dk[mt][i] = dv[mt][i] = 0.f;
+
+  if (tiles > 0) {
+    const int64_t key = (l32 < 16 ? key_lo : key_hi) + (l32 & 15);
+    Parts xk[D / 16], xv[D / 16];
+    const bf16 *k_row = reinterpret_cast<const bf16 *>(a.k) + (zh * a.keys + key) * (3 * D) + 8 * half;
+    const bf16 *v_row = reinterpret_cast<const bf16 *>(a.v) + (zh * a.keys + key) * (3 * D) + 8 * half;
+    const float sc = a.scale * kLog2e, kp = KPM ? pad_term((reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz)[key], a.kpm_mul) : 0.f;
+    const char *pq = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.q) + zh * a.rows * (3 * D));
+    const char *pdo = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.d_o) + zh * a.rows * (3 * D));
+    const char *pstat = reinterpret_cast<const char *>(a.lse + zh * a.row_sh), *pdelta = reinterpret_cast<const char *>(a.delta + zh * a.rows);
+    const uint32_t to_inv = lane & 16 ? (uint32_t)a.rest * 4u : 0u;
+    PieceLoad<D> load;
+    load.init(lane);
+    RowReads<D, true> rows;
+    TrReads<D, true> tr;
+    rows.init(32 * rh, lane);
+    tr.init(lds_address(smem), 32 * rh, lane);
+    const float *rv = side + 2 * rh * 128 + 8 * half;   // per group of sixteen rows: m (16 floats), 1 / l (16), 32 more; -delta
+    int pos_next = core[wave], pos = 0, bits = 0, bits_next = core[4];
+    auto issue_q = [&](int n, int slot) {
+      pos = pos_next;
+      load.issue(pq, pos, lds_address(smem) + slot * R::PIECE, wave);
+      const uint32_t at = (uint32_t)(pos + (lane & 15)) * 4u, to = lds_address(side) + slot * R::SIDE + wave * 512;
+      load_to_lds<4>(pstat, at + to_inv, 0, to);
+      load_to_lds<4>(pdelta, at, 0, to + 256);
+      pos_next = core[kEntry * (n + 1 < tiles ? n + 1 : n) + wave];
+    };
+    auto issue_do = [&](int n, int slot) {              // (pos is still that of tile n: the next tile's q is asked for after it)
+      load.issue(pdo, pos, lds_address(smem) + slot * R::PIECE, wave);
+      bits = bits_next;
+      bits_next = core[kEntry * (n + 1 < tiles ? n + 1 : n) + 4];
+    };
+    float p[16];
+    auto run = [&](auto whole) {
+      constexpr bool W = decltype(whole)::value;
+      if constexpr (!W) {
+        own_parts<D>(xk, smem + R::PIECE, 32 * kh + l32, half);
+        own_parts<D>(xv, smem + 2 * R::PIECE, 32 * kh + l32, half);
+      }
+      int here = 0;
+      walk_x_twice<NX>(tiles, issue_q, issue_do,
+        [&](int x, int) {
+          f32x16 s;
+#pragma unroll
+          for (int i = 0; i < 16; i++) s[i] = 0.f;
+          s = rows_times<W, true, D>(smem + x * R::PIECE, rows, xk, k_row, s);
+          here = bits >> (2 * kh + 8 * rh);
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            const float *at = rv + x * (R::SIDE / 4) + (g >> 1) * 128 + 4 * (g & 1);
+            const f32x4 m = *reinterpret_cast<const f32x4 *>(at), inv = *reinterpret_cast<const f32x4 *>(at + 16);
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[4 * g + i] = __builtin_amdgcn_exp2f((KPM ? fmaf(s[4 * g + i], sc, kp) : s[4 * g + i] * sc) - m[i]) * inv[i];
+          }
+          if ((here & 0x33) != 0x33) {                  // pieces without a block (a row that is masked everywhere has NaN here, which its other keys must not take up)
+            const int mine = here >> ((lane >> 4) & 1);
+#pragma unroll
+            for (int i = 0; i < 16; i++) p[i] = mine >> 4 * (i >> 3) & 1 ? p[i] : 0.f;
+          }
+        },
+        [&](int x, int y, int) {
+          const int mine = here >> ((lane >> 4) & 1);
+          f32x16 dp;
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            const f32x4 nd = *reinterpret_cast<const f32x4 *>(rv + x * (R::SIDE / 4) + (g >> 1) * 128 + 4 * (g & 1) + 64);
+#pragma unroll
+            for (int i = 0; i < 4; i++) dp[4 * g + i] = nd[i];
+          }
+          dp = rows_times<W, false, D>(smem + y * R::PIECE, rows, xv, v_row, dp);
+          float e[16];
+#pragma unroll
+          for (int i = 0; i < 16; i++) e[i] = p[i] * dp[i];
+          if ((here & 0x33) != 0x33)
+#pragma unroll
+            for (int i = 0; i < 16; i++) e[i] = mine >> 4 * (i >> 3) & 1 ? e[i] : 0.f;
+          {
+            const Parts pf[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(p[0])), split8<W>(reinterpret_cast<const float (&)[8]>(p[8]))};
+            columns_times<W, true, D>(dv, y * R::PIECE, tr, pf, mine & 1, mine & 16);
+          }
+          const Parts df[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(e[0])), split8<W>(reinterpret_cast<const float (&)[8]>(e[8]))};
+          columns_times<W, true, D>(dk, x * R::PIECE, tr, df, mine & 1, mine & 16);
+        });
+    };
+    issue_q(0, 0);
+    // the column's own rows through the slots that are free yet: fetched by whole lines
+    load.issue(reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D)), head[8 + wave], lds_address(smem) + R::PIECE, wave);
+    load.issue(reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D)), head[8 + wave], lds_address(smem) + 2 * R::PIECE, wave);
+    const int large = flags_of(a.fq, zh, a.rows / 32, lane) | flags_of(a.fdo, zh, a.rows / 32, lane) | flags_of(a.fk, zh, a.keys / 64, lane) | flags_of(a.fv, zh, a.keys / 64, lane);
+    wait_barrier<0>();
+    if (__builtin_amdgcn_ballot_w64(large != 0)) run(Const<1>{});
+    else run(Const<0>{});
+  }
+  float *other = reinterpret_cast<float *>(smem) + kh * (2 * 16 * MT * 64);
+  wait_barrier<0>();
+  if (rh) {
+    put_sums<D>(other, dk, lane);
+    put_sums<D>(other + 16 * MT * 64, dv, lane);
+  }
+  wait_barrier<0>();
+  if (!rh) {
+    take_sums<D>(other, dk, lane, [&](float a0, float a1) { return (a0 + a1) * a.scale; });
+    take_sums<D>(other + 16 * MT * 64, dv, lane, [&](float a0, float a1) { return a0 + a1; });
+  }
+  wait_barrier<0>();
+  if (rh) return;
+  if (slot_no >= 0) {                                   // a part of a long column: its sums to its slot [dk, dv][64 keys][D]
+    float *ws = a.partial + ((int64_t)z * a.n_slots * a.sub + slot_no) * (2 * 64 * D) + (32 * kh + l32) * D + 4 * half;
+#pragma unroll
+    for (int j = 0; j < MT; j++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        *reinterpret_cast<f32x4 *>(ws + 32 * j + 8 * g) = f32x4{dk[j][4 * g], dk[j][4 * g + 1], dk[j][4 * g + 2], dk[j][4 * g + 3]};
+        *reinterpret_cast<f32x4 *>(ws + 64 * D + 32 * j + 8 * g) = f32x4{dv[j][4 * g], dv[j][4 * g + 1], dv[j][4 * g + 2], dv[j][4 * g + 3]};
+      }
+    return;
+  }
+  float *stage = reinterpret_cast<float *>(smem) + kh * 32 * (D + 4);
+  float *pdk = reinterpret_cast<float *>(a.o) + z * a.o_sz + h * a.o_sh, *pdv = reinterpret_cast<float *>(a.o2) + z * a.o2_sz + h * a.o2_sh;
+  store_32_f32<D>(stage, pdk + key_lo * a.o_ld, pdk + key_hi * a.o_ld, a.o_ld, dk, lane);
+  store_32_f32<D>(stage, pdv + key_lo * a.o2_ld, pdv + key_hi * a.o2_ld, a.o2_ld, dv, lane);
+}
+
+// dk and dv of the columns computed in parts: the slots of a column in order (split_lut as in attention_bwd.hip)
+template <int D> __global__ void __launch_bounds__(256) k_attn32_cols_sum(F32Args a) {
+  constexpr int WGS = 2 * 64 * D / 4 / 256;            // four values a thread
+  const int piece = blockIdx.x % WGS, col = (blockIdx.x / WGS) % a.n_split, z = (blockIdx.x / WGS) / a.n_split;
+  const table_ptr lut = as_table(a.split_lut) + 8 * col;
+  const int h = lut[0], first = lut[2] * a.sub, parts = lut[3] * a.sub;
+  const float *ws = a.partial + ((int64_t)z * a.n_slots * a.sub + first) * (2 * 64 * D);
+  const int g = piece * 256 + threadIdx.x, which = g / (16 * D), rem = g % (16 * D), key = rem / (D / 4), d4 = rem % (D / 4);
+  f32x4 sum = *reinterpret_cast<const f32x4 *>(ws + 4 * g);
+  for (int part = 1; part < parts; part++) {
+    const f32x4 v = *reinterpret_cast<const f32x4 *>(ws + (int64_t)part * (2 * 64 * D) + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; e++) sum[e] += v[e];
+  }
+  const int64_t pos = (key < 32 ? (key < 16 ? lut[4] : lut[5]) : (key < 48 ? lut[6] : lut[7])) + (key & 15);
+  float *dst = which ? reinterpret_cast<float *>(a.o2) + z * a.o2_sz + h * a.o2_sh + pos * a.o2_ld
+                     : reinterpret_cast<float *>(a.o) + z * a.o_sz + h * a.o_sh + pos * a.o_ld;
+  *reinterpret_cast<f32x4 *>(dst + 4 * d4) = sum;
+}
+
+// the kernels' LDS is more than a launch may ask for by default: raised once per device and kernel
+template <class K> int big_lds(K kernel, int bytes, std::atomic<uint64_t> &done) {
+  int dev = 0;
+  BSP_HIP_CHECK(hipGetDevice(&dev));
+  const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
+  if (bit && (done.load(std::memory_order_acquire) & bit)) return BSP_OK;
+  BSP_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  done.fetch_or(bit, std::memory_order_release);
+  return BSP_OK;
+}
+
+template <int D, bool KPM, int WHICH> int launch(const F32Args &a, unsigned n_wg, hipStream_t st) {
+  static std::atomic<uint64_t> done{0};
+  void (*kernel)(F32Args) = WHICH == 0 ? k_attn32_fwd<D, KPM> : WHICH == 1 ? k_attn32_bwd_rows<D, KPM> : k_attn32_bwd_cols<D, KPM>;
+  const int rc = big_lds(kernel, Ring<D>::BYTES, done);
+  if (rc != BSP_OK) return rc;
+  hipLaunchKernelGGL(kernel, dim3(n_wg), dim3(256), Ring<D>::BYTES, st, a);
+  return BSP_OK;
+}
+template <int WHICH> int launch_d(const F32Args &a, int D, int64_t n_wg, hipStream_t st) {
+  if (D == 64) return a.kpm ? launch<64, true, WHICH>(a, (unsigned)n_wg, st) : launch<64, false, WHICH>(a, (unsigned)n_wg, st);
+  return a.kpm ? launch<128, true, WHICH>(a, (unsigned)n_wg, st) : launch<128, false, WHICH>(a, (unsigned)n_wg, st);
+}
+
+// planes of a tensor of n rows in all: [n][3][D] bf16, then its flags, at most one int for 32 rows; a multiple of 16 bytes
+inline int64_t plane_bytes(int64_t n, int D) { return n * 3 * D * 2 + (n / 32 * 4 + 15) / 16 * 16; }
+inline int32_t *flags_in(void *planes, int64_t n, int D) { return reinterpret_cast<int32_t *>(reinterpret_cast<char *>(planes) + n * 3 * D * 2); }
+
+// sizes, 16-byte alignment of pointers (NULL is aligned) and strides (n tensors: batch, head, row; multiples of 4 floats), rows that hold D
+int f32_check(const bsp_attention_f32_call &c, const void *const *ptrs, int n_ptrs, int n) {
+  if (c.Z <= 0 || c.H <= 0 || c.R <= 0 || c.keys <= 0 || c.keys % 64 || !c.planes) return BSP_ERR_ARG;
+  if (c.D != 64 && c.D != 128) return BSP_ERR_UNSUPPORTED;
+  for (int i = 0; i < n_ptrs; i++)
+    if (reinterpret_cast<uintptr_t>(ptrs[i]) & 15) return BSP_ERR_ARG;
+  for (int i = 0; i < 3 * n; i++)
+    if (c.strides[i] % 4 || (i % 3 == 2 && c.strides[i] < c.D)) return BSP_ERR_ARG;
+  const int64_t most = c.keys > (int64_t)c.R * 64 ? c.keys : (int64_t)c.R * 64;
+  // workgroups of a launch, and byte offsets within a head's planes, in 32 bits
+  return (int64_t)c.Z * c.H * c.R >= ((int64_t)1 << 31) || most * 3 * c.D * 2 >= ((int64_t)1 << 32) ? BSP_ERR_UNSUPPORTED : BSP_OK;
+}
+
+// what both directions take from the call: sizes, masks, the parts of the buffer of k, v and q
+F32Args f32_args(const bsp_attention_f32_call &c) {
+  F32Args a{};
+  a.Z = c.Z; a.H = c.H; a.R = c.R;
+  a.rows = (int64_t)c.R * 64; a.keys = c.keys;
+  a.lse = c.stats; a.rest = a.rows; a.row_sh = 2 * a.rows;
+  a.scale = c.scale;
+  a.kpm = c.kpm; a.kpm_sz = c.kpm_stride_z; a.kpm_mul = c.kpm_mul;
+  const int64_t n = (int64_t)c.Z * c.H * c.keys;
+  char *p = reinterpret_cast<char *>(c.planes);
+  a.k = p; a.fk = flags_in(p, n, c.D);
+  p += plane_bytes(n, c.D);
+  a.v = p; a.fv = flags_in(p, n, c.D);
+  p += plane_bytes(n, c.D);
+  a.q = p; a.fq = flags_in(p, (int64_t)c.Z * c.H * a.rows, c.D);
+  return a;
+}
+void take_strides(const int64_t *s, int64_t &z, int64_t &h, int64_t &row) { z = s[0]; h = s[1]; row = s[2]; }
+
+// Pieces of the parts of long columns.  A part is up to sixteen tiles, eight times as long as the short columns of the layouts that have
+// any, and takes 70 us: a launch whose parts do not fill the chip twice (two workgroups a CU) ends with them.  Every piece is a slot written
+// and read once more.  Module in fp32, 2 x 8 heads of 2048 positions, stride 128 of blocks of 32, 256 parts: @@
+int pieces(int64_t parts) { return parts == 0 ? 1 : parts >= 2048 ? 1 : parts > 128 ? 2 : 4; }
+
+}  // namespace
+}  // namespace bsp
+
+using namespace bsp;
+
+extern "C" int64_t bsp_attention_f32_bytes(int Z, int H, int64_t rows, int64_t keys, int D) {
+  const int64_t heads = (int64_t)Z * H;
+  return plane_bytes(heads * rows, D) + (keys ? 2 * plane_bytes(heads * keys, D) : 0);
+}
+extern "C" int64_t bsp_attention_f32_slots(int Z, int n_slots) { return (int64_t)Z * n_slots * pieces((int64_t)Z * n_slots); }
+
+extern "C" int bsp_attention_f32_fwd(const bsp_attention_f32_call *c, const float *q, const float *k, const float *v, float *o, void *stream) {
+  if (!c || !q || !k || !v || !o || !c->d_rows) return BSP_ERR_ARG;
+  const void *ptrs[] = {q, k, v, o, c->planes, c->stats, c->kpm};
+  const int rc = f32_check(*c, ptrs, 7, 4);
+  if (rc != BSP_OK) return rc;
+  F32Args a = f32_args(*c);
+  const int64_t heads = (int64_t)a.Z * a.H, per_tensor = heads * (a.keys / 64);
+  if (2 * per_tensor >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
+  PlaneArgs pl{};
+  pl.x[0] = k; pl.x[1] = v;
+  const void *const to[] = {a.k, a.v};
+  pl.chunks = (int)(a.keys / 64); pl.H = a.H; pl.per_tensor = (uint32_t)per_tensor;
+  for (int t = 0; t < 2; t++) {
+    pl.planes[t] = reinterpret_cast<bf16 *>(const_cast<void *>(to[t]));
+    pl.flags[t] = flags_in(pl.planes[t], heads * a.keys, c->D);
+    take_strides(c->strides + 3 * (t + 1), pl.sz[t], pl.sh[t], pl.ld[t]);
+  }
+  hipStream_t st = as_stream(stream);
+  if (c->D == 64) hipLaunchKernelGGL(k_attn32_planes<64>, dim3((unsigned)(2 * per_tensor)), dim3(256), 0, st, pl);
+  else hipLaunchKernelGGL(k_attn32_planes<128>, dim3((unsigned)(2 * per_tensor)), dim3(256), 0, st, pl);
+  if (c->stats) {
+    a.planes_out = reinterpret_cast<bf16 *>(const_cast<void *>(a.q));
+    a.flags_out = const_cast<int32_t *>(a.fq);
+  }
+  a.q = q;
+  take_strides(c->strides, a.q_sz, a.q_sh, a.q_ld);
+  a.o = o;
+  take_strides(c->strides + 9, a.o_sz, a.o_sh, a.o_ld);
+  a.lut = c->d_rows;
+  const int rl = launch_d<0>(a, c->D, heads * a.R, st);
+  if (rl != BSP_OK) return rl;
+  BSP_LAUNCH_CHECK();
+  return BSP_OK;
+}
+
+extern "C" int bsp_attention_f32_bwd(const bsp_attention_f32_call *c, const float *d_o, const float *o, float *dq, float *dk, float *dv, void *do_planes, float *neg_delta,
+                                     const int32_t *d_items, int n_items, float *partial, int n_slots, const int32_t *d_split, int n_split, void *stream) {
+  if (!c || !d_o || !o || !dq || !c->stats || !c->d_rows || (dk == nullptr) != (dv == nullptr) || (dk && (!do_planes || !neg_delta || !d_items))) return BSP_ERR_ARG;
+  if (n_slots < 0 || n_split < 0 || (n_slots > 0) != (n_split > 0) || (dk && n_slots > 0 && (!partial || !d_split))) return BSP_ERR_ARG;
+  const void *ptrs[] = {d_o, o, dq, dk, dv, do_planes, c->planes, c->stats, neg_delta, partial, c->kpm};
+  const int rc = f32_check(*c, ptrs, 11, dk ? 5 : 3);
+  if (rc != BSP_OK) return rc;
+  F32Args a = f32_args(*c);
+  a.sub = pieces((int64_t)a.Z * n_slots);
+  if (dk && (n_items < (int64_t)a.H * (a.keys / 64) || n_items > (int64_t)a.H * (a.keys / 64) + n_slots || (int64_t)a.Z * n_items * a.sub >= ((int64_t)1 << 31) ||
+             (int64_t)a.Z * n_split * 16 >= ((int64_t)1 << 31))) return BSP_ERR_ARG;
+  hipStream_t st = as_stream(stream);
+  const int64_t n = (int64_t)a.Z * a.H * a.rows;
+  a.d_o = d_o; a.o_in = o;
+  if (dk) {
+    a.planes_out = reinterpret_cast<bf16 *>(do_planes);
+    a.flags_out = flags_in(do_planes, n, c->D);
+    a.delta = neg_delta;
+  }
+  take_strides(c->strides, a.do_sz, a.do_sh, a.do_ld);
+  take_strides(c->strides + 3, a.oin_sz, a.oin_sh, a.oin_ld);
+  take_strides(c->strides + 6, a.o_sz, a.o_sh, a.o_ld);
+  a.o = dq; a.lut = c->d_rows;
+  int rl = launch_d<1>(a, c->D, (int64_t)a.Z * a.H * a.R, st);
+  if (rl != BSP_OK) return rl;
+  if (dk) {
+    a.d_o = do_planes; a.fdo = a.flags_out;
+    take_strides(c->strides + 9, a.o_sz, a.o_sh, a.o_ld);
+    take_strides(c->strides + 12, a.o2_sz, a.o2_sh, a.o2_ld);
+    a.o = dk; a.o2 = dv; a.lut = d_items; a.R = n_items;
+    a.partial = partial; a.n_slots = n_slots; a.split_lut = d_split; a.n_split = n_split;
+    rl = launch_d<2>(a, c->D, (int64_t)a.Z * n_items * a.sub, st);
+    if (rl != BSP_OK) return rl;
+    if (n_split > 0) {
+      const unsigned n_wg = (unsigned)((int64_t)a.Z * n_split * (2 * 64 * c->D / 4 / 256));
+      if (c->D == 64) hipLaunchKernelGGL(k_attn32_cols_sum<64>, dim3(n_wg), dim3(256), 0, st, a);
+      else hipLaunchKernelGGL(k_attn32_cols_sum<128>, dim3(n_wg), dim3(256), 0, st, a);
+    }
+  }
+  BSP_LAUNCH_CHECK();
+  return BSP_OK;
+}

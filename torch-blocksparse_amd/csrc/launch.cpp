@@ -452,22 +452,25 @@ bool near_rows(const Operand &t) {
   return t.dim == 4 && t.stride[3] == 1 && !((t.stride[0] | t.stride[1] | t.stride[2]) % 8) && t.stride[2] >= t.size[3] && !(t.ptr & 15) &&
          t.stride[2] * t.size[2] * 2 < (int64_t)1 << 32;
 }
-bool attn_shape(const Attn *s, const Operand &q, const Operand &k, const Operand &v) {
-  if (q.dtype == BSP_F32 || k.dtype != q.dtype || v.dtype != q.dtype || q.dev != s->dev || k.dev != q.dev || v.dev != q.dev) return false;
+bool attn_shape(const Attn *s, const Operand &q, const Operand &k, const Operand &v, bool f32 = false) {
+  if ((q.dtype == BSP_F32) != f32 || k.dtype != q.dtype || v.dtype != q.dtype || q.dev != s->dev || k.dev != q.dev || v.dev != q.dev) return false;
   if (q.dim != 4 || k.dim != 4 || v.dim != 4 || (q.size[3] != 64 && q.size[3] != 128) || q.size[0] <= 0) return false;
   for (const Operand *t : {&q, &k, &v})
     if (t->size[0] != q.size[0] || t->size[1] != s->H || t->size[3] != q.size[3] || t->size[2] != (t == &q ? s->R : s->C) * s->block) return false;
   return true;
 }
 
-// attn_usable(tables, q, k, v): do the kernels take these operands (copied, where they have to be)?
+// attn_usable(tables, q, k, v): do the kernels take these operands (copied, where they have to be)?  (fp32: those of attention_f32.hip,
+// which keep three parts of two bytes an element within 4 GiB of a head's first)
 PyObject *attn_usable(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != 4) { PyErr_SetString(PyExc_TypeError, "attn_usable takes 4 arguments"); return nullptr; }
   const Attn *s = static_cast<const Attn *>(PyCapsule_GetPointer(args[0], kAttn));
   if (!s) return nullptr;
   Operand q, k, v;
   if (!q.read(args[1]) || !k.read(args[2]) || !v.read(args[3])) Py_RETURN_NONE;
-  return PyBool_FromLong(attn_shape(s, q, k, v) && s->longest > 0 && s->longest * 64 < 32768);
+  const bool f32 = q.dtype == BSP_F32;
+  return PyBool_FromLong(attn_shape(s, q, k, v, f32) && s->longest > 0 && s->longest * 64 < 32768 &&
+                         (!f32 || (s->R > s->C ? s->R : s->C) * s->block * q.size[3] * 6 < (int64_t)1 << 32));
 }
 
 // attn_fwd(tables, q, k, v, scale, kpm, kpm_stride, kpm_mul, keep) -> (o, lse or None): bsp_attention_rows_fwd
@@ -549,6 +552,95 @@ PyObject *attn_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   return PyTuple_Pack(3, need_q ? dq.o : Py_None, need_k ? dk.o : Py_None, need_v ? dv.o : Py_None);
 }
 
+// ... in fp32
+bool f32_rows(const Operand &t) {                       // _vec32 in attention_core.py
+  return t.dim == 4 && t.stride[3] == 1 && !((t.stride[0] | t.stride[1] | t.stride[2]) % 4) && t.stride[2] >= t.size[3] && !(t.ptr & 15);
+}
+void put_strides(int64_t *to, const int64_t *size) {    // of a contiguous tensor
+  to[0] = size[1] * size[2] * size[3]; to[1] = size[2] * size[3]; to[2] = size[3];
+}
+// the call's sizes and masks; masks: scale, kpm, kpm_stride, kpm_mul
+bool f32_call(const Attn *s, int64_t Z, int64_t D, PyObject *const *masks, bsp_attention_f32_call *c) {
+  *c = bsp_attention_f32_call{};
+  c->Z = (int)Z; c->H = (int)s->H; c->R = s->lines; c->D = (int)D;
+  c->keys = s->C * s->block;
+  c->d_rows = s->rows;
+  c->scale = (float)PyFloat_AsDouble(masks[0]);
+  c->kpm_stride_z = PyLong_AsLongLong(masks[2]);
+  c->kpm_mul = (int)PyLong_AsLong(masks[3]);
+  void *kpm = nullptr;
+  if (PyErr_Occurred() || (masks[1] != Py_None && !pointer(masks[1], &kpm))) return false;
+  c->kpm = static_cast<const float *>(kpm);
+  return true;
+}
+
+// attn32_fwd(tables, q, k, v, scale, kpm, kpm_stride, kpm_mul, keep) -> (o, planes, stats or None): bsp_attention_f32_fwd
+PyObject *attn32_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  if (n != 9) { PyErr_SetString(PyExc_TypeError, "attn32_fwd takes 9 arguments"); return nullptr; }
+  const Attn *s = static_cast<const Attn *>(PyCapsule_GetPointer(args[0], kAttn));
+  if (!s) return nullptr;
+  Operand q, k, v;
+  if (!q.read(args[1]) || !k.read(args[2]) || !v.read(args[3]) || !attn_shape(s, q, k, v, true) || !f32_rows(q) || !f32_rows(k) || !f32_rows(v)) Py_RETURN_NONE;
+  const int64_t Z = q.size[0], rows = q.size[2], D = q.size[3], shape[4] = {Z, s->H, rows, D}, sshape[4] = {Z, s->H, 2, rows};
+  const bool keep = truth(args[8]);
+  bsp_attention_f32_call c;
+  void *op, *sp = nullptr, *st;
+  if (!f32_call(s, Z, D, args + 4, &c) || !stream_of(q.dev, &st)) return nullptr;
+  Ref planes(empty_bytes(bsp_attention_f32_bytes((int)Z, (int)s->H, keep ? rows : 0, c.keys, (int)D), q.obj)), o(planes.o ? empty_like_type(shape, 4, q) : nullptr), stats;
+  if (!o.o || !pointer(planes.o, &c.planes) || !pointer(o.o, &op)) return nullptr;
+  if (keep) {
+    stats.o = empty_floats(sshape, 4, q.obj);
+    if (!stats.o || !pointer(stats.o, &sp)) return nullptr;
+  }
+  c.stats = static_cast<float *>(sp);
+  for (int i = 0; i < 3; i++) c.strides[i] = q.stride[i], c.strides[3 + i] = k.stride[i], c.strides[6 + i] = v.stride[i];
+  put_strides(c.strides + 9, shape);
+  const int rc = unlocked([&] { return bsp_attention_f32_fwd(&c, static_cast<const float *>(q.data()), static_cast<const float *>(k.data()), static_cast<const float *>(v.data()),
+                                                             static_cast<float *>(op), st); });
+  if (!checked(rc, "bsp_attention_f32_fwd")) return nullptr;
+  return PyTuple_Pack(3, o.o, planes.o, stats.o ? stats.o : Py_None);
+}
+
+// attn32_bwd(tables, do, o, planes, stats, scale, kpm, kpm_stride, kpm_mul, need_q, need_k, need_v) -> (dq, dk, dv): bsp_attention_f32_bwd
+PyObject *attn32_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  if (n != 12) { PyErr_SetString(PyExc_TypeError, "attn32_bwd takes 12 arguments"); return nullptr; }
+  const Attn *s = static_cast<const Attn *>(PyCapsule_GetPointer(args[0], kAttn));
+  if (!s) return nullptr;
+  const bool need_q = truth(args[9]), need_k = truth(args[10]), need_v = truth(args[11]), columns = need_k || need_v;
+  Operand g, o;
+  if (!g.read(args[1]) || !o.read(args[2]) || g.dim != 4 || o.dim != 4 || g.dtype != BSP_F32 || o.dtype != BSP_F32 || g.dev != o.dev || o.dev != s->dev) Py_RETURN_NONE;
+  for (int i = 0; i < 4; i++) if (g.size[i] != o.size[i]) Py_RETURN_NONE;
+  if (o.size[1] != s->H || o.size[2] != (int64_t)s->lines * 64 || !f32_rows(g) || !f32_rows(o)) Py_RETURN_NONE;
+  const int64_t Z = o.size[0], rows = o.size[2], D = o.size[3];
+  bsp_attention_f32_call c;
+  void *sp, *st, *dq_p, *dk_p = nullptr, *dv_p = nullptr, *parts_p = nullptr, *delta_p = nullptr, *slots_p = nullptr;
+  if (!f32_call(s, Z, D, args + 5, &c) || !pointer(args[3], &c.planes) || !pointer(args[4], &sp) || !stream_of(o.dev, &st)) return nullptr;
+  c.stats = static_cast<float *>(sp);
+  const int64_t qs[4] = {Z, s->H, rows, D}, ks[4] = {Z, s->H, c.keys, D}, ds[3] = {Z, s->H, rows}, ps[4] = {bsp_attention_f32_slots((int)Z, s->n_slots), 2, 64, D};
+  Ref dq(empty_like_type(qs, 4, o)), dk, dv, parts, delta, slots;
+  if (!dq.o || !pointer(dq.o, &dq_p)) return nullptr;
+  if (columns) {
+    dk.o = empty_like_type(ks, 4, o);
+    dv.o = dk.o ? empty_like_type(ks, 4, o) : nullptr;
+    delta.o = dv.o ? empty_floats(ds, 3, o.obj) : nullptr;
+    parts.o = delta.o ? empty_bytes(bsp_attention_f32_bytes((int)Z, (int)s->H, rows, 0, (int)D), o.obj) : nullptr;
+    if (!parts.o || !pointer(dk.o, &dk_p) || !pointer(dv.o, &dv_p) || !pointer(delta.o, &delta_p) || !pointer(parts.o, &parts_p)) return nullptr;
+    if (s->n_slots) {
+      slots.o = empty_floats(ps, 4, o.obj);
+      if (!slots.o || !pointer(slots.o, &slots_p)) return nullptr;
+    }
+  }
+  for (int i = 0; i < 3; i++) c.strides[i] = g.stride[i], c.strides[3 + i] = o.stride[i];
+  put_strides(c.strides + 6, qs);
+  put_strides(c.strides + 9, ks);
+  put_strides(c.strides + 12, ks);
+  const int rc = unlocked([&] { return bsp_attention_f32_bwd(&c, static_cast<const float *>(g.data()), static_cast<const float *>(o.data()), static_cast<float *>(dq_p), static_cast<float *>(dk_p),
+                                                             static_cast<float *>(dv_p), parts_p, static_cast<float *>(delta_p), s->items, s->n_items, static_cast<float *>(slots_p), s->n_slots,
+                                                             s->split, s->n_split, st); });
+  if (!checked(rc, "bsp_attention_f32_bwd")) return nullptr;
+  return PyTuple_Pack(3, need_q ? dq.o : Py_None, need_k ? dk.o : Py_None, need_v ? dv.o : Py_None);
+}
+
 // setup(torch, _lib.check, raw stream of a device, Parameter, the class with SPLITK_TARGET_WORKGROUPS)
 PyObject *setup(PyObject *, PyObject *args) {
   PyObject *torch, *check, *stream, *parameter, *cls;
@@ -566,7 +658,7 @@ PyObject *setup(PyObject *, PyObject *args) {
 #define BSP_FAST(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {{"setup", setup, METH_VARARGS, nullptr}, {"make_xsd", make_xsd, METH_VARARGS, nullptr}, {"make_sdd", make_sdd, METH_VARARGS, nullptr},
                          {"make_rows", make_rows, METH_VARARGS, nullptr}, {"make_attn", make_attn, METH_VARARGS, nullptr}, BSP_FAST(xsd), BSP_FAST(sdd), BSP_FAST(softmax_fwd),
-                         BSP_FAST(softmax_bwd), BSP_FAST(attn_usable), BSP_FAST(attn_fwd), BSP_FAST(attn_bwd), {nullptr, nullptr, 0, nullptr}};
+                         BSP_FAST(softmax_bwd), BSP_FAST(attn_usable), BSP_FAST(attn_fwd), BSP_FAST(attn_bwd), BSP_FAST(attn32_fwd), BSP_FAST(attn32_bwd), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", "host side of the launches", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

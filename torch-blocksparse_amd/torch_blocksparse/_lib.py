@@ -90,6 +90,10 @@ SIGNATURES = {
     'bsp_attention_rows_fwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 13 + [_f, _vp, _vp, _i64, _i, _vp]),
     'bsp_attention_rows_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 19 + [_f, _vp, _vp, _i64, _i, _vp]),
     'bsp_attention_cols_bwd': (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i64, _i] + [_i64] * 19 + [_f, _vp, _i, _vp, _i, _vp, _i, _vp, _i64, _i, _vp]),
+    'bsp_attention_f32_bytes': (_i64, [_i, _i, _i64, _i64, _i]),
+    'bsp_attention_f32_slots': (_i64, [_i, _i]),
+    'bsp_attention_f32_fwd': (_i, [_vp] * 6),
+    'bsp_attention_f32_bwd': (_i, [_vp] * 9 + [_i, _vp, _i, _vp, _i, _vp]),
     'bsp_layout_fixed': (_i, [_vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
     'bsp_layout_sparse_transformer': (_i, [_vp, _i, _i, _i, _i, _i, _vp]),
     'bsp_layout_bigbird': (_i, [_vp, _i, _i, _i, _i, _i, _vp, _i, _vp]),

@@ -4,7 +4,8 @@ The reference's modules call three operators, sparse_dot_sdd_nt(q, k), sparse_so
 (deepspeedsparseselfattention.py:152-157; attention.py:190-202).  `attention_chain` takes the same three operator
 objects and the same arguments and returns the same context tensor; when the operators are this package's, built on
 one layout with blocks of 16, 32 or 64, and the tensors are fp16 / bf16 with a head dimension of 64 or 128, it runs fused
-kernels instead.  Without relative position embedding and attention mask no sparse tensor exists (bsp_attention_rows_fwd,
+kernels instead; in fp32 it does so without relative position embedding and attention mask (bsp_attention_f32_fwd,
+bsp_attention_f32_bwd: class _attention_f32).  In 16 bits, without relative position embedding and attention mask no sparse tensor exists (bsp_attention_rows_fwd,
 bsp_attention_rows_bwd, bsp_attention_cols_bwd: class _attention_quad); with one of them the softmax is stored for the backward pass
 (bsp_attention_fwd, bsp_attention_bwd, bsp_attention_bwd_kv: class _attention_core).
 In every other case, and with FUSED = False, it calls the three operators one after the other.
@@ -20,7 +21,8 @@ from .softmax import Softmax, _sparse_softmax
 
 FUSED = os.environ.get('BSP_FUSED_ATTENTION', '1') != '0'
 MAX_ROW_BLOCKS = 8          # BSP_ATTENTION_MAX_ROW_BLOCKS: longer rows are streamed (the library decides)
-fused_calls = 0             # forward calls that took the fused kernels; tests read it
+fused_calls = 0             # forward calls that took the fused kernels for 16-bit tensors; tests read it
+fused_f32_calls = 0         # ... and those for fp32
 # dk and dv from a column kernel (bsp_attention_cols_bwd, bsp_attention_bwd_kv), which computes the softmax gradient again instead
 # of reading it; False: the row kernel stores the gradient and the two products are ordinary dsd operators
 FUSED_KV = os.environ.get('BSP_FUSED_ATTENTION_KV', '1') != '0'
@@ -221,6 +223,14 @@ class AttentionCore:
             return False
         return t.longest * 64 < 32768                           # the softmax operator's bound on a row (softmax.py:225-227)
 
+    def usable_f32(self, q, k, v, rpe=None, attn_mask=None, dropout_p=0.):
+        """The same for fp32: calls without per-element masks.  FUSED_KV = False asks for the gradients through stored softmax
+        gradients, which only the operators have here."""
+        if not (FUSED and FUSED_KV) or rpe is not None or attn_mask is not None or dropout_p or self.block not in (16, 32, 64) or not q.is_cuda:
+            return False
+        tables = self.quad(q.device)
+        return tables is not None and _lib.native().attn_usable(tables.native(), q, k, v) is True
+
     def __call__(self, q, k, v, scale=1., rpe=None, key_padding_mask=None, attn_mask=None,
                  key_padding_mask_mode='add', attn_mask_mode='add'):
         for name, m in (('relative position embedding', rpe), ('Attention mask', attn_mask), ('Key padding mask', key_padding_mask)):
@@ -229,7 +239,8 @@ class AttentionCore:
         if rpe is None and attn_mask is None:
             if key_padding_mask is not None:
                 self._check_masks(q, None, key_padding_mask, None)
-            return _attention_quad.apply(q, k, v, float(scale), key_padding_mask, key_padding_mask_mode, self, torch.is_grad_enabled())
+            chain = _attention_f32 if q.dtype == torch.float32 else _attention_quad
+            return chain.apply(q, k, v, float(scale), key_padding_mask, key_padding_mask_mode, self, torch.is_grad_enabled())
         lut, maxlut, _, rows = self.tables(q.device)[:4]
         # p is kept for the backward pass; a forward pass that no backward pass can follow does not store it
         keep_p = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
@@ -350,6 +361,53 @@ class _attention_quad(torch.autograd.Function):
             dk, dv = (_attention_quad.columns_kernel(ctx, saved, do, delta) if FUSED_KV else
                       _attention_quad.through_stored_gradient(ctx, saved, do, need_k, need_v))
         return (dq if need_q else None, dk if need_k else None, dv if need_v else None) + (None,) * 5
+
+
+def _vec32(t):
+    """fp32 operands: unit inner stride, every other stride a multiple of 4 elements, aligned base, rows that do not overlap"""
+    z, h, row, inner = t.stride()
+    return t if inner == 1 and not (z | h | row) % 4 and row >= t.size(3) and not t.data_ptr() % 16 else _packed(t)
+
+
+class _attention_f32(torch.autograd.Function):
+    """The chain without per-element masks in fp32: what the backward pass needs of q, k and v are their bfloat16 parts, which the
+    forward pass has made, and of the softmax two floats per row."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, scale, key_padding_mask, kp_mask_mode, core, grad_enabled):
+        global fused_f32_calls
+        tables = core.quad(q.device)
+        keep = grad_enabled and any(ctx.needs_input_grad[:3])
+        kpm = None
+        if key_padding_mask is not None:
+            kpm = _sparse_softmax._strided16(key_padding_mask, 'key_padding_mask')
+            if keep and kpm.data_ptr() == key_padding_mask.data_ptr():
+                kpm = _packed(kpm[:, :k.size(2)])          # (as in _attention_quad)
+        kpm_args = (kpm.stride(0) if kpm is not None and kpm.size(0) > 1 else 0, int(kp_mask_mode == 'mul'))
+        launch, native = _lib.native(), tables.native()
+        made = launch.attn32_fwd(native, q, k, v, scale, kpm, *kpm_args, keep)
+        if made is None:                                   # operands that the kernels cannot address are copied to memory of their own
+            made = launch.attn32_fwd(native, _vec32(q), _vec32(k), _vec32(v), scale, kpm, *kpm_args, keep)
+            if made is None:
+                raise _lib.BlocksparseLibraryError('attention: operands %s, %s, %s do not fit the layout' % (tuple(q.shape), tuple(k.shape), tuple(v.shape)))
+        o, planes, stats = made
+        fused_f32_calls += 1
+        if keep:
+            ctx.save_for_backward(planes, o, stats, kpm)
+            ctx.scale, ctx.tables, ctx.kpm_args = scale, tables, kpm_args
+        return o
+
+    @staticmethod
+    def backward(ctx, do):
+        planes, o, stats, kpm = ctx.saved_tensors
+        args = (planes, stats, ctx.scale, kpm, *ctx.kpm_args, *ctx.needs_input_grad[:3])
+        launch, native = _lib.native(), ctx.tables.native()
+        made = launch.attn32_bwd(native, do, o, *args)
+        if made is None:
+            made = launch.attn32_bwd(native, _vec32(do), _vec32(o), *args)
+            if made is None:
+                raise _lib.BlocksparseLibraryError('attention: gradient %s does not fit the result %s' % (tuple(do.shape), tuple(o.shape)))
+        return made + (None,) * 5
 
 
 class _StoredSoftmax:
@@ -480,7 +538,7 @@ def attention_chain(sdd_nt, softmax, dsd_nn, q, k, v, scale=1., rpe=None, key_pa
                     key_padding_mask_mode='add', attn_mask_mode='add', dropout_p=0.):
     """dsd_nn(softmax(sdd_nt(q, k), ...), v): fused when the operators and tensors allow it, else the three calls."""
     core = _core_for(sdd_nt, softmax, dsd_nn)
-    if core is not None and core.usable(q, k, v, dropout_p):
+    if core is not None and (core.usable_f32(q, k, v, rpe, attn_mask, dropout_p) if q.dtype == torch.float32 else core.usable(q, k, v, dropout_p)):
         return core(q, k, v, scale, rpe, key_padding_mask, attn_mask, key_padding_mask_mode, attn_mask_mode)
     w = sdd_nt(q, k)
     kwargs = dict(dropout_p=dropout_p) if dropout_p else {}

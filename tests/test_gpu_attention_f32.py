@@ -54,8 +54,8 @@ def _layout(H, R, C, kind):
     return lay
 
 
-# one tile; a tile of remainders; lines and columns of one to many tiles; parts of long columns in 4, 2 and 1 pieces (1, 66 and 512 batches x
-# heads of one 40-tile column in three parts, 2 of 64); from 32 heads on another order of the workgroups
+# one tile; a tile of remainders; lines and columns of one to many tiles; parts of long columns in 2 and in 1 pieces
+# (66 and 512 batches x heads of a column in three parts); from 32 heads on another order of the workgroups
 @pytest.mark.parametrize('Z,H,R,C,block,D,kind,padded', [
     (1, 1, 1, 1, 64, 64, 'dense', False),
     (2, 1, 4, 4, 16, 128, 'random', True),

@@ -916,9 +916,10 @@ F32Args f32_args(const bsp_attention_f32_call &c) {
 void take_strides(const int64_t *s, int64_t &z, int64_t &h, int64_t &row) { z = s[0]; h = s[1]; row = s[2]; }
 
 // Pieces of the parts of long columns.  A part is up to sixteen tiles, eight times as long as the short columns of the layouts that have
-// any, and takes 70 us: a launch whose parts do not fill the chip twice (two workgroups a CU) ends with them.  Every piece is a slot written
-// and read once more.  Module in fp32, 2 x 8 heads of 2048 positions, stride 128 of blocks of 32, 256 parts: @@
-int pieces(int64_t parts) { return parts == 0 ? 1 : parts >= 2048 ? 1 : parts > 128 ? 2 : 4; }
+// any: a launch whose parts do not fill the chip (two workgroups a CU, 512) ends with them alone and does better on halves, though each costs
+// a workgroup's first loads and a slot written and read once more.  Column kernel in 1 / 2 / 4 pieces, 8 heads of 2048 positions, stride 128 of blocks of
+// 32: 128 parts 55 / 45 / 54 us, 256 parts 86 / 80 / 105, 512 parts 126 / 147 / 181, 1024 parts 241 / 281 / 367.
+int pieces(int64_t parts) { return parts > 0 && parts < 512 ? 2 : 1; }
 
 }  // namespace
 }  // namespace bsp

@@ -117,6 +117,31 @@ def test_every_row_length_bucket(longest):
     run_case(1, 2, 4, C, 32, torch.float32, 0, 300 + longest, scale=0.3, rpe=True, kpm='add', layout=lay)
 
 
+@pytest.mark.parametrize('longest', [5, 6, 7, 8, 9, 16, 17, 18, 27, 32])
+def test_every_row_length_bucket_of_a_full_launch(longest):
+    # from 4097 matrix rows on (2049 where no row has more than 8 blocks) a few lanes work on a row; in smaller launches, as in
+    # the test above, a wavefront does where rows have more than 4 blocks.  Rows of every length up to the longest, and none.
+    C = longest + 1
+    lay = torch.zeros(2, 12, C, dtype=torch.int64)
+    for r in range(12):
+        lay[0, r, r % 3:max(0, longest - r * longest // 11)] = 1
+        lay[1, r, 1:1 + (longest if r % 4 == 0 else r)] = 1
+    run_case(3, 2, 12, C, 64, torch.float16, 0, 700 + longest, scale=0.3, kpm='add', layout=lay)
+    run_case(11, 2, 12, C, 16, torch.bfloat16, 0, 800 + longest, scale=0.3, kpm='mul', attn='add', layout=lay)
+    run_case(6, 2, 12, C, 32, torch.float32, 0, 900 + longest, scale=0.3, rpe=True, kpm='add', layout=lay)
+
+
+@pytest.mark.parametrize('dtype', [torch.float16, torch.float32])
+@pytest.mark.parametrize('Z,R,cols', [(16, 8, 7), (17, 8, 7), (32, 8, 12), (33, 8, 12), (16, 8, 4), (16, 8, 5)])
+def test_rows_on_either_side_of_a_wavefront_each(Z, R, cols, dtype):
+    # 2048 / 2176 rows of up to 7 blocks, 4096 / 4224 of up to 12, 2048 of 4 and of 5: with every mask and without
+    lay = random_layout((1, R, cols), 0.8, Z + cols)
+    lay[0, 0, :] = 1
+    lay[0, 3, :] = 0
+    run_case(Z, 1, R, cols, 16, dtype, 0, Z + cols, scale=0.3, layout=lay)
+    run_case(Z, 1, R, cols, 16, dtype, 0, Z + cols, scale=0.3, rpe=True, kpm='add', attn='mul', layout=lay)
+
+
 def test_rows_without_blocks_and_single_block():
     lay = torch.zeros(2, 4, 4, dtype=torch.int64)
     lay[0, 0, 1] = 1

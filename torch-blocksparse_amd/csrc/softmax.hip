@@ -658,8 +658,16 @@ template <typename T, int BLOCK, int NB> void launch_bwd_nb(const BwdArgs &a, hi
 
 template <typename T> constexpr int dtype_of() { return sizeof(T) == 4 ? BSP_F32 : std::is_same<T, f16>::value ? BSP_F16 : BSP_BF16; }
 
+// Launches that leave most of the chip idle: a wavefront per row, which keeps a long row's serial part (its loads, exponentials and
+// reductions) short.  A few lanes a row take 3.5 us at 6 blocks a row and 8.9 at 32, whatever the launch, until the chip is full;
+// a wavefront a row 2.8-3.6 while its launch is a few thousand rows, and twice the work per row in a full one.  Measured (us, few lanes / a wavefront; forward,
+// fp32): 2048 rows of 4 blocks of 16 3.2 / 3.0, 7 blocks 3.8 / 3.0, 32 blocks 8.9 / 3.6; 4096 rows of 7 blocks of 64 4.6 / 4.4, of
+// 12 7.0 / 5.8, of 2 3.2 / 3.7; 8192 rows of 7 blocks of 16 4.1 / 4.7, of 7 blocks of 64 5.6 / 6.5.  fp16 alike; backward 1.0-1.9 times as fast.
+inline bool row_a_wavefront(int64_t rows, int maxlut) { return rows <= (maxlut > 8 ? 4096 : maxlut > 4 ? 2048 : 0); }
+
 template <typename T, int BLOCK> void launch_fwd(const FwdArgs &a, int maxlut, hipStream_t st) {
   constexpr int MX = max_nb_fwd<T, BLOCK>();
+  if (row_a_wavefront((int64_t)a.Z * a.H * a.R * BLOCK, maxlut) && softmax_row_fwd(dtype_of<T>(), a, BLOCK, maxlut, st)) return;
   if (maxlut <= 1) launch_fwd_nb<T, BLOCK, 1>(a, st);
   else if (maxlut <= 2) launch_fwd_nb<T, BLOCK, 2>(a, st);
   else if (maxlut <= 4) launch_fwd_nb<T, BLOCK, 4>(a, st);
@@ -668,12 +676,13 @@ template <typename T, int BLOCK> void launch_fwd(const FwdArgs &a, int maxlut, h
   else if (maxlut <= 8) launch_fwd_nb<T, BLOCK, 8>(a, st);
   else if (maxlut <= 16 && 16 <= MX) launch_fwd_nb<T, BLOCK, (16 <= MX ? 16 : 0)>(a, st);
   else if (maxlut <= 32 && 32 <= MX) launch_fwd_nb<T, BLOCK, (32 <= MX ? 32 : 0)>(a, st);
-  // longer rows: one wavefront per row while the row fits its registers, else the variant that re-reads x.  (For rows
+  // longer rows: one wavefront per row while the row fits its registers, else the variant that re-reads x.  (In a full launch of rows
   // that the register variants above hold, one wavefront per row is 2-3 x slower: measured on rows of 7, 14 and 28 blocks
   // of 64, 32 and 16, forward 0.22 against 0.08-0.09 ms: a kilobyte of work per wavefront does not pay for its set-up.)
   else if (!softmax_row_fwd(dtype_of<T>(), a, BLOCK, maxlut, st)) launch_fwd_nb<T, BLOCK, 0>(a, st);
 }
 template <typename T, int BLOCK> void launch_bwd(const BwdArgs &a, int maxlut, hipStream_t st) {
+  if (row_a_wavefront((int64_t)a.Z * a.H * a.R * BLOCK, maxlut) && softmax_row_bwd(dtype_of<T>(), a, BLOCK, maxlut, st)) return;
   if (maxlut <= 1) launch_bwd_nb<T, BLOCK, 1>(a, st);
   else if (maxlut <= 2) launch_bwd_nb<T, BLOCK, 2>(a, st);
   else if (maxlut <= 4) launch_bwd_nb<T, BLOCK, 4>(a, st);

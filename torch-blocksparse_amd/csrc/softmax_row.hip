@@ -58,11 +58,12 @@ __global__ void __launch_bounds__(256) k_softmax_row_fwd(FwdArgs a) {
   }
 #pragma unroll
   for (int i = 0; i < NI; i++) px[i].load(xz + (int64_t)bid[i] * (BLOCK * BLOCK));
+  // the mask terms, then the logits: one rounding beside them, as in softmax.hip
 #pragma unroll
   for (int i = 0; i < NI; i++) {
     const bool live = i * BPS + sub < size;
 #pragma unroll
-    for (int e = 0; e < EV; e++) l[i][e] = live ? to_float(px[i].e[e]) * sc : -INFINITY;      // softmax.py:112-116
+    for (int e = 0; e < EV; e++) l[i][e] = live ? 0.f : -INFINITY;
   }
   if (a.kpm) {                                                    // :122-124, 'mul' mode :104-106
 #pragma unroll
@@ -76,15 +77,6 @@ __global__ void __launch_bounds__(256) k_softmax_row_fwd(FwdArgs a) {
       }
     }
   }
-  if (a.rpe) {                                                    // :118-120
-#pragma unroll
-    for (int i = 0; i < NI; i++) {
-      P pr;
-      pr.load(rz + (int64_t)bcol[i] * BLOCK);
-#pragma unroll
-      for (int e = 0; e < EV; e++) l[i][e] = fmaf(to_float(pr.e[e]), unit, l[i][e]);
-    }
-  }
   if (a.attn) {                                                   // :126-128, 'mul' mode :108-110
 #pragma unroll
     for (int i = 0; i < NI; i++) {
@@ -95,6 +87,19 @@ __global__ void __launch_bounds__(256) k_softmax_row_fwd(FwdArgs a) {
         const float m = to_float(pa.e[e]);
         l[i][e] += a.attn_mul ? (m == 0.f ? -INFINITY : 0.f) : m * unit;
       }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NI; i++)
+#pragma unroll
+    for (int e = 0; e < EV; e++) l[i][e] = i * BPS + sub < size ? fmaf(to_float(px[i].e[e]), sc, l[i][e]) : -INFINITY;      // softmax.py:112-116
+  if (a.rpe) {                                                    // :118-120
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      P pr;
+      pr.load(rz + (int64_t)bcol[i] * BLOCK);
+#pragma unroll
+      for (int e = 0; e < EV; e++) l[i][e] = i * BPS + sub < size ? fmaf(to_float(pr.e[e]), unit, l[i][e]) : -INFINITY;
     }
   }
   float mx = -INFINITY;

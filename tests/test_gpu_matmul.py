@@ -36,6 +36,20 @@ def test_other_dtypes(mode, block, dtype):
     run_case(mode, True, False, block, dtype, Z=1, seed=block + 1)
 
 
+# fp32 dsd / dds take the widest tile of the free dimension of which their launch has 512: for 8 lines in 2 heads (blocks of 32 and 128, tiles of
+# up to 256; 64, up to 128) every width, a ragged last tile, and launches just below and at the line.  Reductions of an odd number of steps.
+@pytest.mark.parametrize('block,Z,free', [(32, 1, 76), (32, 16, 300), (32, 16, 256), (32, 11, 260), (128, 32, 200), (128, 16, 516), (128, 8, 260), (64, 32, 64), (64, 16, 204), (64, 2, 132)])
+@pytest.mark.parametrize('mode', ['dsd', 'dds'])
+def test_fp32_tiles_of_the_free_dimension(mode, block, Z, free):
+    lay = random_layout((2, 8, 3), 0.6, free, at_least_one_per_row=True)
+    lay[1, 5, :] = 0
+    lines, red = 8 * block, 3 * block
+    t = Z % 3 == 1
+    sizes = dict(M=lines, K=red, N=free) if mode == 'dsd' else dict(N=lines, K=red, M=free)
+    run_case(mode, t if mode == 'dsd' else False, True if mode == 'dds' else t, block, torch.float32, Z=Z,
+             layout=lay.transpose(1, 2).contiguous() if mode == 'dsd' and t else lay, seed=free, backward=False, dist='randn', scale=red ** -0.5, **sizes)
+
+
 def test_readme_configuration():
     # README of the reference: fp32, Z=4 H=2 M=256 N=512 K=384, block 16, sdd with trans_a, layout randint(0, 2)
     torch.manual_seed(0)

@@ -62,7 +62,12 @@ template <> struct Mma<float, 32> {
   static __device__ __forceinline__ acc_t run(frag_t a, frag_t b, acc_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 };
 
-template <typename T> struct TileK { static constexpr int TK = 64 / sizeof(T), PAD = 16 / sizeof(T); };  // 64-byte rows + 16 bytes
+// Reduction step: 64 bytes; rows of the tiles 16 bytes more.  fp32 sdd in blocks of 32 takes steps of 128 bytes, whole cache lines and half the
+// barriers (a tenth / four tenths of the blocks, 2048^2 x 1024 in 2 heads: 45-48 -> 41-43 us / 89-95 -> 83-87; 512^2 x 128 in 8 heads and batches
+// 14-15 -> 13 / 28.5-29.5 -> 28.8-29.5).  Blocks of 16 lose up to 12 % where the reduction is short, of 64 and 128 up to 11 %; dsd and
+// dds lose up to 20 % in large launches.
+template <typename T> struct TileK { static constexpr int TK = 64 / sizeof(T), PAD = 16 / sizeof(T); };
+template <typename T, int BLOCK> constexpr int sdd_step() { return sizeof(T) == 4 && BLOCK == 32 ? 32 : TileK<T>::TK; }
 
 // ---------------------------------------------------------------------------------------------------------
 // One operand tile: ROWS x TK, fetched by NT threads in 16-byte chunks, kept in registers until the LDS
@@ -76,23 +81,26 @@ template <typename T> struct TileK { static constexpr int TK = 64 / sizeof(T), P
 // ---------------------------------------------------------------------------------------------------------
 struct Part { int64_t off; bool ok; int sel; int k; };
 
-template <typename T, int ROWS, int NT, bool KCONTIG> struct TileLoader {
-  static constexpr int TK = TileK<T>::TK, LDK = TK + TileK<T>::PAD;
+// MS: rows of the MFMA tiles that read it
+template <typename T, int ROWS, int NT, bool KCONTIG, int MS, int TK> struct TileLoader {
+  static constexpr int LDK = TK + TileK<T>::PAD;
   static constexpr int VE = 16 / sizeof(T);
-  static constexpr int NCH = ROWS * TK / VE;
+  static constexpr int NCH = ROWS * TK / VE, THREADS = NT;
   static constexpr int ITER = (NCH + NT - 1) / NT;
   static constexpr int CPR = TK / VE;    // chunks per row when the reduction is contiguous
   static constexpr int RCH = ROWS / VE;  // chunks per reduction index otherwise
   // An operand stored with the reduction dimension strided is kept in LDS as it lies in memory, [TK][ROWS + 8].  A
   // 16-bit one is handed to the MFMA through the transposing LDS read; a 32-bit one needs no transposition at all:
-  // its MFMA operand is a single element per lane, (row lane % MS, reduction index lane / MS), read where it lies.
+  // its MFMA operand is a single element per lane, read where it lies.
   static constexpr bool ASIS = !KCONTIG;
   static constexpr bool TR = ASIS && sizeof(T) == 2;
   // Padding of a row of the as-is layout.  16-bit: the transposing read of a 16-lane group takes 32 contiguous bytes from
   // each of four consecutive reduction rows, and two groups half a row block apart are served together; with rows of
   // 64 bytes more than a multiple of 256 these eight pieces fall into different banks (the LDS serves 256 bytes per
   // clock: measured, bank-conflict cycles 46-50 % -> 10-20 % of the LDS-active cycles against a padding of 16 bytes).
-  static constexpr int LDR = ROWS + (sizeof(T) == 2 ? 32 : 8);
+  // 32-bit: a read takes MS elements of each of 64 / MS rows that are four apart (frag4): with 8 elements more than a multiple of
+  // 16 (MS 16: 4 more) four rows are half (a quarter) of the 64 banks.
+  static constexpr int LDR = ROWS + (sizeof(T) == 2 ? 32 : MS == 16 ? 4 : 8);
   static constexpr int ELEMS = ASIS ? TK * LDR : ROWS * LDK;
   u32x4 reg[ITER];
   bool ok[ITER];
@@ -112,8 +120,23 @@ template <typename T, int ROWS, int NT, bool KCONTIG> struct TileLoader {
       }
     }
   }
-  // operand fragment of an MS-row MFMA tile starting at tile row `row0`, reduction step kk (KSTEP wide)
-  template <int MS, class M> __device__ __forceinline__ static typename M::frag_t frag(const T *S, int row0, int kk, int lane) {
+  // fp32: the operands of four MFMAs that start at reduction index k0 of the tile.  NEXT: a lane group takes four neighbouring
+  // indices, one an MFMA (which is told two, or four, that are four apart: both operands alike, so that the products are the
+  // same, in another order): where the reduction is contiguous one 128-bit read, in place of four of 32 bits whose rows met in the
+  // same banks.
+  template <class M, bool NEXT> __device__ __forceinline__ static f32x4 frag4(const T *S, int row0, int k0, int lane) {
+    const int k = k0 + (NEXT ? 4 : 1) * (lane / MS), row = row0 + lane % MS;
+    if constexpr (KCONTIG) {
+      static_assert(NEXT, "read as one");
+      return *reinterpret_cast<const f32x4 *>(S + row * LDK + k);
+    } else {
+      constexpr int D = (NEXT ? 1 : M::KSTEP) * LDR;
+      const T *p = S + k * LDR + row;
+      return f32x4{p[0], p[D], p[2 * D], p[3 * D]};
+    }
+  }
+  // operand fragment of an MS-row MFMA tile starting at tile row `row0`, reduction step kk (KSTEP wide); 16-bit types
+  template <class M> __device__ __forceinline__ static typename M::frag_t frag(const T *S, int row0, int kk, int lane) {
     if constexpr (TR) {
       typedef s16x4 __attribute__((address_space(3))) * lds_ptr;
       const int t = lane & 15, gi = lane >> 4;
@@ -125,9 +148,6 @@ template <typename T, int ROWS, int NT, bool KCONTIG> struct TileLoader {
       typedef short s16x8 __attribute__((ext_vector_type(8)));
       s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       return __builtin_bit_cast(typename M::frag_t, v);
-    } else if constexpr (ASIS) {
-      static_assert(M::KV == 1, "32-bit operands: one element per lane");
-      return S[(kk * M::KSTEP + lane / MS) * LDR + row0 + lane % MS];
     } else {
       return *reinterpret_cast<const typename M::frag_t *>(S + (row0 + lane % MS) * LDK + (lane / MS) * M::KV + kk * M::KSTEP);
     }
@@ -135,14 +155,14 @@ template <typename T, int ROWS, int NT, bool KCONTIG> struct TileLoader {
 };
 
 // The thread-invariant half of a loader's addressing (one per operand, shared by all ring stages).
-template <typename T, int ROWS, int NT, bool KCONTIG> struct TileAddr {
-  typedef TileLoader<T, ROWS, NT, KCONTIG> L;
+template <class Loader, bool KCONTIG> struct TileAddr {
+  typedef Loader L;
   Part part[L::ITER];
   template <class View> __device__ __forceinline__ void init(const View &v, int tid) {
 #pragma unroll
     for (int it = 0; it < L::ITER; it++) {
-      int c = tid + it * NT;
-      if (L::NCH % NT != 0 && c >= L::NCH) c = L::NCH - 1;
+      int c = tid + it * L::THREADS;
+      if (L::NCH % L::THREADS != 0 && c >= L::NCH) c = L::NCH - 1;
       if constexpr (KCONTIG) part[it] = v.part_k(c / L::CPR, (c % L::CPR) * L::VE);
       else part[it] = v.part_r((c % L::RCH) * L::VE, c / L::RCH);
     }
@@ -181,15 +201,15 @@ constexpr int stage_tiles(int nc, int ms, int ve, int bytes_per_elem_all_waves, 
   return cg;
 }
 
-template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_KCONTIG, bool OUT_NCONTIG> struct TileGemm {
+template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_KCONTIG, bool OUT_NCONTIG, int TK_> struct TileGemm {
   static constexpr int NT = 64 * WGM * WGN;
-  static constexpr int TK = TileK<T>::TK, LDK = TK + TileK<T>::PAD;
+  static constexpr int TK = TK_;
   // 32x32 MFMA tiles when a wavefront's region allows it (half the LDS operand traffic per flop), 16x16 otherwise
   static constexpr int MS = (TM / WGM >= 32 && TN / WGN >= 32) ? 32 : 16;
   static constexpr int RM = TM / (MS * WGM), RN = TN / (MS * WGN);
   typedef Mma<T, MS> M;
-  typedef TileLoader<T, TM, NT, X_KCONTIG> XL;
-  typedef TileLoader<T, TN, NT, Y_KCONTIG> YL;
+  typedef TileLoader<T, TM, NT, X_KCONTIG, MS, TK> XL;
+  typedef TileLoader<T, TN, NT, Y_KCONTIG, MS, TK> YL;
   static constexpr int X_ELEMS = (XL::ELEMS + 7) & ~7, Y_ELEMS = (YL::ELEMS + 7) & ~7;
   static constexpr int SMEM_BYTES = 2 * (X_ELEMS + Y_ELEMS) * (int)sizeof(T);
 
@@ -220,8 +240,8 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
     static_assert(NS % 2 == 0, "the LDS buffer of a step is chosen by the ring slot's parity");
     XL xl[NS];
     YL yl[NS];
-    TileAddr<T, TM, NT, X_KCONTIG> xa;
-    TileAddr<T, TN, NT, Y_KCONTIG> ya;
+    TileAddr<XL, X_KCONTIG> xa;
+    TileAddr<YL, Y_KCONTIG> ya;
     xa.init(xv, tid);
     ya.init(yv, tid);
 #pragma unroll
@@ -246,20 +266,38 @@ template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_K
         xl[u1].store(Xs[nxt], tid);   // stage s + 1; this buffer was last read in step s - 1, before the previous barrier
         yl[u1].store(Ys[nxt], tid);
         // (steps past the end multiply zeros: cheaper than a branch, which would copy the accumulators around)
-#pragma unroll
-        for (int kk = 0; kk < TK / M::KSTEP; kk++) {
-          typename M::frag_t xf[RM], yf[RN];
-#pragma unroll
-          for (int i = 0; i < RM; i++) xf[i] = XL::template frag<MS, M>(Xs[cur], (wm * RM + i) * MS, kk, lane);
-#pragma unroll
-          for (int j = 0; j < RN; j++) yf[j] = YL::template frag<MS, M>(Ys[cur], (wn * RN + j) * MS, kk, lane);
+        auto product = [&](auto &xf, auto &yf, auto &&of) {
 #pragma unroll
           for (int i = 0; i < RM; i++)
 #pragma unroll
             for (int j = 0; j < RN; j++) {
-              if constexpr (OUT_NCONTIG) acc[i][j] = M::run(yf[j], xf[i], acc[i][j]);   // result rows = n, column = m
-              else acc[i][j] = M::run(xf[i], yf[j], acc[i][j]);                          // result rows = m, column = n
+              if constexpr (OUT_NCONTIG) acc[i][j] = M::run(of(yf[j]), of(xf[i]), acc[i][j]);   // result rows = n, column = m
+              else acc[i][j] = M::run(of(xf[i]), of(yf[j]), acc[i][j]);                          // result rows = m, column = n
             }
+        };
+        if constexpr (sizeof(T) == 4) {
+          // with the reduction strided in both operands rows of 32 lose 2-7 % to NEXT, rows of 16 win 2-8 %
+          constexpr bool NEXT = X_KCONTIG || Y_KCONTIG || MS == 16;
+#pragma unroll
+          for (int k0 = 0; k0 < TK; k0 += 4 * M::KSTEP) {
+            f32x4 xf[RM], yf[RN];
+#pragma unroll
+            for (int i = 0; i < RM; i++) xf[i] = XL::template frag4<M, NEXT>(Xs[cur], (wm * RM + i) * MS, k0, lane);
+#pragma unroll
+            for (int j = 0; j < RN; j++) yf[j] = YL::template frag4<M, NEXT>(Ys[cur], (wn * RN + j) * MS, k0, lane);
+#pragma unroll
+            for (int e = 0; e < 4; e++) product(xf, yf, [&](const f32x4 &v) { return v[e]; });
+          }
+        } else {
+#pragma unroll
+          for (int kk = 0; kk < TK / M::KSTEP; kk++) {
+            typename M::frag_t xf[RM], yf[RN];
+#pragma unroll
+            for (int i = 0; i < RM; i++) xf[i] = XL::template frag<M>(Xs[cur], (wm * RM + i) * MS, kk, lane);
+#pragma unroll
+            for (int j = 0; j < RN; j++) yf[j] = YL::template frag<M>(Ys[cur], (wn * RN + j) * MS, kk, lane);
+            product(xf, yf, [](const typename M::frag_t &v) { return v; });
+          }
         }
         const auto xnext = xv.step((s + NS + 2) * TK);
         const auto ynext = yv.step((s + NS + 2) * TK);
@@ -417,7 +455,7 @@ template <int T_> struct SddShape { static constexpr int WG = T_ >= 32 ? 2 : 1; 
 template <typename T, int BLOCK, int PACK, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __device__ __forceinline__ void sdd_super_block(const SddArgs &g, const int32_t *lut, const uint8_t *all_valid, int part, int z, int64_t grp, bool keep, unsigned char *smem) {
   constexpr int TT = BLOCK * PACK, WG = SddShape<TT>::WG;
-  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
+  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true, sdd_step<T, BLOCK>()> G;
   const table_ptr e = as_table(lut) + grp * (PACK * PACK * 4);
   const int h = e[0];
   SddView<T, BLOCK, PACK, A_KCONTIG> av;
@@ -504,7 +542,7 @@ template <int BLOCK> struct SddLevels {
 constexpr int max_of(int a, int b) { return a > b ? a : b; }
 template <typename T, int BLOCK, bool AK, bool BK> struct SddLevelsShape {
   static constexpr int PACK0 = 64 / BLOCK, LAST_PER_WG = BLOCK == 16 ? 4 : 1;
-  template <int P> using G = TileGemm<T, BLOCK * P, BLOCK * P, SddShape<BLOCK * P>::WG, SddShape<BLOCK * P>::WG, AK, BK, true>;
+  template <int P> using G = TileGemm<T, BLOCK * P, BLOCK * P, SddShape<BLOCK * P>::WG, SddShape<BLOCK * P>::WG, AK, BK, true, sdd_step<T, BLOCK>()>;
   static constexpr int SMEM = max_of(max_of(G<PACK0>::SMEM_BYTES, G<PACK0 / 2>::SMEM_BYTES), LAST_PER_WG * G<1>::SMEM_BYTES);
 };
 
@@ -545,7 +583,7 @@ __global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> 
 template <typename T, int BLOCK, int SPLIT, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __global__ void __launch_bounds__(64 * SddShape<BLOCK / SPLIT>::WG * SddShape<BLOCK / SPLIT>::WG) k_sdd_split(SddArgs g) {
   constexpr int TT = BLOCK / SPLIT, WG = SddShape<TT>::WG;
-  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
+  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true, sdd_step<T, BLOCK>()> G;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int64_t n_wg = g.n_groups * g.Z * (SPLIT * SPLIT);
   const uint32_t w = (uint32_t)xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg);
@@ -694,7 +732,7 @@ __device__ __forceinline__ void xsd_work_item(const XsdArgs &g, int n_tiles, uin
 template <typename T, int BLOCK, int TN_, bool SP_TRANS, bool DN_KCONTIG, bool OUT_NCONTIG, bool PARTS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_xsd(XsdArgs g) {
   typedef XsdShape<BLOCK, TN_> S;
-  typedef TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !SP_TRANS, DN_KCONTIG, OUT_NCONTIG> G;
+  typedef TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !SP_TRANS, DN_KCONTIG, OUT_NCONTIG, TileK<T>::TK> G;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int n_tiles = (g.NF + S::TN - 1) / S::TN;
   const int64_t n_wg = (int64_t)g.width * n_tiles * g.Z;
@@ -794,7 +832,7 @@ template <typename T, int BLOCK> int launch_sdd_b(const SddArgs &g, bool a_kc, b
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true>::SMEM_BYTES;                            \
+    constexpr int SMEM = TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true, sdd_step<T, BLOCK>()>::SMEM_BYTES;      \
     if (g.parts > 1) hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, true>), grid, blockdim, SMEM, st, g);           \
     else hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, false>), grid, blockdim, SMEM, st, g);                      \
   } while (0)
@@ -842,7 +880,7 @@ template <typename T, int BLOCK, int SPLIT> int launch_sdd_split(const SddArgs &
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, TT, TT, WG, WG, AK, BK, true>::SMEM_BYTES;                                  \
+    constexpr int SMEM = TileGemm<T, TT, TT, WG, WG, AK, BK, true, sdd_step<T, BLOCK>()>::SMEM_BYTES;            \
     if (g.parts > 1) hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, true>), grid, blockdim, SMEM, st, g); \
     else hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, false>), grid, blockdim, SMEM, st, g);         \
   } while (0)
@@ -889,7 +927,7 @@ template <typename T, int BLOCK, int TN_> int launch_xsd_bw(const XsdArgs &g0, b
   dim3 grid((unsigned)(n_wg * g.parts)), blockdim(256);
 #define BSP_XSD_LAUNCH(ST, DK, ON)                                                                               \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON>::SMEM_BYTES;                     \
+    constexpr int SMEM = TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON, TileK<T>::TK>::SMEM_BYTES; \
     if constexpr (sizeof(T) == 4)                                                                                \
       if (g.parts > 1) {                                                                                         \
         hipLaunchKernelGGL((k_xsd<T, BLOCK, TN_, ST, DK, ON, true>), grid, blockdim, SMEM, st, g);              \
@@ -919,6 +957,11 @@ template <typename T, int BLOCK> int launch_xsd_b(const XsdArgs &g, bool sp_tran
   // steps in flight, and tiles of 128 are twice as many.  Tiles of 256 / 128, us, of the launches on 256: 128 of them 20.7 / 16.3 (31 blocks
   // a line) and 7.9 / 6.3 (8), 256 20.1 / 17.2, 384 25.7 / 23.4; 512 10.6 / 10.9, 14.3 / 14.3, 17.6 / 20.3; 768 18.2 / 19.1, 25.2 / 27.6.
   if (sizeof(T) == 2 && BLOCK == 32 && tile == 256 && (int64_t)g.width * ((g.NF + 255) / 256) * g.Z < 512) tile = 128;
+  // fp32, whose matrix pipe makes long steps: tiles as narrow as it takes to have two workgroups a compute unit.  1024^3 in 8 heads and batches, a
+  // quarter of the blocks, blocks of 128: tiles of 256 94-103 us, of 128 79-86; 512^3 in 2 heads, of 128 55-61 -> 20-21 on tiles of 64, of 64
+  // 18-20 -> 11-12, of 32 17-22 -> 8-10.  (Parts have their own rule, on the width that xsd_tile gives.)
+  if (sizeof(T) == 4 && g.parts <= 1)
+    while (tile > 64 && (int64_t)g.width * ((g.NF + tile - 1) / tile) * g.Z < 512) tile /= 2;
   if constexpr (BLOCK == 32 || BLOCK == 128)
     if (tile == 256) return launch_xsd_bw<T, BLOCK, 256>(g, sp_trans, dn_kc, out_nc, st);
   if constexpr (BLOCK != 16)

@@ -50,6 +50,22 @@ def test_fp32_tiles_of_the_free_dimension(mode, block, Z, free):
              layout=lay.transpose(1, 2).contiguous() if mode == 'dsd' and t else lay, seed=free, backward=False, dist='randn', scale=red ** -0.5, **sizes)
 
 
+# 16-bit dsd / dds in blocks of 64 and 128 take the widest tile of which their launch has 256, and from 128 workgroups on tiles of 256 the wide
+# kernel: for 8 lines in 2 heads every width, ragged last tiles, launches just below and at the lines
+@pytest.mark.parametrize('block,Z,free', [(128, 1, 72), (128, 16, 200), (128, 8, 264), (128, 3, 520), (128, 8, 512), (128, 7, 256), (64, 15, 72), (64, 16, 136), (64, 7, 257), (64, 8, 512), (64, 1, 776)])
+@pytest.mark.parametrize('mode', ['dsd', 'dds'])
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+def test_16_bit_tiles_of_the_free_dimension(mode, block, Z, free, dtype):
+    lay = random_layout((2, 8, 3), 0.6, free, at_least_one_per_row=True)
+    lay[1, 5, :] = 0
+    lines, red = 8 * block, 3 * block
+    t = Z % 2 == 0
+    sizes = dict(M=lines, K=red, N=free) if mode == 'dsd' else dict(N=lines, K=red, M=free)
+    odd = free % 8 != 0                                       # (the free dimension along whole rows)
+    run_case(mode, t if mode == 'dsd' else False, odd or t if mode == 'dsd' else True, block, dtype, Z=Z,
+             layout=lay.transpose(1, 2).contiguous() if mode == 'dsd' and t else lay, seed=free, backward=False, dist='randn', scale=red ** -0.5, **sizes)
+
+
 def test_readme_configuration():
     # README of the reference: fp32, Z=4 H=2 M=256 N=512 K=384, block 16, sdd with trans_a, layout randint(0, 2)
     torch.manual_seed(0)

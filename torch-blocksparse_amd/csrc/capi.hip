@@ -228,7 +228,7 @@ static int xsd_dispatch(int dtype, XsdArgs g, int block, bool sp_trans, bool dn_
   if (rc < 0) return rc;
   if (rc == 1) { BSP_LAUNCH_CHECK(); return BSP_OK; }
   if (chunks) g.gplan = nullptr;                       // (the chunks serve no other kernel)
-  rc = general_only(flags) ? 0 : xsd_fast64(dtype, g, block, sp_trans, dn_kc, out_nc, st);
+  rc = general_only(flags) || rc == 2 ? 0 : xsd_fast64(dtype, g, block, sp_trans, dn_kc, out_nc, st);
   if (rc < 0) return rc;
   if (rc == 1) { BSP_LAUNCH_CHECK(); return BSP_OK; }
   switch (dtype) {

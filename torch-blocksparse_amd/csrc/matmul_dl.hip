@@ -1380,7 +1380,7 @@ template <typename T, int BLOCK> int launch_dl(const XsdArgs &g0, bool sp_trans,
 // gathered operand of sdd_dl, from its first row).
 static bool near_rows(int64_t rows, int64_t ld) { return ld >= 0 && ld < ((int64_t)1 << 31) / rows; }
 
-// 1 = launched, 0 = not applicable (the caller takes another kernel), < 0 = error
+// 1 = launched, 0 = not applicable (the caller takes another kernel), 2 = the general kernel's, < 0 = error
 int xsd_dl(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bool out_nc, hipStream_t st) {
   if (dtype == BSP_F32 || g.NF < 256 || !near_rows(kTN, g.ldd)) return 0;
   if (block == 32) {   // needs the group plan (whole blocks, no split chains)
@@ -1398,7 +1398,13 @@ int xsd_dl(int dtype, const XsdArgs &g, int block, bool sp_trans, bool dn_kc, bo
   // ... the same at blocks of 64 with the dense reduction contiguous, whose tiles the general kernel reads well: 1024^3 (64
   // workgroups here) 13.7 / 12.2 us, 4096 x 2048 x 4096 (512) 56.7 / 55.5, 8 products of 2048^3 (2048) 89 / 104; with it
   // strided 13.9 / 15.0, 52.4 / 75.1 and 76 / 110
-  if (block == 64 && dn_kc && (int64_t)g.width * ((g.NF + kTN - 1) / kTN) * g.Z <= 512) return 0;
+  const int64_t n_wg = (int64_t)g.width * ((g.NF + kTN - 1) / kTN) * g.Z;
+  if (block == 64 && dn_kc && n_wg <= 512) return 0;
+  // Tiles of 256 on less than half of the compute units: the general kernel's narrower ones.  fp16, this kernel / the general one, us:
+  // blocks of 128, a tenth to half of the blocks there, 512^3 (8 workgroups here) 8-12 / 6-8, 1024 x 512 x 2048 in 2 heads (32) 16-29 / 10-21,
+  // 1024^3 in 3 (96) 13-19 / 10-15; on 128 13-31 / 8-27, but 16 x 512^3 up to 12.8 / 13.9; on 160 17.8 / 20.1.  Blocks of 64, 16 workgroups 6-8 / 5-6,
+  // 64 8-18 / 7-14; 192 8-14 / 7-15.
+  if (n_wg < 128) return 2;
   int rc;
   if (dtype == BSP_F16) rc = block == 128 ? launch_dl<f16, 128>(g, sp_trans, dn_kc, out_nc, st) : launch_dl<f16, 64>(g, sp_trans, dn_kc, out_nc, st);
   else rc = block == 128 ? launch_dl<bf16, 128>(g, sp_trans, dn_kc, out_nc, st) : launch_dl<bf16, 64>(g, sp_trans, dn_kc, out_nc, st);

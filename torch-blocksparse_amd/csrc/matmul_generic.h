@@ -960,8 +960,10 @@ template <typename T, int BLOCK> int launch_xsd_b(const XsdArgs &g, bool sp_tran
   // fp32, whose matrix pipe makes long steps: tiles as narrow as it takes to have two workgroups a compute unit.  1024^3 in 8 heads and batches, a
   // quarter of the blocks, blocks of 128: tiles of 256 94-103 us, of 128 79-86; 512^3 in 2 heads, of 128 55-61 -> 20-21 on tiles of 64, of 64
   // 18-20 -> 11-12, of 32 17-22 -> 8-10.  (Parts have their own rule, on the width that xsd_tile gives.)
-  if (sizeof(T) == 4 && g.parts <= 1)
-    while (tile > 64 && (int64_t)g.width * ((g.NF + tile - 1) / tile) * g.Z < 512) tile /= 2;
+  // 16-bit, blocks of 64 and 128: one a compute unit (1024 x 200 x 1024 in 4 heads, of 128, 14-23 -> 8-13 us, of 64 7-13 -> 6-10; 256
+  // workgroups on tiles of 128 lose 4-10 % on twice as many of 64: 1024 x 128 x 1024 in 16 heads, of 64, half of the blocks, 11.9 -> 13.2).
+  if (sizeof(T) == 4 ? g.parts <= 1 : BLOCK >= 64)
+    while (tile > 64 && (int64_t)g.width * ((g.NF + tile - 1) / tile) * g.Z < (sizeof(T) == 4 ? 512 : 256)) tile /= 2;
   if constexpr (BLOCK == 32 || BLOCK == 128)
     if (tile == 256) return launch_xsd_bw<T, BLOCK, 256>(g, sp_trans, dn_kc, out_nc, st);
   if constexpr (BLOCK != 16)

@@ -62,12 +62,9 @@ template <> struct Mma<float, 32> {
   static __device__ __forceinline__ acc_t run(frag_t a, frag_t b, acc_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 };
 
-// Reduction step: 64 bytes; rows of the tiles 16 bytes more.  fp32 sdd in blocks of 32 takes steps of 128 bytes, whole cache lines and half the
-// barriers (a tenth / four tenths of the blocks, 2048^2 x 1024 in 2 heads: 45-48 -> 41-43 us / 89-95 -> 83-87; 512^2 x 128 in 8 heads and batches
-// 14-15 -> 13 / 28.5-29.5 -> 28.8-29.5).  Blocks of 16 lose up to 12 % where the reduction is short, of 64 and 128 up to 11 %; dsd and
-// dds lose up to 20 % in large launches.
+// Reduction step: 64 bytes; rows of the tiles 16 bytes more.  Steps of 128 bytes in fp32 win up to 15 % in sdd at blocks of 32 with a long
+// reduction and lose 60 % with one of 32; blocks of 16, 64 and 128 lose up to 12 %, dsd and dds up to 20 % in large launches.
 template <typename T> struct TileK { static constexpr int TK = 64 / sizeof(T), PAD = 16 / sizeof(T); };
-template <typename T, int BLOCK> constexpr int sdd_step() { return sizeof(T) == 4 && BLOCK == 32 ? 32 : TileK<T>::TK; }
 
 // ---------------------------------------------------------------------------------------------------------
 // One operand tile: ROWS x TK, fetched by NT threads in 16-byte chunks, kept in registers until the LDS
@@ -82,8 +79,8 @@ template <typename T, int BLOCK> constexpr int sdd_step() { return sizeof(T) == 
 struct Part { int64_t off; bool ok; int sel; int k; };
 
 // MS: rows of the MFMA tiles that read it
-template <typename T, int ROWS, int NT, bool KCONTIG, int MS, int TK> struct TileLoader {
-  static constexpr int LDK = TK + TileK<T>::PAD;
+template <typename T, int ROWS, int NT, bool KCONTIG, int MS> struct TileLoader {
+  static constexpr int TK = TileK<T>::TK, LDK = TK + TileK<T>::PAD;
   static constexpr int VE = 16 / sizeof(T);
   static constexpr int NCH = ROWS * TK / VE, THREADS = NT;
   static constexpr int ITER = (NCH + NT - 1) / NT;
@@ -201,15 +198,15 @@ constexpr int stage_tiles(int nc, int ms, int ve, int bytes_per_elem_all_waves, 
   return cg;
 }
 
-template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_KCONTIG, bool OUT_NCONTIG, int TK_> struct TileGemm {
+template <typename T, int TM, int TN, int WGM, int WGN, bool X_KCONTIG, bool Y_KCONTIG, bool OUT_NCONTIG> struct TileGemm {
   static constexpr int NT = 64 * WGM * WGN;
-  static constexpr int TK = TK_;
+  static constexpr int TK = TileK<T>::TK;
   // 32x32 MFMA tiles when a wavefront's region allows it (half the LDS operand traffic per flop), 16x16 otherwise
   static constexpr int MS = (TM / WGM >= 32 && TN / WGN >= 32) ? 32 : 16;
   static constexpr int RM = TM / (MS * WGM), RN = TN / (MS * WGN);
   typedef Mma<T, MS> M;
-  typedef TileLoader<T, TM, NT, X_KCONTIG, MS, TK> XL;
-  typedef TileLoader<T, TN, NT, Y_KCONTIG, MS, TK> YL;
+  typedef TileLoader<T, TM, NT, X_KCONTIG, MS> XL;
+  typedef TileLoader<T, TN, NT, Y_KCONTIG, MS> YL;
   static constexpr int X_ELEMS = (XL::ELEMS + 7) & ~7, Y_ELEMS = (YL::ELEMS + 7) & ~7;
   static constexpr int SMEM_BYTES = 2 * (X_ELEMS + Y_ELEMS) * (int)sizeof(T);
 
@@ -455,7 +452,7 @@ template <int T_> struct SddShape { static constexpr int WG = T_ >= 32 ? 2 : 1; 
 template <typename T, int BLOCK, int PACK, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __device__ __forceinline__ void sdd_super_block(const SddArgs &g, const int32_t *lut, const uint8_t *all_valid, int part, int z, int64_t grp, bool keep, unsigned char *smem) {
   constexpr int TT = BLOCK * PACK, WG = SddShape<TT>::WG;
-  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true, sdd_step<T, BLOCK>()> G;
+  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
   const table_ptr e = as_table(lut) + grp * (PACK * PACK * 4);
   const int h = e[0];
   SddView<T, BLOCK, PACK, A_KCONTIG> av;
@@ -542,7 +539,7 @@ template <int BLOCK> struct SddLevels {
 constexpr int max_of(int a, int b) { return a > b ? a : b; }
 template <typename T, int BLOCK, bool AK, bool BK> struct SddLevelsShape {
   static constexpr int PACK0 = 64 / BLOCK, LAST_PER_WG = BLOCK == 16 ? 4 : 1;
-  template <int P> using G = TileGemm<T, BLOCK * P, BLOCK * P, SddShape<BLOCK * P>::WG, SddShape<BLOCK * P>::WG, AK, BK, true, sdd_step<T, BLOCK>()>;
+  template <int P> using G = TileGemm<T, BLOCK * P, BLOCK * P, SddShape<BLOCK * P>::WG, SddShape<BLOCK * P>::WG, AK, BK, true>;
   static constexpr int SMEM = max_of(max_of(G<PACK0>::SMEM_BYTES, G<PACK0 / 2>::SMEM_BYTES), LAST_PER_WG * G<1>::SMEM_BYTES);
 };
 
@@ -583,7 +580,7 @@ __global__ void __launch_bounds__(256) k_sdd_levels(SddArgs g, SddLevels<BLOCK> 
 template <typename T, int BLOCK, int SPLIT, bool A_KCONTIG, bool B_KCONTIG, bool PARTS>
 __global__ void __launch_bounds__(64 * SddShape<BLOCK / SPLIT>::WG * SddShape<BLOCK / SPLIT>::WG) k_sdd_split(SddArgs g) {
   constexpr int TT = BLOCK / SPLIT, WG = SddShape<TT>::WG;
-  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true, sdd_step<T, BLOCK>()> G;
+  typedef TileGemm<T, TT, TT, WG, WG, A_KCONTIG, B_KCONTIG, true> G;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int64_t n_wg = g.n_groups * g.Z * (SPLIT * SPLIT);
   const uint32_t w = (uint32_t)xcd_remap(blockIdx.x, PARTS ? n_wg * g.parts : n_wg);
@@ -732,7 +729,7 @@ __device__ __forceinline__ void xsd_work_item(const XsdArgs &g, int n_tiles, uin
 template <typename T, int BLOCK, int TN_, bool SP_TRANS, bool DN_KCONTIG, bool OUT_NCONTIG, bool PARTS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_xsd(XsdArgs g) {
   typedef XsdShape<BLOCK, TN_> S;
-  typedef TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !SP_TRANS, DN_KCONTIG, OUT_NCONTIG, TileK<T>::TK> G;
+  typedef TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !SP_TRANS, DN_KCONTIG, OUT_NCONTIG> G;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int n_tiles = (g.NF + S::TN - 1) / S::TN;
   const int64_t n_wg = (int64_t)g.width * n_tiles * g.Z;
@@ -832,7 +829,7 @@ template <typename T, int BLOCK> int launch_sdd_b(const SddArgs &g, bool a_kc, b
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true, sdd_step<T, BLOCK>()>::SMEM_BYTES;      \
+    constexpr int SMEM = TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true>::SMEM_BYTES;      \
     if (g.parts > 1) hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, true>), grid, blockdim, SMEM, st, g);           \
     else hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, false>), grid, blockdim, SMEM, st, g);                      \
   } while (0)
@@ -880,7 +877,7 @@ template <typename T, int BLOCK, int SPLIT> int launch_sdd_split(const SddArgs &
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, TT, TT, WG, WG, AK, BK, true, sdd_step<T, BLOCK>()>::SMEM_BYTES;            \
+    constexpr int SMEM = TileGemm<T, TT, TT, WG, WG, AK, BK, true>::SMEM_BYTES;            \
     if (g.parts > 1) hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, true>), grid, blockdim, SMEM, st, g); \
     else hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, false>), grid, blockdim, SMEM, st, g);         \
   } while (0)
@@ -927,7 +924,7 @@ template <typename T, int BLOCK, int TN_> int launch_xsd_bw(const XsdArgs &g0, b
   dim3 grid((unsigned)(n_wg * g.parts)), blockdim(256);
 #define BSP_XSD_LAUNCH(ST, DK, ON)                                                                               \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON, TileK<T>::TK>::SMEM_BYTES; \
+    constexpr int SMEM = TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON>::SMEM_BYTES; \
     if constexpr (sizeof(T) == 4)                                                                                \
       if (g.parts > 1) {                                                                                         \
         hipLaunchKernelGGL((k_xsd<T, BLOCK, TN_, ST, DK, ON, true>), grid, blockdim, SMEM, st, g);              \

@@ -519,8 +519,9 @@ template <typename T> int launch_rg_dl(const XsdArgs &g, bool sp_trans, bool dn_
 // every SIMD has all the blocks of a chunk to multiply, however they fall.  The dense operands of a chunk stay in registers
 // for all of its lines; a block is 2 LDS reads and 2 matrix instructions behind a bit of the chunk's mask.  Two stages of 80 KiB: one
 // workgroup a compute unit, which stays for many tiles, so that the next chunk is in flight while this one is multiplied, also where it
-// is the first of the next tile, during this one's stores.  What bounds it now is latency, of the chunk's loads, of the LDS reads
-// behind the branches and at the tile's end: matrix units busy 22 % of the cycles, LDS 20 %, a feed of 7.8 TB/s where 11.6 were reached.
+// is the first of the next tile, during this one's stores.  What bounds it now is the chunk's loads, of which one chunk's are in flight:
+// 1060 us take 700 without them and 1000 without the products (matrix units busy 22 % of the cycles, LDS 20 %, 8 TB/s into LDS where
+// whole lines from L2 reach 35).  Touching the lines of the chunk after next, so that they are in L2 by then: 1200.
 // 16 heads of 64 x 64 blocks, a quarter of them there, batch 8, free dimension 2048, fp16: 1175 -> 1054 us (519 TFLOP/s), with the dense
 // operand's reduction contiguous 1500 -> 1045.  A workgroup a tile with the whole tile staged in LDS at its end: 1277; the results
 // stored from registers: 1105.

@@ -111,6 +111,25 @@ def test_values_without_parts(where, value, block, D):
         assert float((g[1, 0] - c[1, 0]).norm() / c[1, 0].norm()) < 2e-6
 
 
+# A mask value that makes NaN of the rows that see its key: no other row takes notice, also where the key's tile is theirs
+@pytest.mark.parametrize('value', [float('nan'), float('inf')])
+@pytest.mark.parametrize('block,D', [(16, 64), (32, 64), (16, 128), (32, 128)])
+def test_mask_values_of_keys_that_a_row_does_not_see(value, block, D):
+    torch.manual_seed(block + D)
+    n = 256 // block
+    lay = _layout(2, n, n, 'random')
+    ops = _ops(lay, block)
+    q, k, v, do = [torch.randn(2, 2, 256, D, device=DEV) for _ in range(4)]
+    kpm = torch.zeros(2, 256, device=DEV)
+    kpm[0, 101] = value
+    got, other = [_run(ops, q, k, v, do, fused, scale=D ** -0.5, key_padding_mask=kpm) for fused in (True, False)]
+    for name, g, c in zip(('o', 'dq', 'dk', 'dv'), got, other):
+        finite = torch.isfinite(c)
+        assert bool((torch.isfinite(g) == finite).all()) and bool((torch.isnan(g) == torch.isnan(c)).all()), name
+        assert float((g[finite] - c[finite]).norm() / c[finite].norm()) < 2e-6, name
+    assert bool(torch.isfinite(got[0][0]).any()) and bool(torch.isnan(got[0][0]).any())
+
+
 def test_padding_values_that_leave_no_score():
     """The lowest finite value (and -1e9) on every key of a sequence: fp32 rounds the scores away beside it and every key gets the same
     share, as from the operators; -inf on every key gives NaN for that sequence alone."""

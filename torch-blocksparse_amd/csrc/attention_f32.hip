@@ -467,14 +467,16 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           for_16<0>([&](auto ic) { s[decltype(ic)::value] = KPM ? fmaf(s[decltype(ic)::value], sc, row_bcast<decltype(ic)::value>(kp)) : s[decltype(ic)::value] * sc; });
           float sum;
           auto exponentials = [&]() {
-            const float ms = m == -INFINITY ? 0.f : m, off[2] = {here0 ? ms : INFINITY, here1 ? ms : INFINITY};
+            const float ms = m == -INFINITY ? 0.f : m;
+#pragma unroll
+            for (int i = 0; i < 16; i++) e[i] = __builtin_amdgcn_exp2f(s[i] - ms);
+            if ((here & 0x33) != 0x33) {                // (whatever the logits came out as there: a mask may hold NaN or an infinity, the scale may make one)
+#pragma unroll
+              for (int i = 0; i < 16; i++) e[i] = (i < 8 ? here0 : here1) ? e[i] : 0.f;
+            }
             sum = 0.f;
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-              e[i] = __builtin_amdgcn_exp2f(s[i] - off[i >> 3]);
-              if constexpr (W) e[i] = (i < 8 ? here0 : here1) ? e[i] : 0.f;            // (the score may be anything there)
-              sum += e[i];
-            }
+            for (int i = 0; i < 16; i++) sum += e[i];
           };
           exponentials();
           if (__builtin_amdgcn_ballot_w64(!(sum <= 8192.f) || m == -INFINITY)) {      // (also where an exponential overflowed)

@@ -111,6 +111,30 @@ def test_values_without_parts(where, value, block, D):
         assert float((g[1, 0] - c[1, 0]).norm() / c[1, 0].norm()) < 2e-6
 
 
+# Scores so large that one unit of theirs in the last place counts in the softmax, and one value elsewhere in the head that sends products to
+# the fp32 units: the backward kernels must have the forward pass's scores, bit for bit, for every other row.  Bound: four times the
+# operators' error, relative 2-norm over the rows and keys that have nothing to do with the value (both errors are the rounding of the
+# scores in the few rows with two shares of the same size; scores of two kinds make it eight times and more).
+@pytest.mark.parametrize('where', ['q', 'do'])
+@pytest.mark.parametrize('block,D', [(64, 64), (32, 128)])
+@pytest.mark.parametrize('large', [100., 1000.])
+def test_all_passes_have_the_same_scores(where, block, D, large):
+    torch.manual_seed(block + D)
+    n = 512 // block
+    lay = _layout(2, n, n, 'random')
+    lay[:, 0, n // 2:] = 0                                                # (keys that the value's row does not see)
+    x = {t: torch.randn(1, 2, 512, D, device=DEV) for t in ('q', 'k', 'v', 'do')}
+    x['q'] *= large
+    x[where][0, 1, 7, 5] = 2. ** 31
+    ops = _ops(lay, block)
+    got, other = [_run(ops, x['q'], x['k'], x['v'], x['do'], fused, scale=D ** -0.5) for fused in (True, False)]
+    ref = _dense(x['q'], x['k'], x['v'], x['do'], lay, block, D ** -0.5)
+    for name, g, c, r in zip(('o', 'dq', 'dk', 'dv'), got, other, ref):
+        part = (0, 1, slice(64, None)) if name in ('o', 'dq') else (0, 1, slice(256, None))
+        err, bound = [float((t[part].double() - r[part]).norm() / r[part].norm()) for t in (g, c)]
+        assert err <= 4 * bound + 2 ** -23, (name, err, bound)
+
+
 # A mask value that makes NaN of the rows that see its key: no other row takes notice, also where the key's tile is theirs
 @pytest.mark.parametrize('value', [float('nan'), float('inf')])
 @pytest.mark.parametrize('block,D', [(16, 64), (32, 64), (16, 128), (32, 128)])

@@ -29,9 +29,7 @@ namespace {
 
 struct F32Args : QuadArgs {            // k, v: the planes; q: forward q itself, backward the planes; d_o: row kernel do itself, column kernel
                                        // the planes; lse: per row the reference m of its exponentials, rest floats on 1 / l
-  bf16 *planes_out;                    // forward: planes of q (NULL: no backward pass to follow); row kernel: planes of do
-  int32_t *flags_out;                  // ... and their flags
-  const int32_t *fq, *fk, *fv, *fdo;   // flags [Z][H]: of 32 rows each (q, do) or 64 (k, v)
+  const int32_t *fq, *fk, *fv, *fdo;   // flags [Z][H][pieces of 64 rows]; fq (forward) and fdo (row kernel) NULL: not there, no other kernel follows
   int64_t rows, keys;
   int sub;                             // column kernel: pieces that a part of a long column is cut into
 };
@@ -105,9 +103,10 @@ template <int D> struct Ring {
 // acc[i] += (32 rows of the piece, dealt by deal_row) . b, as in attention_quad.h
 // The scores come out the same, bit for bit, with the rows of q or those of k in LDS (SWAP: the parts of b are taken as the first factor's), so
 // that the backward pass has the forward pass's probabilities however large the scores are.
-// (WHOLE: b is fetched again for each product, from its planes or as it is, which leaves its registers to the fp32 units' way of working)
-template <bool WHOLE, bool SWAP, int D, typename S>
-__device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const RowReads<D, true> &reads, const Parts (&b)[D / 16], const S *b_row, f32x16 acc) {
+// (FETCH: b is fetched again for each product, from its planes or as it is, which leaves its registers to the fp32 units' way of working;
+// by_parts: the product is made of parts all the same, which only planes can be)
+template <bool FETCH, bool SWAP, int D, typename S>
+__device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const RowReads<D, true> &reads, const Parts (&b)[D / 16], const S *b_row, bool by_parts, f32x16 acc) {
   uint32_t at[D / 16];
   reads.get(at);
 #pragma unroll
@@ -115,7 +114,12 @@ __device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const R
     Parts f;
 #pragma unroll
     for (int p = 0; p < 3; p++) f.p[p] = *reinterpret_cast<const bf16x8 *>(piece + p * Ring<D>::PLANE + at[s]);
-    if constexpr (WHOLE) {
+    auto terms = [&](const Parts &own) {
+      const Parts &x = SWAP ? own : f, &y = SWAP ? f : own;
+      auto term = [&](int i, int j) { acc = SWAP ? mma(y.p[j], x.p[i], acc) : mma(x.p[i], y.p[j], acc); };
+      term(2, 0); term(0, 2); term(1, 1); term(0, 1); term(1, 0); term(0, 0);
+    };
+    if constexpr (FETCH) {
       asm volatile("" : "+v"(b_row));
       if constexpr (sizeof(S) == 4) {
         const f32x4 lo = *reinterpret_cast<const f32x4 *>(b_row + 16 * s), hi = *reinterpret_cast<const f32x4 *>(b_row + 16 * s + 4);
@@ -124,12 +128,15 @@ __device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const R
         Parts mine;
 #pragma unroll
         for (int p = 0; p < 3; p++) mine.p[p] = *reinterpret_cast<const bf16x8 *>(b_row + p * D + 16 * s);
-        acc = whole_parts_product(f, mine, acc);
+        if (by_parts) {
+          terms(mine);
+          __builtin_amdgcn_sched_barrier(0);
+        } else {
+          acc = whole_parts_product(f, mine, acc);
+        }
       }
     } else {
-      const Parts &x = SWAP ? b[s] : f, &y = SWAP ? f : b[s];
-      auto term = [&](int i, int j) { acc = SWAP ? mma(y.p[j], x.p[i], acc) : mma(x.p[i], y.p[j], acc); };
-      term(2, 0); term(0, 2); term(1, 1); term(0, 1); term(1, 0); term(0, 0);
+      terms(b[s]);
     }
   }
   return acc;
@@ -221,6 +228,12 @@ __device__ __forceinline__ int32_t flags_of(const int32_t *f, int64_t zh, int64_
   int32_t set = f[zh * n + (lane < n ? lane : 0)];
   for (int64_t i = lane + 64; i < n; i += 64) set |= f[zh * n + i];
   return set;
+}
+
+// The way of a product is the head's (n_rows: pieces of 64 rows of q): the scores' that of the forward pass, which knows q, k and v, so that the
+// backward kernels have its probabilities also where only do is flagged.
+__device__ __forceinline__ int32_t forward_flags(const F32Args &a, int64_t zh, int64_t n_rows, int lane) {
+  return flags_of(a.fq, zh, n_rows, lane) | flags_of(a.fk, zh, a.keys / 64, lane) | flags_of(a.fv, zh, a.keys / 64, lane);
 }
 
 // the wavefront's sixteen rows of a piece (its group), three planes
@@ -332,9 +345,8 @@ template <int D> __device__ __forceinline__ void fetch_row(f32x4 (&v)[D / 8], co
 #pragma unroll
     for (int j = 0; j < 2; j++) v[2 * s + j] = *reinterpret_cast<const f32x4 *>(row + 16 * s + 4 * j);
 }
-// its parts; those of the steps s that are `mine` also to the planes row `out` unless NULL.  -> does it (in this lane) hold a value that is
-// not below kLargest?
-template <int D> __device__ __forceinline__ int take_parts(Parts (&f)[D / 16], const f32x4 (&v)[D / 8], bf16 *out, int mine) {
+// its parts.  -> does it (in this lane) hold a value that is not below kLargest?
+template <int D> __device__ __forceinline__ int take_parts(Parts (&f)[D / 16], const f32x4 (&v)[D / 8]) {
   int large = 0;
 #pragma unroll
   for (int s = 0; s < D / 16; s++) {
@@ -345,36 +357,35 @@ template <int D> __device__ __forceinline__ int take_parts(Parts (&f)[D / 16], c
       large |= !(fabsf(e[j]) < kLargest);
     }
     f[s] = split8<true>(e);
-    if (out != nullptr && (s & 1) == mine) {
-#pragma unroll
-      for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8 *>(out + p * D + 16 * s) = f[s].p[p];
-    }
   }
   return large;
 }
 
 // ---- planes ----
 struct PlaneArgs {
-  const float *x[2];
-  bf16 *planes[2];
-  int32_t *flags[2];
-  int64_t sz[2], sh[2], ld[2];
-  int chunks, H;                       // pieces of 64 rows of a head; heads of a batch
-  uint32_t per_tensor;                 // workgroups
+  struct Tensor {
+    const float *x;
+    bf16 *planes;
+    int32_t *flags;
+    int64_t sz, sh, ld;
+    uint32_t chunks, end;              // pieces of 64 rows of a head; the first workgroup behind the tensor's
+  } t[3];
+  int H;                               // heads of a batch
 };
 template <int D> __global__ void __launch_bounds__(256) k_attn32_planes(PlaneArgs a) {
-  const int t = blockIdx.x >= a.per_tensor;
-  const uint32_t wg = blockIdx.x - t * a.per_tensor;
-  const Quotient head(wg, a.chunks), zh(head.q, a.H);
-  const float *x = a.x[t] + zh.q * a.sz[t] + zh.r * a.sh[t] + (int64_t)head.r * 64 * a.ld[t];
-  bf16 *to = a.planes[t] + (int64_t)wg * (64 * 3 * D);
+  const int t = blockIdx.x < a.t[0].end ? 0 : blockIdx.x < a.t[1].end ? 1 : 2;
+  const PlaneArgs::Tensor &own = a.t[t];
+  const uint32_t wg = blockIdx.x - (t ? a.t[t - 1].end : 0u);
+  const Quotient head(wg, own.chunks), zh(head.q, a.H);
+  const float *x = own.x + zh.q * own.sz + zh.r * own.sh + (int64_t)head.r * 64 * own.ld;
+  bf16 *to = own.planes + (int64_t)wg * (64 * 3 * D);
   int large = 0;
   constexpr int PER = 64 * D / 8 / 256;
   f32x4 v[PER][2];
 #pragma unroll
   for (int i = 0; i < PER; i++) {
     const int c = threadIdx.x + 256 * i, row = c / (D / 8), col = 8 * (c % (D / 8));
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(x + row * a.ld[t] + col);
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(x + row * own.ld + col);
     v[i][0] = src[0]; v[i][1] = src[1];
   }
 #pragma unroll
@@ -391,7 +402,7 @@ template <int D> __global__ void __launch_bounds__(256) k_attn32_planes(PlaneArg
     for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8 *>(to + row * (3 * D) + p * D + col) = s.p[p];
   }
   const int any = __syncthreads_or(large);
-  if (threadIdx.x == 0) a.flags[t][wg] = any;
+  if (threadIdx.x == 0) own.flags[wg] = any;
 }
 
 // ---- forward ----
@@ -417,11 +428,6 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     for (int i = 0; i < 16; i++) o[mt][i] = 0.f;
   float m = -INFINITY, l = 0.f;
   int rows_seen = 0;
-  bf16 *q_out = a.planes_out ? a.planes_out + (zh * a.rows + row) * (3 * D) + 8 * half : nullptr;
-  auto put_flag = [&](int large) {
-    const bool any = __builtin_amdgcn_ballot_w64(large != 0);
-    if (q_out != nullptr && kh == 0 && lane == 0) a.flags_out[(zh * a.rows + row) / 32] = any;
-  };
 
   if (tiles > 0) {
     Parts xq[D / 16];
@@ -458,7 +464,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           f32x16 s;
 #pragma unroll
           for (int i = 0; i < 16; i++) s[i] = 0.f;
-          s = rows_times<W, false, D>(smem + x * R::PIECE, rows_k, xq, q_row, s);
+          s = rows_times<W, false, D>(smem + x * R::PIECE, rows_k, xq, q_row, false, s);
           here = bits_next >> (8 * rh + 2 * kh);
           rows_seen |= here & 0x33;
           const float kp = KPM ? pad_term(kp_lane[x * (R::SIDE / 4)], a.kpm_mul) : 0.f;
@@ -505,16 +511,10 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     f32x4 q[D / 8];
     fetch_row<D>(q, q_row);
     int large = flags_of(a.fk, zh, a.keys / 64, lane) | flags_of(a.fv, zh, a.keys / 64, lane);
-    const int mine = take_parts<D>(xq, q, q_out, kh);
-    put_flag(mine);
-    large |= mine;
+    const int mine = take_parts<D>(xq, q);
+    large |= a.fq ? flags_of(a.fq, zh, a.R, lane) : mine;
     if (__builtin_amdgcn_ballot_w64(large != 0)) run(Const<1>{});
     else run(Const<0>{});
-  } else if (q_out != nullptr) {                        // (the column kernel multiplies nothing of these rows, but takes the head's flags)
-    Parts none[D / 16];
-    f32x4 q[D / 8];
-    fetch_row<D>(q, reinterpret_cast<const float *>(a.q) + z * a.q_sz + h * a.q_sh + row * a.q_ld + 8 * half);
-    put_flag(take_parts<D>(none, q, q_out, kh));
   }
 
   // the two halves of the columns, each with its own reference m
@@ -570,7 +570,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
     for (int i = 0; i < 16; i++) dq[mt][i] = 0.f;
-  // the rows' do: its parts, also for the column kernel, and delta
+  // the rows' do, and delta
   const float *do_row = reinterpret_cast<const float *>(a.d_o) + z * a.do_sz + h * a.do_sh + row * a.do_ld + 8 * half;
   const float *o_row = reinterpret_cast<const float *>(a.o_in) + z * a.oin_sz + h * a.oin_sh + row * a.oin_ld + 8 * half;
   auto sums = [&](const f32x4 (&d)[D / 8], const f32x4 (&o)[D / 8]) {
@@ -583,18 +583,11 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     if (a.delta != nullptr && half == 0 && kh == 0) a.delta[zh * a.rows + row] = -delta;
     return delta;
   };
-  bf16 *do_out = a.planes_out ? a.planes_out + (zh * a.rows + row) * (3 * D) + 8 * half : nullptr;
-  auto put_flag = [&](int large) {
-    const bool any = __builtin_amdgcn_ballot_w64(large != 0);
-    if (do_out != nullptr && kh == 0 && lane == 0) a.flags_out[(zh * a.rows + row) / 32] = any;
-  };
   if (tiles == 0) {
-    Parts none[D / 16];
     f32x4 g[D / 8], o[D / 8];
     fetch_row<D>(g, do_row);
     fetch_row<D>(o, o_row);
     sums(g, o);
-    put_flag(take_parts<D>(none, g, do_out, kh));
   }
 
   if (tiles > 0) {
@@ -628,11 +621,11 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     fetch_row<D>(g, do_row);
     fetch_row<D>(o, o_row);
     load_parts<D>(xq, q_row);
-    int large = a.fq[(zh * a.rows + row) / 32] | flags_of(a.fk, zh, a.keys / 64, lane) | flags_of(a.fv, zh, a.keys / 64, lane);
+    int large = forward_flags(a, zh, a.R, lane);
+    const bool by_parts = !__builtin_amdgcn_ballot_w64(large != 0);   // the scores, as in the forward pass
     const float delta = sums(g, o);
-    const int mine = take_parts<D>(xo, g, do_out, kh);
-    put_flag(mine);
-    large |= mine;
+    const int mine = take_parts<D>(xo, g);
+    large |= a.fdo ? flags_of(a.fdo, zh, a.R, lane) : mine;
     f32x16 dp;
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
@@ -642,13 +635,13 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           here = bits_next >> (8 * rh + 2 * kh);
 #pragma unroll
           for (int i = 0; i < 16; i++) dp[i] = 0.f;
-          dp = rows_times<W, false, D>(smem + x * R::PIECE, rows, xo, do_row, dp);
+          dp = rows_times<W, false, D>(smem + x * R::PIECE, rows, xo, do_row, false, dp);
         },
         [&](int y, int) {
           f32x16 s;
 #pragma unroll
           for (int i = 0; i < 16; i++) s[i] = 0.f;
-          s = rows_times<W, false, D>(smem + y * R::PIECE, rows, xq, q_row, s);
+          s = rows_times<W, false, D>(smem + y * R::PIECE, rows, xq, q_row, by_parts, s);
           const float kp = KPM ? pad_term(kp_lane[y * (R::SIDE / 4)], a.kpm_mul) : 0.f;
           const int mine = here >> ((lane >> 4) & 1) * 4;
           float e[16];                                  // (1 / l of the row comes last, on dq)
@@ -747,6 +740,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
       bits_next = core[kEntry * (n + 1 < tiles ? n + 1 : n) + 4];
     };
     float p[16];
+    bool by_parts;
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
       if constexpr (!W) {
@@ -759,7 +753,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           f32x16 s;
 #pragma unroll
           for (int i = 0; i < 16; i++) s[i] = 0.f;
-          s = rows_times<W, true, D>(smem + x * R::PIECE, rows, xk, k_row, s);
+          s = rows_times<W, true, D>(smem + x * R::PIECE, rows, xk, k_row, by_parts, s);
           here = bits >> (2 * kh + 8 * rh);
 #pragma unroll
           for (int g = 0; g < 4; g++) {
@@ -783,7 +777,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
 #pragma unroll
             for (int i = 0; i < 4; i++) dp[4 * g + i] = nd[i];
           }
-          dp = rows_times<W, false, D>(smem + y * R::PIECE, rows, xv, v_row, dp);
+          dp = rows_times<W, false, D>(smem + y * R::PIECE, rows, xv, v_row, false, dp);
           float e[16];
 #pragma unroll
           for (int i = 0; i < 16; i++) e[i] = p[i] * dp[i];
@@ -802,7 +796,9 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     // the column's own rows through the slots that are free yet: fetched by whole lines
     load.issue(reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D)), head[8 + wave], lds_address(smem) + R::PIECE, wave);
     load.issue(reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D)), head[8 + wave], lds_address(smem) + 2 * R::PIECE, wave);
-    const int large = flags_of(a.fq, zh, a.rows / 32, lane) | flags_of(a.fdo, zh, a.rows / 32, lane) | flags_of(a.fk, zh, a.keys / 64, lane) | flags_of(a.fv, zh, a.keys / 64, lane);
+    int large = forward_flags(a, zh, a.rows / 64, lane);
+    by_parts = !__builtin_amdgcn_ballot_w64(large != 0);
+    large |= flags_of(a.fdo, zh, a.rows / 64, lane);
     wait_barrier<0>();
     if (__builtin_amdgcn_ballot_w64(large != 0)) run(Const<1>{});
     else run(Const<0>{});
@@ -881,8 +877,8 @@ template <int WHICH> int launch_d(const F32Args &a, int D, int64_t n_wg, hipStre
   return a.kpm ? launch<128, true, WHICH>(a, (unsigned)n_wg, st) : launch<128, false, WHICH>(a, (unsigned)n_wg, st);
 }
 
-// planes of a tensor of n rows in all: [n][3][D] bf16, then its flags, at most one int for 32 rows; a multiple of 16 bytes
-inline int64_t plane_bytes(int64_t n, int D) { return n * 3 * D * 2 + (n / 32 * 4 + 15) / 16 * 16; }
+// planes of a tensor of n rows in all: [n][3][D] bf16, then its flags, an int for 64 rows; a multiple of 16 bytes
+inline int64_t plane_bytes(int64_t n, int D) { return n * 3 * D * 2 + (n / 64 * 4 + 15) / 16 * 16; }
 inline int32_t *flags_in(void *planes, int64_t n, int D) { return reinterpret_cast<int32_t *>(reinterpret_cast<char *>(planes) + n * 3 * D * 2); }
 
 // sizes, 16-byte alignment of pointers (NULL is aligned) and strides (n tensors: batch, head, row; multiples of 4 floats), rows that hold D
@@ -917,6 +913,32 @@ F32Args f32_args(const bsp_attention_f32_call &c) {
 }
 void take_strides(const int64_t *s, int64_t &z, int64_t &h, int64_t &row) { z = s[0]; h = s[1]; row = s[2]; }
 
+// the planes of up to three tensors of rows rows a head and their flags (no planes: left out)
+struct ToPlanes { const float *x; const void *planes; const int64_t *strides; int64_t rows; };
+int launch_planes(const bsp_attention_f32_call &c, const ToPlanes (&tensors)[3], hipStream_t st) {
+  const int64_t heads = (int64_t)c.Z * c.H;
+  PlaneArgs pl{};
+  pl.H = c.H;
+  int64_t end = 0;
+  for (int i = 0; i < 3; i++) {
+    const ToPlanes &from = tensors[i];
+    PlaneArgs::Tensor &t = pl.t[i];
+    if (from.planes) {
+      t.x = from.x;
+      t.planes = reinterpret_cast<bf16 *>(const_cast<void *>(from.planes));
+      t.flags = flags_in(t.planes, heads * from.rows, c.D);
+      take_strides(from.strides, t.sz, t.sh, t.ld);
+      t.chunks = (uint32_t)(from.rows / 64);
+      end += heads * t.chunks;
+    }
+    if (end >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
+    t.end = (uint32_t)end;
+  }
+  if (c.D == 64) hipLaunchKernelGGL(k_attn32_planes<64>, dim3((unsigned)end), dim3(256), 0, st, pl);
+  else hipLaunchKernelGGL(k_attn32_planes<128>, dim3((unsigned)end), dim3(256), 0, st, pl);
+  return BSP_OK;
+}
+
 // Pieces of the parts of long columns.  A part is up to sixteen tiles, eight times as long as the short columns of the layouts that have
 // any: a launch whose parts do not fill the chip (two workgroups a CU, 512) ends with them alone and does better on halves, though each costs
 // a workgroup's first loads and a slot written and read once more.  Column kernel in 1 / 2 / 4 pieces, 8 heads of 2048 positions, stride 128 of blocks of
@@ -940,24 +962,11 @@ extern "C" int bsp_attention_f32_fwd(const bsp_attention_f32_call *c, const floa
   const int rc = f32_check(*c, ptrs, 7, 4);
   if (rc != BSP_OK) return rc;
   F32Args a = f32_args(*c);
-  const int64_t heads = (int64_t)a.Z * a.H, per_tensor = heads * (a.keys / 64);
-  if (2 * per_tensor >= ((int64_t)1 << 31)) return BSP_ERR_UNSUPPORTED;
-  PlaneArgs pl{};
-  pl.x[0] = k; pl.x[1] = v;
-  const void *const to[] = {a.k, a.v};
-  pl.chunks = (int)(a.keys / 64); pl.H = a.H; pl.per_tensor = (uint32_t)per_tensor;
-  for (int t = 0; t < 2; t++) {
-    pl.planes[t] = reinterpret_cast<bf16 *>(const_cast<void *>(to[t]));
-    pl.flags[t] = flags_in(pl.planes[t], heads * a.keys, c->D);
-    take_strides(c->strides + 3 * (t + 1), pl.sz[t], pl.sh[t], pl.ld[t]);
-  }
+  const int64_t heads = (int64_t)a.Z * a.H;
   hipStream_t st = as_stream(stream);
-  if (c->D == 64) hipLaunchKernelGGL(k_attn32_planes<64>, dim3((unsigned)(2 * per_tensor)), dim3(256), 0, st, pl);
-  else hipLaunchKernelGGL(k_attn32_planes<128>, dim3((unsigned)(2 * per_tensor)), dim3(256), 0, st, pl);
-  if (c->stats) {
-    a.planes_out = reinterpret_cast<bf16 *>(const_cast<void *>(a.q));
-    a.flags_out = const_cast<int32_t *>(a.fq);
-  }
+  const int rp = launch_planes(*c, {{k, a.k, c->strides + 3, a.keys}, {v, a.v, c->strides + 6, a.keys}, {q, c->stats ? a.q : nullptr, c->strides, a.rows}}, st);
+  if (rp != BSP_OK) return rp;
+  if (!c->stats) a.fq = nullptr;
   a.q = q;
   take_strides(c->strides, a.q_sz, a.q_sh, a.q_ld);
   a.o = o;
@@ -981,11 +990,11 @@ extern "C" int bsp_attention_f32_bwd(const bsp_attention_f32_call *c, const floa
   if (dk && (n_items < (int64_t)a.H * (a.keys / 64) || n_items > (int64_t)a.H * (a.keys / 64) + n_slots || (int64_t)a.Z * n_items * a.sub >= ((int64_t)1 << 31) ||
              (int64_t)a.Z * n_split * 16 >= ((int64_t)1 << 31))) return BSP_ERR_ARG;
   hipStream_t st = as_stream(stream);
-  const int64_t n = (int64_t)a.Z * a.H * a.rows;
   a.d_o = d_o; a.o_in = o;
   if (dk) {
-    a.planes_out = reinterpret_cast<bf16 *>(do_planes);
-    a.flags_out = flags_in(do_planes, n, c->D);
+    const int rp = launch_planes(*c, {{d_o, do_planes, c->strides, a.rows}}, st);
+    if (rp != BSP_OK) return rp;
+    a.fdo = flags_in(do_planes, (int64_t)a.Z * a.H * a.rows, c->D);
     a.delta = neg_delta;
   }
   take_strides(c->strides, a.do_sz, a.do_sh, a.do_ld);
@@ -995,7 +1004,7 @@ extern "C" int bsp_attention_f32_bwd(const bsp_attention_f32_call *c, const floa
   int rl = launch_d<1>(a, c->D, (int64_t)a.Z * a.H * a.R, st);
   if (rl != BSP_OK) return rl;
   if (dk) {
-    a.d_o = do_planes; a.fdo = a.flags_out;
+    a.d_o = do_planes;
     take_strides(c->strides + 9, a.o_sz, a.o_sh, a.o_ld);
     take_strides(c->strides + 12, a.o2_sz, a.o2_sh, a.o2_ld);
     a.o = dk; a.o2 = dv; a.lut = d_items; a.R = n_items;

@@ -460,7 +460,7 @@ int bsp_attention_cols_bwd(int dtype, const void *d_o, const void *q, const void
  * elements, three per tensor in the order of the call's tensor arguments (fwd: q, k, v, o; bwd: d_o, o, dq, dk, dv); multiples of 4,
  * unit inner stride, 16-byte aligned pointers.  kpm: element (z, key) at kpm[z * kpm_stride_z + key], or NULL.
  * planes: bsp_attention_f32_bytes(Z, H, 64 R, keys, D) bytes (rows 0 where stats is NULL), written by fwd and read by bwd.  stats:
- * [Z][H][2][64 R] floats, written by fwd (NULL: no backward pass to follow) and read by bwd: the reference of the row's exponentials (log2
+ * [Z][H][2][64 R] floats, written by fwd (NULL: no backward pass to follow) and read by bwd: the reference of the row's exponentials (natural
  * domain), one over their sum.
  * bwd: do_planes: bsp_attention_f32_bytes(Z, H, 64 R, 0, D) bytes of scratch; neg_delta: [Z][H][64 R] floats of scratch.  dk and dv are
  * computed together; without them (both NULL) do_planes, neg_delta and what follows may be NULL and 0.  d_items .. n_split: as for

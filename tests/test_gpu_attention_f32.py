@@ -172,6 +172,25 @@ def test_padding_values_that_leave_no_score():
             assert float((got[0][0] - other[0][0]).norm() / other[0][0].norm()) < 2e-6
 
 
+# Finite padding on every key of a sequence: the logits are rounded where they lie beside it, which is most of the error, and no more than
+# the softmax operator rounds them.  Against 64 bits; a tenth for what rounding by other scores' last bits may do to it.
+@pytest.mark.parametrize('value', [-100., -300., -1000., -10000., -65504., 1000.])
+@pytest.mark.parametrize('block,D', [(32, 64), (64, 128)])
+def test_padded_sequences_against_64_bits(value, block, D):
+    torch.manual_seed(block)
+    n = 256 // block
+    lay = _layout(2, n, n, 'random')
+    ops = _ops(lay, block)
+    q, k, v, do = [torch.randn(2, 2, 256, D, device=DEV) for _ in range(4)]
+    kpm = torch.zeros(2, 256, device=DEV)
+    kpm[0] = value
+    ref = _dense(q, k, v, do, lay, block, D ** -0.5, kpm)
+    got, other = [_run(ops, q, k, v, do, fused, scale=D ** -0.5, key_padding_mask=kpm) for fused in (True, False)]
+    for name, g, c, r in zip(('o', 'dq', 'dk', 'dv'), got, other, ref):
+        err, bound = [float((x.double() - r).norm() / r.norm()) for x in (g, c)]
+        assert err <= 1.1 * bound + 2 ** -23, (name, err, bound)
+
+
 def test_operands_that_are_copied_and_inference():
     """Odd strides, an expanded gradient, gradients of some operands only, and a forward pass alone (which keeps no parts of q)."""
     torch.manual_seed(4)

@@ -21,7 +21,7 @@
 #include "attention_quad.h"
 #include <atomic>
 
-// (a multiplication and the subtraction behind it stay two roundings: see pad_term)
+// (a multiplication and the addition behind it stay two roundings, as in the operators)
 #pragma clang fp contract(off)
 
 namespace bsp {
@@ -209,13 +209,22 @@ __device__ __forceinline__ void columns_times(f32x16 (&acc)[D / 32], uint32_t pi
   }
 }
 
-// key-padding value -> addend of the logits (softmax.py:104-106, 122-124), which are in the log2 domain and rounded to fp32 before the row's
-// reference m is taken off, as the softmax operator does it (so that a padding value of -1e9 leaves nothing of a score).
-// (Finite values stay finite: the lowest one is a usual padding value, and a row of nothing else has equal shares.)
-__device__ __forceinline__ float pad_term(float v, int mul) {
-  const float t = v * kLog2e;
-  return mul ? (v == 0.f ? -INFINITY : 0.f) : fabsf(v) < INFINITY && fabsf(t) == INFINITY ? copysignf(3.402823466e38f, v) : t;
+// Logits are what the softmax operator forms in fp32, in the natural domain and rounded once: score * scale + mask.
+// key-padding value -> mask (softmax.py:104-106, 122-124)
+__device__ __forceinline__ float pad_term(float v, int mul) { return mul ? (v == 0.f ? -INFINITY : 0.f) : v; }
+
+// e^y for y up to some ten.  v_exp_f32 of the rounded product y log2 e, times one plus what its rounding left out: within two units in the last
+// place for every y, where the product alone is off by |y| / 2 of them.  (Below -87 zero.  WHOLE: the library's, whose tiny values
+// make infinities of infinities as the operators' do.)
+template <bool WHOLE> __device__ __forceinline__ float exp_of(float y) {
+  if constexpr (WHOLE) return expf(y);
+  constexpr double kLn2 = 0.69314718055994530942;
+  constexpr float hi = (float)kLn2, lo = (float)(kLn2 - (double)hi);
+  y = __builtin_elementwise_maximum(y, -110.f);         // (NaN stays; minus infinity would become it)
+  const float product = y * kLog2e, left = fmaf(product, -lo, fmaf(product, -hi, y)), e = __builtin_amdgcn_exp2f(product);
+  return fmaf(e, left, e);
 }
+
 // The work of a workgroup.  The tables have the long lines (columns) of four heads at a time first; from eight such groups on each XCD takes
 // its own ones, so that their rows meet in its L2.  Fewer groups would leave the XCDs that begin in the middle of one with its short lines alone: they
 // are dealt in turn.
@@ -432,7 +441,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   if (tiles > 0) {
     Parts xq[D / 16];
     const float *q_row = reinterpret_cast<const float *>(a.q) + z * a.q_sz + h * a.q_sh + row * a.q_ld + 8 * half;
-    const float sc = a.scale * kLog2e;
+    const float sc = a.scale;
     const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D));
     const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D));
     const char *pkpm = reinterpret_cast<const char *>(reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz);
@@ -475,7 +484,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           auto exponentials = [&]() {
             const float ms = m == -INFINITY ? 0.f : m;
 #pragma unroll
-            for (int i = 0; i < 16; i++) e[i] = __builtin_amdgcn_exp2f(s[i] - ms);
+            for (int i = 0; i < 16; i++) e[i] = exp_of<W>(s[i] - ms);
             if ((here & 0x33) != 0x33) {                // (whatever the logits came out as there: a mask may hold NaN or an infinity, the scale may make one)
 #pragma unroll
               for (int i = 0; i < 16; i++) e[i] = (i < 8 ? here0 : here1) ? e[i] : 0.f;
@@ -489,7 +498,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
             float top = -INFINITY;
 #pragma unroll
             for (int i = 0; i < 16; i++) top = fmaxf(top, (i < 8 ? here0 : here1) ? s[i] : -INFINITY);
-            const float mn = fmaxf(m, fmaxf(top, swap32(top))), f = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+            const float mn = fmaxf(m, fmaxf(top, swap32(top))), f = exp_of<W>(m - (mn == -INFINITY ? 0.f : mn));
             l *= f;
 #pragma unroll
             for (int mt = 0; mt < MT; mt++)
@@ -531,7 +540,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   if (!kh) {
     const float m1 = other[16 * MT * 64 + lane], l1 = other[16 * MT * 64 + 64 + lane];
     rows_seen |= reinterpret_cast<const int *>(other)[16 * MT * 64 + 128 + lane];
-    const float top = fmaxf(m, m1), ms = top == -INFINITY ? 0.f : top, f0 = __builtin_amdgcn_exp2f(m - ms), f1 = __builtin_amdgcn_exp2f(m1 - ms);
+    const float top = fmaxf(m, m1), ms = top == -INFINITY ? 0.f : top, f0 = exp_of<false>(m - ms), f1 = exp_of<false>(m1 - ms);
     const float sum = l * f0 + l1 * f1;
     const bool any_block = (rows_seen >> 4 * ((lane >> 4) & 1)) & 15;
     const float inv = any_block ? 1.f / sum : 0.f;      // masked everywhere: 0 * inf = NaN, as the softmax operator gives; no block at all: zeros
@@ -593,7 +602,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   if (tiles > 0) {
     Parts xq[D / 16], xo[D / 16];
     const bf16 *q_row = reinterpret_cast<const bf16 *>(a.q) + (zh * a.rows + row) * (3 * D) + 8 * half;
-    const float sc = a.scale * kLog2e, m = a.lse[zh * a.row_sh + row];
+    const float sc = a.scale, m = a.lse[zh * a.row_sh + row];
     const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D));
     const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D));
     const char *pkpm = reinterpret_cast<const char *>(reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz);
@@ -647,7 +656,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           float e[16];                                  // (1 / l of the row comes last, on dq)
           for_16<0>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            e[i] = __builtin_amdgcn_exp2f((KPM ? fmaf(s[i], sc, row_bcast<i>(kp)) : s[i] * sc) - m) * (dp[i] - delta);
+            e[i] = exp_of<W>((KPM ? fmaf(s[i], sc, row_bcast<i>(kp)) : s[i] * sc) - m) * (dp[i] - delta);
           });
           if ((here & 0x33) != 0x33) {                  // pieces without a block
 #pragma unroll
@@ -713,7 +722,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     Parts xk[D / 16], xv[D / 16];
     const bf16 *k_row = reinterpret_cast<const bf16 *>(a.k) + (zh * a.keys + key) * (3 * D) + 8 * half;
     const bf16 *v_row = reinterpret_cast<const bf16 *>(a.v) + (zh * a.keys + key) * (3 * D) + 8 * half;
-    const float sc = a.scale * kLog2e, kp = KPM ? pad_term((reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz)[key], a.kpm_mul) : 0.f;
+    const float sc = a.scale, kp = KPM ? pad_term((reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz)[key], a.kpm_mul) : 0.f;
     const char *pq = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.q) + zh * a.rows * (3 * D));
     const char *pdo = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.d_o) + zh * a.rows * (3 * D));
     const char *pstat = reinterpret_cast<const char *>(a.lse + zh * a.row_sh), *pdelta = reinterpret_cast<const char *>(a.delta + zh * a.rows);
@@ -760,7 +769,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
             const float *at = rv + x * (R::SIDE / 4) + (g >> 1) * 128 + 4 * (g & 1);
             const f32x4 m = *reinterpret_cast<const f32x4 *>(at), inv = *reinterpret_cast<const f32x4 *>(at + 16);
 #pragma unroll
-            for (int i = 0; i < 4; i++) p[4 * g + i] = __builtin_amdgcn_exp2f((KPM ? fmaf(s[4 * g + i], sc, kp) : s[4 * g + i] * sc) - m[i]) * inv[i];
+            for (int i = 0; i < 4; i++) p[4 * g + i] = exp_of<W>((KPM ? fmaf(s[4 * g + i], sc, kp) : s[4 * g + i] * sc) - m[i]) * inv[i];
           }
           if ((here & 0x33) != 0x33) {                  // pieces without a block (a row that is masked everywhere has NaN here, which its other keys must not take up)
             const int mine = here >> ((lane >> 4) & 1);

@@ -95,14 +95,22 @@ __device__ __forceinline__ f32x16 whole_parts_product(const Parts &a, const Part
   return whole_product(a, [&](int i) { return whole(y, i); }, acc);
 }
 
+// the same of parts, in the order of the parts' sizes; SWAP: those of b count as the first factor's
+template <bool SWAP> __device__ __forceinline__ f32x16 parts_product(const Parts &a, const Parts &b, f32x16 acc) {
+  const Parts &x = SWAP ? b : a, &y = SWAP ? a : b;
+  auto term = [&](int i, int j) { acc = SWAP ? mma(y.p[j], x.p[i], acc) : mma(x.p[i], y.p[j], acc); };
+  term(2, 0); term(0, 2); term(1, 1); term(0, 1); term(1, 0); term(0, 0);
+  return acc;
+}
+
 template <int D> struct Ring {
   static constexpr int PLANE = 64 * D * 2, PIECE = 3 * PLANE, SIDE = 4 * 512;   // SIDE: two words a lane for each wavefront, beside a piece
   static constexpr int BYTES = 3 * (PIECE + SIDE);
 };
 
 // acc[i] += (32 rows of the piece, dealt by deal_row) . b, as in attention_quad.h
-// The scores come out the same, bit for bit, with the rows of q or those of k in LDS (SWAP: the parts of b are taken as the first factor's), so
-// that the backward pass has the forward pass's probabilities however large the scores are.
+// The sums come out the same, bit for bit, with either factor's rows in LDS (SWAP: the parts of b are taken as the first factor's): the
+// backward pass has the forward pass's probabilities however large the scores are, and dp minus delta is zero where it is (see delta_of).
 // (FETCH: b is fetched again for each product, from its planes or as it is, which leaves its registers to the fp32 units' way of working;
 // by_parts: the product is made of parts all the same, which only planes can be)
 template <bool FETCH, bool SWAP, int D, typename S>
@@ -114,11 +122,7 @@ __device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const R
     Parts f;
 #pragma unroll
     for (int p = 0; p < 3; p++) f.p[p] = *reinterpret_cast<const bf16x8 *>(piece + p * Ring<D>::PLANE + at[s]);
-    auto terms = [&](const Parts &own) {
-      const Parts &x = SWAP ? own : f, &y = SWAP ? f : own;
-      auto term = [&](int i, int j) { acc = SWAP ? mma(y.p[j], x.p[i], acc) : mma(x.p[i], y.p[j], acc); };
-      term(2, 0); term(0, 2); term(1, 1); term(0, 1); term(1, 0); term(0, 0);
-    };
+    auto terms = [&](const Parts &own) { acc = parts_product<SWAP>(f, own, acc); };
     if constexpr (FETCH) {
       asm volatile("" : "+v"(b_row));
       if constexpr (sizeof(S) == 4) {
@@ -370,6 +374,34 @@ template <int D> __device__ __forceinline__ int take_parts(Parts (&f)[D / 16], c
   return large;
 }
 
+// delta = sum_d do . o of the lane's row.  ds = p (dp - delta), so in a row whose share is one key's delta has to be that key's dp to the last bit
+// (what is left of the two, 1e-7 of |do| |v|, would be multiplied by rows of q and k that may be of any size): o is that key's v there, and
+// the sum is taken from the same unit's products in the same order as dp, off the diagonal of do . o^T.
+// (do with an infinity: sums of infinities of both signs in the operators, so NaN)
+template <bool WHOLE, int D> __device__ __forceinline__ float delta_of(const f32x4 (&o)[D / 8], const Parts (&do_parts)[D / 16], const f32x4 (&d_o)[D / 8], int lane) {
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[i] = 0.f;
+#pragma unroll
+  for (int s = 0; s < D / 16; s++) {
+    if constexpr (WHOLE) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(o[2 * s + (i >> 2)][i & 3], d_o[2 * s + (i >> 2)][i & 3], acc, 0, 0, 0);
+    } else {
+      float e[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) e[i] = o[2 * s + (i >> 2)][i & 3];
+      acc = parts_product<false>(split8<true>(e), do_parts[s], acc);
+    }
+  }
+  const int r = lane & 31, at = 4 * (r >> 3) + (r & 3);  // acc[i]: row 8 (i / 4) + 4 (lane / 32) + i % 4 of o, column r of do
+  float own = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) own = at == i ? acc[i] : own;
+  const float other = swap32(own), delta = ((r >> 2) & 1) == (lane >> 5) ? own : other;
+  return WHOLE && !(fabsf(delta) < INFINITY) ? NAN : delta;
+}
+
 // ---- planes ----
 struct PlaneArgs {
   struct Tensor {
@@ -582,23 +614,6 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   // the rows' do, and delta
   const float *do_row = reinterpret_cast<const float *>(a.d_o) + z * a.do_sz + h * a.do_sh + row * a.do_ld + 8 * half;
   const float *o_row = reinterpret_cast<const float *>(a.o_in) + z * a.oin_sz + h * a.oin_sh + row * a.oin_ld + 8 * half;
-  auto sums = [&](const f32x4 (&d)[D / 8], const f32x4 (&o)[D / 8]) {
-    float delta = 0.f;
-#pragma unroll
-    for (int s = 0; s < D / 8; s++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) delta = fmaf(d[s][i], o[s][i], delta);
-    delta += swap32(delta);
-    if (a.delta != nullptr && half == 0 && kh == 0) a.delta[zh * a.rows + row] = -delta;
-    return delta;
-  };
-  if (tiles == 0) {
-    f32x4 g[D / 8], o[D / 8];
-    fetch_row<D>(g, do_row);
-    fetch_row<D>(o, o_row);
-    sums(g, o);
-  }
-
   if (tiles > 0) {
     Parts xq[D / 16], xo[D / 16];
     const bf16 *q_row = reinterpret_cast<const bf16 *>(a.q) + (zh * a.rows + row) * (3 * D) + 8 * half;
@@ -629,15 +644,17 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     f32x4 g[D / 8], o[D / 8];
     fetch_row<D>(g, do_row);
     fetch_row<D>(o, o_row);
-    load_parts<D>(xq, q_row);
     int large = forward_flags(a, zh, a.R, lane);
     const bool by_parts = !__builtin_amdgcn_ballot_w64(large != 0);   // the scores, as in the forward pass
-    const float delta = sums(g, o);
     const int mine = take_parts<D>(xo, g);
     large |= a.fdo ? flags_of(a.fdo, zh, a.R, lane) : mine;
     f32x16 dp;
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
+      const float delta = delta_of<W, D>(o, xo, g, lane);
+      if (a.delta != nullptr && half == 0 && kh == 0) a.delta[zh * a.rows + row] = -delta;
+      __builtin_amdgcn_sched_barrier(0);                // (q takes the registers of o and do)
+      if constexpr (!W) load_parts<D>(xq, q_row);
       int here = 0;
       walk<PieceLoad<D>::COUNT, NK>(tiles, issue_v, issue_k,
         [&](int x, int) {
@@ -781,15 +798,15 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           const int mine = here >> ((lane >> 4) & 1);
           f32x16 dp;
 #pragma unroll
+          for (int i = 0; i < 16; i++) dp[i] = 0.f;
+          dp = rows_times<W, true, D>(smem + y * R::PIECE, rows, xv, v_row, false, dp);
+          float e[16];
+#pragma unroll
           for (int g = 0; g < 4; g++) {
             const f32x4 nd = *reinterpret_cast<const f32x4 *>(rv + x * (R::SIDE / 4) + (g >> 1) * 128 + 4 * (g & 1) + 64);
 #pragma unroll
-            for (int i = 0; i < 4; i++) dp[4 * g + i] = nd[i];
+            for (int i = 0; i < 4; i++) e[4 * g + i] = p[4 * g + i] * (dp[4 * g + i] + nd[i]);
           }
-          dp = rows_times<W, false, D>(smem + y * R::PIECE, rows, xv, v_row, false, dp);
-          float e[16];
-#pragma unroll
-          for (int i = 0; i < 16; i++) e[i] = p[i] * dp[i];
           if ((here & 0x33) != 0x33)
 #pragma unroll
             for (int i = 0; i < 16; i++) e[i] = mine >> 4 * (i >> 3) & 1 ? e[i] : 0.f;

@@ -461,7 +461,8 @@ int bsp_attention_cols_bwd(int dtype, const void *d_o, const void *q, const void
  * unit inner stride, 16-byte aligned pointers.  kpm: element (z, key) at kpm[z * kpm_stride_z + key], or NULL.
  * planes: bsp_attention_f32_bytes(Z, H, 64 R, keys, D) bytes (rows 0 where stats is NULL), written by fwd and read by bwd.  stats:
  * [Z][H][2][64 R] floats, written by fwd (NULL: no backward pass to follow) and read by bwd: the reference of the row's exponentials (natural
- * domain), one over their sum.
+ * domain), one over their sum.  o_copy: NULL, or [Z][H][64 R][D] floats that fwd writes o to once more, for callers whose o may change before
+ * bwd, which reads it.
  * bwd: do_planes: bsp_attention_f32_bytes(Z, H, 64 R, 0, D) bytes of scratch; neg_delta: [Z][H][64 R] floats of scratch.  dk and dv are
  * computed together; without them (both NULL) do_planes, neg_delta and what follows may be NULL and 0.  d_items .. n_split: as for
  * bsp_attention_cols_bwd; partial: bsp_attention_f32_slots(Z, n_slots) slots of 2 x 64 x D floats. */
@@ -476,6 +477,7 @@ typedef struct {
   float *stats;
   float scale;
   int kpm_mul;
+  float *o_copy;
 } bsp_attention_f32_call;
 int64_t bsp_attention_f32_bytes(int Z, int H, int64_t rows, int64_t keys, int D);
 int64_t bsp_attention_f32_slots(int Z, int n_slots);

@@ -225,3 +225,21 @@ def test_operands_that_are_copied_and_inference():
         assert torch.equal(grad, want[1 + i])
     with torch.no_grad():
         assert torch.equal(ac.attention_chain(*ops, q, k, v, scale=0.125), want[0])
+
+
+def test_result_may_change_before_the_backward_pass():
+    """The operators keep neither the result nor anything that shares its memory: a program may change it in place."""
+    torch.manual_seed(5)
+    lay = _layout(2, 8, 8, 'random')
+    ops = _ops(lay, 32)
+    q, k, v, do = [torch.randn(2, 2, 256, 64, device=DEV) for _ in range(4)]
+    want = _run(ops, q, k, v, do, True, scale=0.125)
+    xs = [t.clone().requires_grad_() for t in (q, k, v)]
+    o = ac.attention_chain(*ops, *xs, scale=0.125)
+    o += 7.
+    o.mul_(0.)
+    grads = torch.autograd.grad(o, xs, do)
+    assert all(float(g.abs().max()) == 0. for g in grads)
+    o = ac.attention_chain(*ops, *xs, scale=0.125)
+    o += 7.
+    assert all(torch.equal(g, w) for g, w in zip(torch.autograd.grad(o, xs, do), want[1:]))

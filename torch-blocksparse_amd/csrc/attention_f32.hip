@@ -586,7 +586,12 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   wait_barrier<0>();
   if (!kh) {
     float *po = reinterpret_cast<float *>(a.o) + z * a.o_sz + h * a.o_sh + ((int64_t)line * 64 + 32 * rh) * a.o_ld;
-    store_32_f32<D>(reinterpret_cast<float *>(smem) + rh * 32 * (D + 4), po, po + 16 * a.o_ld, a.o_ld, o, lane);
+    float *stage = reinterpret_cast<float *>(smem) + rh * 32 * (D + 4);
+    store_32_f32<D>(stage, po, po + 16 * a.o_ld, a.o_ld, o, lane);
+    if (a.o2 != nullptr) {
+      float *copy = reinterpret_cast<float *>(a.o2) + (zh * a.rows + (int64_t)line * 64 + 32 * rh) * D;
+      store_32_f32<D>(stage, copy, copy + 16 * D, D, o, lane);
+    }
   }
 }
 
@@ -984,8 +989,8 @@ extern "C" int64_t bsp_attention_f32_slots(int Z, int n_slots) { return (int64_t
 
 extern "C" int bsp_attention_f32_fwd(const bsp_attention_f32_call *c, const float *q, const float *k, const float *v, float *o, void *stream) {
   if (!c || !q || !k || !v || !o || !c->d_rows) return BSP_ERR_ARG;
-  const void *ptrs[] = {q, k, v, o, c->planes, c->stats, c->kpm};
-  const int rc = f32_check(*c, ptrs, 7, 4);
+  const void *ptrs[] = {q, k, v, o, c->planes, c->stats, c->kpm, c->o_copy};
+  const int rc = f32_check(*c, ptrs, 8, 4);
   if (rc != BSP_OK) return rc;
   F32Args a = f32_args(*c);
   const int64_t heads = (int64_t)a.Z * a.H;
@@ -995,7 +1000,7 @@ extern "C" int bsp_attention_f32_fwd(const bsp_attention_f32_call *c, const floa
   if (!c->stats) a.fq = nullptr;
   a.q = q;
   take_strides(c->strides, a.q_sz, a.q_sh, a.q_ld);
-  a.o = o;
+  a.o = o; a.o2 = c->o_copy;
   take_strides(c->strides + 9, a.o_sz, a.o_sh, a.o_ld);
   a.lut = c->d_rows;
   const int rl = launch_d<0>(a, c->D, heads * a.R, st);

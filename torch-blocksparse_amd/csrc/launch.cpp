@@ -574,7 +574,7 @@ bool f32_call(const Attn *s, int64_t Z, int64_t D, PyObject *const *masks, bsp_a
   return true;
 }
 
-// attn32_fwd(tables, q, k, v, scale, kpm, kpm_stride, kpm_mul, keep) -> (o, planes, stats or None): bsp_attention_f32_fwd
+// attn32_fwd(tables, q, k, v, scale, kpm, kpm_stride, kpm_mul, keep) -> (o, planes, stats or None, copy of o or None): bsp_attention_f32_fwd
 PyObject *attn32_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != 9) { PyErr_SetString(PyExc_TypeError, "attn32_fwd takes 9 arguments"); return nullptr; }
   const Attn *s = static_cast<const Attn *>(PyCapsule_GetPointer(args[0], kAttn));
@@ -584,21 +584,23 @@ PyObject *attn32_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const int64_t Z = q.size[0], rows = q.size[2], D = q.size[3], shape[4] = {Z, s->H, rows, D}, sshape[4] = {Z, s->H, 2, rows};
   const bool keep = truth(args[8]);
   bsp_attention_f32_call c;
-  void *op, *sp = nullptr, *st;
+  void *op, *sp = nullptr, *cp = nullptr, *st;
   if (!f32_call(s, Z, D, args + 4, &c) || !stream_of(q.dev, &st)) return nullptr;
-  Ref planes(empty_bytes(bsp_attention_f32_bytes((int)Z, (int)s->H, keep ? rows : 0, c.keys, (int)D), q.obj)), o(planes.o ? empty_like_type(shape, 4, q) : nullptr), stats;
+  Ref planes(empty_bytes(bsp_attention_f32_bytes((int)Z, (int)s->H, keep ? rows : 0, c.keys, (int)D), q.obj)), o(planes.o ? empty_like_type(shape, 4, q) : nullptr), stats, copy;
   if (!o.o || !pointer(planes.o, &c.planes) || !pointer(o.o, &op)) return nullptr;
   if (keep) {
     stats.o = empty_floats(sshape, 4, q.obj);
-    if (!stats.o || !pointer(stats.o, &sp)) return nullptr;
+    copy.o = stats.o ? empty_like_type(shape, 4, q) : nullptr;
+    if (!copy.o || !pointer(stats.o, &sp) || !pointer(copy.o, &cp)) return nullptr;
   }
   c.stats = static_cast<float *>(sp);
+  c.o_copy = static_cast<float *>(cp);
   for (int i = 0; i < 3; i++) c.strides[i] = q.stride[i], c.strides[3 + i] = k.stride[i], c.strides[6 + i] = v.stride[i];
   put_strides(c.strides + 9, shape);
   const int rc = unlocked([&] { return bsp_attention_f32_fwd(&c, static_cast<const float *>(q.data()), static_cast<const float *>(k.data()), static_cast<const float *>(v.data()),
                                                              static_cast<float *>(op), st); });
   if (!checked(rc, "bsp_attention_f32_fwd")) return nullptr;
-  return PyTuple_Pack(3, o.o, planes.o, stats.o ? stats.o : Py_None);
+  return PyTuple_Pack(4, o.o, planes.o, stats.o ? stats.o : Py_None, copy.o ? copy.o : Py_None);
 }
 
 // attn32_bwd(tables, do, o, planes, stats, scale, kpm, kpm_stride, kpm_mul, need_q, need_k, need_v) -> (dq, dk, dv): bsp_attention_f32_bwd

@@ -390,10 +390,10 @@ class _attention_f32(torch.autograd.Function):
             made = launch.attn32_fwd(native, _vec32(q), _vec32(k), _vec32(v), scale, kpm, *kpm_args, keep)
             if made is None:
                 raise _lib.BlocksparseLibraryError('attention: operands %s, %s, %s do not fit the layout' % (tuple(q.shape), tuple(k.shape), tuple(v.shape)))
-        o, planes, stats = made
+        o, planes, stats, o_copy = made
         fused_f32_calls += 1
-        if keep:
-            ctx.save_for_backward(planes, o, stats, kpm)
+        if keep:                                           # (a copy of o: a program may add to the result in place, which none of the operators reads again)
+            ctx.save_for_backward(planes, o_copy, stats, kpm)
             ctx.scale, ctx.tables, ctx.kpm_args = scale, tables, kpm_args
         return o
 

@@ -209,6 +209,60 @@ def test_saturated_rows(where, size, block, D):
         assert err <= 4 * bound + 2 ** -23, (name, err, bound)
 
 
+def _rows_error(x, r):
+    """relative error of a row (2-norm), root mean square over the rows that are not zero"""
+    e, n = (x.double() - r).norm(dim=-1), r.norm(dim=-1)
+    return float(((e[n > 0] / n[n > 0]) ** 2).mean().sqrt())
+
+
+# One value that sends a head's products to the fp32 units.  Against 64 bits row by row, since it dwarfs what has to do with it (and without its
+# column where it only reaches that); twice the operators' error, which is of the same units in another order.
+@pytest.mark.parametrize('where', ['q', 'k', 'v', 'do'])
+@pytest.mark.parametrize('Z,H,R,C,block,D,kind,padded', [
+    (2, 2, 16, 24, 32, 64, 'holes', True),
+    (1, 2, 12, 8, 16, 64, 'holes', False),
+    (1, 3, 40, 6, 64, 64, 'random', False),
+    (1, 2, 40, 6, 64, 128, 'random', True),
+    (1, 2, 8, 8, 16, 128, 'random', True),
+])
+def test_whole_values_against_64_bits(where, Z, H, R, C, block, D, kind, padded):
+    torch.manual_seed(R + C + D)
+    lay = _layout(H, R, C, kind)
+    x = {t: torch.randn(Z, H, (R if t in ('q', 'do') else C) * block, D, device=DEV) for t in ('q', 'k', 'v', 'do')}
+    x[where][0, 1, 37, 5] = 2. ** 31
+    kw = dict(scale=D ** -0.5)
+    if padded:
+        kpm = torch.zeros(Z, C * block, device=DEV)
+        kpm[0, block:block + 9] = float('-inf')
+        kpm[-1, block + 5:] = -2.
+        kw['key_padding_mask'] = kpm
+    ops = _ops(lay, block)
+    ref = _dense(x['q'], x['k'], x['v'], x['do'], lay, block, D ** -0.5, kw.get('key_padding_mask'))
+    got, other = [_run(ops, x['q'], x['k'], x['v'], x['do'], fused, **kw) for fused in (True, False)]
+    for name, g, c, r in zip(('o', 'dq', 'dk', 'dv'), got, other, ref):
+        if (where, name) in (('v', 'o'), ('do', 'dv'), ('k', 'dq'), ('q', 'dk')):
+            g, c, r = [torch.cat((t[..., :5], t[..., 6:]), -1) for t in (g, c, r)]
+        err, bound = _rows_error(g, r), _rows_error(c, r)
+        assert err <= 2 * bound + 2 ** -22, (name, err, bound)
+
+
+def test_sums_that_fp32_holds():
+    """Values near the largest of fp32: shares times them add up to less than it, numerators would not."""
+    torch.manual_seed(6)
+    lay = _layout(2, 8, 8, 'random')
+    ops = _ops(lay, 32)
+    q, k, v, do = [torch.randn(2, 2, 256, 64, device=DEV) for _ in range(4)]
+    huge = v.clone()
+    huge[0, 1, ::3] = 3e38
+    do *= 3e36
+    for x, names in (((q, k, huge, do * 1e-38), ('o',)), ((q, k, v, do), ('o', 'dq', 'dk', 'dv'))):
+        ref = _dense(*x, lay, 32, 0.125)
+        got, other = [_run(ops, *x, fused, scale=0.125) for fused in (True, False)]
+        for name, g, c, r in zip(names, got, other, ref):
+            assert bool(torch.isfinite(c).all()) and bool(torch.isfinite(g).all()), name
+            assert _rows_error(g, r) <= 2 * _rows_error(c, r) + 2 ** -22, name
+
+
 def test_operands_that_are_copied_and_inference():
     """Odd strides, an expanded gradient, gradients of some operands only, and a forward pass alone (which keeps no parts of q)."""
     torch.manual_seed(4)

@@ -38,6 +38,10 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 struct Parts { bf16x8 p[3]; };
 constexpr float kLargest = 1073741824.f;               // 2^30
+// Where products are of whole values, those may be as large as fp32 holds.  The operators multiply shares, which add up to one; the kernels
+// then take every exponential against the row's maximum and 2^-16 of it (a row has fewer keys), p and not its numerator in the
+// row kernel, and the scale with ds instead of with its sums, so that no sum overflows which theirs do not.
+constexpr float kWholeShare = 1.f / 65536.f;
 
 // the parts of eight values; WHOLE: also of those that are not below kLargest (infinities and NaN in the first part alone)
 template <bool WHOLE> __device__ __forceinline__ Parts split8(const float (&v)[8]) {
@@ -149,7 +153,12 @@ __device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const R
 // rows of a block that does not exist may reach the sums, and an infinity among them would).  Two chains of products at a time: two groups
 // of columns, each step's 32 terms added up first; TIGHT (where registers are short): one group, the smaller products of a step and the others.
 template <bool WHOLE, bool TIGHT, int D>
-__device__ __forceinline__ void columns_times(f32x16 (&acc)[D / 32], uint32_t piece, const TrReads<D, true> &reads, const Parts (&b)[2], bool here0, bool here1) {
+__device__ __forceinline__ void columns_times(f32x16 (&acc)[D / 32], uint32_t piece, const TrReads<D, true> &reads, const float (&e)[16], bool here0, bool here1) {
+  Parts b[2];
+  if constexpr (!WHOLE) {
+    b[0] = split8<false>(reinterpret_cast<const float (&)[8]>(e[0]));
+    b[1] = split8<false>(reinterpret_cast<const float (&)[8]>(e[8]));
+  }
   uint32_t lo[D / 32], hi[D / 32];
   reads.get(lo, hi);
   auto fetch = [&](int mt, int ks) {
@@ -170,7 +179,7 @@ __device__ __forceinline__ void columns_times(f32x16 (&acc)[D / 32], uint32_t pi
     for (int mt = 0; mt < D / 32; mt++)
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) {
-        const f32x16 sum = whole_parts_product(fetch(mt, ks), b[ks], acc[mt]);
+        const f32x16 sum = whole_product(fetch(mt, ks), [&](int i) { return e[8 * ks + i]; }, acc[mt]);
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[mt][i] = (ks ? here1 : here0) ? sum[i] : acc[mt][i];
         __builtin_amdgcn_sched_barrier(0);
@@ -467,7 +476,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
     for (int i = 0; i < 16; i++) o[mt][i] = 0.f;
-  float m = -INFINITY, l = 0.f;
+  float m = -INFINITY, l = 0.f, share = 1.f;            // share: what l and o are in units of
   int rows_seen = 0;
 
   if (tiles > 0) {
@@ -499,6 +508,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     float e[16];
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
+      share = W ? kWholeShare : 1.f;
       int here = 0;
       walk<NK, PieceLoad<D>::COUNT>(tiles, issue_k, issue_v,
         [&](int x, int) {
@@ -512,11 +522,15 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           const int mine = here >> ((lane >> 4) & 1) * 4;
           const bool here0 = mine & 1, here1 = mine & 2;        // pieces without a block take no part in the row
           for_16<0>([&](auto ic) { s[decltype(ic)::value] = KPM ? fmaf(s[decltype(ic)::value], sc, row_bcast<decltype(ic)::value>(kp)) : s[decltype(ic)::value] * sc; });
-          float sum;
+          float sum, top = -INFINITY;
+          auto highest = [&]() {
+#pragma unroll
+            for (int i = 0; i < 16; i++) top = fmaxf(top, (i < 8 ? here0 : here1) ? s[i] : -INFINITY);
+          };
           auto exponentials = [&]() {
             const float ms = m == -INFINITY ? 0.f : m;
 #pragma unroll
-            for (int i = 0; i < 16; i++) e[i] = exp_of<W>(s[i] - ms);
+            for (int i = 0; i < 16; i++) e[i] = exp_of<W>(s[i] - ms) * (W ? kWholeShare : 1.f);
             if ((here & 0x33) != 0x33) {                // (whatever the logits came out as there: a mask may hold NaN or an infinity, the scale may make one)
 #pragma unroll
               for (int i = 0; i < 16; i++) e[i] = (i < 8 ? here0 : here1) ? e[i] : 0.f;
@@ -525,11 +539,10 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
 #pragma unroll
             for (int i = 0; i < 16; i++) sum += e[i];
           };
-          exponentials();
-          if (__builtin_amdgcn_ballot_w64(!(sum <= 8192.f) || m == -INFINITY)) {      // (also where an exponential overflowed)
-            float top = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < 16; i++) top = fmaxf(top, (i < 8 ? here0 : here1) ? s[i] : -INFINITY);
+          if constexpr (W) highest();
+          else exponentials();
+          if (__builtin_amdgcn_ballot_w64(W ? top > m || m == -INFINITY : !(sum <= 8192.f) || m == -INFINITY)) {      // (also where an exponential overflowed)
+            if constexpr (!W) highest();
             const float mn = fmaxf(m, fmaxf(top, swap32(top))), f = exp_of<W>(m - (mn == -INFINITY ? 0.f : mn));
             l *= f;
 #pragma unroll
@@ -537,14 +550,14 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
 #pragma unroll
               for (int i = 0; i < 16; i++) o[mt][i] *= f;
             m = mn;
-            exponentials();
+            if constexpr (!W) exponentials();
           }
+          if constexpr (W) exponentials();
           l += sum;
         },
         [&](int y, int) {
-          const Parts pf[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(e[0])), split8<W>(reinterpret_cast<const float (&)[8]>(e[8]))};
           const int mine = here >> ((lane >> 4) & 1) * 4;
-          columns_times<W, false, D>(o, y * R::PIECE, tr_v, pf, mine & 1, mine & 2);
+          columns_times<W, false, D>(o, y * R::PIECE, tr_v, e, mine & 1, mine & 2);
         });
     };
     issue_k(0, 0);
@@ -580,7 +593,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     if (a.lse != nullptr && half == 0) {
       float *to = a.lse + zh * a.row_sh + row;
       to[0] = ms;
-      to[a.rest] = inv;
+      to[a.rest] = inv * share;
     }
   }
   wait_barrier<0>();
@@ -611,6 +624,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   const int tiles = lut[2 * (h * a.R + line)];
   const table_ptr core = lut + lut[2 * (h * a.R + line) + 1];
   const int64_t row = (int64_t)line * 64 + 32 * rh + l32;
+  float last = 1.f;
   f32x16 dq[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
@@ -622,7 +636,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   if (tiles > 0) {
     Parts xq[D / 16], xo[D / 16];
     const bf16 *q_row = reinterpret_cast<const bf16 *>(a.q) + (zh * a.rows + row) * (3 * D) + 8 * half;
-    const float sc = a.scale, m = a.lse[zh * a.row_sh + row];
+    const float sc = a.scale, m = a.lse[zh * a.row_sh + row], inv = a.lse[zh * a.row_sh + a.rest + row];
     const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D));
     const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D));
     const char *pkpm = reinterpret_cast<const char *>(reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz);
@@ -657,6 +671,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
       const float delta = delta_of<W, D>(o, xo, g, lane);
+      last = W ? 1.f : inv * a.scale;
       if (a.delta != nullptr && half == 0 && kh == 0) a.delta[zh * a.rows + row] = -delta;
       __builtin_amdgcn_sched_barrier(0);                // (q takes the registers of o and do)
       if constexpr (!W) load_parts<D>(xq, q_row);
@@ -675,17 +690,17 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           s = rows_times<W, false, D>(smem + y * R::PIECE, rows, xq, q_row, by_parts, s);
           const float kp = KPM ? pad_term(kp_lane[y * (R::SIDE / 4)], a.kpm_mul) : 0.f;
           const int mine = here >> ((lane >> 4) & 1) * 4;
-          float e[16];                                  // (1 / l of the row comes last, on dq)
+          float e[16];                                  // (1 / l of the row and the scale come last, on dq, unless W)
           for_16<0>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            e[i] = exp_of<W>((KPM ? fmaf(s[i], sc, row_bcast<i>(kp)) : s[i] * sc) - m) * (dp[i] - delta);
+            const float x = exp_of<W>((KPM ? fmaf(s[i], sc, row_bcast<i>(kp)) : s[i] * sc) - m);
+            e[i] = W ? x * inv * (dp[i] - delta) * sc : x * (dp[i] - delta);
           });
           if ((here & 0x33) != 0x33) {                  // pieces without a block
 #pragma unroll
             for (int i = 0; i < 16; i++) e[i] = mine >> (i >> 3) & 1 ? e[i] : 0.f;
           }
-          const Parts df[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(e[0])), split8<W>(reinterpret_cast<const float (&)[8]>(e[8]))};
-          columns_times<W, false, D>(dq, y * R::PIECE, tr, df, mine & 1, mine & 2);
+          columns_times<W, false, D>(dq, y * R::PIECE, tr, e, mine & 1, mine & 2);
         });
     };
     if (__builtin_amdgcn_ballot_w64(large != 0)) run(Const<1>{});
@@ -696,7 +711,6 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   if (kh) put_sums<D>(other, dq, lane);
   wait_barrier<0>();
   if (!kh) {
-    const float last = a.lse[zh * a.row_sh + a.rest + row] * a.scale;
     take_sums<D>(other, dq, lane, [&](float a0, float a1) { return (a0 + a1) * last; });
   }
   wait_barrier<0>();
@@ -733,6 +747,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     }
   }
   const int64_t key_lo = head[8 + 2 * kh], key_hi = head[8 + 2 * kh + 1], zh = (int64_t)z * a.H + h;
+  float last = 1.f;
   f32x16 dk[MT], dv[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
@@ -774,6 +789,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     bool by_parts;
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
+      last = W ? 1.f : a.scale;
       if constexpr (!W) {
         own_parts<D>(xk, smem + R::PIECE, 32 * kh + l32, half);
         own_parts<D>(xv, smem + 2 * R::PIECE, 32 * kh + l32, half);
@@ -810,17 +826,13 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           for (int g = 0; g < 4; g++) {
             const f32x4 nd = *reinterpret_cast<const f32x4 *>(rv + x * (R::SIDE / 4) + (g >> 1) * 128 + 4 * (g & 1) + 64);
 #pragma unroll
-            for (int i = 0; i < 4; i++) e[4 * g + i] = p[4 * g + i] * (dp[4 * g + i] + nd[i]);
+            for (int i = 0; i < 4; i++) e[4 * g + i] = p[4 * g + i] * (dp[4 * g + i] + nd[i]) * (W ? sc : 1.f);
           }
           if ((here & 0x33) != 0x33)
 #pragma unroll
             for (int i = 0; i < 16; i++) e[i] = mine >> 4 * (i >> 3) & 1 ? e[i] : 0.f;
-          {
-            const Parts pf[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(p[0])), split8<W>(reinterpret_cast<const float (&)[8]>(p[8]))};
-            columns_times<W, true, D>(dv, y * R::PIECE, tr, pf, mine & 1, mine & 16);
-          }
-          const Parts df[2] = {split8<W>(reinterpret_cast<const float (&)[8]>(e[0])), split8<W>(reinterpret_cast<const float (&)[8]>(e[8]))};
-          columns_times<W, true, D>(dk, x * R::PIECE, tr, df, mine & 1, mine & 16);
+          columns_times<W, true, D>(dv, y * R::PIECE, tr, p, mine & 1, mine & 16);
+          columns_times<W, true, D>(dk, x * R::PIECE, tr, e, mine & 1, mine & 16);
         });
     };
     issue_q(0, 0);
@@ -842,7 +854,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   }
   wait_barrier<0>();
   if (!rh) {
-    take_sums<D>(other, dk, lane, [&](float a0, float a1) { return (a0 + a1) * a.scale; });
+    take_sums<D>(other, dk, lane, [&](float a0, float a1) { return (a0 + a1) * last; });
     take_sums<D>(other + 16 * MT * 64, dv, lane, [&](float a0, float a1) { return a0 + a1; });
   }
   wait_barrier<0>();

@@ -454,14 +454,14 @@ int bsp_attention_cols_bwd(int dtype, const void *d_o, const void *q, const void
                            const void *kpm, int64_t kpm_stride_z, int kpm_mul, void *stream);
 
 /* The same chain in fp32, D = 64 or 128, with the tables of bsp_attention_tables_build.  The operands are kept as three bfloat16 parts
- * each, whose products add up to fp32 products (heads that hold a value of 2^30 or more, an infinity or a NaN are computed on the
+ * each, whose products add up to fp32 products (heads that hold a value of 2^20 or more, an infinity or a NaN are computed on the
  * fp32 matrix units instead).
  * Z, H, R: batches, heads, lines of 64 rows; keys: positions of k and v (a multiple of 64).  strides: of batch, head and row, in
  * elements, three per tensor in the order of the call's tensor arguments (fwd: q, k, v, o; bwd: d_o, o, dq, dk, dv); multiples of 4,
  * unit inner stride, 16-byte aligned pointers.  kpm: element (z, key) at kpm[z * kpm_stride_z + key], or NULL.
  * planes: bsp_attention_f32_bytes(Z, H, 64 R, keys, D) bytes (rows 0 where stats is NULL), written by fwd and read by bwd.  stats:
  * [Z][H][2][64 R] floats, written by fwd (NULL: no backward pass to follow) and read by bwd: the reference of the row's exponentials (natural
- * domain), one over their sum.  o_copy: NULL, or [Z][H][64 R][D] floats that fwd writes o to once more, for callers whose o may change before
+ * domain), 2^16 over their sum.  o_copy: NULL, or [Z][H][64 R][D] floats that fwd writes o to once more, for callers whose o may change before
  * bwd, which reads it.
  * bwd: do_planes: bsp_attention_f32_bytes(Z, H, 64 R, 0, D) bytes of scratch; neg_delta: [Z][H][64 R] floats of scratch.  dk and dv are
  * computed together; without them (both NULL) do_planes, neg_delta and what follows may be NULL and 0.  d_items .. n_split: as for

@@ -263,6 +263,25 @@ def test_sums_that_fp32_holds():
             assert _rows_error(g, r) <= 2 * _rows_error(c, r) + 2 ** -22, name
 
 
+# Operands and gradients of the scores far below one: they keep their 24 bits.  Against 64 bits, bound as in test_against_64_bits.
+@pytest.mark.parametrize('sizes,scale', [(dict(do=-115), 0), (dict(v=-115), 0), (dict(v=-60, do=-60), 0), (dict(q=-118), 118), (dict(q=-60, k=-60), 120), (dict(k=-20, v=19, do=-100), 20)])
+@pytest.mark.parametrize('block,D', [(32, 64), (64, 128)])
+def test_small_operands(sizes, scale, block, D):
+    torch.manual_seed(block)
+    n = 256 // block
+    lay = _layout(2, n, n, 'random')
+    x = {t: torch.randn(2, 2, 256, D, device=DEV) for t in ('q', 'k', 'v', 'do')}
+    for t, power in sizes.items():
+        x[t].clamp_(-8, 8).mul_(2. ** (power if power < 0 else power - 3))
+    scale = D ** -0.5 * 2. ** scale
+    ops = _ops(lay, block)
+    ref = _dense(x['q'], x['k'], x['v'], x['do'], lay, block, scale)
+    got, other = [_run(ops, x['q'], x['k'], x['v'], x['do'], fused, scale=scale) for fused in (True, False)]
+    for name, g, c, r in zip(('o', 'dq', 'dk', 'dv'), got, other, ref):
+        err, bound = [float((t.double() - r).norm() / r.norm()) for t in (g, c)]
+        assert err <= bound + 2 ** -23, (name, err, bound)
+
+
 def test_operands_that_are_copied_and_inference():
     """Odd strides, an expanded gradient, gradients of some operands only, and a forward pass alone (which keeps no parts of q)."""
     torch.manual_seed(4)

@@ -1,15 +1,16 @@
 // The attention chain without sparse tensors in fp32 (head dimension 64 or 128; calls without relative position embedding and attention
 // mask): what attention_fwd.hip and attention_bwd.hip do for 16-bit tensors, in single precision and on the bfloat16 matrix units.
 //
-// Products.  A number of 24 bits is the sum of three bfloat16 numbers, each rounded to nearest: x = x0 + x1 + x2 (exactly, down
-// to 2^-110).  A product is the sum of the six products of such parts that count in 24 bits, smallest first, in one fp32
+// Products.  A number of 24 bits is the sum of three bfloat16 numbers, each rounded to nearest: x = x0 + x1 + x2, exactly down
+// to 2^-110.  The parts are those of 2^16 x, so of every number that fp32 has, and the sums are scaled back where they are used (powers of
+// two, in factors that are there).  A product is the sum of the six products of such parts that count in 24 bits, smallest first, in one fp32
 // accumulator: x2 y0 + x1 y1 + x0 y2 + x1 y0 + x0 y1 + x0 y0.  Six MFMAs of bfloat16 do in 6 x 32 cycles what eight of fp32 do in
 // 8 x 64, and round less often (once a step of sixteen instead of two).  Error against 64 bits of 32 x 32 products of N(0, 1) operands, relative 2-norm, this /
 // fp32 MFMA: 64 terms 1.1e-7 / 1.5e-7, 512 terms 3.4e-7 / 4.0e-7, 4096 terms 9.9e-7 / 1.15e-6; uniform operands 0.9e-7 / 1.2e-7, 2.4e-7 /
 // 2.9e-7, 5.2e-7 / 8.3e-7.  (Parts cut off instead of rounded: 1e-5 for 4096 uniform terms, their sums being one-sided.)
-// Infinities have no such parts, and their products with zero parts would be NaN: where a head's operands hold a value of 2^30 or
+// Infinities have no such parts, and their products with zero parts would be NaN: where a head's operands hold a value of 2^20 or
 // more, an infinity or a NaN (a flag per 64 rows, made beside the parts), the kernels compute its products from the whole
-// values on the fp32 units, as the operators do.  Below 2^30 no product overflows.
+// values on the fp32 units, as the operators do.  Below 2^20 no sum of products of parts overflows.
 //
 // Launches.  k_attn32_planes writes the three parts of q, k and v (backward: do) as planes, [row][part][D], so that the other
 // kernels fetch them tile by tile straight into LDS.  Those walk the same tables and 64 x 64 tiles as the 16-bit kernels; a
@@ -28,7 +29,7 @@ namespace bsp {
 namespace {
 
 struct F32Args : QuadArgs {            // k, v: the planes; q: forward q itself, backward the planes; d_o: row kernel do itself, column kernel
-                                       // the planes; lse: per row the reference m of its exponentials, rest floats on 1 / l
+                                       // the planes; lse: per row the reference m of its exponentials, rest floats on kUp / l
   const int32_t *fq, *fk, *fv, *fdo;   // flags [Z][H][pieces of 64 rows]; fq (forward) and fdo (row kernel) NULL: not there, no other kernel follows
   int64_t rows, keys;
   int sub;                             // column kernel: pieces that a part of a long column is cut into
@@ -37,14 +38,16 @@ struct F32Args : QuadArgs {            // k, v: the planes; q: forward q itself,
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 struct Parts { bf16x8 p[3]; };
-constexpr float kLargest = 1073741824.f;               // 2^30
+constexpr float kLargest = 1048576.f;                  // 2^20
+constexpr float kUp = 65536.f, kDown = 1.f / kUp, kDown2 = kDown * kDown;   // parts are those of kUp x
+constexpr float kReversed = 1267650600228229401496703205376.f;              // 2^100
 // Where products are of whole values, those may be as large as fp32 holds.  The operators multiply shares, which add up to one; the kernels
 // then take every exponential against the row's maximum and 2^-16 of it (a row has fewer keys), p and not its numerator in the
 // row kernel, and the scale with ds instead of with its sums, so that no sum overflows which theirs do not.
 constexpr float kWholeShare = 1.f / 65536.f;
 
-// the parts of eight values; WHOLE: also of those that are not below kLargest (infinities and NaN in the first part alone)
-template <bool WHOLE> __device__ __forceinline__ Parts split8(const float (&v)[8]) {
+// the parts of eight values
+__device__ __forceinline__ Parts split8(const float (&v)[8]) {
   union { bf16x2 two[4]; bf16x8 all; } h, m, l;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
@@ -54,26 +57,34 @@ template <bool WHOLE> __device__ __forceinline__ Parts split8(const float (&v)[8
     m.two[i] = __builtin_convertvector(r, bf16x2);
     l.two[i] = __builtin_convertvector(r - __builtin_convertvector(m.two[i], f32x2), bf16x2);
   }
-  if constexpr (WHOLE) {
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-      if (!(fabsf(v[i]) < kLargest)) {
-        const bool finite = fabsf(v[i]) < INFINITY;
-        const float a = finite ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i]) & 0xffff0000u) : v[i], r = finite ? v[i] - a : 0.f;
-        const float b = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xffff0000u);
-        h.all[i] = (bf16)a; m.all[i] = (bf16)b; l.all[i] = (bf16)(r - b);
-      }
-  }
   Parts s;
   s.p[0] = h.all; s.p[1] = m.all; s.p[2] = l.all;
   return s;
 }
+// ... of an operand's, scaled up.  What fp32 does not hold then is kept as it is, for `whole` to find: from 2^100 on with the smallest part first,
+// infinities and NaN in the first part alone.
+__device__ __forceinline__ Parts split_operand(const float (&v)[8]) {
+  float x[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) x[i] = v[i] * kUp;
+  Parts s = split8(x);
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    if (!(fabsf(v[i]) < kReversed)) {
+      const bool finite = fabsf(v[i]) < INFINITY;
+      const float a = finite ? __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[i]) & 0xffff0000u) : 0.f, r = finite ? v[i] - a : 0.f;
+      const float b = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xffff0000u);
+      s.p[0][i] = finite ? (bf16)(r - b) : (bf16)v[i]; s.p[1][i] = (bf16)b; s.p[2][i] = (bf16)a;
+    }
+  return s;
+}
 
 __device__ __forceinline__ f32x16 mma(const bf16x8 &a, const bf16x8 &b, const f32x16 &c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
-// value i of eight that are held as parts
+// value i of eight that are held as parts (split_operand)
 __device__ __forceinline__ float whole(const u32x4 (&v)[3], int i) {
   auto part = [&](int p) { return __builtin_bit_cast(float, i & 1 ? v[p][i >> 1] & 0xffff0000u : v[p][i >> 1] << 16); };
-  return part(0) + part(1) + part(2);
+  const float a = part(0), c = part(2), sum = a + part(1) + c;
+  return fabsf(c) > fabsf(a) ? sum : sum * kDown;
 }
 // acc += a . b over sixteen indices from the whole values, on the fp32 units.  (The empty assembly keeps whole values from being held
 // beside the parts, the barrier keeps the next operands from being fetched ahead: this way is about registers, not time.)
@@ -106,6 +117,13 @@ template <bool SWAP> __device__ __forceinline__ f32x16 parts_product(const Parts
   term(2, 0); term(0, 2); term(1, 1); term(0, 1); term(1, 0); term(0, 0);
   return acc;
 }
+
+// a sum of products of parts -> what it stands for, times scale (in the order in which nothing that fp32 holds is lost on the way)
+struct ScaledDown {
+  float first, then;
+  __device__ __forceinline__ explicit ScaledDown(float scale) : first(fabsf(scale) < 1.f ? scale : scale * kDown2), then(fabsf(scale) < 1.f ? kDown2 : 1.f) {}
+  __device__ __forceinline__ float operator()(float sum) const { return sum * first * then; }
+};
 
 template <int D> struct Ring {
   static constexpr int PLANE = 64 * D * 2, PIECE = 3 * PLANE, SIDE = 4 * 512;   // SIDE: two words a lane for each wavefront, beside a piece
@@ -155,9 +173,9 @@ __device__ __forceinline__ f32x16 rows_times(const unsigned char *piece, const R
 template <bool WHOLE, bool TIGHT, int D>
 __device__ __forceinline__ void columns_times(f32x16 (&acc)[D / 32], uint32_t piece, const TrReads<D, true> &reads, const float (&e)[16], bool here0, bool here1) {
   Parts b[2];
-  if constexpr (!WHOLE) {
-    b[0] = split8<false>(reinterpret_cast<const float (&)[8]>(e[0]));
-    b[1] = split8<false>(reinterpret_cast<const float (&)[8]>(e[8]));
+  if constexpr (!WHOLE) {                               // (e is kUp times what it stands for)
+    b[0] = split8(reinterpret_cast<const float (&)[8]>(e[0]));
+    b[1] = split8(reinterpret_cast<const float (&)[8]>(e[8]));
   }
   uint32_t lo[D / 32], hi[D / 32];
   reads.get(lo, hi);
@@ -378,7 +396,7 @@ template <int D> __device__ __forceinline__ int take_parts(Parts (&f)[D / 16], c
       e[j] = v[2 * s + (j >> 2)][j & 3];
       large |= !(fabsf(e[j]) < kLargest);
     }
-    f[s] = split8<true>(e);
+    f[s] = split_operand(e);
   }
   return large;
 }
@@ -400,7 +418,7 @@ template <bool WHOLE, int D> __device__ __forceinline__ float delta_of(const f32
       float e[8];
 #pragma unroll
       for (int i = 0; i < 8; i++) e[i] = o[2 * s + (i >> 2)][i & 3];
-      acc = parts_product<false>(split8<true>(e), do_parts[s], acc);
+      acc = parts_product<false>(split_operand(e), do_parts[s], acc);
     }
   }
   const int r = lane & 31, at = 4 * (r >> 3) + (r & 3);  // acc[i]: row 8 (i / 4) + 4 (lane / 32) + i % 4 of o, column r of do
@@ -408,7 +426,7 @@ template <bool WHOLE, int D> __device__ __forceinline__ float delta_of(const f32
 #pragma unroll
   for (int i = 0; i < 16; i++) own = at == i ? acc[i] : own;
   const float other = swap32(own), delta = ((r >> 2) & 1) == (lane >> 5) ? own : other;
-  return WHOLE && !(fabsf(delta) < INFINITY) ? NAN : delta;
+  return !WHOLE ? delta * kDown2 : fabsf(delta) < INFINITY ? delta : NAN;
 }
 
 // ---- planes ----
@@ -447,7 +465,7 @@ template <int D> __global__ void __launch_bounds__(256) k_attn32_planes(PlaneArg
       e[j] = v[i][j >> 2][j & 3];
       large |= !(fabsf(e[j]) < kLargest);
     }
-    const Parts s = split8<true>(e);
+    const Parts s = split_operand(e);
 #pragma unroll
     for (int p = 0; p < 3; p++) *reinterpret_cast<bf16x8 *>(to + row * (3 * D) + p * D + col) = s.p[p];
   }
@@ -476,13 +494,13 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
     for (int i = 0; i < 16; i++) o[mt][i] = 0.f;
-  float m = -INFINITY, l = 0.f, share = 1.f;            // share: what l and o are in units of
+  float m = -INFINITY, l = 0.f, share = 1.f, down = 1.f;   // l and o are `share` times what they stand for; down: takes the scale of v off o
   int rows_seen = 0;
 
   if (tiles > 0) {
     Parts xq[D / 16];
     const float *q_row = reinterpret_cast<const float *>(a.q) + z * a.q_sz + h * a.q_sh + row * a.q_ld + 8 * half;
-    const float sc = a.scale;
+    float sc = a.scale * kDown2;
     const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D));
     const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D));
     const char *pkpm = reinterpret_cast<const char *>(reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz);
@@ -508,7 +526,9 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     float e[16];
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
-      share = W ? kWholeShare : 1.f;
+      share = W ? kWholeShare : kUp;
+      down = W ? 1.f : kDown;
+      if constexpr (W) sc = a.scale;
       int here = 0;
       walk<NK, PieceLoad<D>::COUNT>(tiles, issue_k, issue_v,
         [&](int x, int) {
@@ -530,7 +550,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           auto exponentials = [&]() {
             const float ms = m == -INFINITY ? 0.f : m;
 #pragma unroll
-            for (int i = 0; i < 16; i++) e[i] = exp_of<W>(s[i] - ms) * (W ? kWholeShare : 1.f);
+            for (int i = 0; i < 16; i++) e[i] = exp_of<W>(s[i] - ms) * (W ? kWholeShare : kUp);
             if ((here & 0x33) != 0x33) {                // (whatever the logits came out as there: a mask may hold NaN or an infinity, the scale may make one)
 #pragma unroll
               for (int i = 0; i < 16; i++) e[i] = (i < 8 ? here0 : here1) ? e[i] : 0.f;
@@ -541,7 +561,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           };
           if constexpr (W) highest();
           else exponentials();
-          if (__builtin_amdgcn_ballot_w64(W ? top > m || m == -INFINITY : !(sum <= 8192.f) || m == -INFINITY)) {      // (also where an exponential overflowed)
+          if (__builtin_amdgcn_ballot_w64(W ? top > m || m == -INFINITY : !(sum <= 8192.f * kUp) || m == -INFINITY)) {      // (also where an exponential overflowed)
             if constexpr (!W) highest();
             const float mn = fmaxf(m, fmaxf(top, swap32(top))), f = exp_of<W>(m - (mn == -INFINITY ? 0.f : mn));
             l *= f;
@@ -589,11 +609,12 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     const float sum = l * f0 + l1 * f1;
     const bool any_block = (rows_seen >> 4 * ((lane >> 4) & 1)) & 15;
     const float inv = any_block ? 1.f / sum : 0.f;      // masked everywhere: 0 * inf = NaN, as the softmax operator gives; no block at all: zeros
-    take_sums<D>(other, o, lane, [&](float a0, float a1) { return (a0 * f0 + a1 * f1) * inv; });
+    const float last = inv * down;
+    take_sums<D>(other, o, lane, [&](float a0, float a1) { return (a0 * f0 + a1 * f1) * last; });
     if (a.lse != nullptr && half == 0) {
       float *to = a.lse + zh * a.row_sh + row;
       to[0] = ms;
-      to[a.rest] = inv * share;
+      to[a.rest] = inv * share * kUp;
     }
   }
   wait_barrier<0>();
@@ -625,6 +646,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   const table_ptr core = lut + lut[2 * (h * a.R + line) + 1];
   const int64_t row = (int64_t)line * 64 + 32 * rh + l32;
   float last = 1.f;
+  bool parts = false;
   f32x16 dq[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
@@ -636,7 +658,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   if (tiles > 0) {
     Parts xq[D / 16], xo[D / 16];
     const bf16 *q_row = reinterpret_cast<const bf16 *>(a.q) + (zh * a.rows + row) * (3 * D) + 8 * half;
-    const float sc = a.scale, m = a.lse[zh * a.row_sh + row], inv = a.lse[zh * a.row_sh + a.rest + row];
+    const float m = a.lse[zh * a.row_sh + row], inv = a.lse[zh * a.row_sh + a.rest + row];
     const char *pk = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.k) + zh * a.keys * (3 * D));
     const char *pv = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.v) + zh * a.keys * (3 * D));
     const char *pkpm = reinterpret_cast<const char *>(reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz);
@@ -665,13 +687,16 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     fetch_row<D>(o, o_row);
     int large = forward_flags(a, zh, a.R, lane);
     const bool by_parts = !__builtin_amdgcn_ballot_w64(large != 0);   // the scores, as in the forward pass
+    const float sc = by_parts ? a.scale * kDown2 : a.scale;
     const int mine = take_parts<D>(xo, g);
     large |= a.fdo ? flags_of(a.fdo, zh, a.R, lane) : mine;
     f32x16 dp;
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
       const float delta = delta_of<W, D>(o, xo, g, lane);
-      last = W ? 1.f : inv * a.scale;
+      const float up = delta * -kUp;
+      parts = !W;
+      last = inv * kDown;
       if (a.delta != nullptr && half == 0 && kh == 0) a.delta[zh * a.rows + row] = -delta;
       __builtin_amdgcn_sched_barrier(0);                // (q takes the registers of o and do)
       if constexpr (!W) load_parts<D>(xq, q_row);
@@ -694,7 +719,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           for_16<0>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
             const float x = exp_of<W>((KPM ? fmaf(s[i], sc, row_bcast<i>(kp)) : s[i] * sc) - m);
-            e[i] = W ? x * inv * (dp[i] - delta) * sc : x * (dp[i] - delta);
+            e[i] = W ? x * (inv * kDown) * (dp[i] - delta) * a.scale : x * fmaf(dp[i], kDown, up);
           });
           if ((here & 0x33) != 0x33) {                  // pieces without a block
 #pragma unroll
@@ -711,7 +736,8 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   if (kh) put_sums<D>(other, dq, lane);
   wait_barrier<0>();
   if (!kh) {
-    take_sums<D>(other, dq, lane, [&](float a0, float a1) { return (a0 + a1) * last; });
+    const ScaledDown scaled(a.scale);
+    take_sums<D>(other, dq, lane, [&](float a0, float a1) { return parts ? scaled((a0 + a1) * last) : a0 + a1; });
   }
   wait_barrier<0>();
   if (!kh) {
@@ -747,7 +773,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     }
   }
   const int64_t key_lo = head[8 + 2 * kh], key_hi = head[8 + 2 * kh + 1], zh = (int64_t)z * a.H + h;
-  float last = 1.f;
+  bool parts = false;
   f32x16 dk[MT], dv[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
@@ -759,7 +785,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     Parts xk[D / 16], xv[D / 16];
     const bf16 *k_row = reinterpret_cast<const bf16 *>(a.k) + (zh * a.keys + key) * (3 * D) + 8 * half;
     const bf16 *v_row = reinterpret_cast<const bf16 *>(a.v) + (zh * a.keys + key) * (3 * D) + 8 * half;
-    const float sc = a.scale, kp = KPM ? pad_term((reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz)[key], a.kpm_mul) : 0.f;
+    const float kp = KPM ? pad_term((reinterpret_cast<const float *>(a.kpm) + z * a.kpm_sz)[key], a.kpm_mul) : 0.f;
     const char *pq = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.q) + zh * a.rows * (3 * D));
     const char *pdo = reinterpret_cast<const char *>(reinterpret_cast<const bf16 *>(a.d_o) + zh * a.rows * (3 * D));
     const char *pstat = reinterpret_cast<const char *>(a.lse + zh * a.row_sh), *pdelta = reinterpret_cast<const char *>(a.delta + zh * a.rows);
@@ -789,7 +815,8 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
     bool by_parts;
     auto run = [&](auto whole) {
       constexpr bool W = decltype(whole)::value;
-      last = W ? 1.f : a.scale;
+      parts = !W;
+      const float sc = by_parts ? a.scale * kDown2 : a.scale;
       if constexpr (!W) {
         own_parts<D>(xk, smem + R::PIECE, 32 * kh + l32, half);
         own_parts<D>(xv, smem + 2 * R::PIECE, 32 * kh + l32, half);
@@ -807,7 +834,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
             const float *at = rv + x * (R::SIDE / 4) + (g >> 1) * 128 + 4 * (g & 1);
             const f32x4 m = *reinterpret_cast<const f32x4 *>(at), inv = *reinterpret_cast<const f32x4 *>(at + 16);
 #pragma unroll
-            for (int i = 0; i < 4; i++) p[4 * g + i] = exp_of<W>((KPM ? fmaf(s[4 * g + i], sc, kp) : s[4 * g + i] * sc) - m[i]) * inv[i];
+            for (int i = 0; i < 4; i++) p[4 * g + i] = exp_of<W>((KPM ? fmaf(s[4 * g + i], sc, kp) : s[4 * g + i] * sc) - m[i]) * (W ? inv[i] * kDown : inv[i]);
           }
           if ((here & 0x33) != 0x33) {                  // pieces without a block (a row that is masked everywhere has NaN here, which its other keys must not take up)
             const int mine = here >> ((lane >> 4) & 1);
@@ -826,7 +853,7 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
           for (int g = 0; g < 4; g++) {
             const f32x4 nd = *reinterpret_cast<const f32x4 *>(rv + x * (R::SIDE / 4) + (g >> 1) * 128 + 4 * (g & 1) + 64);
 #pragma unroll
-            for (int i = 0; i < 4; i++) e[4 * g + i] = p[4 * g + i] * (dp[4 * g + i] + nd[i]) * (W ? sc : 1.f);
+            for (int i = 0; i < 4; i++) e[4 * g + i] = W ? p[4 * g + i] * (dp[4 * g + i] + nd[i]) * a.scale : p[4 * g + i] * fmaf(dp[4 * g + i], kDown2, nd[i]);
           }
           if ((here & 0x33) != 0x33)
 #pragma unroll
@@ -854,8 +881,9 @@ template <int D, bool KPM> __global__ void __launch_bounds__(256, D == 64 ? 2 : 
   }
   wait_barrier<0>();
   if (!rh) {
-    take_sums<D>(other, dk, lane, [&](float a0, float a1) { return (a0 + a1) * last; });
-    take_sums<D>(other + 16 * MT * 64, dv, lane, [&](float a0, float a1) { return a0 + a1; });
+    const ScaledDown scaled(a.scale);
+    take_sums<D>(other, dk, lane, [&](float a0, float a1) { return parts ? scaled(a0 + a1) : a0 + a1; });
+    take_sums<D>(other + 16 * MT * 64, dv, lane, [&](float a0, float a1) { return parts ? (a0 + a1) * kDown2 : a0 + a1; });
   }
   wait_barrier<0>();
   if (rh) return;

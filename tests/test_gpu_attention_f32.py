@@ -54,8 +54,8 @@ def _layout(H, R, C, kind):
     return lay
 
 
-# one tile; a tile of remainders; lines and columns of one to many tiles; parts of long columns in 2 and in 1 pieces
-# (66 and 512 batches x heads of a column in three parts); from 32 heads on another order of the workgroups
+# one tile; a tile of remainders; lines and columns of one to many tiles; parts of long columns (6 and 128 of them, in halves; 192,
+# whole); from 32 heads on another order of the workgroups
 @pytest.mark.parametrize('Z,H,R,C,block,D,kind,padded', [
     (1, 1, 1, 1, 64, 64, 'dense', False),
     (2, 1, 4, 4, 16, 128, 'random', True),
@@ -66,6 +66,7 @@ def _layout(H, R, C, kind):
     (11, 6, 80, 8, 32, 64, 'random', False),
     (2, 32, 40, 4, 64, 128, 'random', True),
     (64, 8, 40, 2, 64, 64, 'random', False),
+    (3, 32, 40, 4, 64, 64, 'random', False),
     (1, 2, 32, 32, 64, 128, 'dense', False),
 ])
 def test_against_64_bits(Z, H, R, C, block, D, kind, padded):

@@ -17,7 +17,7 @@
 // workgroup is four wavefronts, one per 32 x 32 quadrant, since a line is few tiles and 64 rows with two wavefronts would leave
 // half of the SIMDs of a launch of a few hundred lines without any.  The quadrants of the same rows add up at the end through LDS.
 // A tile's operands come in two pieces (k, v; columns: q, do) of 64 rows x 3 parts, 24 KiB at head dimension 64; the ring has
-// three slots of a piece, so two workgroups share a CU: while a piece is used the next is on its way, and the one after that
+// three slots of a piece, so two workgroups share a CU (one at 128): while a piece is used the next is on its way, and the one after that
 // where a slot is free.
 #include "attention_quad.h"
 #include <atomic>
@@ -1011,10 +1011,11 @@ int launch_planes(const bsp_attention_f32_call &c, const ToPlanes (&tensors)[3],
 }
 
 // Pieces of the parts of long columns.  A part is up to sixteen tiles, eight times as long as the short columns of the layouts that have
-// any: a launch whose parts do not fill the chip (two workgroups a CU, 512) ends with them alone and does better on halves, though each costs
-// a workgroup's first loads and a slot written and read once more.  Column kernel in 1 / 2 / 4 pieces, 8 heads of 2048 positions, stride 128 of blocks of
-// 32: 128 parts 55 / 45 / 54 us, 256 parts 86 / 80 / 105, 512 parts 126 / 147 / 181, 1024 parts 241 / 281 / 367.
-int pieces(int64_t parts) { return parts > 0 && parts < 512 ? 2 : 1; }
+// any: a launch of few parts ends with them alone and does better on halves, as long as every half has a compute unit of its own; each half costs
+// a workgroup's first loads and a slot written and read once more.  Backward pass in 1 / 2 pieces, us: head dimension 64, 128 parts 100.6 / 92.9,
+// 192 parts 157 / 176 and (columns of 128 keys' blocks) 278 / 269, 256 parts 155 / 155, 384 parts 197 / 204, 512 parts 233 / 248; 128, whose workgroups
+// have a compute unit each: 128 parts 183 / 171, 192 parts 340 / 400, 256 parts 283 / 328, 512 parts 569 / 656.
+int pieces(int64_t parts) { return parts > 0 && parts <= 128 ? 2 : 1; }
 
 }  // namespace
 }  // namespace bsp

@@ -317,3 +317,17 @@ def test_result_may_change_before_the_backward_pass():
     o = ac.attention_chain(*ops, *xs, scale=0.125)
     o += 7.
     assert all(torch.equal(g, w) for g, w in zip(torch.autograd.grad(o, xs, do), want[1:]))
+
+
+def test_calls_for_the_operators_make_no_tables():
+    """A head dimension, or shapes, that the kernels do not take: the operators run (or raise), and no table of tiles is made for them."""
+    lay = _layout(2, 8, 8, 'random')
+    ops = _ops(lay, 32)
+    q, k, v = [torch.randn(2, 2, 256, 32, device=DEV) for _ in range(3)]
+    before = ac.fused_f32_calls
+    ac.attention_chain(*ops, q, k, v)
+    with pytest.raises(ValueError):
+        ac.attention_chain(*ops, *[torch.randn(2, 3, 256, 64, device=DEV) for _ in range(3)])
+    assert ac.fused_f32_calls == before and not ac._core_for(*ops)._tables
+    ac.attention_chain(*ops, *[torch.randn(2, 2, 256, 64, device=DEV) for _ in range(3)])
+    assert ac.fused_f32_calls == before + 1 and ac._core_for(*ops)._tables

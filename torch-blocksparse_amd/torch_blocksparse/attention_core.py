@@ -210,24 +210,28 @@ class AttentionCore:
             usable = _lib.native().attn_usable(tables[0].native(), q, k, v)
             if usable is not None:
                 return usable
-        if not (q.is_cuda and q.dtype in (torch.float16, torch.bfloat16) and k.dtype == q.dtype and v.dtype == q.dtype):
-            return False
-        if q.dim() != 4 or k.dim() != 4 or v.dim() != 4 or q.size(3) not in (64, 128):
-            return False
-        H, R, C = self.spdims
-        Z, D, b = q.size(0), q.size(3), self.block
-        if tuple(q.shape) != (Z, H, R * b, D) or tuple(k.shape) != (Z, H, C * b, D) or tuple(v.shape) != (Z, H, C * b, D):
+        if not (q.is_cuda and q.dtype in (torch.float16, torch.bfloat16) and self._fits(q, k, v)):
             return False
         t = self.quad(q.device)
         if t is None or t.longest <= 0:
             return False
         return t.longest * 64 < 32768                           # the softmax operator's bound on a row (softmax.py:225-227)
 
+    def _fits(self, q, k, v):
+        """three operands of one type that fit the layout, of a head dimension that there are kernels for"""
+        if k.dtype != q.dtype or v.dtype != q.dtype or q.dim() != 4 or k.dim() != 4 or v.dim() != 4 or q.size(3) not in (64, 128):
+            return False
+        H, R, C = self.spdims
+        Z, D, b = q.size(0), q.size(3), self.block
+        return tuple(q.shape) == (Z, H, R * b, D) and tuple(k.shape) == (Z, H, C * b, D) and tuple(v.shape) == (Z, H, C * b, D)
+
     def usable_f32(self, q, k, v, rpe=None, attn_mask=None, dropout_p=0.):
         """The same for fp32: calls without per-element masks.  FUSED_KV = False asks for the gradients through stored softmax
         gradients, which only the operators have here."""
         if not (FUSED and FUSED_KV) or rpe is not None or attn_mask is not None or dropout_p or self.block not in (16, 32, 64) or not q.is_cuda:
             return False
+        if str(q.device) not in self._tables and not self._fits(q, k, v):
+            return False                                        # (no tables for calls that never use them)
         tables = self.quad(q.device)
         return tables is not None and _lib.native().attn_usable(tables.native(), q, k, v) is True
 

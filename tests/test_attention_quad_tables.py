@@ -115,3 +115,33 @@ def test_tables_of_the_kernels_that_store_p(block, H, R, C):
     odd = ctypes.c_int64(0)
     assert _lib.load().bsp_attention_stored_tables_build(_lib.ptr(lay.bool()), None, H, R, C, block, 0, ctypes.byref(odd), 1, ctypes.byref(info)) == _lib.ERR_CAPACITY
     assert info.total == host.numel()
+
+
+@pytest.mark.parametrize('block,H,R,C,density', [(64, 2, 6, 9, 0.4), (32, 3, 8, 12, 0.3), (16, 2, 16, 8, 0.1)])
+def test_counts_that_fp32_calls_are_routed_by(block, H, R, C, density):
+    """tiles and pieces as the tables have them, also in operators saved before these were kept"""
+    torch.manual_seed(block)
+    lay = torch.rand(H, R, C) < density
+    core = AttentionCore(lay, block)
+    t = core.quad('cpu')
+    rows = t.rows.tolist()
+    lines = [(rows[2 * i], rows[2 * i + 1]) for i in range(H * t.lines)]
+    assert t.tiles == sum(n for n, _ in lines)
+    assert t.pieces == sum(bin(rows[first + 8 * e + 4] & 0xffff).count('1') for n, first in lines for e in range(n))
+    kept = t.tiles, t.pieces
+    del t.tiles, t.pieces
+    again = AttentionCore.__new__(AttentionCore)
+    again.__setstate__(core.__dict__)
+    assert (again.quad('cpu').tiles, again.quad('cpu').pieces) == kept
+
+
+def test_fp32_calls_take_the_faster_way():
+    def pays(lay, block, Z, D, backward=True):
+        return _QuadTables(lay, block, 'cpu').pays_f32(Z, D, backward)
+    dense, diagonal = torch.ones(8, 32, 32, dtype=torch.int64), torch.eye(64, dtype=torch.int64).expand(16, 64, 64)
+    few = (torch.rand((8, 128, 128), generator=torch.Generator().manual_seed(1)) < 0.05).long() | torch.eye(128, dtype=torch.int64)
+    for D in (64, 128):
+        assert pays(dense, 64, 2, D) and pays(dense, 64, 2, D, False)
+        assert not pays(diagonal, 64, 4, D) and not pays(few, 16, 2, D)
+    assert pays(dense[:, :8, :8], 64, 1, 64, False) and pays(dense[:, :3, :3], 64, 1, 128, True)
+    assert not pays(dense[:, :3, :3], 64, 1, 128, False)

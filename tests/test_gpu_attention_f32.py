@@ -13,6 +13,12 @@ pytestmark = pytest.mark.gpu
 DEV = 'cuda'
 
 
+@pytest.fixture(autouse=True)
+def _kernels_for_every_layout(request, monkeypatch):
+    if 'layouts_of_both_routes' not in request.node.name:
+        monkeypatch.setattr(ac._QuadTables, 'pays_f32', lambda *args: True)
+
+
 def _ops(lay, block):
     return tb.MatMul(lay, block, 'sdd', trans_b=True), tb.Softmax(lay, block), tb.MatMul(lay, block, 'dsd')
 
@@ -331,3 +337,17 @@ def test_calls_for_the_operators_make_no_tables():
     assert ac.fused_f32_calls == before and not ac._core_for(*ops)._tables
     ac.attention_chain(*ops, *[torch.randn(2, 2, 256, 64, device=DEV) for _ in range(3)])
     assert ac.fused_f32_calls == before + 1 and ac._core_for(*ops)._tables
+
+
+# (random layouts of few blocks: tiles that are mostly holes, lines of a tile or two)
+@pytest.mark.parametrize('Z,H,n,block,D,density,fused', [(2, 8, 128, 16, 64, 0.05, False), (4, 16, 64, 64, 64, 0.005, False), (2, 8, 32, 64, 64, 1., True),
+                                                         (2, 8, 64, 32, 128, 0.05, False), (2, 8, 32, 64, 128, 1., True)])
+def test_layouts_of_both_routes(Z, H, n, block, D, density, fused):
+    """fp32 calls take the kernels where they are faster, the operators elsewhere"""
+    g = torch.Generator().manual_seed(7)
+    lay = (torch.rand((H, n, n), generator=g) < density).long()
+    lay[:, range(n), range(n)] = 1
+    q, k, v = [torch.randn(Z, H, n * block, D, device=DEV, requires_grad=True) for _ in range(3)]
+    before = ac.fused_f32_calls
+    ac.attention_chain(*_ops(lay, block), q, k, v, scale=D ** -0.5).sum().backward()
+    assert ac.fused_f32_calls - before == int(fused)

@@ -4,8 +4,8 @@ The reference's modules call three operators, sparse_dot_sdd_nt(q, k), sparse_so
 (deepspeedsparseselfattention.py:152-157; attention.py:190-202).  `attention_chain` takes the same three operator
 objects and the same arguments and returns the same context tensor; when the operators are this package's, built on
 one layout with blocks of 16, 32 or 64, and the tensors are fp16 / bf16 with a head dimension of 64 or 128, it runs fused
-kernels instead; in fp32 it does so without relative position embedding and attention mask (bsp_attention_f32_fwd,
-bsp_attention_f32_bwd: class _attention_f32).  In 16 bits, without relative position embedding and attention mask no sparse tensor exists (bsp_attention_rows_fwd,
+kernels instead; in fp32 it does so without relative position embedding and attention mask, for layouts that make it pay
+(_QuadTables.pays_f32; bsp_attention_f32_fwd, bsp_attention_f32_bwd: class _attention_f32).  In 16 bits, without relative position embedding and attention mask no sparse tensor exists (bsp_attention_rows_fwd,
 bsp_attention_rows_bwd, bsp_attention_cols_bwd: class _attention_quad); with one of them the softmax is stored for the backward pass
 (bsp_attention_fwd, bsp_attention_bwd, bsp_attention_bwd_kv: class _attention_core).
 In every other case, and with FUSED = False, it calls the three operators one after the other.
@@ -114,6 +114,27 @@ class _QuadTables:
         self.lines, self.longest, self.columns = info.lines, info.longest_line, info.columns
         self.n_items, self.n_slots, self.n_split = info.n_items, info.n_slots, info.n_split
         self.shape = (H, R, C, block)
+        self._count(host, int(torch.count_nonzero(lay)))
+
+    def _count(self, tables, blocks):
+        """tiles of the lines, and the 16 x 16 pieces of score that have a block"""
+        self.tiles = int(tables[0:2 * self.shape[0] * self.lines:2].sum())
+        self.pieces = blocks * (self.shape[3] // 16) ** 2
+
+    def pays_f32(self, Z, D, backward):
+        """Is a call in fp32 faster here than through the three operators?  The kernels work on whole tiles and have a cost a line, the
+        operators work on blocks alone.  Fitted to layouts of all kinds (random ones of a hundredth to a quarter of the blocks, fixed,
+        transformer, BigBird, dense; blocks of 16 to 64; 64 to 8192 lines in the launch).  Head dimension 64, training / inference, us of operators and
+        kernels: per 1000 lines 29 and 79 / 8 and 24, per 10000 pieces 35 / 11, per 1000 tiles 21 / 5.  Beside the line, training: 2048 lines of
+        2.5 tiles with 12.8 pieces each 352 and 331, 4096 of 1.6 with 16 405 and 499, 4096 of 13 with 4.2 1040 and 1539, 512 of 23 with 5.8 306
+        and 337, of 15 with 9.0 286 and 261.  Head dimension 128, one workgroup a compute unit: 512 lines of 6 tiles with 16 pieces 347 and 395, of 10
+        with 15.2 452 and 396, 2048 of 3 with 16 667 and 953, of 6 with 16 1131 and 1098, 8192 of 4 with 16 3247 and 3423; the operators take longer
+        over blocks of 16 (2048 lines of 5.2 with 13.7: 1542 and 1063).  A short training pass waits for the host, which makes five launches
+        for eleven: 64 lines of 3 tiles with head dimension 128 163 and 127, 512 lines of 2.6 with 64, 3.5 pieces a tile, 172 and 125."""
+        lines, tiles, pieces = [Z * n for n in (self.shape[0] * self.lines, self.tiles, self.pieces)]
+        if D == 64:
+            return (backward and tiles + 4 * lines <= 4000) or pieces > 6 * tiles + 20 * lines - 8000
+        return (backward and lines <= 128) or pieces * (1.1 if self.shape[3] == 16 else 1.) > 12 * tiles + 10 * lines + 7000
 
     def __getstate__(self):
         return {k: v for k, v in self.__dict__.items() if k != '_native'}
@@ -163,9 +184,11 @@ class AttentionCore:
 
     def __setstate__(self, state):
         self.__dict__.update(state)
-        for quad, _ in self._tables.values():              # (saved before the tables kept their shape)
+        for quad, _ in self._tables.values():              # (saved before the tables kept their shape, or their counts)
             if quad is not None and not hasattr(quad, 'shape'):
                 quad.shape = tuple(int(n) for n in self.spdims) + (self.block,)
+            if quad is not None and not hasattr(quad, 'pieces'):
+                quad._count(quad.rows.cpu(), int((self.layout != 0).sum()))
 
     def blocks(self):
         if self.nnz is None:
@@ -226,14 +249,16 @@ class AttentionCore:
         return tuple(q.shape) == (Z, H, R * b, D) and tuple(k.shape) == (Z, H, C * b, D) and tuple(v.shape) == (Z, H, C * b, D)
 
     def usable_f32(self, q, k, v, rpe=None, attn_mask=None, dropout_p=0.):
-        """The same for fp32: calls without per-element masks.  FUSED_KV = False asks for the gradients through stored softmax
-        gradients, which only the operators have here."""
+        """The same for fp32: calls without per-element masks, where the kernels are faster.  FUSED_KV = False asks for the gradients through
+        stored softmax gradients, which only the operators have here."""
         if not (FUSED and FUSED_KV) or rpe is not None or attn_mask is not None or dropout_p or self.block not in (16, 32, 64) or not q.is_cuda:
             return False
         if str(q.device) not in self._tables and not self._fits(q, k, v):
             return False                                        # (no tables for calls that never use them)
         tables = self.quad(q.device)
-        return tables is not None and _lib.native().attn_usable(tables.native(), q, k, v) is True
+        if tables is None or _lib.native().attn_usable(tables.native(), q, k, v) is not True:
+            return False
+        return tables.pays_f32(q.size(0), q.size(3), torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad))
 
     def __call__(self, q, k, v, scale=1., rpe=None, key_padding_mask=None, attn_mask=None,
                  key_padding_mask_mode='add', attn_mask_mode='add'):

@@ -1,8 +1,9 @@
 """GPU: the attention chain in fp32 on the bfloat16 matrix units (bsp_attention_f32_fwd / _bwd behind attention_chain) against dense 64-bit
 arithmetic and against the three operators, which compute on the fp32 units.
 
-Tolerance: a product keeps what counts in 24 bits and is rounded less often than on the fp32 units, so every result is at least as
-close to 64 bits as the operators' one, give or take a unit of 2^-23 for the softmax (relative 2-norm)."""
+Tolerance: a product keeps what counts in 24 bits and is rounded less often than on the fp32 units, and the softmax is formed as the
+operator forms it.  So over a tensor the error to 64 bits is no more than the operators', give or take a unit of 2^-23 (relative 2-norm); single rows
+may be further off than theirs as they may be closer, which is where a factor stands beside the bound."""
 import pytest
 import torch
 
@@ -351,3 +352,87 @@ def test_layouts_of_both_routes(Z, H, n, block, D, density, fused):
     before = ac.fused_f32_calls
     ac.attention_chain(*_ops(lay, block), q, k, v, scale=D ** -0.5).sum().backward()
     assert ac.fused_f32_calls - before == int(fused)
+
+
+@pytest.mark.parametrize('rows_of_mask', [1, 2])
+@pytest.mark.parametrize('block,D', [(16, 64), (64, 128)])
+def test_multiplied_masks_and_one_mask_for_all_batches(rows_of_mask, block, D):
+    """mode 'mul': zeros are padding, every other value is none; a mask of one row serves all batches"""
+    torch.manual_seed(8)
+    n = 256 // block
+    lay = _layout(2, n, n, 'random')
+    q, k, v, do = [torch.randn(2, 2, 256, D, device=DEV) for _ in range(4)]
+    keep = (torch.rand(rows_of_mask, 256, device=DEV) < 0.7).float() * 3.
+    keep[:, 0] = 1.                                                       # (every row sees its key)
+    add = torch.where(keep == 0, float('-inf'), 0.)
+    ref = _dense(q, k, v, do, lay, block, 0.125, add.expand(2, 256))
+    ops = _ops(lay, block)
+    got, other = [_run(ops, q, k, v, do, fused, scale=0.125, key_padding_mask=keep, key_padding_mask_mode='mul') for fused in (True, False)]
+    for name, g, c, r in zip(('o', 'dq', 'dk', 'dv'), got, other, ref):
+        err, bound = [float((x.double() - r).norm() / r.norm()) for x in (g, c)]
+        assert err <= bound + 2 ** -23, (name, err, bound)
+    assert all(torch.equal(a, b) for a, b in zip(got, _run(ops, q, k, v, do, True, scale=0.125, key_padding_mask=add)))
+
+
+# Logits up to some hundreds: most rows have one or two shares.  Bound as in test_against_64_bits.
+@pytest.mark.parametrize('times', [4., 16., 64.])
+@pytest.mark.parametrize('block,D', [(32, 64), (64, 64), (16, 128)])
+def test_large_logits(times, block, D):
+    torch.manual_seed(block)
+    n = 512 // block
+    lay = _layout(2, n, n, 'random')
+    q, k, v, do = [torch.randn(2, 2, 512, D, device=DEV) for _ in range(4)]
+    ref = _dense(q, k, v, do, lay, block, times * D ** -0.5)
+    ops = _ops(lay, block)
+    got, other = [_run(ops, q, k, v, do, fused, scale=times * D ** -0.5) for fused in (True, False)]
+    for name, g, c, r in zip(('o', 'dq', 'dk', 'dv'), got, other, ref):
+        err, bound = [float((x.double() - r).norm() / r.norm()) for x in (g, c)]
+        assert err <= 1.1 * bound + 2 ** -23, (name, err, bound)
+
+
+@pytest.mark.parametrize('Z,R,block,D', [(2, 8, 32, 64), (1, 40, 64, 128)])
+def test_capture_and_another_stream(Z, R, block, D):
+    """A training step captured in a graph, replayed on new inputs with eager work between; and on a stream of its own."""
+    torch.manual_seed(9)
+    lay = _layout(3, R, 8, 'random')
+    ops = _ops(lay, block)
+    q, do = [torch.randn(Z, 3, R * block, D, device=DEV) for _ in range(2)]
+    k, v = [torch.randn(Z, 3, 8 * block, D, device=DEV) for _ in range(2)]
+    kpm = torch.zeros(Z, 8 * block, device=DEV)
+    kpm[:, 3:9] = float('-inf')
+    xs = [t.clone().requires_grad_() for t in (q, k, v)]
+
+    def step():
+        o = ac.attention_chain(*ops, *xs, scale=0.125, key_padding_mask=kpm)
+        return (o.detach(),) + torch.autograd.grad(o, xs, do)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        on_side = step()
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.equal(a, b) for a, b in zip(on_side, step()))
+    graph = torch.cuda.CUDAGraph()
+    before = ac.fused_f32_calls
+    with torch.cuda.graph(graph):
+        out = step()
+    assert ac.fused_f32_calls == before + 1
+    for i in range(3):
+        for x in xs:
+            x.data.normal_()
+        do.normal_()
+        graph.replay()
+        replayed = [t.clone() for t in out]
+        assert all(torch.equal(a, b) for a, b in zip(replayed, step())), i
+
+
+def test_gradients_through_stored_softmax_gradients(monkeypatch):
+    """FUSED_KV = False: fp32 has no kernels for it, the operators run."""
+    monkeypatch.setattr(ac, 'FUSED_KV', False)
+    torch.manual_seed(10)
+    lay = _layout(2, 8, 8, 'random')
+    ops = _ops(lay, 32)
+    xs = [torch.randn(2, 2, 256, 64, device=DEV, requires_grad=True) for _ in range(3)]
+    before = ac.fused_f32_calls
+    o = ac.attention_chain(*ops, *xs, scale=0.125)
+    assert ac.fused_f32_calls == before
+    assert torch.equal(o, ops[2](ops[1](ops[0](xs[0], xs[1]), scale=0.125), xs[2]))

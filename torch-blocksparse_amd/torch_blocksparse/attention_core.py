@@ -104,7 +104,8 @@ class _QuadTables:
         H, R, C = lay.shape
         lib = _lib.load()
         info = _lib.AttentionTables()
-        cap = 32 * H * (R + C) + 16 * int(torch.count_nonzero(lay)) + 64
+        blocks = int(torch.count_nonzero(lay))
+        cap = 32 * H * (R + C) + 16 * blocks + 64
         host = torch.empty(cap, dtype=torch.int32)
         _lib.check(lib.bsp_attention_tables_build(_lib.ptr(lay), H, R, C, block, _lib.ptr(host), cap, ctypes.byref(info)),
                    'bsp_attention_tables_build')
@@ -114,11 +115,11 @@ class _QuadTables:
         self.lines, self.longest, self.columns = info.lines, info.longest_line, info.columns
         self.n_items, self.n_slots, self.n_split = info.n_items, info.n_slots, info.n_split
         self.shape = (H, R, C, block)
-        self._count(host, int(torch.count_nonzero(lay)))
+        self._count(blocks)
 
-    def _count(self, tables, blocks):
-        """tiles of the lines, and the 16 x 16 pieces of score that have a block"""
-        self.tiles = int(tables[0:2 * self.shape[0] * self.lines:2].sum())
+    def _count(self, blocks):
+        """tiles of the lines (what lies between the lines' heads and the items, eight ints each), and the 16 x 16 pieces of score that have a block"""
+        self.tiles = (self.rows.numel() - self.items.numel() - 2 * self.shape[0] * self.lines) // 8
         self.pieces = blocks * (self.shape[3] // 16) ** 2
 
     def pays_f32(self, Z, D, backward):
@@ -188,7 +189,7 @@ class AttentionCore:
             if quad is not None and not hasattr(quad, 'shape'):
                 quad.shape = tuple(int(n) for n in self.spdims) + (self.block,)
             if quad is not None and not hasattr(quad, 'pieces'):
-                quad._count(quad.rows.cpu(), int((self.layout != 0).sum()))
+                quad._count(self.blocks())
 
     def blocks(self):
         if self.nnz is None:

@@ -20,7 +20,6 @@
 // three slots of a piece, so two workgroups share a CU (one at 128): while a piece is used the next is on its way, and the one after that
 // where a slot is free.
 #include "attention_quad.h"
-#include <atomic>
 
 // (a multiplication and the addition behind it stay two roundings, as in the operators)
 #pragma clang fp contract(off)
@@ -924,22 +923,10 @@ template <int D> __global__ void __launch_bounds__(256) k_attn32_cols_sum(F32Arg
   *reinterpret_cast<f32x4 *>(dst + 4 * d4) = sum;
 }
 
-// the kernels' LDS is more than a launch may ask for by default: raised once per device and kernel
-template <class K> int big_lds(K kernel, int bytes, std::atomic<uint64_t> &done) {
-  int dev = 0;
-  BSP_HIP_CHECK(hipGetDevice(&dev));
-  const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
-  if (bit && (done.load(std::memory_order_acquire) & bit)) return BSP_OK;
-  BSP_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-  done.fetch_or(bit, std::memory_order_release);
-  return BSP_OK;
-}
-
 template <int D, bool KPM, int WHICH> int launch(const F32Args &a, unsigned n_wg, hipStream_t st) {
   static std::atomic<uint64_t> done{0};
   void (*kernel)(F32Args) = WHICH == 0 ? k_attn32_fwd<D, KPM> : WHICH == 1 ? k_attn32_bwd_rows<D, KPM> : k_attn32_bwd_cols<D, KPM>;
-  const int rc = big_lds(kernel, Ring<D>::BYTES, done);
-  if (rc != BSP_OK) return rc;
+  if (!raise_lds_limit(reinterpret_cast<const void *>(kernel), Ring<D>::BYTES, done)) return BSP_ERR_HIP;
   hipLaunchKernelGGL(kernel, dim3(n_wg), dim3(256), Ring<D>::BYTES, st, a);
   return BSP_OK;
 }

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <atomic>
 #include "../../include/bsp.h"
 
 #define BSP_HIP_CHECK(expr)                       \
@@ -25,6 +26,18 @@ template <class F> int no_throw(F &&build) {
   } catch (...) {
     return BSP_ERR_UNSUPPORTED;
   }
+}
+
+// Kernels that use more dynamic LDS than a launch may ask for by default: the limit of a kernel is raised once per device
+// (a bit per device; devices past the 64th set it at every launch), from whichever thread gets there.
+inline bool raise_lds_limit(const void *kernel, int bytes, std::atomic<uint64_t> &done) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
+  if (bit && (done.load(std::memory_order_acquire) & bit)) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
+  done.fetch_or(bit, std::memory_order_release);
+  return true;
 }
 
 typedef _Float16 f16;

@@ -24,23 +24,10 @@
 // product where the register-staged general kernel reaches 0.75.
 #include "matmul_generic.h"
 #include <algorithm>
-#include <atomic>
 #include <vector>
 
 namespace bsp {
 namespace {
-
-// The kernels of this file use more dynamic LDS than a launch may ask for by default: the limit of a kernel is raised
-// once per device (a bit per device; devices past the 64th set it at every launch), from whichever thread gets there.
-inline bool raise_lds_limit(const void *kernel, int bytes, std::atomic<uint64_t> &done) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
-  if (bit && (done.load(std::memory_order_acquire) & bit)) return true;
-  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
-  done.fetch_or(bit, std::memory_order_release);
-  return true;
-}
 
 constexpr int kTK = 32;          // reduction step (elements)
 constexpr int kTN = 256;         // tile of the dense free dimension

@@ -829,7 +829,7 @@ template <typename T, int BLOCK> int launch_sdd_b(const SddArgs &g, bool a_kc, b
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true>::SMEM_BYTES;      \
+    constexpr int SMEM = TileGemm<T, BLOCK, BLOCK, WG, WG, AK, BK, true>::SMEM_BYTES;                            \
     if (g.parts > 1) hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, true>), grid, blockdim, SMEM, st, g);           \
     else hipLaunchKernelGGL((k_sdd<T, BLOCK, AK, BK, false>), grid, blockdim, SMEM, st, g);                      \
   } while (0)
@@ -877,7 +877,7 @@ template <typename T, int BLOCK, int SPLIT> int launch_sdd_split(const SddArgs &
   dim3 grid((unsigned)n_wg), blockdim(64 * WG * WG);
 #define BSP_SDD_LAUNCH(AK, BK)                                                                                   \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, TT, TT, WG, WG, AK, BK, true>::SMEM_BYTES;            \
+    constexpr int SMEM = TileGemm<T, TT, TT, WG, WG, AK, BK, true>::SMEM_BYTES;                                  \
     if (g.parts > 1) hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, true>), grid, blockdim, SMEM, st, g); \
     else hipLaunchKernelGGL((k_sdd_split<T, BLOCK, SPLIT, AK, BK, false>), grid, blockdim, SMEM, st, g);         \
   } while (0)
@@ -924,7 +924,7 @@ template <typename T, int BLOCK, int TN_> int launch_xsd_bw(const XsdArgs &g0, b
   dim3 grid((unsigned)(n_wg * g.parts)), blockdim(256);
 #define BSP_XSD_LAUNCH(ST, DK, ON)                                                                               \
   do {                                                                                                           \
-    constexpr int SMEM = TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON>::SMEM_BYTES; \
+    constexpr int SMEM = TileGemm<T, BLOCK, S::TN, S::WGM, S::WGN, !ST, DK, ON>::SMEM_BYTES;                     \
     if constexpr (sizeof(T) == 4)                                                                                \
       if (g.parts > 1) {                                                                                         \
         hipLaunchKernelGGL((k_xsd<T, BLOCK, TN_, ST, DK, ON, true>), grid, blockdim, SMEM, st, g);              \
